@@ -20,6 +20,7 @@ int ensure_device(int *cus);
 
 // Per-device grow-only scratch allocation owned by the library.
 int workspace(size_t bytes, void **ptr);
+bool workspace_holds(size_t bytes);  // workspace(bytes) would not have to grow it
 void workspace_release();
 
 // Streams the library forks independent work onto, kHelperStreams per device,

@@ -88,6 +88,11 @@ int workspace(size_t bytes, void **ptr) {
   return SPSIM_HIP_OK;
 }
 
+bool workspace_holds(size_t bytes) {
+  DeviceState *st = state_for_current(nullptr);
+  return st && st->ws_bytes >= bytes;
+}
+
 int helper_streams(hipStream_t streams[kHelperStreams], hipEvent_t events[kHelperStreams + 1]) {
   DeviceState *st = state_for_current(nullptr);
   if (!st) return fail(SPSIM_HIP_ERR_NODEVICE, "no HIP device is available");

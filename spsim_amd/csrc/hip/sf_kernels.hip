@@ -22,6 +22,7 @@
 //    amplitude into one exp2: w_j e^{-B_j s^2} = 2^(log2 w_j - B_j s^2 log2 e).
 #include "sf_kernels.hpp"
 #include "form_factor.hpp"
+#include "surface.hpp"
 
 #include <algorithm>
 #include <cmath>
@@ -618,6 +619,7 @@ __device__ __forceinline__ void octant_tile(const float *__restrict__ hkl, int n
 
 template <int K, int CHUNK, bool HAS_B>
 __global__ __launch_bounds__(kThreads) void sf_pattern_kernel(PatternLaunch a, double2 *__restrict__ partial) {
+  if (a.skip && *a.skip) return;
   __shared__ AtomLds sm[CHUNK];
   const int split = blockIdx.y, nsplit = gridDim.y;
   const int a_begin = (int)(((long long)a.natoms * split) / nsplit);
@@ -643,6 +645,7 @@ __global__ __launch_bounds__(kThreads) void sf_pattern_kernel(PatternLaunch a, d
 template <int K, int CHUNK, bool HAS_B>
 __global__ __launch_bounds__(kThreads) void sf_grid_kernel(PatternLaunch a, int nx, int ny,
                                                            double2 *__restrict__ partial) {
+  if (a.skip && *a.skip) return;
   __shared__ AtomLds sm[CHUNK];
   const int split = blockIdx.y, nsplit = gridDim.y;
   const int a_begin = (int)(((long long)a.natoms * split) / nsplit);
@@ -659,6 +662,7 @@ __global__ __launch_bounds__(kThreads) void sf_grid_kernel(PatternLaunch a, int 
 template <int CHUNK, bool HAS_B>
 __global__ __launch_bounds__(kThreads) void sf_octant_kernel(PatternLaunch a, int n, int ny_unused,
                                                              double2 *__restrict__ partial) {
+  if (a.skip && *a.skip) return;
   __shared__ AtomLds sm[CHUNK];
   const int split = blockIdx.y, nsplit = gridDim.y;
   const int a_begin = (int)(((long long)a.natoms * split) / nsplit);
@@ -675,6 +679,7 @@ __global__ __launch_bounds__(kThreads) void sf_octant_kernel(PatternLaunch a, in
 template <int K, int CHUNK, bool HAS_B>
 __global__ __launch_bounds__(kThreads) void sf_spectrum_kernel(PatternLaunch a, Spectrum sp,
                                                                double2 *__restrict__ partial) {
+  if (a.skip && *a.skip) return;
   __shared__ AtomLds sm[CHUNK];
   const int split = blockIdx.y, nsplit = gridDim.y;
   const int a_begin = (int)(((long long)a.natoms * split) / nsplit);
@@ -699,7 +704,9 @@ __global__ __launch_bounds__(kThreads) void sf_spectrum_kernel(PatternLaunch a, 
 
 // Deterministic reduction of the atom splits of one pattern, in split order.
 __global__ __launch_bounds__(kThreads) void sf_reduce_kernel(const double2 *__restrict__ partial, int nsplit, int npix,
-                                                             float2 *__restrict__ F, float *__restrict__ I) {
+                                                             const int *skip, float2 *__restrict__ F,
+                                                             float *__restrict__ I) {
+  if (skip && *skip) return;
   const int pix = blockIdx.x * kThreads + threadIdx.x;
   if (pix >= npix) return;
   double re = 0.0, im = 0.0;
@@ -920,7 +927,7 @@ int launch_single(Kind kind, const PatternLaunch &a, int nx, int ny, const spsim
   }
   if (splits > 1) {
     hipLaunchKernelGGL(sf_reduce_kernel, dim3((a.npix + kThreads - 1) / kThreads), dim3(kThreads), 0, s,
-                       (const double2 *)partial, splits, a.npix, a.F, a.I);
+                       (const double2 *)partial, splits, a.npix, a.skip, a.F, a.I);
     SPSIM_HIP_TRY(hipGetLastError());
   }
   return SPSIM_HIP_OK;
@@ -955,7 +962,31 @@ PatternLaunch make_launch(const float *d_hkl, int npix, const spsim_hip_atom *d_
   a.I = d_I;
   a.has_rot = rot9 != nullptr;
   for (int i = 0; i < 9; ++i) a.rot.r[i] = rot9 ? rot9[i] : (i % 4 == 0 ? 1.0 : 0.0);
+  a.skip = nullptr;
   return a;
+}
+
+// A pattern on an nx x ny list with the automatic tile: interpolated over the
+// detector surface when the list and molecule are smooth enough (surface.hip
+// decides on the device, without a host round trip), and by the direct kernel
+// `kind` otherwise, which is launched behind it and finds the outputs written.
+// Both use the library workspace, the direct sums' partials past the flag.
+int launch_smooth(Kind kind, const PatternLaunch &a, int nx, int ny, const spsim_hip_tile &t, int splits, int cus,
+                  hipStream_t s) {
+  if (!surf_worth(nx, ny, a.natoms)) return launch_single(kind, a, nx, ny, t, splits, s);
+  constexpr size_t kFlag = (sizeof(SurfJob) + 255) / 256 * 256;
+  const size_t bytes = std::max(surf_single_bytes(nx, ny, a.natoms), kFlag + sizeof(double2) * (size_t)splits * a.npix);
+  if (!workspace_holds(bytes)) {
+    // A capture cannot grow the workspace: it takes the direct kernel, as long as that one's partials fit.
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(s, &st) != hipSuccess || st != hipStreamCaptureStatusNone)
+      return launch_single(kind, a, nx, ny, t, splits, s);
+  }
+  void *ws = nullptr;
+  SPSIM_TRY(workspace(bytes, &ws));
+  PatternLaunch direct = a;
+  SPSIM_TRY(launch_surface(a, nx, ny, cus, ws, &direct.skip, s));
+  return launch_single(kind, direct, nx, ny, t, splits, s, nullptr, (double2 *)((char *)ws + kFlag));
 }
 
 }  // namespace
@@ -1237,8 +1268,11 @@ extern "C" int spsim_hip_sf_grid(const float *d_hkl, int nx, int ny, const spsim
   SPSIM_TRY(grid_setup(d_hkl, nx, ny, d_atoms, d_atom_b != nullptr, d_segs, nsegs, natoms, d_ff, tile,
                        kWorkspacePartials, &t, &splits, &explicit_splits, &npix));
   if (npix == 0) return SPSIM_HIP_OK;
+  int cus = 0;
+  SPSIM_TRY(ensure_device(&cus));
   const PatternLaunch a =
       make_launch(d_hkl, npix, d_atoms, d_atom_b, d_segs, nsegs, natoms, d_ff, b_global, rot9, d_F, d_I);
+  if (!tile) return launch_smooth(Kind::kGrid, a, nx, ny, t, splits, cus, (hipStream_t)stream);
   return launch_grid(a, nx, ny, t, splits, (hipStream_t)stream);
 }
 

@@ -55,6 +55,7 @@ struct PatternLaunch {
   float *I;   // may be null
   int has_rot;
   Rot rot;
+  const int *skip;  // may be null; a device int, non-zero: the outputs are already written
 };
 
 // One work item of the batched kernels: the atoms [a_begin, a_end) (relative

@@ -1,0 +1,1137 @@
+// Structure factor of a detector by interpolation over the detector surface,
+// for gfx950 (MI355X).
+//
+// The direct sum F(q) = sum_j f_j(|q|) w_j exp(-2 pi i q.r_j) of a molecule of
+// radius R varies over the detector no faster than the phase of its outermost
+// atom: along one detector axis by theta = 2 pi R |dq/du| radians per unit of
+// u in [-1, 1], some tens of radians over hundreds of pixels on an oversampled
+// detector. So F is summed directly at n_x x n_y nodes, n a little above
+// theta, and every pixel interpolates from them:
+//
+//  1. Surface. q(x, y) is replaced by the polynomial qs(u, v) through 16 x 16
+//     of its pixels (Chebyshev form, FP64). What the list has beyond it,
+//     d = q - qs, is the FP32 rounding of the list and must be small:
+//     2 pi R |d| <= 2e-4 at every pixel, otherwise the list is not taken.
+//  2. Nodes. u_i = asin(a cos t_i) / asin(a), t_i = (2 i + 1) pi / (2 n), the
+//     Chebyshev points stretched towards even spacing (Kosloff & Tal-Ezer,
+//     J. Comput. Phys. 104 (1993) 457), with a = 1 / cosh(20.7 / n), so that
+//     the stretch itself errs by e^-20.7 = 1e-9. Chebyshev coefficients of
+//     exp(i theta u) fall off like Bessel functions beyond theta:
+//     n = theta + 4 theta^(1/3) + 8 leaves 1e-9..1e-8 of |F| (measured against
+//     FP64 sums), a tenth of the FP32 sums' own error.
+//  3. Node sums. F and its gradient G = dF/dq at the nodes, by the arithmetic
+//     of the direct kernels (FP64 phase reduced to turns, FP32 sine and
+//     cosine, FP32 sums over 64 atoms folded into FP64).
+//  4. Interpolation along the rows, then along the columns: two small dense
+//     products with FP64 weights for F (FP32 for G), then per pixel
+//     F(q) = e^{-2 pi i q.r0} (F(qs) + d.G(qs)),
+//     which takes the list's rounding into account to first order (second
+//     order: (2 pi R |d|)^2 / 2 <= 2e-8).
+//
+// The cost is n_x n_y natoms terms instead of npix natoms: 35 times fewer on
+// 100,000 atoms x 1024^2 at 0.15 nm (n = 160). The interpolation weights add
+// no error of their own: the sum of their squares is 1 at every pixel.
+#include "surface.hpp"
+
+#include <algorithm>
+#include <cmath>
+
+#include "form_factor.hpp"
+
+namespace spsim {
+
+namespace {
+
+constexpr int kT = 256;
+constexpr int D = kSurfDeg;
+constexpr double kPi = 3.14159265358979323846;
+constexpr float kStretch = 20.7f;       // -ln of the node map's own error
+constexpr double kMaxPhaseDev = 2e-4;   // largest 2 pi R |q - surface|
+constexpr float kMinWeakest = 0.02f;    // see surf_terms
+constexpr float kMaxGauss = 60.0f;      // largest exponent B s^2 over the detector
+
+// a-th of the kSurfDeg sample pixels of an axis: the pixel nearest to the
+// Chebyshev-Lobatto point (distinct for 64 pixels and more).
+__device__ __forceinline__ int sample_pixel(int a, int n) {
+  return (int)rint(0.5 * (1.0 - cospi((double)a / (D - 1))) * (n - 1));
+}
+__device__ __forceinline__ double pixel_u(int x, int n) { return (2.0 * x - (n - 1)) / (double)(n - 1); }
+
+// Largest (sum for SUM) of N values over the workgroup, given to every thread.
+template <int N, bool SUM = false>
+__device__ __forceinline__ void block_reduce(double (&v)[N]) {
+  __shared__ double part[kT / 64][N];
+#pragma unroll
+  for (int i = 0; i < N; ++i)
+    for (int o = 32; o > 0; o >>= 1) {
+      const double w = __shfl_xor(v[i], o);
+      v[i] = SUM ? v[i] + w : fmax(v[i], w);
+    }
+  __syncthreads();
+  if ((threadIdx.x & 63) == 0)
+    for (int i = 0; i < N; ++i) part[threadIdx.x / 64][i] = v[i];
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    v[i] = part[0][i];
+    for (int w = 1; w < kT / 64; ++w) v[i] = SUM ? v[i] + part[w][i] : fmax(v[i], part[w][i]);
+  }
+}
+
+// ---- 1. scan: the list's surface and deviations, the molecule's radius -------
+
+// C[m][a]: weight of sample a in Chebyshev coefficient m of the polynomial
+// through the samples at us: the polynomial at the 16 Chebyshev points
+// (barycentric formula), then their cosine transform. cosines[k] = cos(pi k / 32).
+__device__ void sample_to_chebyshev(const double *us, const double *cosines, double (*C)[D], double (*tmp)[D]) {
+  const int t = threadIdx.x, p = t / D, a = t % D;
+  double w = 1.0;
+#pragma unroll
+  for (int c = 0; c < D; ++c)
+    if (c != a) w *= 2.0 * (us[a] - us[c]);
+  const double up = cosines[2 * p + 1], d = up - us[a];
+  const double v = d == 0.0 ? 0.0 : 1.0 / (w * d);
+  tmp[p][a] = v;
+  __syncthreads();
+  double den = 0.0;
+  int hit = -1;
+#pragma unroll
+  for (int c = 0; c < D; ++c) {
+    den += tmp[p][c];
+    if (up == us[c]) hit = c;
+  }
+  __syncthreads();
+  tmp[p][a] = hit >= 0 ? (hit == a ? 1.0 : 0.0) : v / den;
+  __syncthreads();
+  double s = 0.0;
+#pragma unroll
+  for (int k = 0; k < D; ++k) {
+    int j = p * (2 * k + 1) % (4 * D);  // cos(pi j / 32)
+    if (j > 2 * D) j = 4 * D - j;
+    s += tmp[k][a] * cosines[j];
+  }
+  C[p][a] = s * (p == 0 ? 1.0 : 2.0) / D;
+  __syncthreads();
+}
+
+// Chebyshev series of 3 components at u (c[m][3]).
+__device__ __forceinline__ void clenshaw3(const double (*c)[3], double u, double out[3]) {
+  double b1[3] = {0, 0, 0}, b2[3] = {0, 0, 0};
+  const double u2 = 2.0 * u;
+#pragma unroll
+  for (int m = D - 1; m >= 1; --m) {
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      const double b = __builtin_fma(u2, b1[k], c[m][k] - b2[k]);
+      b2[k] = b1[k];
+      b1[k] = b;
+    }
+  }
+#pragma unroll
+  for (int k = 0; k < 3; ++k) out[k] = __builtin_fma(u, b1[k], c[0][k] - b2[k]);
+}
+
+// Coefficients along u of the surface's line v (or of its derivative in v):
+// row[m][k] = sum_n T_n(v) coef[n][m][k]. Threads 0..47.
+__device__ __forceinline__ void surface_row(const double (*coef)[D][3], double v, double (*row)[3]) {
+  if (threadIdx.x < 3 * D) {
+    const int m = threadIdx.x / 3, k = threadIdx.x % 3;
+    double t0 = 1.0, t1 = v, s = coef[0][m][k];
+    for (int n = 1; n < D; ++n) {
+      s = __builtin_fma(t1, coef[n][m][k], s);
+      const double t2 = __builtin_fma(2.0 * v, t1, -t0);
+      t0 = t1;
+      t1 = t2;
+    }
+    row[m][k] = s;
+  }
+}
+
+struct ScanArgs {
+  const float *hkl;
+  int nx, ny;
+  int list_blocks;
+  const spsim_hip_atom *atoms;
+  const float *atom_b;
+  const MolInfo *mols;  // null: one molecule of natoms atoms
+  int natoms;
+  SurfFit *fit;
+  float *dev;
+  SurfRecord *records;  // [list_blocks + nmol * kSurfAtomBlocks]
+  double *centres;      // [nmol][3]
+};
+
+__device__ void scan_list(const ScanArgs &a) {
+  __shared__ double C[2][D][D], tmp[D][D], Q[D][D][3], P[D][D][3], row[D][3], us[2][D], cosines[2 * D + 1];
+  __shared__ int px[2][D];
+  const int t = threadIdx.x, b = t / D, i = t % D;
+  if (t < 2 * D) {
+    const int n = b ? a.ny : a.nx;
+    px[b][i] = sample_pixel(i, n);
+    us[b][i] = pixel_u(px[b][i], n);
+  }
+  if (t >= 64 && t <= 64 + 2 * D) cosines[t - 64] = cospi((t - 64) / (2.0 * D));
+  __syncthreads();
+  {
+    const size_t p = (size_t)px[1][b] * a.nx + px[0][i];
+    for (int k = 0; k < 3; ++k) Q[b][i][k] = a.hkl[3 * p + k];
+  }
+  sample_to_chebyshev(us[0], cosines, C[0], tmp);
+  sample_to_chebyshev(us[1], cosines, C[1], tmp);
+  // along x: P[b][m], then along y in place of Q
+  for (int k = 0; k < 3; ++k) {
+    double s = 0.0;
+#pragma unroll
+    for (int c = 0; c < D; ++c) s = __builtin_fma(C[0][i][c], Q[b][c][k], s);
+    P[b][i][k] = s;
+  }
+  __syncthreads();
+  for (int k = 0; k < 3; ++k) {
+    double s = 0.0;
+#pragma unroll
+    for (int c = 0; c < D; ++c) s = __builtin_fma(C[1][b][c], P[c][i][k], s);
+    Q[b][i][k] = s;
+  }
+  __syncthreads();
+  if (blockIdx.x == 0) {
+    // slopes |dq/du|, |dq/dv| and s^2 on the 16 x 16 Lobatto points: T_m and
+    // m U_{m-1} at the points, then the rows' sums, then the points'
+    double(*T)[D] = C[0], (*U)[D] = C[1];  // [m][point]
+    __shared__ double R[D][D][6];          // [n][point of u]: q, dq/du along row n
+    if (t < D) {
+      const double u = cospi((double)t / (D - 1));
+      double t0 = 1.0, t1 = u, u0 = 0.0, u1 = 1.0;
+      for (int m = 0; m < D; ++m) {
+        T[m][t] = t0;
+        U[m][t] = m * u0;
+        const double tn = 2.0 * u * t1 - t0, un = 2.0 * u * u1 - u0;
+        t0 = t1;
+        t1 = tn;
+        u0 = u1;
+        u1 = un;
+      }
+    }
+    __syncthreads();
+    for (int k = 0; k < 3; ++k) {
+      double r = 0.0, rd = 0.0;
+      for (int m = 0; m < D; ++m) {
+        r = __builtin_fma(T[m][i], Q[b][m][k], r);
+        rd = __builtin_fma(U[m][i], Q[b][m][k], rd);
+      }
+      R[b][i][k] = r;
+      R[b][i][3 + k] = rd;
+    }
+    __syncthreads();
+    double du = 0.0, dv = 0.0, s2[1] = {0.0};
+    for (int k = 0; k < 3; ++k) {
+      double q = 0.0, qu = 0.0, qv = 0.0;
+      for (int n = 0; n < D; ++n) {
+        q = __builtin_fma(T[n][b], R[n][i][k], q);
+        qu = __builtin_fma(T[n][b], R[n][i][3 + k], qu);
+        qv = __builtin_fma(U[n][b], R[n][i][k], qv);
+      }
+      s2[0] += q * q * 2.5e-21;
+      du += qu * qu;
+      dv += qv * qv;
+    }
+    block_reduce(s2);
+    tmp[b][i] = du;
+    P[b][i][0] = dv;
+    __syncthreads();
+    if (t < D) {
+      double sx = 0.0, sy = 0.0;
+      for (int c = 0; c < D; ++c) {
+        sx = fmax(sx, tmp[c][t]);
+        sy = fmax(sy, P[t][c][0]);
+      }
+      a.fit->slope_x[t] = (float)sqrt(sx);
+      a.fit->slope_y[t] = (float)sqrt(sy);
+    }
+    if (t == 0) a.fit->s2max = (float)s2[0];
+    for (int c = t; c < D * D * 3; c += kT) (&a.fit->coef[0][0][0])[c] = (&Q[0][0][0])[c];
+  }
+  double m[4] = {0, 0, 0, 0};
+  for (int y = blockIdx.x; y < a.ny; y += a.list_blocks) {
+    __syncthreads();
+    surface_row(Q, pixel_u(y, a.ny), row);
+    __syncthreads();
+    for (int x = t; x < a.nx; x += kT) {
+      double s[3];
+      clenshaw3(row, pixel_u(x, a.nx), s);
+      const size_t p = 3 * ((size_t)y * a.nx + x);
+#pragma unroll
+      for (int k = 0; k < 3; ++k) {
+        const double d = (double)a.hkl[p + k] - s[k];
+        a.dev[p + k] = (float)d;
+        if (!(fabs(d) < 1e30)) m[3] = 1.0;
+        m[k] = fmax(m[k], fabs(d));
+      }
+    }
+  }
+  block_reduce(m);
+  if (t == 0) a.records[blockIdx.x] = SurfRecord{{m[0], m[1], m[2]}, 0.0, 0.0f, 0.0f, m[3] > 0.0, 0};
+}
+
+// The molecule's centre is the mean of 1024 evenly spaced atoms: any point near
+// the middle serves, and every workgroup forms the same one.
+__device__ void scan_atoms(const ScanArgs &a) {
+  const int t = threadIdx.x;
+  const int mol = ((int)blockIdx.x - a.list_blocks) / kSurfAtomBlocks;
+  const int part = ((int)blockIdx.x - a.list_blocks) % kSurfAtomBlocks;
+  const int begin = a.mols ? a.mols[mol].atom_begin : 0;
+  const int n = a.mols ? a.mols[mol].atom_end - begin : a.natoms;
+  const spsim_hip_atom *atoms = a.atoms + begin;
+  double c[3] = {0, 0, 0};
+  if (n > 0)
+    for (int i = 0; i < 4; ++i) {
+      const spsim_hip_atom at = atoms[(int)((long long)(4 * t + i) * n / (4 * kT))];
+      c[0] += at.x;
+      c[1] += at.y;
+      c[2] += at.z;
+    }
+  block_reduce<3, true>(c);
+  for (int k = 0; k < 3; ++k) c[k] /= 4.0 * kT;
+  if (part == 0 && t == 0)
+    for (int k = 0; k < 3; ++k) a.centres[3 * mol + k] = c[k];
+  // |r - r0|^2, -B, B, not finite
+  double m[4] = {0.0, -3.4e38, -3.4e38, fabs(c[0]) + fabs(c[1]) + fabs(c[2]) < 1e30 ? 0.0 : 1.0};
+  for (int j = part * kT + t; j < n; j += kSurfAtomBlocks * kT) {
+    const spsim_hip_atom at = atoms[j];
+    const double x = at.x - c[0], y = at.y - c[1], z = at.z - c[2];
+    const double d2 = x * x + y * y + z * z;
+    if (!(d2 < 1e30) || !(fabsf(at.w) < 3.4e38f)) m[3] = 1.0;
+    m[0] = fmax(m[0], d2);
+    if (a.atom_b) {
+      const float b = a.atom_b[begin + j];
+      if (!(fabsf(b) < 1e30f)) m[3] = 1.0;
+      m[1] = fmax(m[1], -(double)b);
+      m[2] = fmax(m[2], (double)b);
+    }
+  }
+  block_reduce(m);
+  if (t == 0)
+    a.records[blockIdx.x] = SurfRecord{{0, 0, 0}, m[0], (float)-m[1], (float)m[2], m[3] > 0.0, 0};
+}
+
+__global__ __launch_bounds__(kT) void surface_scan_kernel(ScanArgs a) {
+  if ((int)blockIdx.x < a.list_blocks)
+    scan_list(a);
+  else
+    scan_atoms(a);
+}
+
+// ---- 2. nodes -------------------------------------------------------------------
+
+// The stretch parameter of n nodes, and the nodes that phases of the given
+// slopes need at that stretch. 2 % are added to the slopes for their sampling.
+__host__ __device__ inline float axis_stretch(int n) { return 1.0f / coshf(kStretch / n); }
+
+__host__ __device__ inline float fast_sin(float x) {
+#ifdef __HIP_DEVICE_COMPILE__
+  return __sinf(x);
+#else
+  return std::sin(x);
+#endif
+}
+__host__ __device__ inline float fast_cos(float x) {
+#ifdef __HIP_DEVICE_COMPILE__
+  return __cosf(x);
+#else
+  return std::cos(x);
+#endif
+}
+
+__host__ __device__ inline float axis_need(const float *slope, float radius, float gauss, float a) {
+  const float as = asinf(a);
+  float w = 0.0f;
+  for (int k = 0; k < D; ++k) {
+    // lines mirrored about the middle share their stretch
+    const float u = fabsf(fast_cos((float)kPi * k / (D - 1)));
+    const float s = fminf(1.0f, fast_sin(u * as) / a), c = fast_cos(u * as);
+    w = fmaxf(w, slope[k] * sqrtf(fmaxf(0.0f, 1.0f - s * s)) * a / (as * fmaxf(c, 1e-6f)));
+  }
+  const float theta = 1.02f * 2.0f * (float)kPi * radius * w;
+  return theta + 4.0f * cbrtf(theta) + 8.0f + 2.0f * sqrtf(fmaxf(gauss, 0.0f));
+}
+
+__host__ __device__ inline bool worth(double nodes_x, double nodes_y, double nx, double ny, double natoms) {
+  // Issue cycles per lane: a term of the node sums 62, of the direct sums 26
+  // to 40; the interpolation 25 per node row and pixel. Measured on the MI355X.
+  const double surf = nodes_x * nodes_y * natoms * 62.0 + 25.0 * (nx * ny * nodes_y + nx * nodes_x * nodes_y);
+  return surf < 0.8 * 26.0 * nx * ny * natoms;
+}
+
+__host__ __device__ inline bool smooth(const SurfMol &m, float s2max) {
+  return !m.bad && 2.0 * kPi * m.radius * m.dev <= kMaxPhaseDev && m.weakest >= kMinWeakest &&
+         m.b_smooth * s2max <= kMaxGauss;
+}
+
+// Amplitude of a term over the detector, per species: the interpolation's error
+// is relative to the strongest part of the pattern, the direct sum's to the
+// pixel's own terms, so terms that fade below kMinWeakest of their value at
+// the beam are left to the direct sum.
+__host__ __device__ inline void species_terms(const float *c, float Bs, float bmin, float bmax, float s2max,
+                                              float *b_smooth, float *weakest) {
+  float f0 = c[8], f1 = c[8], b = 0.0f;
+  for (int i = 0; i < 4; ++i) {
+    f0 += c[i];
+    f1 += c[i] * expf(-c[4 + i] * s2max);
+    b = fmaxf(b, fabsf(c[4 + i]));
+  }
+  const float lo = Bs + bmin, hi = Bs + bmax;
+  const float e0 = fmaxf(1.0f, expf(-lo * s2max)), e1 = fminf(1.0f, expf(-hi * s2max));
+  const float ratio = fabsf(f1) * e1 / (fabsf(f0) * e0);
+  *b_smooth = fmaxf(*b_smooth, b + fmaxf(fabsf(lo), fabsf(hi)));
+  *weakest = ratio < *weakest || !(ratio < 1e30f) ? (ratio < 1e30f ? ratio : 0.0f) : *weakest;
+}
+
+// Atom records of the node sums: position relative
+// to the centre, rotated (FP64), and the amplitude with its products with the
+// position; with per-atom B, v holds log2 of the amplitude, B and the position.
+struct __align__(16) NodeAtom {
+  double x, y, z;
+  float v[6];
+};
+static_assert(sizeof(NodeAtom) == 48, "node-sum atom record");
+
+__device__ __forceinline__ void prepare_atoms(const SurfJob &jb, bool has_b, int first, int step) {
+  NodeAtom *out = (NodeAtom *)jb.prep;
+  for (int j = first; j < jb.natoms; j += step) {
+    const spsim_hip_atom at = jb.atoms[j];
+    const double x = at.x - jb.r0[0], y = at.y - jb.r0[1], z = at.z - jb.r0[2];
+    NodeAtom r;
+    if (jb.has_rot) {
+      const double *R = jb.rot;
+      r.x = __builtin_fma(R[6], z, __builtin_fma(R[3], y, R[0] * x));
+      r.y = __builtin_fma(R[7], z, __builtin_fma(R[4], y, R[1] * x));
+      r.z = __builtin_fma(R[8], z, __builtin_fma(R[5], y, R[2] * x));
+    } else {
+      r.x = x;
+      r.y = y;
+      r.z = z;
+    }
+    const float xf = (float)r.x, yf = (float)r.y, zf = (float)r.z;
+    if (has_b) {
+      r.v[0] = log2f(at.w);
+      r.v[1] = xf;
+      r.v[2] = yf;
+      r.v[3] = zf;
+      r.v[4] = jb.atom_b[j];
+    } else {
+      r.v[0] = at.w;
+      r.v[1] = at.w * xf;
+      r.v[2] = at.w * yf;
+      r.v[3] = at.w * zf;
+      r.v[4] = 0.0f;
+    }
+    r.v[5] = 0.0f;
+    out[j] = r;
+  }
+}
+
+// Nodes per lane of the node sums: four share an atom's LDS read (2.27 ms
+// against 2.42 ms on 35,344 nodes x 100,000 atoms), two make twice the work
+// items (17.6 us against 24 us on 1024 nodes x 5,000 atoms).
+__host__ __device__ inline int surf_per_lane(long long nodes, long long natoms) {
+  return nodes * natoms >= 1LL << 28 ? 4 : 2;
+}
+
+// Time of the node sums in atoms per lane with s atom ranges per tile: rounds
+// of `slots` resident workgroups, each of an atom range and a fixed part (the
+// form factors and the loop's start, about 40 atoms), and the ranges' partial
+// sums, which cost about one atom each.
+__host__ __device__ inline float splits_cost(int s, int tiles, int natoms, int slots) {
+  const int rounds = (tiles * s + slots - 1) / slots;
+  return rounds * ((float)natoms / s + 40.0f) + (s > 1 ? 1.5f * s + 40.0f : 0.0f);
+}
+
+struct PlanArgs {
+  SurfJob job;  // template: pointers and sizes set, the choice left open
+  const SurfFit *fit;
+  const SurfRecord *records;
+  int list_blocks;
+  const double *centres;
+  const float *ff;
+  float b_global;
+  bool has_b;
+  int slots;       // resident workgroups of the node sums
+  int slot_cap;    // partial slots that fit
+  int max_nx, max_ny;  // nodes that fit the workspace
+  SurfJob *out;
+};
+
+// Interpolation weights of one axis (node-major [n][npix]), one wave per
+// pixel: barycentric formula in s = cos t, whose weights at the Chebyshev
+// points are (-1)^i sin t_i.
+__device__ __forceinline__ void weight_column(const SurfAxis &ax, int x, int npix, const double *sn, const double *wn,
+                                              double *__restrict__ out) {
+  const int lane = threadIdx.x & 63;
+  const double s = sinpi(pixel_u(x, npix) * (ax.asin_a / kPi)) / ax.a;
+  double sum = 0.0;
+  int hit = -1;
+  for (int i = lane; i < ax.n; i += 64) {
+    const double d = s - sn[i];
+    if (d == 0.0)
+      hit = i;
+    else
+      sum += wn[i] / d;
+  }
+  for (int o = 32; o > 0; o >>= 1) {
+    sum += __shfl_xor(sum, o);
+    hit = max(hit, __shfl_xor(hit, o));
+  }
+  for (int i = lane; i < ax.n; i += 64) {
+    const double d = s - sn[i];
+    out[(size_t)i * npix + x] = hit >= 0 ? (i == hit ? 1.0 : 0.0) : (wn[i] / d) / sum;
+  }
+}
+
+// Part 0: the weights of both axes, part 1: the node q of a shape, spread over
+// gridDim.x workgroups. Called by every thread; sn* and wn* are LDS arrays of
+// kSurfMaxNodes.
+__device__ void build(int part, const SurfFit *fit, const SurfShape &sh, int nx, int ny, double *snx, double *wnx,
+                      double *sny, double *wny) {
+  __shared__ double coef[D][D][3], row[D][3];
+  const int t = threadIdx.x;
+  if (part == 0) {
+    for (int i = t; i < sh.ax.n; i += kT) {
+      const double ph = (2 * i + 1) / (2.0 * sh.ax.n);
+      snx[i] = cospi(ph);
+      wnx[i] = (i & 1) ? -sinpi(ph) : sinpi(ph);
+    }
+    for (int i = t; i < sh.ay.n; i += kT) {
+      const double ph = (2 * i + 1) / (2.0 * sh.ay.n);
+      sny[i] = cospi(ph);
+      wny[i] = (i & 1) ? -sinpi(ph) : sinpi(ph);
+    }
+    __syncthreads();
+    const int waves = kT / 64, wave = t / 64;
+    for (int r = (int)blockIdx.x * waves + wave; r < nx + ny; r += (int)gridDim.x * waves) {
+      if (r < nx)
+        weight_column(sh.ax, r, nx, snx, wnx, sh.tx);
+      else
+        weight_column(sh.ay, r - nx, ny, sny, wny, sh.ty);
+    }
+  } else if (part == 1) {
+    for (int i = t; i < D * D * 3; i += kT) (&coef[0][0][0])[i] = (&fit->coef[0][0][0])[i];
+    for (int i = t; i < sh.ax.n; i += kT)
+      snx[i] = asin(sh.ax.a * cospi((2 * i + 1) / (2.0 * sh.ax.n))) / sh.ax.asin_a;
+    for (int i = t; i < sh.ay.n; i += kT)
+      sny[i] = asin(sh.ay.a * cospi((2 * i + 1) / (2.0 * sh.ay.n))) / sh.ay.asin_a;
+    // node (i, k) -> index i ay.n + k: a row of 16 nodes is contiguous for the first product
+    for (int k = blockIdx.x; k < sh.ay.n; k += gridDim.x) {
+      __syncthreads();
+      surface_row(coef, sny[k], row);
+      __syncthreads();
+      for (int i = t; i < sh.ax.n; i += kT) {
+        double q[3];
+        clenshaw3(row, snx[i], q);
+        double *o = sh.nodes + 3 * ((size_t)i * sh.ay.n + k);
+        o[0] = q[0];
+        o[1] = q[1];
+        o[2] = q[2];
+      }
+    }
+  }
+}
+
+__global__ __launch_bounds__(kT) void surface_plan_kernel(PlanArgs a) {
+  __shared__ double snx[kSurfMaxNodes], wnx[kSurfMaxNodes], sny[kSurfMaxNodes], wny[kSurfMaxNodes];
+  __shared__ SurfMol mol;
+  __shared__ int best[2], split[1];
+  __shared__ SurfJob job;
+  const int t = threadIdx.x;
+  double m[7] = {0, 0, 0, 0, -3.4e38, -3.4e38, 0};  // dev, r2, -B, B, not finite
+  for (int i = t; i < a.list_blocks + kSurfAtomBlocks; i += kT) {
+    const SurfRecord r = a.records[i];
+    for (int k = 0; k < 3; ++k) m[k] = fmax(m[k], r.dev[k]);
+    m[3] = fmax(m[3], r.r2);
+    if (i >= a.list_blocks) {
+      m[4] = fmax(m[4], -(double)r.bmin);
+      m[5] = fmax(m[5], (double)r.bmax);
+    }
+    if (r.bad) m[6] = 1.0;
+  }
+  block_reduce(m);
+  // every form-factor row that is used, one thread each
+  float bs = 0.0f, weak = 1.0f;
+  for (int i = t; i < a.job.nsegs; i += kT) {
+    const int sp = a.job.segs[i].species;
+    species_terms(a.ff + sp * SPSIM_HIP_FF_STRIDE, sp == SPSIM_HIP_UNIT_SPECIES ? 0.0f : a.b_global,
+                  a.has_b ? (float)-m[4] : 0.0f, a.has_b ? (float)m[5] : 0.0f, a.fit->s2max, &bs, &weak);
+  }
+  double e[2] = {(double)bs, -(double)weak};
+  block_reduce(e);
+  if (t == 0) {
+    mol.radius = sqrt(m[3]);
+    mol.dev = sqrt(m[0] * m[0] + m[1] * m[1] + m[2] * m[2]);
+    mol.b_smooth = (float)e[0];
+    mol.weakest = (float)-e[1];
+    mol.bad = m[6] > 0.0;
+    best[0] = best[1] = 1 << 30;
+  }
+  __syncthreads();
+  {  // smallest sufficient node count of each axis, one candidate per thread
+    const int axis = t / 128, n = kSurfMinNodes + 4 * (t % 128);
+    const float *slope = axis ? a.fit->slope_y : a.fit->slope_x;
+    if (n <= kSurfMaxNodes &&
+        axis_need(slope, (float)mol.radius, mol.b_smooth * a.fit->s2max, axis_stretch(n)) <= (float)n)
+      atomicMin(&best[axis], n);
+  }
+  __syncthreads();
+  const int nx = best[0], ny = best[1];
+  const bool ok = smooth(mol, a.fit->s2max) && nx <= a.max_nx && ny <= a.max_ny &&
+                  worth(nx, ny, a.job.nx, a.job.ny, a.job.natoms);
+  if (!ok) {
+    if (blockIdx.x == 0 && blockIdx.y == 0 && t == 0) a.out->ok = 0;
+    return;
+  }
+  const int per_lane = surf_per_lane((long long)nx * ny, a.job.natoms), tile = per_lane * kT;
+  const int tiles = (nx * ny + tile - 1) / tile;
+  if (t < 64) {  // the cheapest number of atom ranges, two candidates per lane
+    float c = 3.0e38f;
+    int n = 1;
+    for (int s = t + 1; s <= kSurfMaxSplits; s += 64)
+      if (s == 1 || ((long long)tiles * tile * s <= a.slot_cap && a.job.natoms / s >= 32)) {
+        const float k = splits_cost(s, tiles, a.job.natoms, a.slots);
+        if (k < c) {
+          c = k;
+          n = s;
+        }
+      }
+    for (int o = 32; o > 0; o >>= 1) {
+      const float c2 = __shfl_xor(c, o);
+      const int n2 = __shfl_xor(n, o);
+      if (c2 < c || (c2 == c && n2 < n)) {
+        c = c2;
+        n = n2;
+      }
+    }
+    if (t == 0) split[0] = n;
+  } else if (t == 64) {
+    job = a.job;
+    job.ok = 1;
+    job.sh.ax = SurfAxis{nx, axis_stretch(nx), 0.0};
+    job.sh.ay = SurfAxis{ny, axis_stretch(ny), 0.0};
+    job.sh.ax.asin_a = asin(job.sh.ax.a);
+    job.sh.ay.asin_a = asin(job.sh.ay.a);
+    job.per_lane = per_lane;
+    job.tiles = tiles;
+    for (int k = 0; k < 3; ++k) job.r0[k] = a.centres[k];
+  }
+  __syncthreads();
+  if (t == 0) {
+    job.splits = split[0];
+    if (blockIdx.x == 0 && blockIdx.y == 0) *a.out = job;
+  }
+  __syncthreads();
+  build(blockIdx.y, a.fit, job.sh, job.nx, job.ny, snx, wnx, sny, wny);
+  if (blockIdx.y == 2) prepare_atoms(job, a.has_b, (int)(blockIdx.x * kT) + t, (int)gridDim.x * kT);
+}
+
+__global__ __launch_bounds__(kT) void surface_tables_kernel(const SurfFit *fit, SurfShape sh, int nx, int ny) {
+  __shared__ double snx[kSurfMaxNodes], wnx[kSurfMaxNodes], sny[kSurfMaxNodes], wny[kSurfMaxNodes];
+  build(blockIdx.y, fit, sh, nx, ny, snx, wnx, sny, wny);
+}
+
+// ---- 3. node sums ---------------------------------------------------------------
+//
+// One work item: two or four nodes per lane x one atom range, whose records are
+// staged in LDS 256 at a time; every lane reads the same record, and its terms
+// share the read (surf_per_lane). Per node and atom: 3 FP64 FMAs, a fraction and a
+// conversion, a sine and cosine, 8 FP32 FMAs (F and the three components of G):
+// 62 issue cycles. (The records through scalar loads instead, one node per
+// lane: 128 cycles; the waves drift apart and miss the scalar cache.) A tile's
+// atom ranges leave partial sums, which surface_reduce_kernel adds in range
+// order (added by the tile's last workgroup instead, 64 ranges took 30 us: one
+// lane per node waits for every slot). The form factor is evaluated in FP64:
+// its rounding at a node would be shared by all the pixels around it.
+
+constexpr int kNodeChunk = 256;  // atoms staged at once
+constexpr int kNodeFold = 64;  // atoms per FP32 partial sum
+
+struct __align__(16) NodeSlot {
+  double fc, fs;
+  float g[8];  // sin, cos of x, y, z; 2 unused
+};
+
+__device__ __forceinline__ double form_factor64(const float *__restrict__ c, double s2, float B) {
+  double f = c[8] * exp(-(double)B * s2);
+#pragma unroll
+  for (int i = 0; i < 4; ++i) f += c[i] * exp(-((double)c[4 + i] + B) * s2);
+  return f;
+}
+
+template <int K, bool HAS_B>
+__device__ __forceinline__ void node_item(const SurfJob &jb, int tile, int split, const float *__restrict__ ff,
+                                          float b_global, NodeAtom *sm) {
+  constexpr int kTile = K * kT;
+  const int nodes = jb.sh.ax.n * jb.sh.ay.n;
+  const int a_begin = (int)((long long)jb.natoms * split / jb.splits);
+  const int a_end = (int)((long long)jb.natoms * (split + 1) / jb.splits);
+  double qx[K], qy[K], qz[K], s2[K], Fc[K], Fs[K];
+  float nl2[K], gc[K][3], gs[K][3];
+#pragma unroll
+  for (int k = 0; k < K; ++k) {
+    const double *q = jb.sh.nodes + 3 * (size_t)min(tile * kTile + k * kT + (int)threadIdx.x, nodes - 1);
+    qx[k] = q[0];
+    qy[k] = q[1];
+    qz[k] = q[2];
+    s2[k] = (qx[k] * qx[k] + qy[k] * qy[k] + qz[k] * qz[k]) * 2.5e-21;
+    nl2[k] = (float)(-s2[k] * kLog2e);
+    Fc[k] = Fs[k] = 0.0;
+#pragma unroll
+    for (int i = 0; i < 3; ++i) gc[k][i] = gs[k][i] = 0.0f;
+  }
+  const NodeAtom *atoms = (const NodeAtom *)jb.prep;
+  for (int sg = 0; sg < jb.nsegs; ++sg) {
+    const spsim_hip_segment seg = jb.segs[sg];
+    const int lo = max(seg.start, a_begin), hi = min(seg.start + seg.count, a_end);
+    if (lo >= hi) continue;
+    double f[K];
+#pragma unroll
+    for (int k = 0; k < K; ++k)
+      f[k] = form_factor64(ff + seg.species * SPSIM_HIP_FF_STRIDE, s2[k],
+                           seg.species == SPSIM_HIP_UNIT_SPECIES ? 0.0f : b_global);
+    for (int c0 = lo; c0 < hi; c0 += kNodeChunk) {
+      const int n = min(kNodeChunk, hi - c0);
+      __syncthreads();
+      if ((int)threadIdx.x < n) sm[threadIdx.x] = atoms[c0 + threadIdx.x];
+      __syncthreads();
+      for (int j0 = 0; j0 < n; j0 += kNodeFold) {
+        const int j1 = min(n, j0 + kNodeFold);
+        float c[K][4], s[K][4];
+#pragma unroll
+        for (int k = 0; k < K; ++k)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) c[k][i] = s[k][i] = 0.0f;
+        for (int j = j0; j < j1; ++j) {
+          const NodeAtom at = sm[j];
+#pragma unroll
+          for (int k = 0; k < K; ++k) {
+            const double t = __builtin_fma(qz[k], at.z, __builtin_fma(qy[k], at.y, qx[k] * at.x));
+            const float ph = (float)__builtin_amdgcn_fract(t);
+            float cs = __builtin_amdgcn_cosf(ph), sn = __builtin_amdgcn_sinf(ph);
+            if constexpr (HAS_B) {
+              const float w = __builtin_amdgcn_exp2f(__builtin_fmaf(at.v[4], nl2[k], at.v[0]));
+              cs *= w;
+              sn *= w;
+              c[k][0] += cs;
+              s[k][0] += sn;
+            } else {
+              c[k][0] = __builtin_fmaf(at.v[0], cs, c[k][0]);
+              s[k][0] = __builtin_fmaf(at.v[0], sn, s[k][0]);
+            }
+#pragma unroll
+            for (int i = 1; i < 4; ++i) {
+              c[k][i] = __builtin_fmaf(at.v[i], cs, c[k][i]);
+              s[k][i] = __builtin_fmaf(at.v[i], sn, s[k][i]);
+            }
+          }
+        }
+#pragma unroll
+        for (int k = 0; k < K; ++k) {
+          Fc[k] = __builtin_fma(f[k], (double)c[k][0], Fc[k]);
+          Fs[k] = __builtin_fma(f[k], (double)s[k][0], Fs[k]);
+          const float f32 = (float)f[k];
+#pragma unroll
+          for (int i = 0; i < 3; ++i) {
+            gc[k][i] = __builtin_fmaf(f32, c[k][i + 1], gc[k][i]);
+            gs[k][i] = __builtin_fmaf(f32, s[k][i + 1], gs[k][i]);
+          }
+        }
+      }
+    }
+  }
+#pragma unroll
+  for (int k = 0; k < K; ++k) {
+    const int l = k * kT + threadIdx.x, node = tile * kTile + l;
+    if (jb.splits > 1) {
+      ((NodeSlot *)jb.slots)[((size_t)tile * jb.splits + split) * kTile + l] =
+          NodeSlot{Fc[k], Fs[k], {gs[k][0], gc[k][0], gs[k][1], gc[k][1], gs[k][2], gc[k][2], 0.0f, 0.0f}};
+    } else if (node < nodes) {
+      // G = dF/dq = -2 pi i sum w f r e^{-i phi}: (re, im) = -2 pi (gs, gc)
+      jb.f[node] = make_double2(Fc[k], -Fs[k]);
+      float2 *g = (float2 *)(jb.g + 6 * (size_t)node);
+#pragma unroll
+      for (int i = 0; i < 3; ++i)
+        g[i] = make_float2(-2.0f * (float)kPi * gs[k][i], -2.0f * (float)kPi * gc[k][i]);
+    }
+  }
+}
+
+template <bool HAS_B>
+__global__ __launch_bounds__(kT) void surface_nodes_kernel(const SurfJob *jobs, const SurfItem *items, int nitems,
+                                                           const float *__restrict__ ff, float b_global) {
+  __shared__ NodeAtom sm[kNodeChunk];
+  if (!items) {  // one pattern: every (tile, range) of job 0
+    if (!jobs->ok) return;
+    nitems = jobs->tiles * jobs->splits;
+  }
+  for (int it = blockIdx.x; it < nitems; it += gridDim.x) {
+    const SurfItem m = items ? items[it] : SurfItem{0, it % jobs->tiles, it / jobs->tiles, 0};
+    const SurfJob &jb = jobs[m.job];
+    if (jb.per_lane == 4)
+      node_item<4, HAS_B>(jb, m.tile, m.split, ff, b_global, sm);
+    else
+      node_item<2, HAS_B>(jb, m.tile, m.split, ff, b_global, sm);
+  }
+}
+
+// Adds the atom ranges of every node: one lane per third of a node's slot, so
+// that a wave reads contiguous 16-byte parts and keeps 8 ranges in flight.
+__global__ __launch_bounds__(kT) void surface_reduce_kernel(const SurfJob *jobs, int first) {
+  const SurfJob &jb = jobs[first + blockIdx.z];
+  if (!jb.ok || jb.splits == 1) return;
+  const int nodes = jb.sh.ax.n * jb.sh.ay.n;
+  const int id = (int)blockIdx.x * kT + threadIdx.x, node = id / 3, part = id % 3;
+  if (node >= nodes) return;
+  const int size = jb.per_lane * kT, tile = node / size, lane = node % size, splits = jb.splits;
+  const char *slot = (const char *)((const NodeSlot *)jb.slots + (size_t)tile * splits * size + lane) + 16 * part;
+  const size_t step = sizeof(NodeSlot) * size;
+  if (part == 0) {
+    double c = 0.0, s = 0.0;
+#pragma unroll 8
+    for (int i = 0; i < splits; ++i) {
+      const double2 v = *(const double2 *)(slot + i * step);
+      c += v.x;
+      s += v.y;
+    }
+    jb.f[node] = make_double2(c, -s);
+  } else {
+    float4 a = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+#pragma unroll 8
+    for (int i = 0; i < splits; ++i) {
+      const float4 v = *(const float4 *)(slot + i * step);
+      a.x += v.x;
+      a.y += v.y;
+      a.z += v.z;
+      a.w += v.w;
+    }
+    const float k = -2.0f * (float)kPi;
+    float2 *g = (float2 *)(jb.g + 6 * (size_t)node) + 2 * (part - 1);
+    g[0] = make_float2(k * a.x, k * a.y);
+    if (part == 1) g[1] = make_float2(k * a.z, k * a.w);
+  }
+}
+
+// ---- 4. interpolation -----------------------------------------------------------
+//
+// Both products run on the matrix units, in FP64 for F and FP32 for G
+// (16 x 16 x 4 products; 105 and 40 cycles each, as fast as the vector FMAs
+// they replace: 76 and 42). The second product's waves make two 16 x 16
+// tiles that share the operand with the most fields. Lane l of an FP64 product holds rows
+// l / 16 + 4 r (r = 0..3) of column l % 16, of an FP32 product rows
+// 4 (l / 16) + r: the FP32 products take their rows in the order `prow`, so
+// that a lane's F and G belong to the same pixels. (Scalar operands and vector
+// FMAs instead: 18 us for the rows of a 256 x 256 detector at 28 nodes, where
+// each step waits for its scalar loads.)
+
+typedef double double4v __attribute__((ext_vector_type(4)));
+typedef float float4v __attribute__((ext_vector_type(4)));
+
+struct Fields {
+  double4v re, im;
+  float4v g[6];
+};
+
+__device__ __forceinline__ void clear(Fields &a) {
+  a.re = a.im = double4v{0, 0, 0, 0};
+#pragma unroll
+  for (int c = 0; c < 6; ++c) a.g[c] = float4v{0, 0, 0, 0};
+}
+
+// Row of an FP32 product that puts a lane's results on its FP64 rows.
+__device__ __forceinline__ int prow(int m) { return m / 4 + 4 * (m % 4); }
+
+// t[k][x] = sum_i node[i][k] tx[i][x]: 16 node rows x 16 columns per wave;
+// blockIdx.x: 64 columns, blockIdx.y: 16 node rows, blockIdx.z: pattern.
+__global__ __launch_bounds__(kT) void surface_rows_kernel(const SurfJob *jobs, int first) {
+  const SurfJob &jb = jobs[first + blockIdx.z];
+  if (!jb.ok) return;
+  const int nyn = jb.sh.ay.n, nxn = jb.sh.ax.n, nx = jb.nx;
+  const int l = threadIdx.x & 63, m = l & 15, gq = l >> 4;
+  const int k0 = (int)blockIdx.y * 16, x = (int)blockIdx.x * 64 + (int)(threadIdx.x / 64) * 16 + m;
+  if (k0 >= nyn || x - m >= nx) return;
+  // rows and columns past the end repeat the last one and are not stored
+  const double2 *f = jb.f + (size_t)gq * nyn + min(k0 + m, nyn - 1);
+  const float2 *g = (const float2 *)jb.g + 3 * ((size_t)gq * nyn + min(k0 + prow(m), nyn - 1));
+  const double *tx = jb.sh.tx + (size_t)gq * nx + min(x, nx - 1);
+  Fields acc;
+  clear(acc);
+#pragma unroll 4
+  for (int i = 0; i < nxn; i += 4) {
+    const double2 fv = f[(size_t)i * nyn];
+    const float2 g0 = g[3 * (size_t)i * nyn], g1 = g[3 * (size_t)i * nyn + 1], g2 = g[3 * (size_t)i * nyn + 2];
+    const double b = tx[(size_t)i * nx];
+    const float gv[6] = {g0.x, g0.y, g1.x, g1.y, g2.x, g2.y};
+    acc.re = __builtin_amdgcn_mfma_f64_16x16x4f64(fv.x, b, acc.re, 0, 0, 0);
+    acc.im = __builtin_amdgcn_mfma_f64_16x16x4f64(fv.y, b, acc.im, 0, 0, 0);
+#pragma unroll
+    for (int c = 0; c < 6; ++c) acc.g[c] = __builtin_amdgcn_mfma_f32_16x16x4f32(gv[c], (float)b, acc.g[c], 0, 0, 0);
+  }
+  if (x >= nx) return;
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    const int k = k0 + gq + 4 * r;
+    if (k >= nyn) continue;
+    const size_t o = (size_t)k * nx + x;
+    jb.t64[o] = make_double2(acc.re[r], acc.im[r]);
+    float2 *t = (float2 *)jb.t32 + 3 * o;
+#pragma unroll
+    for (int c = 0; c < 3; ++c) t[c] = make_float2(acc.g[2 * c][r], acc.g[2 * c + 1][r]);
+  }
+}
+
+// F(y, x) = sum_k ty[k][y] t[k][x], the list's deviation, the centre's phase
+// and the intensity: J tiles of 16 x 16 pixels per wave (one above the other),
+// 2 x 2 waves per workgroup. One tile where two would leave SIMDs without a
+// wave (a 256 x 256 detector has 256 tiles).
+template <int J>
+__global__ __launch_bounds__(kT) void surface_cols_kernel(const SurfJob *jobs, int first, const float *__restrict__ dev,
+                                                          const float *__restrict__ hkl, float2 *__restrict__ F,
+                                                          float *__restrict__ I) {
+  const SurfJob &jb = jobs[first + blockIdx.z];
+  if (!jb.ok) return;
+  const int nyn = jb.sh.ay.n, nx = jb.nx, ny = jb.ny;
+  const int wave = threadIdx.x / 64, l = threadIdx.x & 63, m = l & 15, gq = l >> 4;
+  const int x = (int)blockIdx.x * 32 + (wave & 1) * 16 + m, y0 = ((int)blockIdx.y * 2 + (wave >> 1)) * 16 * J;
+  if (x - m >= nx || y0 >= ny) return;
+  const size_t xc = (size_t)gq * nx + min(x, nx - 1);
+  const double2 *t64 = jb.t64 + xc;
+  const float2 *t32 = (const float2 *)jb.t32 + 3 * xc;
+  const double *w[J], *wp[J];
+#pragma unroll
+  for (int j = 0; j < J; ++j) {
+    w[j] = jb.sh.ty + (size_t)gq * ny + min(y0 + 16 * j + m, ny - 1);
+    wp[j] = jb.sh.ty + (size_t)gq * ny + min(y0 + 16 * j + prow(m), ny - 1);
+  }
+  Fields acc[J];
+#pragma unroll
+  for (int j = 0; j < J; ++j) clear(acc[j]);
+#pragma unroll 4
+  for (int k = 0; k < nyn; k += 4) {
+    const double2 v = t64[(size_t)k * nx];
+    const float2 g0 = t32[3 * (size_t)k * nx], g1 = t32[3 * (size_t)k * nx + 1], g2 = t32[3 * (size_t)k * nx + 2];
+    const float gv[6] = {g0.x, g0.y, g1.x, g1.y, g2.x, g2.y};
+#pragma unroll
+    for (int j = 0; j < J; ++j) {
+      const double a = w[j][(size_t)k * ny];
+      const float a32 = (float)wp[j][(size_t)k * ny];
+      acc[j].re = __builtin_amdgcn_mfma_f64_16x16x4f64(a, v.x, acc[j].re, 0, 0, 0);
+      acc[j].im = __builtin_amdgcn_mfma_f64_16x16x4f64(a, v.y, acc[j].im, 0, 0, 0);
+#pragma unroll
+      for (int c = 0; c < 6; ++c) acc[j].g[c] = __builtin_amdgcn_mfma_f32_16x16x4f32(a32, gv[c], acc[j].g[c], 0, 0, 0);
+    }
+  }
+  if (x >= nx) return;
+  double cx = jb.r0[0], cy = jb.r0[1], cz = jb.r0[2];
+  if (jb.has_rot) {
+    const double *R = jb.rot;
+    const double ax = cx, ay = cy, az = cz;
+    cx = __builtin_fma(R[6], az, __builtin_fma(R[3], ay, R[0] * ax));
+    cy = __builtin_fma(R[7], az, __builtin_fma(R[4], ay, R[1] * ax));
+    cz = __builtin_fma(R[8], az, __builtin_fma(R[5], ay, R[2] * ax));
+  }
+  const size_t out = (size_t)jb.pattern * ((size_t)nx * ny);
+#pragma unroll
+  for (int j = 0; j < J; ++j)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int y = y0 + 16 * j + gq + 4 * r;
+      if (y >= ny) continue;
+      const size_t p = (size_t)y * nx + x;
+      const float dx = dev[3 * p], dy = dev[3 * p + 1], dz = dev[3 * p + 2];
+      const Fields &v = acc[j];
+      const double re =
+          v.re[r] + (double)__builtin_fmaf(dz, v.g[4][r], __builtin_fmaf(dy, v.g[2][r], dx * v.g[0][r]));
+      const double im =
+          v.im[r] + (double)__builtin_fmaf(dz, v.g[5][r], __builtin_fmaf(dy, v.g[3][r], dx * v.g[1][r]));
+      if (I) I[out + p] = (float)(re * re + im * im);
+      if (F) {
+        const double t = __builtin_fma((double)hkl[3 * p + 2], cz,
+                                       __builtin_fma((double)hkl[3 * p + 1], cy, (double)hkl[3 * p] * cx));
+        double sn, cs;
+        sincospi(2.0 * __builtin_amdgcn_fract(t), &sn, &cs);
+        F[out + p] = make_float2((float)(re * cs + im * sn), (float)(im * cs - re * sn));
+      }
+    }
+}
+
+size_t align_up(size_t n) { return (n + 255) / 256 * 256; }
+
+// Workspace of one pattern: the nodes of an axis are limited to what can pay
+// (worth() needs n_x n_y below about a third of the pixels).
+struct SingleLayout {
+  int max_nx, max_ny, slot_cap;
+  size_t fit, records, centres, job, dev, nodes, tx, ty, prep, f, g, slots, t64, t32, total;
+};
+
+SingleLayout single_layout(int nx, int ny, int natoms) {
+  SingleLayout l;
+  auto cap = [](int n) { return std::max(kSurfMinNodes, std::min(kSurfMaxNodes, (int)(0.6 * n) / 4 * 4)); };
+  l.max_nx = cap(nx);
+  l.max_ny = cap(ny);
+  const size_t nodes = (size_t)l.max_nx * l.max_ny, npix = (size_t)nx * ny;
+  l.slot_cap = std::max(1 << 20, (int)(nodes + 4 * kT));
+  size_t at = 0;
+  auto take = [&](size_t bytes) {
+    const size_t o = at;
+    at += align_up(bytes);
+    return o;
+  };
+  l.job = take(sizeof(SurfJob));
+  l.fit = take(sizeof(SurfFit));
+  l.records = take(sizeof(SurfRecord) * (kSurfListBlocks + kSurfAtomBlocks));
+  l.centres = take(sizeof(double) * 3);
+  l.dev = take(sizeof(float) * 3 * npix);
+  l.nodes = take(sizeof(double) * 3 * nodes);
+  l.tx = take(sizeof(double) * (size_t)l.max_nx * nx);
+  l.ty = take(sizeof(double) * (size_t)l.max_ny * ny);
+  l.prep = take(sizeof(NodeAtom) * (size_t)natoms);
+  l.f = take(sizeof(double2) * nodes);
+  l.g = take(sizeof(float) * 6 * nodes);
+  l.slots = take(sizeof(NodeSlot) * (size_t)l.slot_cap);
+  l.t64 = take(sizeof(double2) * (size_t)l.max_ny * nx);
+  l.t32 = take(sizeof(float) * 6 * (size_t)l.max_ny * nx);
+  l.total = at;
+  return l;
+}
+
+void launch_interpolation(const SurfJob *jobs, int first, int count, int nx, int ny, int max_nodes, int max_ny,
+                          const float *dev, const float *hkl, float2 *F, float *I, hipStream_t s) {
+  hipLaunchKernelGGL(surface_reduce_kernel, dim3((3 * max_nodes + kT - 1) / kT, 1, count), dim3(kT), 0, s, jobs, first);
+  hipLaunchKernelGGL(surface_rows_kernel, dim3((nx + 63) / 64, (max_ny + 15) / 16, count), dim3(kT), 0, s, jobs,
+                     first);
+  if ((long long)nx * ny * count >= 1 << 20)  // at least two waves of two tiles per SIMD
+    hipLaunchKernelGGL(surface_cols_kernel<2>, dim3((nx + 31) / 32, (ny + 63) / 64, count), dim3(kT), 0, s, jobs, first,
+                       dev, hkl, F, I);
+  else
+    hipLaunchKernelGGL(surface_cols_kernel<1>, dim3((nx + 31) / 32, (ny + 31) / 32, count), dim3(kT), 0, s, jobs, first,
+                       dev, hkl, F, I);
+}
+
+const void *nodes_kernel(bool has_b) {
+  return has_b ? (const void *)&surface_nodes_kernel<true> : (const void *)&surface_nodes_kernel<false>;
+}
+
+}  // namespace
+
+void surf_terms(const float *ff, const spsim_hip_segment *segs, int nsegs, float b_global, float bmin, float bmax,
+                float s2max, SurfMol *mol) {
+  mol->b_smooth = 0.0f;
+  mol->weakest = 1.0f;
+  for (int i = 0; i < nsegs; ++i)
+    species_terms(ff + segs[i].species * SPSIM_HIP_FF_STRIDE,
+                  segs[i].species == SPSIM_HIP_UNIT_SPECIES ? 0.0f : b_global, bmin, bmax, s2max, &mol->b_smooth,
+                  &mol->weakest);
+}
+
+bool surf_choose(const SurfFit &fit, const SurfMol &mol, int nx, int ny, int natoms, SurfAxis *ax, SurfAxis *ay) {
+  if (!smooth(mol, fit.s2max)) return false;
+  SurfAxis *out[2] = {ax, ay};
+  for (int k = 0; k < 2; ++k) {
+    const float *slope = k ? fit.slope_y : fit.slope_x;
+    int n = kSurfMinNodes;
+    while (n <= kSurfMaxNodes &&
+           !(axis_need(slope, (float)mol.radius, mol.b_smooth * fit.s2max, axis_stretch(n)) <= (float)n))
+      n += n < 64 ? 4 : 8;
+    if (n > kSurfMaxNodes) return false;
+    out[k]->n = n;
+    out[k]->a = axis_stretch(n);
+    out[k]->asin_a = std::asin(out[k]->a);
+  }
+  return worth(ax->n, ay->n, nx, ny, natoms);
+}
+
+bool surf_worth(long long nx, long long ny, long long natoms) {
+  // Below 2e8 terms the direct sum takes less than the interpolation's six
+  // launches (about 40 us).
+  return nx >= kSurfMinSide && ny >= kSurfMinSide && nx * ny * natoms >= 200000000LL;
+}
+
+size_t surf_single_bytes(int nx, int ny, int natoms) { return single_layout(nx, ny, natoms).total; }
+
+int launch_surface(const PatternLaunch &a, int nx, int ny, int cus, void *ws, const int **ok_flag, hipStream_t s) {
+  const SingleLayout l = single_layout(nx, ny, a.natoms);
+  char *w = (char *)ws;
+  const bool has_b = a.atom_b != nullptr;
+  const int slots = resident_slots(nodes_kernel(has_b), cus);
+  PlanArgs p{};
+  p.job.nx = nx;
+  p.job.ny = ny;
+  p.job.sh.nodes = (double *)(w + l.nodes);
+  p.job.sh.tx = (double *)(w + l.tx);
+  p.job.sh.ty = (double *)(w + l.ty);
+  p.job.atoms = a.atoms;
+  p.job.atom_b = a.atom_b;
+  p.job.segs = a.segs;
+  p.job.nsegs = a.nsegs;
+  p.job.natoms = a.natoms;
+  p.job.has_rot = a.has_rot;
+  std::copy(a.rot.r, a.rot.r + 9, p.job.rot);
+  p.job.f = (double2 *)(w + l.f);
+  p.job.g = (float *)(w + l.g);
+  p.job.slots = w + l.slots;
+  p.job.prep = w + l.prep;
+  p.job.t64 = (double2 *)(w + l.t64);
+  p.job.t32 = (float *)(w + l.t32);
+  p.fit = (const SurfFit *)(w + l.fit);
+  p.records = (const SurfRecord *)(w + l.records);
+  p.list_blocks = std::min(kSurfListBlocks, ny);
+  p.centres = (const double *)(w + l.centres);
+  p.ff = a.ff;
+  p.b_global = a.b_global;
+  p.has_b = has_b;
+  p.slots = slots;
+  p.slot_cap = l.slot_cap;
+  p.max_nx = l.max_nx;
+  p.max_ny = l.max_ny;
+  p.out = (SurfJob *)(w + l.job);
+  const SurfJob *job = p.out;
+  ScanArgs sc{a.hkl,    nx, ny, p.list_blocks, a.atoms, a.atom_b, nullptr, a.natoms, (SurfFit *)(w + l.fit),
+              (float *)(w + l.dev), (SurfRecord *)(w + l.records), (double *)(w + l.centres)};
+  hipLaunchKernelGGL(surface_scan_kernel, dim3(p.list_blocks + kSurfAtomBlocks), dim3(kT), 0, s, sc);
+  hipLaunchKernelGGL(surface_plan_kernel, dim3(std::max(1, 2 * cus / 3), 3), dim3(kT), 0, s, p);
+  if (has_b)
+    hipLaunchKernelGGL(surface_nodes_kernel<true>, dim3(slots), dim3(kT), 0, s, job, (const SurfItem *)nullptr, 0,
+                       a.ff, a.b_global);
+  else
+    hipLaunchKernelGGL(surface_nodes_kernel<false>, dim3(slots), dim3(kT), 0, s, job, (const SurfItem *)nullptr, 0,
+                       a.ff, a.b_global);
+  launch_interpolation(job, 0, 1, nx, ny, l.max_nx * l.max_ny, l.max_ny, (const float *)(w + l.dev), a.hkl, a.F, a.I, s);
+  SPSIM_HIP_TRY(hipGetLastError());
+  *ok_flag = &job->ok;
+  return SPSIM_HIP_OK;
+}
+
+int surf_scan(const float *hkl, int nx, int ny, const spsim_hip_atom *atoms, const float *atom_b, const MolInfo *mols,
+              int nmol, SurfFit *fit, float *dev, SurfRecord *records, double *centres, hipStream_t s) {
+  const int lb = std::min(kSurfListBlocks, ny);
+  ScanArgs sc{hkl, nx, ny, lb, atoms, atom_b, mols, 0, fit, dev, records, centres};
+  hipLaunchKernelGGL(surface_scan_kernel, dim3(lb + nmol * kSurfAtomBlocks), dim3(kT), 0, s, sc);
+  SPSIM_HIP_TRY(hipGetLastError());
+  return SPSIM_HIP_OK;
+}
+
+int surf_tables(const SurfFit *fit, const SurfShape &sh, int nx, int ny, hipStream_t s) {
+  hipLaunchKernelGGL(surface_tables_kernel, dim3(256, 2), dim3(kT), 0, s, fit, sh, nx, ny);
+  SPSIM_HIP_TRY(hipGetLastError());
+  return SPSIM_HIP_OK;
+}
+
+int surf_run(const SurfRun &r, int cus, hipStream_t s) {
+  if (r.count <= 0) return SPSIM_HIP_OK;
+  const int blocks = std::min(r.nitems, resident_slots(nodes_kernel(r.has_b), cus));
+  if (r.has_b)
+    hipLaunchKernelGGL(surface_nodes_kernel<true>, dim3(blocks), dim3(kT), 0, s, r.jobs, r.items, r.nitems, r.ff,
+                       r.b_global);
+  else
+    hipLaunchKernelGGL(surface_nodes_kernel<false>, dim3(blocks), dim3(kT), 0, s, r.jobs, r.items, r.nitems, r.ff,
+                       r.b_global);
+  launch_interpolation(r.jobs, r.first, r.count, r.nx, r.ny, r.max_nodes, r.max_ny, r.dev, r.hkl, r.F, r.I, s);
+  SPSIM_HIP_TRY(hipGetLastError());
+  return SPSIM_HIP_OK;
+}
+
+}  // namespace spsim

@@ -1,0 +1,126 @@
+// Structure factor of a smooth detector list by interpolation over the
+// detector surface (surface.hip): descriptions shared with the batched plans.
+#pragma once
+
+#include "common.hpp"
+#include "sf_kernels.hpp"
+
+namespace spsim {
+
+constexpr int kSurfDeg = 16;         // sample lines per axis of the list's surface (degree kSurfDeg - 1)
+constexpr int kSurfMinSide = 64;     // shortest detector side that is tried
+constexpr int kSurfMinNodes = 16;    // fewest and most nodes per axis, a multiple of 4
+constexpr int kSurfMaxNodes = 512;
+constexpr int kSurfMaxSplits = 128;  // atom ranges per node tile
+constexpr int kSurfListBlocks = 512;
+constexpr int kSurfAtomBlocks = 64;  // per molecule
+
+// What one workgroup of the scan saw: the largest |q - surface| per component
+// (list blocks), or the largest |r - r0|^2 and the range of B (atom blocks).
+struct SurfRecord {
+  double dev[3];
+  double r2;
+  float bmin, bmax;
+  int bad;  // some value was not finite
+  int pad;
+};
+
+// The list's surface: Chebyshev coefficients of a polynomial through q at
+// kSurfDeg x kSurfDeg pixels, in the pixel coordinates u, v in [-1, 1]
+// (coef[n][m][k]: T_n(v) T_m(u), component k), and its steepest slopes:
+// slope_x[j] is the largest |dq/du| on the line u = cos(pi j / (kSurfDeg - 1)).
+struct SurfFit {
+  double coef[kSurfDeg][kSurfDeg][3];
+  float slope_x[kSurfDeg], slope_y[kSurfDeg];
+  float s2max;  // largest s^2 = (|q| 1e-10 / 2)^2 seen
+};
+
+// Nodes of one axis: u_i = asin(a cos t_i) / asin(a), t_i = (2 i + 1) pi / (2 n);
+// n = 0: the axis needs more than kSurfMaxNodes.
+struct SurfAxis {
+  int n;
+  double a, asin_a;
+};
+
+// One detector shape at one node count: node q [ay.n][ax.n][3] and the
+// interpolation weights, node-major (tx [ax.n][nx], ty [ay.n][ny]).
+struct SurfShape {
+  SurfAxis ax, ay;
+  double *nodes, *tx, *ty;
+};
+
+// One pattern. The node sums f (F) and g (its gradient in q, 3 complex) are
+// [ay.n][ax.n]; t64 and t32 are the same fields along the detector's rows,
+// [ay.n][nx].
+struct SurfJob {
+  int ok;
+  int nx, ny;
+  SurfShape sh;
+  const spsim_hip_atom *atoms;
+  const float *atom_b;
+  const spsim_hip_segment *segs;
+  int nsegs, natoms;
+  int has_rot;
+  double rot[9];
+  double r0[3];  // subtracted from every atom
+  int per_lane, tiles, splits;  // node tiles of 256 per_lane nodes, atom ranges per tile
+  double2 *f;
+  float *g;
+  void *prep;   // atom records of the node sums [natoms]
+  void *slots;  // partial sums [tile * splits + split][256 per_lane]
+  double2 *t64;
+  float *t32;
+  long long pattern;  // index of the outputs
+};
+
+struct SurfItem {
+  int job, tile, split, pad;
+};
+
+// Everything about the molecule that the choice of nodes depends on.
+struct SurfMol {
+  double radius;     // largest |r - r0|
+  double dev;        // largest |q - surface| of the list
+  float b_smooth;    // largest Gaussian coefficient of the terms (form factor + B), A^2
+  float weakest;     // smallest ratio of a term's amplitude at s2max to that at 0
+  int bad;
+};
+
+// Node counts of the pattern, and whether interpolating beats the direct sum.
+bool surf_choose(const SurfFit &fit, const SurfMol &mol, int nx, int ny, int natoms, SurfAxis *ax, SurfAxis *ay);
+// Fills b_smooth and weakest from a form-factor table and the species of a molecule.
+void surf_terms(const float *ff, const spsim_hip_segment *segs, int nsegs, float b_global, float bmin, float bmax,
+                float s2max, SurfMol *mol);
+
+// Host sizes only: is the pattern large enough to look at its list?
+bool surf_worth(long long nx, long long ny, long long natoms);
+
+// One pattern on the device alone (no host decision). On return *ok_flag points
+// to a device int that is non-zero when the outputs were written and zero when
+// the list or molecule is not smooth enough, in which case nothing was.
+size_t surf_single_bytes(int nx, int ny, int natoms);
+int launch_surface(const PatternLaunch &a, int nx, int ny, int cus, void *ws, const int **ok_flag, hipStream_t s);
+
+// For plans: scan a list and nmol molecules into device memory, build a
+// shape's tables, and run a list of patterns.
+int surf_scan(const float *hkl, int nx, int ny, const spsim_hip_atom *atoms, const float *atom_b, const MolInfo *mols,
+              int nmol, SurfFit *fit, float *dev, SurfRecord *records, double *centres, hipStream_t s);
+int surf_tables(const SurfFit *fit, const SurfShape &sh, int nx, int ny, hipStream_t s);
+struct SurfRun {
+  const SurfJob *jobs;    // device
+  int first, count;       // jobs [first, first + count) of this run
+  const SurfItem *items;  // device, of this run
+  int nitems;
+  int max_nodes, max_ny;  // most nodes of these jobs
+  int nx, ny;
+  const float *dev;
+  const float *hkl;
+  const float *ff;
+  float b_global;
+  bool has_b;
+  float2 *F;
+  float *I;
+};
+int surf_run(const SurfRun &r, int cus, hipStream_t s);
+
+}  // namespace spsim

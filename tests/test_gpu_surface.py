@@ -1,0 +1,131 @@
+"""Interpolation over the detector surface (csrc/hip/surface.hip), which large
+patterns on a smooth list take with the automatic tile, against the FP64 oracle
+and against the direct kernels (an explicit tile).
+
+Tolerance: the interpolation's own error is below 3e-8 of |F| (normwise), the
+FP32 sums' error 1e-7 of F and 2e-7 of I, as for the direct kernels: 4e-7
+leaves a factor of two."""
+import numpy as np
+import pytest
+
+import oracle
+from spsim_amd import device as dv
+from spsim_amd import workloads as wl
+from tests.conftest import oracle_threads, rel_l2
+
+pytestmark = pytest.mark.gpu
+
+TOL = 4e-7
+
+
+def _run(gpu, hkl, nx, ny, Z, pos, atom_b=None, amp=None, B=0.0, R=None, tile=None):
+    import torch
+
+    atoms = dv.DeviceAtoms(dv.pack_atoms(Z, pos, atom_b=atom_b, amp=amp), gpu)
+    q = torch.from_numpy(np.ascontiguousarray(hkl, np.float32)).to(gpu)
+    F, I = dv.structure_factor_grid(q, nx, ny, atoms, dv.form_factor_table(device=gpu), B=B, R=R, tile=tile)
+    torch.cuda.synchronize()
+    F = F.cpu().numpy()
+    return F[:, 0] + 1j * F[:, 1], I.cpu().numpy()
+
+
+def _list(nx, ny, pixel=75e-6, distance=0.1, wavelength=0.2e-9, cx=0.0, cy=0.0, spherical=0):
+    return oracle.hkl_detector(nx, ny, np.float32(nx * pixel).item(), np.float32(ny * pixel).item(), distance, cx, cy,
+                               spherical, wavelength)
+
+
+# (nx, ny, atoms, radius, list, per-atom B, rotation): the shortest sides, odd
+# and unequal ones, one that ends inside every tile, a long wavelength (fewest
+# nodes), a wide angle (most nodes), a molecule far from the origin
+CASES = [
+    (64, 64, 60_000, 4e-9, {"pixel": 3e-4}, False, False),
+    (65, 67, 50_000, 5e-9, {}, True, True),
+    (333, 217, 4_000, 5e-9, {"cx": 1.3e-3, "wavelength": 0.15e-9}, False, True),
+    (129, 257, 9_000, 6e-9, {}, True, False),
+    (400, 400, 3_000, 5e-9, {"pixel": 20e-6, "distance": 0.05, "wavelength": 1.3e-9}, False, True),
+    (512, 512, 3_000, 14e-9, {"pixel": 150e-6}, True, True),
+    (300, 300, 3_000, 4e-9, {"spherical": 1}, False, False),
+]
+
+
+@pytest.mark.parametrize("nx,ny,natoms,radius,geometry,with_b,rotated", CASES)
+def test_interpolated_pattern_vs_f64_and_direct(gpu, nx, ny, natoms, radius, geometry, with_b, rotated):
+    rng = np.random.default_rng(nx * 1000 + ny)
+    Z, pos, b = wl.random_molecule(natoms, radius, rng, atom_b_range=(5.0, 40.0))
+    pos = (pos + np.array([3e-9, -2e-9, 1e-9])).astype(np.float32)
+    Z[: natoms // 50] = 1
+    b = b if with_b else None
+    R = wl.uniform_rotations(1, rng)[0] if rotated else None
+    hkl = _list(nx, ny, **geometry)
+    F, I = _run(gpu, hkl, nx, ny, Z, pos, atom_b=b, B=2.0, R=R)
+    Fd, Id = _run(gpu, hkl, nx, ny, Z, pos, atom_b=b, B=2.0, R=R, tile=dv.make_tile(1, 256, 0))
+    assert not np.array_equal(I, Id)  # the interpolation ran
+    # the corners, the edges and a random sample
+    sub = np.unique(np.concatenate([[0, nx - 1, nx * ny - nx, nx * ny - 1], np.arange(0, nx * ny, 7 * nx),
+                                    rng.choice(nx * ny, 1500, replace=False)]))
+    F_ref, I_ref = oracle.sf_f64(hkl[sub], Z, pos, atom_b=b, B=2.0, R=R, threads=oracle_threads())
+    e, ed = rel_l2(I[sub], I_ref), rel_l2(Id[sub], I_ref)
+    ef = np.linalg.norm(F[sub] - F_ref) / np.linalg.norm(F_ref)
+    print(f"{nx}x{ny}: I {e:.2e} (direct {ed:.2e}), F {ef:.2e}", flush=True)
+    assert e < TOL and ef < TOL
+    assert np.linalg.norm(F - Fd) / np.linalg.norm(Fd) < 2 * TOL
+
+
+@pytest.mark.parametrize("what", ["pixel", "noise", "nan pixel", "wide B", "infinite weight", "huge molecule"])
+def test_rough_inputs_keep_the_direct_sum(gpu, what):
+    """Lists and molecules that do not vary smoothly over the detector give
+    the direct kernel's results bit for bit."""
+    rng = np.random.default_rng(5)
+    n, natoms = 200, 6_000
+    Z, pos, b = wl.random_molecule(natoms, 5e-9, rng, atom_b_range=(5.0, 40.0))
+    hkl, amp, B = _list(n, n).copy(), None, 0.0
+    if what == "pixel":
+        hkl[123 * n + 77, 1] *= np.float32(1.001)
+    elif what == "noise":
+        hkl = (hkl * (1.0 + 1e-4 * rng.normal(size=hkl.shape))).astype(np.float32)
+    elif what == "nan pixel":
+        hkl[31, 2] = np.nan
+    elif what == "wide B":
+        b = b * np.float32(1e4)
+    elif what == "infinite weight":
+        amp = np.ones(natoms, np.float32)
+        amp[10] = np.inf
+    else:
+        pos = pos * np.float32(300.0)
+    F, I = _run(gpu, hkl, n, n, Z, pos, atom_b=b, amp=amp, B=B)
+    Fd, Id = _run(gpu, hkl, n, n, Z, pos, atom_b=b, amp=amp, B=B, tile=dv.make_tile(8, 256, 0))
+    assert np.array_equal(I, Id, equal_nan=True) and np.array_equal(F, Fd, equal_nan=True)
+
+
+def test_interpolated_pattern_repeats_and_captures(gpu):
+    """The same bits on every call, with the workspace used by other calls in
+    between, and on every replay of a captured graph."""
+    import torch
+
+    rng = np.random.default_rng(8)
+    n = 256
+    Z, pos, _ = wl.random_molecule(5_000, 5e-9, rng)
+    atoms = dv.DeviceAtoms(dv.pack_atoms(Z, pos), gpu)
+    ff = dv.form_factor_table(device=gpu)
+    q = torch.from_numpy(_list(n, n)).to(gpu)
+    small = torch.from_numpy(_list(128, 128)).to(gpu)
+    F0, I0 = dv.structure_factor_grid(q, n, n, atoms, ff)
+    dv.structure_factor_grid(small, 128, 128, atoms, ff)
+    F1, I1 = dv.structure_factor_grid(q, n, n, atoms, ff)
+    torch.cuda.synchronize()
+    assert torch.equal(I0, I1) and torch.equal(F0, F1)
+    stream = torch.cuda.Stream()
+    with torch.cuda.stream(stream):
+        dv.structure_factor_grid(q, n, n, atoms, ff, F=F1, I=I1, stream=stream)
+    stream.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=stream):
+        dv.structure_factor_grid(q, n, n, atoms, ff, F=F1, I=I1, stream=torch.cuda.current_stream())
+    for _ in range(3):
+        I1.fill_(float("nan"))
+        F1.fill_(float("nan"))
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(I0, I1) and torch.equal(F0, F1)
+        dv.structure_factor_grid(small, 128, 128, atoms, ff)
