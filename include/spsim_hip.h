@@ -141,7 +141,14 @@ int spsim_hip_sf_pattern(const float *d_hkl, int npix, const spsim_hip_atom *d_a
    workgroups without that symmetry fall back to two quads. tile->pixels_per_lane
    is the quads per lane here (1 or 2), or 8 for one octant per lane (nx == ny
    only; the default for square detectors, with atom_splits chosen to fill the
-   GPU). tile may be NULL. */
+   GPU). tile may be NULL.
+   With tile == NULL, a detector of at least 64 x 64 pixels and 2e8 pixel-atom
+   terms, F is summed only at the nodes of a grid over the detector surface and
+   interpolated from there (error below 3e-8 of |F|, less than the direct sums'
+   own rounding), when the list and the molecule are smooth enough for it; the
+   device checks both, and everything else takes the direct sum. Such a call
+   uses the library workspace (about 100 MiB at 1024 x 1024); while the stream
+   is being captured it does so only if the workspace is already that large. */
 int spsim_hip_sf_grid(const float *d_hkl, int nx, int ny, const spsim_hip_atom *d_atoms, const float *d_atom_b,
                       const spsim_hip_segment *d_segs, int nsegs, int natoms, const float *d_ff, float b_global,
                       const double *rot9, float *d_F, float *d_I, const spsim_hip_tile *tile, void *stream);
@@ -307,7 +314,10 @@ typedef struct spsim_hip_batch spsim_hip_batch;
    default there); otherwise the per-pixel kernel. The plan copies everything
    to the device, builds the cost-sorted (pattern, tile, atom range) work list
    and owns its device memory until spsim_hip_batch_destroy. tile may be NULL
-   (default tiling). A pattern whose molecule has more atoms than the plan's
+   (default tiling); without one, patterns that are smooth enough are
+   interpolated over the detector surface as in spsim_hip_sf_grid (decided here,
+   pattern by pattern; the plan then holds up to a few hundred MiB for them),
+   and what follows applies to the others. A pattern whose molecule has more atoms than the plan's
    item bound (spsim_hip_batch_set_item_atoms) is split into near-equal atom
    ranges, one work item per range and tile; the tile's last item to finish
    adds the ranges' FP64 partial sums in range order, so results do not depend
@@ -316,7 +326,7 @@ int spsim_hip_batch_create(const float *hkl, int nx, int ny, int nmol, const int
                            const float *pos, const float *amp, const float *atom_b, int delta_atoms,
                            int npatterns, const int *pattern_mol, const double *rot9, const float *ff,
                            float b_global, const spsim_hip_tile *tile, spsim_hip_batch **out);
-/* Runs the persistent kernel: d_I [npatterns][npix] (required), d_F [npatterns][npix][2]
+/* Runs the plan: d_I [npatterns][npix] (required), d_F [npatterns][npix][2]
    (may be NULL). use_graph != 0 replays a captured hipGraph (captured on first use
    for this stream and these output pointers; the stream must not be NULL). */
 int spsim_hip_batch_run(spsim_hip_batch *b, float *d_F, float *d_I, int use_graph, void *stream);
@@ -325,19 +335,20 @@ int spsim_hip_batch_run(spsim_hip_batch *b, float *d_F, float *d_I, int use_grap
 int spsim_hip_batch_run_plain(spsim_hip_batch *b, float *d_F, float *d_I, void *stream);
 /* 1 when the plan runs the mirror-symmetric quad kernel, 0 for the per-pixel kernel. */
 int spsim_hip_batch_uses_grid(const spsim_hip_batch *b);
-/* Tile of the persistent kernel; setting it rebuilds the work list. */
+/* Tile of the persistent kernel; setting it rebuilds the work list, which then
+   takes every pattern. */
 int spsim_hip_batch_set_tile(spsim_hip_batch *b, const spsim_hip_tile *tile);
 int spsim_hip_batch_get_tile(const spsim_hip_batch *b, spsim_hip_tile *tile, int *blocks);
 /* Bound on the atoms of one work item; rebuilds the work list. 0 (the default):
    automatic, about an eighth of one resident workgroup's share of the whole
    run and at least 4 LDS chunks; > 0: that many atoms; < 0: never split a
-   pattern's atoms. */
+   pattern's atoms. A bound other than 0 also puts every pattern on the list. */
 int spsim_hip_batch_set_item_atoms(spsim_hip_batch *b, int item_atoms);
-/* Work items of one run, the item bound in effect (0: no pattern is split) and
+/* Work items of a run of all patterns by the persistent kernel, the item bound in effect (0: no pattern is split) and
    the number of (pattern, tile) pairs split over several items. Any pointer
    may be NULL. */
 int spsim_hip_batch_describe(const spsim_hip_batch *b, int *nitems, int *item_atoms, int *split_tiles);
-/* Autotuner: times every supported tile (pixels per lane x LDS chunk) on a
+/* Autotuner of the persistent kernel: times every supported tile (pixels per lane x LDS chunk) on a
    slice of the plan's own work (patterns spread over its atom-count range),
    keeps the kernel family (pixels or quads per lane, octants) with the
    highest pixel-atom terms/s and, within it, the LDS chunk whose sample runs

@@ -1,5 +1,7 @@
-// Batched structure factors: many molecules and orientations in one persistent
-// launch over a cost-sorted (pattern, pixel-tile, atom-range) work list,
+// Batched structure factors: many molecules and orientations. Patterns whose
+// list and molecule are smooth enough are interpolated over the detector
+// surface (surface.hip), unless the caller names a tile or an item bound of the
+// direct kernels; the others run in one persistent launch over a cost-sorted (pattern, pixel-tile, atom-range) work list,
 // optionally replayed from a captured hipGraph, plus the plain
 // one-launch-per-pattern path and the tile autotuner.
 //
@@ -19,6 +21,7 @@
 
 #include "common.hpp"
 #include "sf_kernels.hpp"
+#include "surface.hpp"
 
 using spsim::BatchItem;
 using spsim::MolInfo;
@@ -37,6 +40,13 @@ struct spsim_hip_batch {
   int item_atoms = 0;      // in effect (0: no pattern split)
   int split_tiles = 0;     // (pattern, tile) pairs with more than one item
   double terms = 0.0;
+
+  // Patterns interpolated over the detector surface (null: none), and whether
+  // runs use it: not after a tile or an item bound was asked for, which name
+  // the direct kernels. run_items: the items of the other patterns.
+  spsim::SurfPlan *surf = nullptr;
+  bool direct = false;
+  int run_items = 0;
 
   // device memory
   float *hkl = nullptr;
@@ -84,6 +94,7 @@ int dupload(T **p, const T *h, size_t n) {
 void free_batch(spsim_hip_batch *b) {
   if (!b) return;
   if (b->exec) (void)hipGraphExecDestroy(b->exec);
+  surf_plan_destroy(b->surf);
   void *ptrs[] = {b->hkl,  b->atoms, b->atom_b,   b->segs,     b->mols, b->pattern_mol,
                   b->rot,  b->items, b->counters, b->partials, b->queue, b->ff};
   for (void *p : ptrs)
@@ -227,14 +238,31 @@ int set_tile(spsim_hip_batch *b, const spsim_hip_tile &t) {
   b->items = nullptr;
   b->counters = nullptr;
   b->partials = nullptr;
-  SPSIM_TRY(dupload(&b->items, L.items.data(), L.items.size()));
-  SPSIM_TRY(alloc_split_state(L, t, b->grid, &b->counters, &b->partials));
   b->nitems = (int)L.items.size();
   b->item_atoms = item_atoms;
   b->split_tiles = L.groups;
+  if (b->surf && !b->direct) {  // the direct kernels run what is left over
+    std::vector<int> rest;
+    for (int p = 0; p < b->npatterns; ++p)
+      if (!surf_plan_takes(b->surf, p)) rest.push_back(p);
+    L = build_items(*b, t, item_atoms, &rest);
+  }
+  SPSIM_TRY(dupload(&b->items, L.items.data(), L.items.size()));
+  SPSIM_TRY(alloc_split_state(L, t, b->grid, &b->counters, &b->partials));
+  b->run_items = (int)L.items.size();
   b->tile = t;
   b->blocks = blocks;
   return SPSIM_HIP_OK;
+}
+
+// One run of the plan: the interpolated patterns, then the others.
+int launch_plan(const spsim_hip_batch *b, float *F, float *I, hipStream_t s) {
+  if (b->surf && !b->direct) {
+    SPSIM_TRY(surf_plan_run(b->surf, (float2 *)F, I, s));
+    if (b->run_items == 0) return SPSIM_HIP_OK;
+  }
+  const BatchLaunch a = launch_args(b, b->items, b->run_items, b->queue, b->counters, b->partials, F, I);
+  return launch_batch(a, b->tile, b->grid, b->blocks, s);
 }
 
 }  // namespace
@@ -321,6 +349,13 @@ int spsim_hip_batch_create(const float *hkl, int nx, int ny, int nmol, const int
     free_batch(b);
     return rc;
   }
+  if (tile) b->direct = true;
+  if (!tile && (rc = surf_plan_create(b->hkl, nx, ny, b->atoms, b->atom_b, b->segs, b->mols, b->h_mols.data(), nmol,
+                                      h_segs.data(), npatterns, pattern_mol, rot9, b->ff, ffh, b_global, cus,
+                                      &b->surf)) != SPSIM_HIP_OK) {
+    free_batch(b);
+    return rc;
+  }
   const int avg_atoms = packed_total / std::max(nmol, 1);
   spsim_hip_tile t = tile ? *tile : default_tile(avg_atoms, npix, b->grid);
   if (!tile && b->square) t.pixels_per_lane = kOctantLane;
@@ -335,7 +370,11 @@ int spsim_hip_batch_create(const float *hkl, int nx, int ny, int nmol, const int
 int spsim_hip_batch_set_tile(spsim_hip_batch *b, const spsim_hip_tile *tile) {
   using namespace spsim;
   if (!b || !tile) return fail(SPSIM_HIP_ERR_INVALID, "NULL argument");
-  return set_tile(b, *tile);
+  const bool old = b->direct;
+  b->direct = true;
+  const int rc = set_tile(b, *tile);
+  if (rc != SPSIM_HIP_OK) b->direct = old;
+  return rc;
 }
 
 int spsim_hip_batch_get_tile(const spsim_hip_batch *b, spsim_hip_tile *tile, int *blocks) {
@@ -350,9 +389,14 @@ int spsim_hip_batch_set_item_atoms(spsim_hip_batch *b, int item_atoms) {
   using namespace spsim;
   if (!b) return fail(SPSIM_HIP_ERR_INVALID, "NULL plan");
   const int old = b->item_atoms_req;
+  const bool old_direct = b->direct;
   b->item_atoms_req = item_atoms;
+  if (item_atoms != 0) b->direct = true;
   const int rc = set_tile(b, b->tile);
-  if (rc != SPSIM_HIP_OK) b->item_atoms_req = old;
+  if (rc != SPSIM_HIP_OK) {
+    b->item_atoms_req = old;
+    b->direct = old_direct;
+  }
   return rc;
 }
 
@@ -369,8 +413,7 @@ int spsim_hip_batch_run(spsim_hip_batch *b, float *d_F, float *d_I, int use_grap
   using namespace spsim;
   if (!b || !d_I) return fail(SPSIM_HIP_ERR_INVALID, "NULL argument");
   hipStream_t s = (hipStream_t)stream;
-  BatchLaunch a = launch_args(b, b->items, b->nitems, b->queue, b->counters, b->partials, d_F, d_I);
-  if (!use_graph) return launch_batch(a, b->tile, b->grid, b->blocks, s);
+  if (!use_graph) return launch_plan(b, d_F, d_I, s);
   if (!s) return fail(SPSIM_HIP_ERR_INVALID, "graph replay needs a non-default stream");
   if (!b->exec || b->g_stream != s || b->g_F != d_F || b->g_I != d_I) {
     if (b->exec) {
@@ -379,7 +422,7 @@ int spsim_hip_batch_run(spsim_hip_batch *b, float *d_F, float *d_I, int use_grap
     }
     hipGraph_t g = nullptr;
     SPSIM_HIP_TRY(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
-    int rc = launch_batch(a, b->tile, b->grid, b->blocks, s);
+    int rc = launch_plan(b, d_F, d_I, s);
     hipError_t e = hipStreamEndCapture(s, &g);
     if (rc != SPSIM_HIP_OK) {
       if (g) (void)hipGraphDestroy(g);

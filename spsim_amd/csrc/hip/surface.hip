@@ -35,6 +35,7 @@
 
 #include <algorithm>
 #include <cmath>
+#include <vector>
 
 #include "form_factor.hpp"
 
@@ -1000,7 +1001,9 @@ SingleLayout single_layout(int nx, int ny, int natoms) {
 
 void launch_interpolation(const SurfJob *jobs, int first, int count, int nx, int ny, int max_nodes, int max_ny,
                           const float *dev, const float *hkl, float2 *F, float *I, hipStream_t s) {
-  hipLaunchKernelGGL(surface_reduce_kernel, dim3((3 * max_nodes + kT - 1) / kT, 1, count), dim3(kT), 0, s, jobs, first);
+  if (max_nodes > 0)  // some pattern's atoms are split
+    hipLaunchKernelGGL(surface_reduce_kernel, dim3((3 * max_nodes + kT - 1) / kT, 1, count), dim3(kT), 0, s, jobs,
+                       first);
   hipLaunchKernelGGL(surface_rows_kernel, dim3((nx + 63) / 64, (max_ny + 15) / 16, count), dim3(kT), 0, s, jobs,
                      first);
   if ((long long)nx * ny * count >= 1 << 20)  // at least two waves of two tiles per SIMD
@@ -1016,33 +1019,6 @@ const void *nodes_kernel(bool has_b) {
 }
 
 }  // namespace
-
-void surf_terms(const float *ff, const spsim_hip_segment *segs, int nsegs, float b_global, float bmin, float bmax,
-                float s2max, SurfMol *mol) {
-  mol->b_smooth = 0.0f;
-  mol->weakest = 1.0f;
-  for (int i = 0; i < nsegs; ++i)
-    species_terms(ff + segs[i].species * SPSIM_HIP_FF_STRIDE,
-                  segs[i].species == SPSIM_HIP_UNIT_SPECIES ? 0.0f : b_global, bmin, bmax, s2max, &mol->b_smooth,
-                  &mol->weakest);
-}
-
-bool surf_choose(const SurfFit &fit, const SurfMol &mol, int nx, int ny, int natoms, SurfAxis *ax, SurfAxis *ay) {
-  if (!smooth(mol, fit.s2max)) return false;
-  SurfAxis *out[2] = {ax, ay};
-  for (int k = 0; k < 2; ++k) {
-    const float *slope = k ? fit.slope_y : fit.slope_x;
-    int n = kSurfMinNodes;
-    while (n <= kSurfMaxNodes &&
-           !(axis_need(slope, (float)mol.radius, mol.b_smooth * fit.s2max, axis_stretch(n)) <= (float)n))
-      n += n < 64 ? 4 : 8;
-    if (n > kSurfMaxNodes) return false;
-    out[k]->n = n;
-    out[k]->a = axis_stretch(n);
-    out[k]->asin_a = std::asin(out[k]->a);
-  }
-  return worth(ax->n, ay->n, nx, ny, natoms);
-}
 
 bool surf_worth(long long nx, long long ny, long long natoms) {
   // Below 2e8 terms the direct sum takes less than the interpolation's six
@@ -1105,33 +1081,300 @@ int launch_surface(const PatternLaunch &a, int nx, int ny, int cus, void *ws, co
   return SPSIM_HIP_OK;
 }
 
-int surf_scan(const float *hkl, int nx, int ny, const spsim_hip_atom *atoms, const float *atom_b, const MolInfo *mols,
-              int nmol, SurfFit *fit, float *dev, SurfRecord *records, double *centres, hipStream_t s) {
-  const int lb = std::min(kSurfListBlocks, ny);
-  ScanArgs sc{hkl, nx, ny, lb, atoms, atom_b, mols, 0, fit, dev, records, centres};
-  hipLaunchKernelGGL(surface_scan_kernel, dim3(lb + nmol * kSurfAtomBlocks), dim3(kT), 0, s, sc);
+// ---- plans --------------------------------------------------------------------
+
+struct SurfPlan {
+  // Patterns that run together and share the workspace.
+  struct Group {
+    int first, count, item_first, nitems, max_nodes, max_ny;
+    bool split;
+  };
+  int nx = 0, ny = 0, cus = 0;
+  bool has_b = false;
+  float b_global = 0.0f;
+  const float *hkl = nullptr, *ff = nullptr;
+  std::vector<char> takes;
+  std::vector<Group> groups;
+  std::vector<void *> owned;  // device memory
+  const SurfJob *jobs = nullptr;
+  const SurfItem *items = nullptr;
+  const float *dev = nullptr;
+};
+
+namespace {
+
+constexpr size_t kGroupBytes = (size_t)256 << 20;  // workspace of a group: about the last-level cache
+
+__global__ __launch_bounds__(kT) void surface_prepare_kernel(const SurfJob *jobs, int first, bool has_b) {
+  prepare_atoms(jobs[first + blockIdx.y], has_b, (int)(blockIdx.x * kT + threadIdx.x), (int)gridDim.x * kT);
+}
+
+bool choose(const SurfFit &fit, const SurfMol &mol, int nx, int ny, int natoms, SurfAxis *ax, SurfAxis *ay) {
+  if (!smooth(mol, fit.s2max)) return false;
+  SurfAxis *out[2] = {ax, ay};
+  for (int k = 0; k < 2; ++k) {
+    const float *slope = k ? fit.slope_y : fit.slope_x;
+    int n = kSurfMinNodes;
+    // steps of 8 from 64 nodes on: molecules of similar size share their tables
+    while (n <= kSurfMaxNodes &&
+           !(axis_need(slope, (float)mol.radius, mol.b_smooth * fit.s2max, axis_stretch(n)) <= (float)n))
+      n += n < 64 ? 4 : 8;
+    if (n > kSurfMaxNodes) return false;
+    *out[k] = SurfAxis{n, axis_stretch(n), 0.0};
+    out[k]->asin_a = std::asin(out[k]->a);
+  }
+  return worth(ax->n, ay->n, nx, ny, natoms);
+}
+
+// Lays the job's buffers out in a workspace from `at` on; returns the end.
+size_t place(SurfJob *j, int nx, char *ws, size_t at) {
+  const size_t nodes = (size_t)j->sh.ax.n * j->sh.ay.n;
+  auto take = [&](size_t bytes) {
+    char *p = ws + at;
+    at += align_up(bytes);
+    return p;
+  };
+  j->prep = take(sizeof(NodeAtom) * (size_t)j->natoms);
+  j->f = (double2 *)take(sizeof(double2) * nodes);
+  j->g = (float *)take(sizeof(float) * 6 * nodes);
+  j->slots = take(j->splits > 1 ? sizeof(NodeSlot) * (size_t)j->tiles * j->per_lane * kT * j->splits : 0);
+  j->t64 = (double2 *)take(sizeof(double2) * (size_t)j->sh.ay.n * nx);
+  j->t32 = (float *)take(sizeof(float) * 6 * (size_t)j->sh.ay.n * nx);
+  return at;
+}
+
+// Splits a group's atoms so that its work items number about four per resident
+// workgroup, and appends the items, largest first.
+void split_group(std::vector<SurfJob> &jobs, int first, int count, int slots, std::vector<SurfItem> *items) {
+  double work = 0.0;
+  for (int i = first; i < first + count; ++i) {
+    SurfJob &j = jobs[i];
+    const int nodes = j.sh.ax.n * j.sh.ay.n;
+    // four nodes per lane, unless two leave much less of the last tile empty
+    const int pad4 = (nodes + 4 * kT - 1) / (4 * kT) * 4 * kT, pad2 = (nodes + 2 * kT - 1) / (2 * kT) * 2 * kT;
+    j.per_lane = pad4 > 1.1 * pad2 ? 2 : 4;
+    j.tiles = (nodes + j.per_lane * kT - 1) / (j.per_lane * kT);
+    work += (double)j.tiles * j.per_lane * j.natoms;
+  }
+  const double share = std::max(work / (4.0 * slots), 512.0);  // nodes per lane x atoms
+  const size_t begin = items->size();
+  for (int i = first; i < first + count; ++i) {
+    SurfJob &j = jobs[i];
+    j.splits = std::max(1, std::min(kSurfMaxSplits, (int)std::ceil(j.per_lane * (double)j.natoms / share)));
+    for (int t = 0; t < j.tiles; ++t)
+      for (int k = 0; k < j.splits; ++k) items->push_back(SurfItem{i, t, k, 0});
+  }
+  std::stable_sort(items->begin() + begin, items->end(), [&](const SurfItem &a, const SurfItem &b) {
+    const SurfJob &x = jobs[a.job], &y = jobs[b.job];
+    return (double)x.per_lane * x.natoms / x.splits > (double)y.per_lane * y.natoms / y.splits;
+  });
+}
+
+template <class T>
+int own(SurfPlan *p, T **out, size_t n) {
+  *out = nullptr;
+  hipError_t e = hipMalloc((void **)out, std::max<size_t>(1, n) * sizeof(T));
+  if (e != hipSuccess) return fail(SPSIM_HIP_ERR_NOMEM, "hipMalloc(%zu) failed: %s", n * sizeof(T), hipGetErrorString(e));
+  p->owned.push_back(*out);
+  return SPSIM_HIP_OK;
+}
+
+int build_plan(SurfPlan *p, const spsim_hip_atom *atoms, const float *atom_b, const spsim_hip_segment *segs,
+               const MolInfo *d_mols, const MolInfo *h_mols, int nmol, const spsim_hip_segment *h_segs, int npatterns,
+               const int *pattern_mol, const double *rot9, const float *h_ff) {
+  const int lb = std::min(kSurfListBlocks, p->ny);
+  SurfFit *d_fit = nullptr;
+  float *dev = nullptr;
+  SPSIM_TRY(own(p, &d_fit, 1));
+  SPSIM_TRY(own(p, &dev, 3 * (size_t)p->nx * p->ny));
+  p->dev = dev;
+  SurfFit fit;
+  std::vector<SurfRecord> rec(lb + (size_t)nmol * kSurfAtomBlocks);
+  std::vector<double> centres(3 * (size_t)nmol);
+  {
+    SurfPlan scratch;  // released below
+    SurfRecord *d_rec = nullptr;
+    double *d_centres = nullptr;
+    int rc = own(&scratch, &d_rec, rec.size());
+    if (rc == SPSIM_HIP_OK) rc = own(&scratch, &d_centres, centres.size());
+    hipError_t e = hipSuccess;
+    if (rc == SPSIM_HIP_OK) {
+      const ScanArgs sc{p->hkl, p->nx, p->ny, lb, atoms, atom_b, d_mols, 0, d_fit, dev, d_rec, d_centres};
+      hipLaunchKernelGGL(surface_scan_kernel, dim3(lb + nmol * kSurfAtomBlocks), dim3(kT), 0, nullptr, sc);
+      e = hipGetLastError();
+      if (e == hipSuccess) e = hipMemcpy(&fit, d_fit, sizeof fit, hipMemcpyDeviceToHost);
+      if (e == hipSuccess) e = hipMemcpy(rec.data(), d_rec, rec.size() * sizeof(SurfRecord), hipMemcpyDeviceToHost);
+      if (e == hipSuccess)
+        e = hipMemcpy(centres.data(), d_centres, centres.size() * sizeof(double), hipMemcpyDeviceToHost);
+    }
+    for (void *m : scratch.owned) (void)hipFree(m);
+    SPSIM_TRY(rc);
+    if (e != hipSuccess) return hip_fail(e, "surface scan");
+  }
+  double d2 = 0.0;
+  bool bad = false;
+  for (int k = 0; k < 3; ++k) {
+    double d = 0.0;
+    for (int i = 0; i < lb; ++i) d = std::max(d, rec[i].dev[k]);
+    d2 += d * d;
+  }
+  for (int i = 0; i < lb; ++i) bad = bad || rec[i].bad;
+  std::vector<SurfShape> shapes;
+  std::vector<int> shape_of(nmol, -1);
+  for (int m = 0; m < nmol; ++m) {
+    const MolInfo &mi = h_mols[m];
+    SurfMol mol{0.0, std::sqrt(d2), 0.0f, 1.0f, bad};
+    float lo = 3.4e38f, hi = -3.4e38f;
+    for (int i = 0; i < kSurfAtomBlocks; ++i) {
+      const SurfRecord &r = rec[lb + (size_t)m * kSurfAtomBlocks + i];
+      mol.radius = std::max(mol.radius, std::sqrt(r.r2));
+      lo = std::min(lo, r.bmin);
+      hi = std::max(hi, r.bmax);
+      mol.bad |= r.bad;
+    }
+    for (int i = 0; i < mi.nseg; ++i) {
+      const int sp = h_segs[mi.seg_begin + i].species;
+      species_terms(h_ff + sp * SPSIM_HIP_FF_STRIDE, sp == SPSIM_HIP_UNIT_SPECIES ? 0.0f : p->b_global,
+                    p->has_b ? lo : 0.0f, p->has_b ? hi : 0.0f, fit.s2max, &mol.b_smooth, &mol.weakest);
+    }
+    SurfShape sh{};
+    if (!choose(fit, mol, p->nx, p->ny, mi.atom_end - mi.atom_begin, &sh.ax, &sh.ay)) continue;
+    for (size_t i = 0; i < shapes.size(); ++i)
+      if (shapes[i].ax.n == sh.ax.n && shapes[i].ay.n == sh.ay.n) shape_of[m] = (int)i;
+    if (shape_of[m] >= 0) continue;
+    SPSIM_TRY(own(p, &sh.nodes, 3 * (size_t)sh.ax.n * sh.ay.n));
+    SPSIM_TRY(own(p, &sh.tx, (size_t)sh.ax.n * p->nx));
+    SPSIM_TRY(own(p, &sh.ty, (size_t)sh.ay.n * p->ny));
+    hipLaunchKernelGGL(surface_tables_kernel, dim3(256, 2), dim3(kT), 0, nullptr, (const SurfFit *)d_fit, sh, p->nx,
+                       p->ny);
+    SPSIM_HIP_TRY(hipGetLastError());
+    shape_of[m] = (int)shapes.size();
+    shapes.push_back(sh);
+  }
+  std::vector<SurfJob> jobs;
+  p->takes.assign(npatterns, 0);
+  for (int i = 0; i < npatterns; ++i) {
+    const int m = pattern_mol[i];
+    if (shape_of[m] < 0) continue;
+    p->takes[i] = 1;
+    SurfJob j{};
+    j.ok = 1;
+    j.nx = p->nx;
+    j.ny = p->ny;
+    j.sh = shapes[shape_of[m]];
+    j.atoms = atoms + h_mols[m].atom_begin;
+    j.atom_b = p->has_b ? atom_b + h_mols[m].atom_begin : nullptr;
+    j.segs = segs + h_mols[m].seg_begin;
+    j.nsegs = h_mols[m].nseg;
+    j.natoms = h_mols[m].atom_end - h_mols[m].atom_begin;
+    j.has_rot = 1;
+    std::copy(rot9 + 9 * (size_t)i, rot9 + 9 * (size_t)(i + 1), j.rot);
+    std::copy(&centres[3 * (size_t)m], &centres[3 * (size_t)m] + 3, j.r0);
+    j.pattern = i;
+    jobs.push_back(j);
+  }
+  if (jobs.empty()) return SPSIM_HIP_OK;
+  // largest first, so that a group's patterns need similar grids
+  std::stable_sort(jobs.begin(), jobs.end(), [](const SurfJob &a, const SurfJob &b) {
+    return (double)a.sh.ax.n * a.sh.ay.n * a.natoms > (double)b.sh.ax.n * b.sh.ay.n * b.natoms;
+  });
+  const int slots = resident_slots(nodes_kernel(p->has_b), p->cus);
+  std::vector<SurfItem> items;
+  size_t ws_bytes = 0;
+  for (int first = 0; first < (int)jobs.size();) {
+    SurfPlan::Group g{first, 0, (int)items.size(), 0, 0, 0, false};
+    size_t at = 0;
+    while (first + g.count < (int)jobs.size() && g.count < 4096) {
+      SurfJob probe = jobs[first + g.count];
+      probe.per_lane = 4;
+      probe.tiles = (probe.sh.ax.n * probe.sh.ay.n + 4 * kT - 1) / (4 * kT);
+      probe.splits = 4;  // a typical group's; only the group's size depends on it
+      const size_t end = place(&probe, p->nx, nullptr, at);
+      if (g.count > 0 && end > kGroupBytes) break;
+      at = end;
+      g.max_nodes = std::max(g.max_nodes, probe.sh.ax.n * probe.sh.ay.n);
+      g.max_ny = std::max(g.max_ny, probe.sh.ay.n);
+      ++g.count;
+    }
+    split_group(jobs, first, g.count, slots, &items);
+    g.nitems = (int)items.size() - g.item_first;
+    at = 0;
+    for (int i = first; i < first + g.count; ++i) {
+      at = place(&jobs[i], p->nx, nullptr, at);
+      g.split = g.split || jobs[i].splits > 1;
+    }
+    ws_bytes = std::max(ws_bytes, at);
+    p->groups.push_back(g);
+    first += g.count;
+  }
+  char *ws = nullptr;
+  SurfJob *d_jobs = nullptr;
+  SurfItem *d_items = nullptr;
+  SPSIM_TRY(own(p, &ws, ws_bytes));
+  for (const SurfPlan::Group &g : p->groups) {
+    size_t at = 0;
+    for (int i = g.first; i < g.first + g.count; ++i) at = place(&jobs[i], p->nx, ws, at);
+  }
+  SPSIM_TRY(own(p, &d_jobs, jobs.size()));
+  SPSIM_TRY(own(p, &d_items, items.size()));
+  SPSIM_HIP_TRY(hipMemcpy(d_jobs, jobs.data(), jobs.size() * sizeof(SurfJob), hipMemcpyHostToDevice));
+  SPSIM_HIP_TRY(hipMemcpy(d_items, items.data(), items.size() * sizeof(SurfItem), hipMemcpyHostToDevice));
+  SPSIM_HIP_TRY(hipStreamSynchronize(nullptr));  // the tables
+  p->jobs = d_jobs;
+  p->items = d_items;
+  return SPSIM_HIP_OK;
+}
+
+}  // namespace
+
+int surf_plan_create(const float *hkl, int nx, int ny, const spsim_hip_atom *atoms, const float *atom_b,
+                     const spsim_hip_segment *segs, const MolInfo *d_mols, const MolInfo *h_mols, int nmol,
+                     const spsim_hip_segment *h_segs, int npatterns, const int *pattern_mol, const double *rot9,
+                     const float *d_ff, const float *h_ff, float b_global, int cus, SurfPlan **out) {
+  *out = nullptr;
+  if (nx < kSurfMinSide || ny < kSurfMinSide) return SPSIM_HIP_OK;
+  SurfPlan *p = new SurfPlan;
+  p->nx = nx;
+  p->ny = ny;
+  p->cus = cus;
+  p->has_b = atom_b != nullptr;
+  p->b_global = b_global;
+  p->hkl = hkl;
+  p->ff = d_ff;
+  const int rc = build_plan(p, atoms, atom_b, segs, d_mols, h_mols, nmol, h_segs, npatterns, pattern_mol, rot9, h_ff);
+  if (rc != SPSIM_HIP_OK || p->groups.empty()) {
+    surf_plan_destroy(p);
+    return rc;
+  }
+  *out = p;
+  return SPSIM_HIP_OK;
+}
+
+bool surf_plan_takes(const SurfPlan *p, int pattern) { return p && p->takes[pattern]; }
+
+int surf_plan_run(const SurfPlan *p, float2 *F, float *I, hipStream_t s) {
+  const int slots = resident_slots(nodes_kernel(p->has_b), p->cus);
+  for (const SurfPlan::Group &g : p->groups) {
+    hipLaunchKernelGGL(surface_prepare_kernel, dim3(16, g.count), dim3(kT), 0, s, p->jobs, g.first, p->has_b);
+    const SurfItem *items = p->items + g.item_first;
+    const int blocks = std::min(g.nitems, slots);
+    if (p->has_b)
+      hipLaunchKernelGGL(surface_nodes_kernel<true>, dim3(blocks), dim3(kT), 0, s, p->jobs, items, g.nitems, p->ff,
+                         p->b_global);
+    else
+      hipLaunchKernelGGL(surface_nodes_kernel<false>, dim3(blocks), dim3(kT), 0, s, p->jobs, items, g.nitems, p->ff,
+                         p->b_global);
+    launch_interpolation(p->jobs, g.first, g.count, p->nx, p->ny, g.split ? g.max_nodes : 0, g.max_ny, p->dev, p->hkl,
+                         F, I, s);
+  }
   SPSIM_HIP_TRY(hipGetLastError());
   return SPSIM_HIP_OK;
 }
 
-int surf_tables(const SurfFit *fit, const SurfShape &sh, int nx, int ny, hipStream_t s) {
-  hipLaunchKernelGGL(surface_tables_kernel, dim3(256, 2), dim3(kT), 0, s, fit, sh, nx, ny);
-  SPSIM_HIP_TRY(hipGetLastError());
-  return SPSIM_HIP_OK;
-}
-
-int surf_run(const SurfRun &r, int cus, hipStream_t s) {
-  if (r.count <= 0) return SPSIM_HIP_OK;
-  const int blocks = std::min(r.nitems, resident_slots(nodes_kernel(r.has_b), cus));
-  if (r.has_b)
-    hipLaunchKernelGGL(surface_nodes_kernel<true>, dim3(blocks), dim3(kT), 0, s, r.jobs, r.items, r.nitems, r.ff,
-                       r.b_global);
-  else
-    hipLaunchKernelGGL(surface_nodes_kernel<false>, dim3(blocks), dim3(kT), 0, s, r.jobs, r.items, r.nitems, r.ff,
-                       r.b_global);
-  launch_interpolation(r.jobs, r.first, r.count, r.nx, r.ny, r.max_nodes, r.max_ny, r.dev, r.hkl, r.F, r.I, s);
-  SPSIM_HIP_TRY(hipGetLastError());
-  return SPSIM_HIP_OK;
+void surf_plan_destroy(SurfPlan *p) {
+  if (!p) return;
+  for (void *m : p->owned) (void)hipFree(m);
+  delete p;
 }
 
 }  // namespace spsim

@@ -2,7 +2,6 @@
 // detector surface (surface.hip): descriptions shared with the batched plans.
 #pragma once
 
-#include "common.hpp"
 #include "sf_kernels.hpp"
 
 namespace spsim {
@@ -86,12 +85,6 @@ struct SurfMol {
   int bad;
 };
 
-// Node counts of the pattern, and whether interpolating beats the direct sum.
-bool surf_choose(const SurfFit &fit, const SurfMol &mol, int nx, int ny, int natoms, SurfAxis *ax, SurfAxis *ay);
-// Fills b_smooth and weakest from a form-factor table and the species of a molecule.
-void surf_terms(const float *ff, const spsim_hip_segment *segs, int nsegs, float b_global, float bmin, float bmax,
-                float s2max, SurfMol *mol);
-
 // Host sizes only: is the pattern large enough to look at its list?
 bool surf_worth(long long nx, long long ny, long long natoms);
 
@@ -101,26 +94,21 @@ bool surf_worth(long long nx, long long ny, long long natoms);
 size_t surf_single_bytes(int nx, int ny, int natoms);
 int launch_surface(const PatternLaunch &a, int nx, int ny, int cus, void *ws, const int **ok_flag, hipStream_t s);
 
-// For plans: scan a list and nmol molecules into device memory, build a
-// shape's tables, and run a list of patterns.
-int surf_scan(const float *hkl, int nx, int ny, const spsim_hip_atom *atoms, const float *atom_b, const MolInfo *mols,
-              int nmol, SurfFit *fit, float *dev, SurfRecord *records, double *centres, hipStream_t s);
-int surf_tables(const SurfFit *fit, const SurfShape &sh, int nx, int ny, hipStream_t s);
-struct SurfRun {
-  const SurfJob *jobs;    // device
-  int first, count;       // jobs [first, first + count) of this run
-  const SurfItem *items;  // device, of this run
-  int nitems;
-  int max_nodes, max_ny;  // most nodes of these jobs
-  int nx, ny;
-  const float *dev;
-  const float *hkl;
-  const float *ff;
-  float b_global;
-  bool has_b;
-  float2 *F;
-  float *I;
-};
-int surf_run(const SurfRun &r, int cus, hipStream_t s);
+// ---- plans that decide on the host (batch.hip) ----
+
+struct SurfPlan;
+
+// Looks at a plan's list and molecules (all in device memory; pattern p shows
+// molecule pattern_mol[p] rotated by rot9 + 9 p) and prepares the patterns that
+// are smooth enough. *out is null when there is none. Synchronises.
+int surf_plan_create(const float *hkl, int nx, int ny, const spsim_hip_atom *atoms, const float *atom_b,
+                     const spsim_hip_segment *segs, const MolInfo *d_mols, const MolInfo *h_mols, int nmol,
+                     const spsim_hip_segment *h_segs, int npatterns, const int *pattern_mol, const double *rot9,
+                     const float *d_ff, const float *h_ff, float b_global, int cus, SurfPlan **out);
+// Whether the plan takes pattern p.
+bool surf_plan_takes(const SurfPlan *p, int pattern);
+// Writes the outputs of the patterns it takes.
+int surf_plan_run(const SurfPlan *p, float2 *F, float *I, hipStream_t s);
+void surf_plan_destroy(SurfPlan *p);
 
 }  // namespace spsim

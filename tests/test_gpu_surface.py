@@ -129,3 +129,66 @@ def test_interpolated_pattern_repeats_and_captures(gpu):
         torch.cuda.synchronize()
         assert torch.equal(I0, I1) and torch.equal(F0, F1)
         dv.structure_factor_grid(small, 128, 128, atoms, ff)
+
+
+@pytest.mark.parametrize("with_b", [False, True])
+def test_plan_mixes_interpolated_and_direct_patterns(gpu, with_b):
+    """A batched plan on a 96 x 80 detector: molecules that are interpolated,
+    one too wide for it (direct kernels) and an empty one, each at its own
+    rotation, against the FP64 oracle; graph replays bit for bit; and the same
+    plan with a tile asked for, which takes the direct kernels throughout."""
+    import ctypes as C
+
+    import torch
+
+    from spsim_amd import _lib
+    from tests.test_gpu_batch import make_plan
+
+    rng = np.random.default_rng(17)
+    nx, ny = 96, 80
+    q = _list(nx, ny, pixel=3e-4, cx=1e-3)
+    mols, Bs = [], []
+    for natoms, radius in ((900, 3e-9), (2500, 4e-9), (400, 2e-7), (0, 0.0)):
+        Z, pos, b = (wl.random_molecule(natoms, radius, rng, atom_b_range=(5.0, 40.0)) if natoms else
+                     (np.zeros(0, np.int32), np.zeros((0, 3), np.float32), np.zeros(0, np.float32)))
+        mols.append((Z, pos))
+        Bs.append(b)
+    pm = np.array([1, 2, 0, 3, 1, 0], np.int32)
+    rots = wl.uniform_rotations(len(pm), rng)
+    L = _lib.load()
+    plan, *_ = make_plan(mols, rots, pm, q, nx, ny, atom_b=np.concatenate(Bs) if with_b else None, b_global=3.0)
+    try:
+        stream = torch.cuda.Stream()
+        sp = C.c_void_p(stream.cuda_stream)
+        I = torch.full((len(pm), nx * ny), float("nan"), dtype=torch.float32, device=gpu)
+        F = torch.full((len(pm), nx * ny, 2), float("nan"), dtype=torch.float32, device=gpu)
+        torch.cuda.synchronize()
+        run = lambda g: _lib.check(L.spsim_hip_batch_run(plan, C.c_void_p(F.data_ptr()), C.c_void_p(I.data_ptr()), g,
+                                                         sp), "run")
+        run(0)
+        stream.synchronize()
+        first, Fh = I.cpu().numpy().copy(), F.cpu().numpy()
+        for p, m in enumerate(pm):
+            Z, pos = mols[m]
+            if not len(Z):
+                assert np.all(first[p] == 0) and np.all(Fh[p] == 0)
+                continue
+            Fr, Ir = oracle.sf_f64(q, Z, pos, atom_b=Bs[m] if with_b else None, B=3.0, R=rots[p],
+                                   threads=oracle_threads())
+            assert rel_l2(first[p], Ir) < TOL, p
+            assert np.linalg.norm(Fh[p, :, 0] + 1j * Fh[p, :, 1] - Fr) / np.linalg.norm(Fr) < TOL, p
+        for _ in range(3):
+            I.fill_(float("nan"))
+            torch.cuda.synchronize()
+            run(1)
+            stream.synchronize()
+            assert np.array_equal(I.cpu().numpy(), first)
+        _lib.check(L.spsim_hip_batch_set_tile(plan, C.byref(dv.make_tile(1, 256, 0))), "set_tile")
+        run(0)
+        stream.synchronize()
+        direct = I.cpu().numpy()
+        same = [np.array_equal(direct[p], first[p]) for p in range(len(pm))]
+        assert same == [False, True, False, True, False, False]
+        assert rel_l2(direct, first) < 2 * TOL
+    finally:
+        L.spsim_hip_batch_destroy(plan)
