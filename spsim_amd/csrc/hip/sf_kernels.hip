@@ -189,7 +189,6 @@ __device__ __forceinline__ void spectrum_sum(const double (&qx)[K], const double
     Fr[k] = 0.0;
     Fi[k] = 0.0;
   }
-  const int ns = sp.n;
   for (int sg = 0; sg < nsegs; ++sg) {
     const int s_start = segs[sg].start;
     const int s_end = s_start + segs[sg].count;
@@ -216,31 +215,8 @@ __device__ __forceinline__ void spectrum_sum(const double (&qx)[K], const double
 #pragma unroll
         for (int k = 0; k < K; ++k) {
           const double t = __builtin_fma(qz[k], a.z, __builtin_fma(qy[k], a.y, qx[k] * a.x));
-          const double tc = sp.sc * t;
-          const float tf = (float)tc;
-          float ur = 0.0f, ui = 0.0f;
-          if (__builtin_fabsf(tf) <= sp.tlim) {
-            const float ph = (float)__builtin_amdgcn_fract(tc);
-            const float cs = __builtin_amdgcn_cosf(ph);
-            const float sn = __builtin_amdgcn_sinf(ph);
-            const float v = tf * sp.inv_tlim;
-            const float u = v * v;
-            float gc = sp.p[kSpectrumDegree], gq = sp.q[kSpectrumDegree];
-#pragma unroll
-            for (int d = kSpectrumDegree - 1; d >= 0; --d) {
-              gc = __builtin_fmaf(gc, u, sp.p[d]);
-              gq = __builtin_fmaf(gq, u, sp.q[d]);
-            }
-            const float gs = v * gq;
-            ur = __builtin_fmaf(cs, gc, -sn * gs);
-            ui = __builtin_fmaf(sn, gc, cs * gs);
-          } else {
-            for (int m = 0; m < ns; ++m) {
-              const float ph = (float)__builtin_amdgcn_fract(sp.s[m] * t);
-              ur = __builtin_fmaf(sp.w[m], __builtin_amdgcn_cosf(ph), ur);
-              ui = __builtin_fmaf(sp.w[m], __builtin_amdgcn_sinf(ph), ui);
-            }
-          }
+          float ur, ui;
+          spectrum_term(sp, t, ur, ui);
           float wt;
           if constexpr (HAS_B) {
             wt = __builtin_amdgcn_exp2f(__builtin_fmaf(a.b, nl2[k], a.w));
@@ -971,22 +947,24 @@ PatternLaunch make_launch(const float *d_hkl, int npix, const spsim_hip_atom *d_
 // decides on the device, without a host round trip), and by the direct kernel
 // `kind` otherwise, which is launched behind it and finds the outputs written.
 // Both use the library workspace, the direct sums' partials past the flag.
+// The interpolation's eight launches take about 60 us, the direct sums that from
+// about min_terms on.
 int launch_smooth(Kind kind, const PatternLaunch &a, int nx, int ny, const spsim_hip_tile &t, int splits, int cus,
-                  hipStream_t s) {
-  if (!surf_worth(nx, ny, a.natoms)) return launch_single(kind, a, nx, ny, t, splits, s);
+                  long long min_terms, const Spectrum *spec, hipStream_t s) {
+  if (!surf_worth(nx, ny, a.natoms, min_terms)) return launch_single(kind, a, nx, ny, t, splits, s, spec);
   constexpr size_t kFlag = (sizeof(SurfJob) + 255) / 256 * 256;
   const size_t bytes = std::max(surf_single_bytes(nx, ny, a.natoms), kFlag + sizeof(double2) * (size_t)splits * a.npix);
   if (!workspace_holds(bytes)) {
     // A capture cannot grow the workspace: it takes the direct kernel, as long as that one's partials fit.
     hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(s, &st) != hipSuccess || st != hipStreamCaptureStatusNone)
-      return launch_single(kind, a, nx, ny, t, splits, s);
+      return launch_single(kind, a, nx, ny, t, splits, s, spec);
   }
   void *ws = nullptr;
   SPSIM_TRY(workspace(bytes, &ws));
   PatternLaunch direct = a;
-  SPSIM_TRY(launch_surface(a, nx, ny, cus, ws, &direct.skip, s));
-  return launch_single(kind, direct, nx, ny, t, splits, s, nullptr, (double2 *)((char *)ws + kFlag));
+  SPSIM_TRY(launch_surface(a, nx, ny, spec, cus, ws, &direct.skip, s));
+  return launch_single(kind, direct, nx, ny, t, splits, s, spec, (double2 *)((char *)ws + kFlag));
 }
 
 }  // namespace
@@ -1189,6 +1167,12 @@ extern "C" int spsim_hip_sf_pattern(const float *d_hkl, int npix, const spsim_hi
                                        (int)std::min<size_t>(64, kWorkspacePartials / (size_t)npix));
   const PatternLaunch a =
       make_launch(d_hkl, npix, d_atoms, d_atom_b, d_segs, nsegs, natoms, d_ff, b_global, rot9, d_F, d_I);
+  // A flat list carries no shape. One of n^2 vectors is taken for an n x n
+  // detector where that can pay; the device's check catches a wrong guess, which
+  // costs its launches (40 us of 250 us and more).
+  const int side = (int)std::lround(std::sqrt((double)npix));
+  if (!tile && (long long)side * side == npix)
+    return launch_smooth(Kind::kPattern, a, side, side, t, splits, cus, 500000000LL, nullptr, (hipStream_t)stream);
   return launch_pattern(a, t, splits, (hipStream_t)stream);
 }
 
@@ -1272,7 +1256,8 @@ extern "C" int spsim_hip_sf_grid(const float *d_hkl, int nx, int ny, const spsim
   SPSIM_TRY(ensure_device(&cus));
   const PatternLaunch a =
       make_launch(d_hkl, npix, d_atoms, d_atom_b, d_segs, nsegs, natoms, d_ff, b_global, rot9, d_F, d_I);
-  if (!tile) return launch_smooth(Kind::kGrid, a, nx, ny, t, splits, cus, (hipStream_t)stream);
+  if (!tile)
+    return launch_smooth(Kind::kGrid, a, nx, ny, t, splits, cus, 200000000LL, nullptr, (hipStream_t)stream);
   return launch_grid(a, nx, ny, t, splits, (hipStream_t)stream);
 }
 
@@ -1339,5 +1324,8 @@ extern "C" int spsim_hip_sf_spectrum(const float *d_hkl, int npix, const spsim_h
                                        (int)std::min<size_t>(64, kWorkspacePartials / (size_t)npix));
   const PatternLaunch a =
       make_launch(d_hkl, npix, d_atoms, d_atom_b, d_segs, nsegs, natoms, d_ff, b_global, rot9, d_F, d_I);
+  const int side = (int)std::lround(std::sqrt((double)npix));  // as in spsim_hip_sf_pattern
+  if (!tile && (long long)side * side == npix)
+    return launch_smooth(Kind::kSpectrum, a, side, side, t, splits, cus, 200000000LL, &sp, (hipStream_t)stream);
   return launch_spectrum(a, sp, t, splits, (hipStream_t)stream);
 }

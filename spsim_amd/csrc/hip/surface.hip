@@ -45,9 +45,11 @@ namespace {
 
 constexpr int kT = 256;
 constexpr int D = kSurfDeg;
+constexpr int kLines = kSurfLines;
 constexpr double kPi = 3.14159265358979323846;
 constexpr float kStretch = 20.7f;       // -ln of the node map's own error
 constexpr double kMaxPhaseDev = 2e-4;   // largest 2 pi R |q - surface|
+constexpr double kMaxSpreadDev = 3e-7;  // the same times the spectrum's largest |s_k / sc - 1|
 constexpr float kMinWeakest = 0.02f;    // see surf_terms
 constexpr float kMaxGauss = 60.0f;      // largest exponent B s^2 over the detector
 
@@ -151,11 +153,12 @@ __device__ __forceinline__ void surface_row(const double (*coef)[D][3], double v
 struct ScanArgs {
   const float *hkl;
   int nx, ny;
-  int list_blocks;
+  int list_blocks;  // the last two measure the slopes
   const spsim_hip_atom *atoms;
   const float *atom_b;
   const MolInfo *mols;  // null: one molecule of natoms atoms
   int natoms;
+  bool centre;  // false: the molecules' centres are the origin
   SurfFit *fit;
   float *dev;
   SurfRecord *records;  // [list_blocks + nmol * kSurfAtomBlocks]
@@ -177,6 +180,9 @@ __device__ void scan_list(const ScanArgs &a) {
     const size_t p = (size_t)px[1][b] * a.nx + px[0][i];
     for (int k = 0; k < 3; ++k) Q[b][i][k] = a.hkl[3 * p + k];
   }
+  // s^2 of the sample pixels, corners among them
+  double s2[1] = {(Q[b][i][0] * Q[b][i][0] + Q[b][i][1] * Q[b][i][1] + Q[b][i][2] * Q[b][i][2]) * 2.5e-21};
+  if ((int)blockIdx.x == a.list_blocks - 2) block_reduce(s2);
   sample_to_chebyshev(us[0], cosines, C[0], tmp);
   sample_to_chebyshev(us[1], cosines, C[1], tmp);
   // along x: P[b][m], then along y in place of Q
@@ -194,13 +200,15 @@ __device__ void scan_list(const ScanArgs &a) {
     Q[b][i][k] = s;
   }
   __syncthreads();
-  if (blockIdx.x == 0) {
-    // slopes |dq/du|, |dq/dv| and s^2 on the 16 x 16 Lobatto points: T_m and
-    // m U_{m-1} at the points, then the rows' sums, then the points'
-    double(*T)[D] = C[0], (*U)[D] = C[1];  // [m][point]
-    __shared__ double R[D][D][6];          // [n][point of u]: q, dq/du along row n
-    if (t < D) {
-      const double u = cospi((double)t / (D - 1));
+  const int rows = a.list_blocks - 2;  // workgroups that take the list's rows
+  if ((int)blockIdx.x >= rows) {
+    // slopes along one axis on the kLines x kLines Lobatto points: T_m and
+    // m U_{m-1} at the points, then dq/du of every row of coefficients, then the points'
+    const bool along_y = (int)blockIdx.x == rows + 1;
+    __shared__ double T[D][kLines], U[D][kLines], R[D][kLines][3];
+    __shared__ unsigned smax[kLines];
+    if (t < kLines) {
+      const double u = cospi((double)t / (kLines - 1));
       double t0 = 1.0, t1 = u, u0 = 0.0, u1 = 1.0;
       for (int m = 0; m < D; ++m) {
         T[m][t] = t0;
@@ -211,48 +219,38 @@ __device__ void scan_list(const ScanArgs &a) {
         u0 = u1;
         u1 = un;
       }
+      smax[t] = 0u;
     }
     __syncthreads();
-    for (int k = 0; k < 3; ++k) {
-      double r = 0.0, rd = 0.0;
-      for (int m = 0; m < D; ++m) {
-        r = __builtin_fma(T[m][i], Q[b][m][k], r);
-        rd = __builtin_fma(U[m][i], Q[b][m][k], rd);
-      }
-      R[b][i][k] = r;
-      R[b][i][3 + k] = rd;
+    for (int c = t; c < D * kLines; c += kT) {
+      const int n = c / kLines, j = c % kLines;
+      double r[3] = {0, 0, 0};
+#pragma unroll
+      for (int m = 0; m < D; ++m)
+        for (int k = 0; k < 3; ++k) r[k] = __builtin_fma(U[m][j], along_y ? Q[m][n][k] : Q[n][m][k], r[k]);
+      for (int k = 0; k < 3; ++k) R[n][j][k] = r[k];
     }
     __syncthreads();
-    double du = 0.0, dv = 0.0, s2[1] = {0.0};
-    for (int k = 0; k < 3; ++k) {
-      double q = 0.0, qu = 0.0, qv = 0.0;
-      for (int n = 0; n < D; ++n) {
-        q = __builtin_fma(T[n][b], R[n][i][k], q);
-        qu = __builtin_fma(T[n][b], R[n][i][3 + k], qu);
-        qv = __builtin_fma(U[n][b], R[n][i][k], qv);
-      }
-      s2[0] += q * q * 2.5e-21;
-      du += qu * qu;
-      dv += qv * qv;
+    for (int c = t; c < kLines * kLines; c += kT) {
+      const int across = c / kLines, line = c % kLines;
+      double d[3] = {0, 0, 0};
+#pragma unroll
+      for (int n = 0; n < D; ++n)
+        for (int k = 0; k < 3; ++k) d[k] = __builtin_fma(T[n][across], R[n][line][k], d[k]);
+      // non-negative floats order as their bits
+      atomicMax(&smax[line], __float_as_uint((float)sqrt(d[0] * d[0] + d[1] * d[1] + d[2] * d[2])));
     }
-    block_reduce(s2);
-    tmp[b][i] = du;
-    P[b][i][0] = dv;
     __syncthreads();
-    if (t < D) {
-      double sx = 0.0, sy = 0.0;
-      for (int c = 0; c < D; ++c) {
-        sx = fmax(sx, tmp[c][t]);
-        sy = fmax(sy, P[t][c][0]);
-      }
-      a.fit->slope_x[t] = (float)sqrt(sx);
-      a.fit->slope_y[t] = (float)sqrt(sy);
+    if (t < kLines) (along_y ? a.fit->slope_y : a.fit->slope_x)[t] = __uint_as_float(smax[t]);
+    if (t == 0) a.records[blockIdx.x] = SurfRecord{{0, 0, 0}, 0.0, 0.0f, 0.0f, 0, 0};
+    if (!along_y) {
+      if (t == 0) a.fit->s2max = (float)s2[0];
+      for (int c = t; c < D * D * 3; c += kT) (&a.fit->coef[0][0][0])[c] = (&Q[0][0][0])[c];
     }
-    if (t == 0) a.fit->s2max = (float)s2[0];
-    for (int c = t; c < D * D * 3; c += kT) (&a.fit->coef[0][0][0])[c] = (&Q[0][0][0])[c];
+    return;
   }
   double m[4] = {0, 0, 0, 0};
-  for (int y = blockIdx.x; y < a.ny; y += a.list_blocks) {
+  for (int y = blockIdx.x; y < a.ny; y += rows) {
     __syncthreads();
     surface_row(Q, pixel_u(y, a.ny), row);
     __syncthreads();
@@ -283,7 +281,7 @@ __device__ void scan_atoms(const ScanArgs &a) {
   const int n = a.mols ? a.mols[mol].atom_end - begin : a.natoms;
   const spsim_hip_atom *atoms = a.atoms + begin;
   double c[3] = {0, 0, 0};
-  if (n > 0)
+  if (n > 0 && a.centre)
     for (int i = 0; i < 4; ++i) {
       const spsim_hip_atom at = atoms[(int)((long long)(4 * t + i) * n / (4 * kT))];
       c[0] += at.x;
@@ -327,39 +325,36 @@ __global__ __launch_bounds__(kT) void surface_scan_kernel(ScanArgs a) {
 // slopes need at that stretch. 2 % are added to the slopes for their sampling.
 __host__ __device__ inline float axis_stretch(int n) { return 1.0f / coshf(kStretch / n); }
 
-__host__ __device__ inline float fast_sin(float x) {
-#ifdef __HIP_DEVICE_COMPILE__
-  return __sinf(x);
-#else
-  return std::sin(x);
-#endif
-}
-__host__ __device__ inline float fast_cos(float x) {
-#ifdef __HIP_DEVICE_COMPILE__
-  return __cosf(x);
-#else
-  return std::cos(x);
-#endif
-}
-
 __host__ __device__ inline float axis_need(const float *slope, float radius, float gauss, float a) {
   const float as = asinf(a);
   float w = 0.0f;
-  for (int k = 0; k < D; ++k) {
-    // lines mirrored about the middle share their stretch
-    const float u = fabsf(fast_cos((float)kPi * k / (D - 1)));
-    const float s = fminf(1.0f, fast_sin(u * as) / a), c = fast_cos(u * as);
-    w = fmaxf(w, slope[k] * sqrtf(fmaxf(0.0f, 1.0f - s * s)) * a / (as * fmaxf(c, 1e-6f)));
+  for (int k = 0; k < kLines; ++k) {
+    // On the line u = cos(pi k / (kLines - 1)), x = u asin(a): s = sin(x) / a,
+    // |du/dt| = sqrt(1 - s^2) a / (asin(a) cos(x)). Lines mirrored about the
+    // middle share them.
+#ifdef __HIP_DEVICE_COMPILE__
+    const float x = fabsf(__builtin_amdgcn_cosf(0.5f * k / (kLines - 1))) * as;
+    const float sx = __builtin_amdgcn_sinf(x * (float)(0.5 / kPi)), cx = __builtin_amdgcn_cosf(x * (float)(0.5 / kPi));
+    const float g = __builtin_amdgcn_sqrtf(fmaxf(0.0f, a * a - sx * sx)) * __builtin_amdgcn_rcpf(fmaxf(cx, 1e-6f));
+#else
+    const float x = std::fabs(std::cos((float)kPi * k / (kLines - 1))) * as;
+    const float sx = std::sin(x), cx = std::cos(x);
+    const float g = std::sqrt(std::max(0.0f, a * a - sx * sx)) / std::max(cx, 1e-6f);
+#endif
+    w = fmaxf(w, slope[k] * g);
   }
-  const float theta = 1.02f * 2.0f * (float)kPi * radius * w;
+  const float theta = 1.02f * 2.0f * (float)kPi * radius * w / as;
   return theta + 4.0f * cbrtf(theta) + 8.0f + 2.0f * sqrtf(fmaxf(gauss, 0.0f));
 }
 
-__host__ __device__ inline bool worth(double nodes_x, double nodes_y, double nx, double ny, double natoms) {
-  // Issue cycles per lane: a term of the node sums 62, of the direct sums 26
-  // to 40; the interpolation 25 per node row and pixel. Measured on the MI355X.
-  const double surf = nodes_x * nodes_y * natoms * 62.0 + 25.0 * (nx * ny * nodes_y + nx * nodes_x * nodes_y);
-  return surf < 0.8 * 26.0 * nx * ny * natoms;
+__host__ __device__ inline bool worth(double nodes_x, double nodes_y, double nx, double ny, double natoms,
+                                      bool spectrum) {
+  // Issue cycles per lane: a term of the node sums 80 (160 with a spectrum), of
+  // the direct sums 26 to 45 (130); the interpolation 25 per node row and pixel.
+  // Measured on the MI355X.
+  const double surf = nodes_x * nodes_y * natoms * (spectrum ? 160.0 : 80.0) +
+                      25.0 * (nx * ny * nodes_y + nx * nodes_x * nodes_y);
+  return surf < 0.8 * (spectrum ? 130.0 : 26.0) * nx * ny * natoms;
 }
 
 __host__ __device__ inline bool smooth(const SurfMol &m, float s2max) {
@@ -431,19 +426,20 @@ __device__ __forceinline__ void prepare_atoms(const SurfJob &jb, bool has_b, int
 }
 
 // Nodes per lane of the node sums: four share an atom's LDS read (2.27 ms
-// against 2.42 ms on 35,344 nodes x 100,000 atoms), two make twice the work
-// items (17.6 us against 24 us on 1024 nodes x 5,000 atoms).
+// against 2.42 ms for two on 35,344 nodes x 100,000 atoms); fewer make more work
+// items (two: 17.6 us against 24 us on 1024 nodes x 5,000 atoms).
 __host__ __device__ inline int surf_per_lane(long long nodes, long long natoms) {
-  return nodes * natoms >= 1LL << 28 ? 4 : 2;
+  const long long terms = nodes * natoms;
+  return terms >= 1LL << 28 ? 4 : (terms >= 1LL << 25 ? 2 : 1);
 }
 
 // Time of the node sums in atoms per lane with s atom ranges per tile: rounds
 // of `slots` resident workgroups, each of an atom range and a fixed part (the
 // form factors and the loop's start, about 40 atoms), and the ranges' partial
-// sums, which cost about one atom each.
+// sums, which cost about half an atom each.
 __host__ __device__ inline float splits_cost(int s, int tiles, int natoms, int slots) {
   const int rounds = (tiles * s + slots - 1) / slots;
-  return rounds * ((float)natoms / s + 40.0f) + (s > 1 ? 1.5f * s + 40.0f : 0.0f);
+  return rounds * ((float)natoms / s + 40.0f) + (s > 1 ? 0.5f * s + 40.0f : 0.0f);
 }
 
 struct PlanArgs {
@@ -458,6 +454,8 @@ struct PlanArgs {
   int slots;       // resident workgroups of the node sums
   int slot_cap;    // partial slots that fit
   int max_nx, max_ny;  // nodes that fit the workspace
+  bool spectrum;
+  double scale, spread;  // of a spectrum: largest s_k, largest |s_k / sc - 1|
   SurfJob *out;
 };
 
@@ -564,7 +562,7 @@ __global__ __launch_bounds__(kT) void surface_plan_kernel(PlanArgs a) {
   double e[2] = {(double)bs, -(double)weak};
   block_reduce(e);
   if (t == 0) {
-    mol.radius = sqrt(m[3]);
+    mol.radius = sqrt(m[3]) * a.scale;
     mol.dev = sqrt(m[0] * m[0] + m[1] * m[1] + m[2] * m[2]);
     mol.b_smooth = (float)e[0];
     mol.weakest = (float)-e[1];
@@ -581,8 +579,10 @@ __global__ __launch_bounds__(kT) void surface_plan_kernel(PlanArgs a) {
   }
   __syncthreads();
   const int nx = best[0], ny = best[1];
-  const bool ok = smooth(mol, a.fit->s2max) && nx <= a.max_nx && ny <= a.max_ny &&
-                  worth(nx, ny, a.job.nx, a.job.ny, a.job.natoms);
+  // G is taken at the spectrum's centre scale, so it is off by the spread
+  const bool ok = smooth(mol, a.fit->s2max) && 2.0 * kPi * mol.radius * mol.dev * a.spread <= kMaxSpreadDev &&
+                  nx <= a.max_nx && ny <= a.max_ny &&
+                  worth(nx, ny, a.job.nx, a.job.ny, a.job.natoms, a.spectrum);
   if (!ok) {
     if (blockIdx.x == 0 && blockIdx.y == 0 && t == 0) a.out->ok = 0;
     return;
@@ -637,7 +637,7 @@ __global__ __launch_bounds__(kT) void surface_tables_kernel(const SurfFit *fit, 
 
 // ---- 3. node sums ---------------------------------------------------------------
 //
-// One work item: two or four nodes per lane x one atom range, whose records are
+// One work item: one, two or four nodes per lane x one atom range, whose records are
 // staged in LDS 256 at a time; every lane reads the same record, and its terms
 // share the read (surf_per_lane). Per node and atom: 3 FP64 FMAs, a fraction and a
 // conversion, a sine and cosine, 8 FP32 FMAs (F and the three components of G):
@@ -663,10 +663,23 @@ __device__ __forceinline__ double form_factor64(const float *__restrict__ c, dou
   return f;
 }
 
-template <int K, bool HAS_B>
+// The spectrum travels in the kernel's arguments only where there is one.
+struct NoSpectrum {};
+template <bool SPEC>
+struct SpectrumArg {
+  using type = NoSpectrum;
+};
+template <>
+struct SpectrumArg<true> {
+  using type = Spectrum;
+};
+
+// SPEC: a wavelength spectrum, the sample sum in place of the sine and cosine
+// (spectrum_term), and the gradient at the centre scale.
+template <int K, bool HAS_B, bool SPEC>
 __device__ __forceinline__ void node_item(const SurfJob &jb, int tile, int split, const float *__restrict__ ff,
-                                          float b_global, NodeAtom *sm) {
-  constexpr int kTile = K * kT;
+                                          float b_global, const typename SpectrumArg<SPEC>::type &sp, NodeAtom *sm) {
+  constexpr int kTile = K * kT, kUnroll = K == 1 ? 4 : (K == 2 ? 2 : 1);
   const int nodes = jb.sh.ax.n * jb.sh.ay.n;
   const int a_begin = (int)((long long)jb.natoms * split / jb.splits);
   const int a_end = (int)((long long)jb.natoms * (split + 1) / jb.splits);
@@ -706,13 +719,20 @@ __device__ __forceinline__ void node_item(const SurfJob &jb, int tile, int split
         for (int k = 0; k < K; ++k)
 #pragma unroll
           for (int i = 0; i < 4; ++i) c[k][i] = s[k][i] = 0.0f;
+#pragma unroll kUnroll
         for (int j = j0; j < j1; ++j) {
           const NodeAtom at = sm[j];
 #pragma unroll
           for (int k = 0; k < K; ++k) {
             const double t = __builtin_fma(qz[k], at.z, __builtin_fma(qy[k], at.y, qx[k] * at.x));
-            const float ph = (float)__builtin_amdgcn_fract(t);
-            float cs = __builtin_amdgcn_cosf(ph), sn = __builtin_amdgcn_sinf(ph);
+            float cs, sn;
+            if constexpr (SPEC) {
+              spectrum_term(sp, t, cs, sn);
+            } else {
+              const float ph = (float)__builtin_amdgcn_fract(t);
+              cs = __builtin_amdgcn_cosf(ph);
+              sn = __builtin_amdgcn_sinf(ph);
+            }
             if constexpr (HAS_B) {
               const float w = __builtin_amdgcn_exp2f(__builtin_fmaf(at.v[4], nl2[k], at.v[0]));
               cs *= w;
@@ -747,6 +767,11 @@ __device__ __forceinline__ void node_item(const SurfJob &jb, int tile, int split
 #pragma unroll
   for (int k = 0; k < K; ++k) {
     const int l = k * kT + threadIdx.x, node = tile * kTile + l;
+    if constexpr (SPEC)
+      for (int i = 0; i < 3; ++i) {
+        gc[k][i] *= (float)sp.sc;
+        gs[k][i] *= (float)sp.sc;
+      }
     if (jb.splits > 1) {
       ((NodeSlot *)jb.slots)[((size_t)tile * jb.splits + split) * kTile + l] =
           NodeSlot{Fc[k], Fs[k], {gs[k][0], gc[k][0], gs[k][1], gc[k][1], gs[k][2], gc[k][2], 0.0f, 0.0f}};
@@ -761,9 +786,10 @@ __device__ __forceinline__ void node_item(const SurfJob &jb, int tile, int split
   }
 }
 
-template <bool HAS_B>
+template <bool HAS_B, bool SPEC>
 __global__ __launch_bounds__(kT) void surface_nodes_kernel(const SurfJob *jobs, const SurfItem *items, int nitems,
-                                                           const float *__restrict__ ff, float b_global) {
+                                                           const float *__restrict__ ff, float b_global,
+                                                           typename SpectrumArg<SPEC>::type sp) {
   __shared__ NodeAtom sm[kNodeChunk];
   if (!items) {  // one pattern: every (tile, range) of job 0
     if (!jobs->ok) return;
@@ -773,14 +799,16 @@ __global__ __launch_bounds__(kT) void surface_nodes_kernel(const SurfJob *jobs, 
     const SurfItem m = items ? items[it] : SurfItem{0, it % jobs->tiles, it / jobs->tiles, 0};
     const SurfJob &jb = jobs[m.job];
     if (jb.per_lane == 4)
-      node_item<4, HAS_B>(jb, m.tile, m.split, ff, b_global, sm);
+      node_item<4, HAS_B, SPEC>(jb, m.tile, m.split, ff, b_global, sp, sm);
+    else if (jb.per_lane == 2)
+      node_item<2, HAS_B, SPEC>(jb, m.tile, m.split, ff, b_global, sp, sm);
     else
-      node_item<2, HAS_B>(jb, m.tile, m.split, ff, b_global, sm);
+      node_item<1, HAS_B, SPEC>(jb, m.tile, m.split, ff, b_global, sp, sm);
   }
 }
 
 // Adds the atom ranges of every node: one lane per third of a node's slot, so
-// that a wave reads contiguous 16-byte parts and keeps 8 ranges in flight.
+// that a wave reads contiguous 16-byte parts and keeps 16 ranges in flight.
 __global__ __launch_bounds__(kT) void surface_reduce_kernel(const SurfJob *jobs, int first) {
   const SurfJob &jb = jobs[first + blockIdx.z];
   if (!jb.ok || jb.splits == 1) return;
@@ -792,7 +820,7 @@ __global__ __launch_bounds__(kT) void surface_reduce_kernel(const SurfJob *jobs,
   const size_t step = sizeof(NodeSlot) * size;
   if (part == 0) {
     double c = 0.0, s = 0.0;
-#pragma unroll 8
+#pragma unroll 16
     for (int i = 0; i < splits; ++i) {
       const double2 v = *(const double2 *)(slot + i * step);
       c += v.x;
@@ -801,7 +829,7 @@ __global__ __launch_bounds__(kT) void surface_reduce_kernel(const SurfJob *jobs,
     jb.f[node] = make_double2(c, -s);
   } else {
     float4 a = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-#pragma unroll 8
+#pragma unroll 16
     for (int i = 0; i < splits; ++i) {
       const float4 v = *(const float4 *)(slot + i * step);
       a.x += v.x;
@@ -1014,25 +1042,35 @@ void launch_interpolation(const SurfJob *jobs, int first, int count, int nx, int
                        dev, hkl, F, I);
 }
 
-const void *nodes_kernel(bool has_b) {
-  return has_b ? (const void *)&surface_nodes_kernel<true> : (const void *)&surface_nodes_kernel<false>;
+const void *nodes_kernel(bool has_b, bool spec) {
+  if (spec)
+    return has_b ? (const void *)&surface_nodes_kernel<true, true> : (const void *)&surface_nodes_kernel<false, true>;
+  return has_b ? (const void *)&surface_nodes_kernel<true, false> : (const void *)&surface_nodes_kernel<false, false>;
+}
+
+int launch_nodes(const SurfJob *jobs, const SurfItem *items, int nitems, int blocks, const float *ff, float b_global,
+                 bool has_b, const Spectrum *sp, hipStream_t s) {
+  NoSpectrum none;
+  void *params[] = {(void *)&jobs, (void *)&items,    (void *)&nitems,
+                    (void *)&ff,   (void *)&b_global, sp ? (void *)sp : (void *)&none};
+  SPSIM_HIP_TRY(hipLaunchKernel(nodes_kernel(has_b, sp != nullptr), dim3(blocks), dim3(kT), params, 0, s));
+  return SPSIM_HIP_OK;
 }
 
 }  // namespace
 
-bool surf_worth(long long nx, long long ny, long long natoms) {
-  // Below 2e8 terms the direct sum takes less than the interpolation's six
-  // launches (about 40 us).
-  return nx >= kSurfMinSide && ny >= kSurfMinSide && nx * ny * natoms >= 200000000LL;
+bool surf_worth(long long nx, long long ny, long long natoms, long long min_terms) {
+  return nx >= kSurfMinSide && ny >= kSurfMinSide && nx * ny * natoms >= min_terms;
 }
 
 size_t surf_single_bytes(int nx, int ny, int natoms) { return single_layout(nx, ny, natoms).total; }
 
-int launch_surface(const PatternLaunch &a, int nx, int ny, int cus, void *ws, const int **ok_flag, hipStream_t s) {
+int launch_surface(const PatternLaunch &a, int nx, int ny, const Spectrum *sp, int cus, void *ws, const int **ok_flag,
+                   hipStream_t s) {
   const SingleLayout l = single_layout(nx, ny, a.natoms);
   char *w = (char *)ws;
   const bool has_b = a.atom_b != nullptr;
-  const int slots = resident_slots(nodes_kernel(has_b), cus);
+  const int slots = resident_slots(nodes_kernel(has_b, sp != nullptr), cus);
   PlanArgs p{};
   p.job.nx = nx;
   p.job.ny = ny;
@@ -1054,7 +1092,7 @@ int launch_surface(const PatternLaunch &a, int nx, int ny, int cus, void *ws, co
   p.job.t32 = (float *)(w + l.t32);
   p.fit = (const SurfFit *)(w + l.fit);
   p.records = (const SurfRecord *)(w + l.records);
-  p.list_blocks = std::min(kSurfListBlocks, ny);
+  p.list_blocks = std::min(kSurfListBlocks, ny + 2);
   p.centres = (const double *)(w + l.centres);
   p.ff = a.ff;
   p.b_global = a.b_global;
@@ -1063,18 +1101,22 @@ int launch_surface(const PatternLaunch &a, int nx, int ny, int cus, void *ws, co
   p.slot_cap = l.slot_cap;
   p.max_nx = l.max_nx;
   p.max_ny = l.max_ny;
+  p.spectrum = sp != nullptr;
+  p.scale = 1.0;
+  if (sp) {
+    p.scale = 0.0;
+    for (int k = 0; k < sp->n; ++k) {
+      p.scale = std::max(p.scale, std::fabs(sp->s[k]));
+      p.spread = std::max(p.spread, std::fabs(sp->s[k] / sp->sc - 1.0));
+    }
+  }
   p.out = (SurfJob *)(w + l.job);
   const SurfJob *job = p.out;
-  ScanArgs sc{a.hkl,    nx, ny, p.list_blocks, a.atoms, a.atom_b, nullptr, a.natoms, (SurfFit *)(w + l.fit),
+  ScanArgs sc{a.hkl,    nx, ny, p.list_blocks, a.atoms, a.atom_b, nullptr, a.natoms, !sp, (SurfFit *)(w + l.fit),
               (float *)(w + l.dev), (SurfRecord *)(w + l.records), (double *)(w + l.centres)};
   hipLaunchKernelGGL(surface_scan_kernel, dim3(p.list_blocks + kSurfAtomBlocks), dim3(kT), 0, s, sc);
   hipLaunchKernelGGL(surface_plan_kernel, dim3(std::max(1, 2 * cus / 3), 3), dim3(kT), 0, s, p);
-  if (has_b)
-    hipLaunchKernelGGL(surface_nodes_kernel<true>, dim3(slots), dim3(kT), 0, s, job, (const SurfItem *)nullptr, 0,
-                       a.ff, a.b_global);
-  else
-    hipLaunchKernelGGL(surface_nodes_kernel<false>, dim3(slots), dim3(kT), 0, s, job, (const SurfItem *)nullptr, 0,
-                       a.ff, a.b_global);
+  SPSIM_TRY(launch_nodes(job, nullptr, 0, slots, a.ff, a.b_global, has_b, sp, s));
   launch_interpolation(job, 0, 1, nx, ny, l.max_nx * l.max_ny, l.max_ny, (const float *)(w + l.dev), a.hkl, a.F, a.I, s);
   SPSIM_HIP_TRY(hipGetLastError());
   *ok_flag = &job->ok;
@@ -1123,7 +1165,7 @@ bool choose(const SurfFit &fit, const SurfMol &mol, int nx, int ny, int natoms, 
     *out[k] = SurfAxis{n, axis_stretch(n), 0.0};
     out[k]->asin_a = std::asin(out[k]->a);
   }
-  return worth(ax->n, ay->n, nx, ny, natoms);
+  return worth(ax->n, ay->n, nx, ny, natoms, false);
 }
 
 // Lays the job's buffers out in a workspace from `at` on; returns the end.
@@ -1182,7 +1224,7 @@ int own(SurfPlan *p, T **out, size_t n) {
 int build_plan(SurfPlan *p, const spsim_hip_atom *atoms, const float *atom_b, const spsim_hip_segment *segs,
                const MolInfo *d_mols, const MolInfo *h_mols, int nmol, const spsim_hip_segment *h_segs, int npatterns,
                const int *pattern_mol, const double *rot9, const float *h_ff) {
-  const int lb = std::min(kSurfListBlocks, p->ny);
+  const int lb = std::min(kSurfListBlocks, p->ny + 2);
   SurfFit *d_fit = nullptr;
   float *dev = nullptr;
   SPSIM_TRY(own(p, &d_fit, 1));
@@ -1199,7 +1241,7 @@ int build_plan(SurfPlan *p, const spsim_hip_atom *atoms, const float *atom_b, co
     if (rc == SPSIM_HIP_OK) rc = own(&scratch, &d_centres, centres.size());
     hipError_t e = hipSuccess;
     if (rc == SPSIM_HIP_OK) {
-      const ScanArgs sc{p->hkl, p->nx, p->ny, lb, atoms, atom_b, d_mols, 0, d_fit, dev, d_rec, d_centres};
+      const ScanArgs sc{p->hkl, p->nx, p->ny, lb, atoms, atom_b, d_mols, 0, true, d_fit, dev, d_rec, d_centres};
       hipLaunchKernelGGL(surface_scan_kernel, dim3(lb + nmol * kSurfAtomBlocks), dim3(kT), 0, nullptr, sc);
       e = hipGetLastError();
       if (e == hipSuccess) e = hipMemcpy(&fit, d_fit, sizeof fit, hipMemcpyDeviceToHost);
@@ -1278,7 +1320,7 @@ int build_plan(SurfPlan *p, const spsim_hip_atom *atoms, const float *atom_b, co
   std::stable_sort(jobs.begin(), jobs.end(), [](const SurfJob &a, const SurfJob &b) {
     return (double)a.sh.ax.n * a.sh.ay.n * a.natoms > (double)b.sh.ax.n * b.sh.ay.n * b.natoms;
   });
-  const int slots = resident_slots(nodes_kernel(p->has_b), p->cus);
+  const int slots = resident_slots(nodes_kernel(p->has_b, false), p->cus);
   std::vector<SurfItem> items;
   size_t ws_bytes = 0;
   for (int first = 0; first < (int)jobs.size();) {
@@ -1353,17 +1395,12 @@ int surf_plan_create(const float *hkl, int nx, int ny, const spsim_hip_atom *ato
 bool surf_plan_takes(const SurfPlan *p, int pattern) { return p && p->takes[pattern]; }
 
 int surf_plan_run(const SurfPlan *p, float2 *F, float *I, hipStream_t s) {
-  const int slots = resident_slots(nodes_kernel(p->has_b), p->cus);
+  const int slots = resident_slots(nodes_kernel(p->has_b, false), p->cus);
   for (const SurfPlan::Group &g : p->groups) {
     hipLaunchKernelGGL(surface_prepare_kernel, dim3(16, g.count), dim3(kT), 0, s, p->jobs, g.first, p->has_b);
     const SurfItem *items = p->items + g.item_first;
     const int blocks = std::min(g.nitems, slots);
-    if (p->has_b)
-      hipLaunchKernelGGL(surface_nodes_kernel<true>, dim3(blocks), dim3(kT), 0, s, p->jobs, items, g.nitems, p->ff,
-                         p->b_global);
-    else
-      hipLaunchKernelGGL(surface_nodes_kernel<false>, dim3(blocks), dim3(kT), 0, s, p->jobs, items, g.nitems, p->ff,
-                         p->b_global);
+    SPSIM_TRY(launch_nodes(p->jobs, items, g.nitems, blocks, p->ff, p->b_global, p->has_b, nullptr, s));
     launch_interpolation(p->jobs, g.first, g.count, p->nx, p->ny, g.split ? g.max_nodes : 0, g.max_ny, p->dev, p->hkl,
                          F, I, s);
   }

@@ -7,11 +7,12 @@
 namespace spsim {
 
 constexpr int kSurfDeg = 16;         // sample lines per axis of the list's surface (degree kSurfDeg - 1)
+constexpr int kSurfLines = 31;       // lines per axis on which its slopes are measured
 constexpr int kSurfMinSide = 64;     // shortest detector side that is tried
 constexpr int kSurfMinNodes = 16;    // fewest and most nodes per axis, a multiple of 4
 constexpr int kSurfMaxNodes = 512;
 constexpr int kSurfMaxSplits = 128;  // atom ranges per node tile
-constexpr int kSurfListBlocks = 512;
+constexpr int kSurfListBlocks = 448;  // with the atom blocks, two workgroups per CU
 constexpr int kSurfAtomBlocks = 64;  // per molecule
 
 // What one workgroup of the scan saw: the largest |q - surface| per component
@@ -27,10 +28,10 @@ struct SurfRecord {
 // The list's surface: Chebyshev coefficients of a polynomial through q at
 // kSurfDeg x kSurfDeg pixels, in the pixel coordinates u, v in [-1, 1]
 // (coef[n][m][k]: T_n(v) T_m(u), component k), and its steepest slopes:
-// slope_x[j] is the largest |dq/du| on the line u = cos(pi j / (kSurfDeg - 1)).
+// slope_x[j] is the largest |dq/du| on the line u = cos(pi j / (kSurfLines - 1)).
 struct SurfFit {
   double coef[kSurfDeg][kSurfDeg][3];
-  float slope_x[kSurfDeg], slope_y[kSurfDeg];
+  float slope_x[kSurfLines], slope_y[kSurfLines];
   float s2max;  // largest s^2 = (|q| 1e-10 / 2)^2 seen
 };
 
@@ -86,13 +87,15 @@ struct SurfMol {
 };
 
 // Host sizes only: is the pattern large enough to look at its list?
-bool surf_worth(long long nx, long long ny, long long natoms);
+bool surf_worth(long long nx, long long ny, long long natoms, long long min_terms);
 
 // One pattern on the device alone (no host decision). On return *ok_flag points
 // to a device int that is non-zero when the outputs were written and zero when
 // the list or molecule is not smooth enough, in which case nothing was.
 size_t surf_single_bytes(int nx, int ny, int natoms);
-int launch_surface(const PatternLaunch &a, int nx, int ny, int cus, void *ws, const int **ok_flag, hipStream_t s);
+// sp: a wavelength spectrum, or null.
+int launch_surface(const PatternLaunch &a, int nx, int ny, const Spectrum *sp, int cus, void *ws, const int **ok_flag,
+                   hipStream_t s);
 
 // ---- plans that decide on the host (batch.hip) ----
 

@@ -192,3 +192,52 @@ def test_plan_mixes_interpolated_and_direct_patterns(gpu, with_b):
         assert rel_l2(direct, first) < 2 * TOL
     finally:
         L.spsim_hip_batch_destroy(plan)
+
+
+@pytest.mark.parametrize("bandwidth,samples,with_b", [(0.02, 5, False), (0.01, 11, True), (0.05, 3, False)])
+def test_interpolated_spectrum_vs_f64(gpu, bandwidth, samples, with_b):
+    """The wavelength spectrum on a flat list of n x n vectors, in the fitted
+    and the per-sample form (3 samples), a molecule off the origin."""
+    import torch
+
+    rng = np.random.default_rng(samples)
+    n, natoms = 160, 12_000
+    Z, pos, b = wl.random_molecule(natoms, 6e-9, rng, atom_b_range=(5.0, 40.0))
+    pos = (pos + np.array([1e-9, 2e-9, -1e-9])).astype(np.float32)
+    b = b if with_b else None
+    hkl = _list(n, n, pixel=1.5e-4)
+    R = wl.uniform_rotations(1, rng)[0]
+    atoms = dv.DeviceAtoms(dv.pack_atoms(Z, pos, atom_b=b), gpu)
+    q, ff = torch.from_numpy(hkl).to(gpu), dv.form_factor_table(device=gpu)
+    sc, w = dv.spectrum_samples(0.2e-9, bandwidth, samples)
+    F, I = dv.structure_factor_spectrum(q, atoms, ff, sc, w, R=R)
+    _, Id = dv.structure_factor_spectrum(q, atoms, ff, sc, w, R=R, tile=dv.make_tile(2, 256, 0))
+    torch.cuda.synchronize()
+    assert not torch.equal(I, Id)
+    sub = np.sort(rng.choice(n * n, 1200, replace=False))
+    F_ref, I_ref = oracle.sf_spectrum_f64(hkl[sub], Z, pos, sc, w, atom_b=b, R=R)
+    Fh = F.cpu().numpy()[sub]
+    e = rel_l2(I.cpu().numpy()[sub], I_ref)
+    print(f"spectrum {bandwidth} {samples}: I {e:.2e} (direct {rel_l2(Id.cpu().numpy()[sub], I_ref):.2e})", flush=True)
+    assert e < TOL
+    assert np.linalg.norm(Fh[:, 0] + 1j * Fh[:, 1] - F_ref) / np.linalg.norm(F_ref) < TOL
+
+
+def test_flat_lists_of_square_length(gpu):
+    """A flat list of n^2 vectors is tried as a detector: a detector's list is
+    interpolated, a 64^3 volume's (512^2 vectors) is not and gives the direct
+    kernel's bits."""
+    import torch
+
+    rng = np.random.default_rng(3)
+    ff = dv.form_factor_table(device=gpu)
+    Z, pos, _ = wl.random_molecule(2_500, 4e-9, rng)
+    atoms = dv.DeviceAtoms(dv.pack_atoms(Z, pos), gpu)
+    flat = torch.from_numpy(_list(512, 512)).to(gpu)
+    volume = dv.hkl_detector_3d(64, 64, 64, 5e-3, 5e-3, 5e-3, 0.1, 0.2e-9, device=gpu)
+    for q, smooth in ((flat, True), (volume, False)):
+        _, I = dv.structure_factor(q, atoms, ff)
+        _, Id = dv.structure_factor(q, atoms, ff, tile=dv.make_tile(2, 256, 0))
+        torch.cuda.synchronize()
+        assert torch.equal(I, Id) != smooth
+        assert rel_l2(I.cpu().numpy(), Id.cpu().numpy()) < 2 * TOL
