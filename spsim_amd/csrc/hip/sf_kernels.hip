@@ -1167,12 +1167,6 @@ extern "C" int spsim_hip_sf_pattern(const float *d_hkl, int npix, const spsim_hi
                                        (int)std::min<size_t>(64, kWorkspacePartials / (size_t)npix));
   const PatternLaunch a =
       make_launch(d_hkl, npix, d_atoms, d_atom_b, d_segs, nsegs, natoms, d_ff, b_global, rot9, d_F, d_I);
-  // A flat list carries no shape. One of n^2 vectors is taken for an n x n
-  // detector where that can pay; the device's check catches a wrong guess, which
-  // costs its launches (40 us of 250 us and more).
-  const int side = (int)std::lround(std::sqrt((double)npix));
-  if (!tile && (long long)side * side == npix)
-    return launch_smooth(Kind::kPattern, a, side, side, t, splits, cus, 500000000LL, nullptr, (hipStream_t)stream);
   return launch_pattern(a, t, splits, (hipStream_t)stream);
 }
 
@@ -1324,7 +1318,10 @@ extern "C" int spsim_hip_sf_spectrum(const float *d_hkl, int npix, const spsim_h
                                        (int)std::min<size_t>(64, kWorkspacePartials / (size_t)npix));
   const PatternLaunch a =
       make_launch(d_hkl, npix, d_atoms, d_atom_b, d_segs, nsegs, natoms, d_ff, b_global, rot9, d_F, d_I);
-  const int side = (int)std::lround(std::sqrt((double)npix));  // as in spsim_hip_sf_pattern
+  // A flat list carries no shape. One of n^2 vectors is taken for an n x n
+  // detector where that can pay; the device's check catches a wrong guess, which
+  // costs its launches (40 us of 130 us and more).
+  const int side = (int)std::lround(std::sqrt((double)npix));
   if (!tile && (long long)side * side == npix)
     return launch_smooth(Kind::kSpectrum, a, side, side, t, splits, cus, 200000000LL, &sp, (hipStream_t)stream);
   return launch_spectrum(a, sp, t, splits, (hipStream_t)stream);
