@@ -121,10 +121,8 @@ int spsim_hip_hkl_detector_3d(int nx, int ny, int nz, float width, float height,
    kernels apply it exactly, in FP64, as R^T to the atoms. d_atom_b may be NULL
    (no per-atom Debye-Waller factor). d_F ([npix][2]) or d_I may be NULL. The
    nsegs segments must tile the packed atoms [0, natoms) in order (as
-   spsim_hip_pack_atoms writes them). tile may be NULL (default tiling; a list of
-   n^2 vectors and 5e8 terms or more is then tried as an n x n detector and
-   interpolated as in spsim_hip_sf_grid if it is one). Uses a library-owned
-   device workspace when atom_splits > 1 or interpolating (grown on demand, kept
+   spsim_hip_pack_atoms writes them). tile may be NULL (default tiling). Uses a
+   library-owned device workspace when atom_splits > 1 (grown on demand, kept
    until spsim_hip_release). */
 int spsim_hip_sf_pattern(const float *d_hkl, int npix, const spsim_hip_atom *d_atoms, const float *d_atom_b,
                          const spsim_hip_segment *d_segs, int nsegs, int natoms, const float *d_ff,
@@ -194,8 +192,9 @@ int spsim_hip_spectrum_samples(double wavelength, double bandwidth, int nsamples
    average over wavelengths with the form factor at the unscaled |q|, as the
    reference's spectrum kernel computes it). scales and weights are host arrays
    of nsamples <= SPSIM_HIP_MAX_SPECTRUM entries. Other arguments as
-   spsim_hip_sf_pattern (with tile == NULL, n x n lists of 2e8 terms or more are
-   interpolated); tile->pixels_per_lane is 1 or 2. */
+   spsim_hip_sf_pattern; tile->pixels_per_lane is 1 or 2. With tile == NULL, a
+   list of n^2 vectors and 2e8 terms or more is tried as an n x n detector and
+   interpolated as in spsim_hip_sf_grid if it is one. */
 int spsim_hip_sf_spectrum(const float *d_hkl, int npix, const spsim_hip_atom *d_atoms, const float *d_atom_b,
                           const spsim_hip_segment *d_segs, int nsegs, int natoms, const float *d_ff,
                           float b_global, const double *rot9, int nsamples, const double *scales,
@@ -427,7 +426,10 @@ int spsim_hip_poisson_nll(const float *d_I, const float *d_y, const float *d_K, 
    metre) and d_grad_b [natoms] = dL/dB_j (units of L per A^2), recomputing the
    phases per pixel chunk instead of storing atom x pixel terms. h_segs is the
    HOST copy of the segments (as spsim_hip_pack_atoms returns them); d_grad_b
-   may be NULL. Uses the library workspace and synchronises the stream. */
+   may be NULL. Uses the library workspace and synchronises the stream. A list of
+   n^2 vectors and 5e8 terms or more is tried as an n x n detector; if it is one
+   (and the molecule smooth over it, as for spsim_hip_sf_grid), the pixels' values
+   are carried to the nodes by the transposed interpolation and the atoms sum nodes. */
 int spsim_hip_sf_adjoint(const float *d_hkl, int npix, const spsim_hip_atom *d_atoms, const float *d_atom_b,
                          const spsim_hip_segment *h_segs, int nsegs, int natoms, const float *d_ff,
                          float b_global, const float *d_F, const float *d_gI, float *d_grad_pos,

@@ -17,10 +17,12 @@
 // Sums are FP32 within a chunk and FP64 across chunks; the pixel ranges of one
 // atom tile are reduced in a fixed order by a second kernel (deterministic).
 #include <algorithm>
+#include <cmath>
 #include <vector>
 
 #include "common.hpp"
 #include "form_factor.hpp"
+#include "surface.hpp"
 
 namespace spsim {
 namespace {
@@ -38,12 +40,7 @@ struct __align__(16) PixRec {
 };
 static_assert(sizeof(PixRec) == 56 || sizeof(PixRec) == 64, "pixel record size");
 
-struct AtomTile {
-  int start;    // first packed atom
-  int count;    // atoms in the tile (<= 256 * KA)
-  int species;
-  int pad;
-};
+using AtomTile = SurfAtomTile;
 
 struct AdjArgs {
   const float *hkl;
@@ -57,10 +54,12 @@ struct AdjArgs {
   const float *gI;
   double4 *partial;  // [nsplit][natoms] {Ux, Uy, Uz, V}
   int natoms;
+  const int *skip;  // may be null; a device int, non-zero: the nodes' partial sums are used instead
 };
 
 template <int KA, bool HAS_B, bool WANT_B>
 __global__ __launch_bounds__(kT) void adjoint_kernel(AdjArgs a) {
+  if (a.skip && *a.skip) return;
   __shared__ PixRec sm[kCP];
   const AtomTile tile = a.tiles[blockIdx.x];
   const int split = blockIdx.y, nsplit = gridDim.y;
@@ -149,12 +148,20 @@ __global__ __launch_bounds__(kT) void adjoint_kernel(AdjArgs a) {
   }
 }
 
+// node_partial: the node_splits ranges that the interpolated adjoint left, when *skip.
 __global__ __launch_bounds__(kT) void adjoint_reduce_kernel(const double4 *__restrict__ partial, int nsplit, int natoms,
+                                                            const int *skip, const double4 *__restrict__ node_partial,
+                                                            int node_splits,
                                                             const spsim_hip_atom *__restrict__ atoms,
                                                             float *__restrict__ grad_pos, float *__restrict__ grad_b) {
   const int j = blockIdx.x * kT + threadIdx.x;
   if (j >= natoms) return;
+  if (skip && *skip) {
+    partial = node_partial;
+    nsplit = node_splits;
+  }
   double ux = 0, uy = 0, uz = 0, v = 0;
+#pragma unroll 4
   for (int s = 0; s < nsplit; ++s) {
     const double4 p = partial[(size_t)s * natoms + j];
     ux += p.x;
@@ -227,7 +234,7 @@ extern "C" int spsim_hip_sf_adjoint(const float *d_hkl, int npix, const spsim_hi
   SPSIM_TRY(ensure_device(&cus));
   hipStream_t s = (hipStream_t)stream;
   if (natoms == 0) return SPSIM_HIP_OK;
-  constexpr int KA = 2;
+  constexpr int KA = kSurfAtomsPerLane;
   const int per_tile = kT * KA;
   std::vector<AtomTile> tiles;
   int covered = 0;
@@ -252,21 +259,51 @@ extern "C" int spsim_hip_sf_adjoint(const float *d_hkl, int npix, const spsim_hi
   int nsplit = (int)std::max<long long>(1, (want + (long long)tiles.size() - 1) / (long long)tiles.size());
   nsplit = std::max(1, std::min(nsplit, std::max(1, npix / (4 * kCP))));
   const size_t tiles_bytes = ((tiles.size() * sizeof(AtomTile) + 255) / 256) * 256;
+  // A list of n^2 vectors is tried as an n x n detector (surface.hip); the
+  // device's check catches a wrong guess, which costs its launches (60 us of
+  // 350 us and more), and the direct kernel stays behind it.
+  const int side = (int)std::lround(std::sqrt((double)npix));
+  const bool smooth = (long long)side * side == npix && surf_worth(side, side, natoms, 500000000LL);
+  const size_t segs_bytes = (((size_t)nsegs * sizeof(spsim_hip_segment) + 255) / 256) * 256;
+  const int node_splits = (int)std::max<long long>(1, std::min<long long>(32, (4LL * cus + tiles.size() - 1) / (long long)tiles.size()));
+  const size_t partial_bytes = sizeof(double4) * (size_t)nsplit * natoms;
+  const size_t node_bytes = smooth ? sizeof(double4) * (size_t)node_splits * natoms : 0;
+  const size_t head = tiles_bytes + segs_bytes + partial_bytes + node_bytes;
+  const size_t surf_at = (head + 255) / 256 * 256;
   void *ws = nullptr;
-  SPSIM_TRY(workspace(tiles_bytes + sizeof(double4) * (size_t)nsplit * natoms, &ws));
+  SPSIM_TRY(workspace(smooth ? surf_at + surf_adjoint_bytes(side, side, natoms) : head, &ws));
   AtomTile *d_tiles = (AtomTile *)ws;
-  double4 *partial = (double4 *)((char *)ws + tiles_bytes);
+  spsim_hip_segment *d_segs = (spsim_hip_segment *)((char *)ws + tiles_bytes);
+  double4 *partial = (double4 *)((char *)ws + tiles_bytes + segs_bytes);
+  double4 *node_partial = (double4 *)((char *)partial + partial_bytes);
   SPSIM_HIP_TRY(hipMemcpyAsync(d_tiles, tiles.data(), tiles.size() * sizeof(AtomTile), hipMemcpyHostToDevice, s));
   if (npix == 0) {
     SPSIM_HIP_TRY(hipMemsetAsync(d_grad_pos, 0, sizeof(float) * 3 * (size_t)natoms, s));
     if (d_grad_b) SPSIM_HIP_TRY(hipMemsetAsync(d_grad_b, 0, sizeof(float) * (size_t)natoms, s));
     return SPSIM_HIP_OK;
   }
-  AdjArgs a{d_hkl, npix, d_atoms, d_atom_b, d_tiles, d_ff, b_global, (const float2 *)d_F, d_gI, partial, natoms};
+  const int *skip = nullptr;
+  if (smooth) {
+    SPSIM_HIP_TRY(hipMemcpyAsync(d_segs, h_segs, (size_t)nsegs * sizeof(spsim_hip_segment), hipMemcpyHostToDevice, s));
+    PatternLaunch f{};
+    f.hkl = d_hkl;
+    f.npix = npix;
+    f.atoms = d_atoms;
+    f.atom_b = d_atom_b;
+    f.segs = d_segs;
+    f.nsegs = nsegs;
+    f.natoms = natoms;
+    f.ff = d_ff;
+    f.b_global = b_global;
+    f.F = (float2 *)const_cast<float *>(d_F);
+    SPSIM_TRY(launch_surface_adjoint(f, d_gI, side, side, d_tiles, (int)tiles.size(), node_splits, wb, node_partial, cus,
+                                     (char *)ws + surf_at, &skip, s));
+  }
+  AdjArgs a{d_hkl, npix, d_atoms, d_atom_b, d_tiles, d_ff, b_global, (const float2 *)d_F, d_gI, partial, natoms, skip};
   void *params[] = {(void *)&a};
   SPSIM_HIP_TRY(hipLaunchKernel(k, dim3((unsigned)tiles.size(), nsplit), dim3(kT), params, 0, s));
   hipLaunchKernelGGL(adjoint_reduce_kernel, dim3((natoms + kT - 1) / kT), dim3(kT), 0, s, (const double4 *)partial,
-                     nsplit, natoms, d_atoms, d_grad_pos, d_grad_b);
+                     nsplit, natoms, skip, (const double4 *)node_partial, node_splits, d_atoms, d_grad_pos, d_grad_b);
   SPSIM_HIP_TRY(hipGetLastError());
   // The tile list was copied from host memory that goes out of scope.
   SPSIM_HIP_TRY(hipStreamSynchronize(s));

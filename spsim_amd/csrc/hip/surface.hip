@@ -347,14 +347,17 @@ __host__ __device__ inline float axis_need(const float *slope, float radius, flo
   return theta + 4.0f * cbrtf(theta) + 8.0f + 2.0f * sqrtf(fmaxf(gauss, 0.0f));
 }
 
+enum class SurfKind { kSum, kSpectrum, kAdjoint };
+
 __host__ __device__ inline bool worth(double nodes_x, double nodes_y, double nx, double ny, double natoms,
-                                      bool spectrum) {
-  // Issue cycles per lane: a term of the node sums 80 (160 with a spectrum), of
-  // the direct sums 26 to 45 (130); the interpolation 25 per node row and pixel.
-  // Measured on the MI355X.
-  const double surf = nodes_x * nodes_y * natoms * (spectrum ? 160.0 : 80.0) +
-                      25.0 * (nx * ny * nodes_y + nx * nodes_x * nodes_y);
-  return surf < 0.8 * (spectrum ? 130.0 : 26.0) * nx * ny * natoms;
+                                      SurfKind kind) {
+  // Issue cycles per lane: a term of the node sums 80 (160 with a spectrum, 120
+  // in the adjoint), of the direct sums 26 to 45 (130, 109); the interpolation
+  // 25 per node row and pixel. Measured on the MI355X.
+  const double node = kind == SurfKind::kSum ? 80.0 : (kind == SurfKind::kSpectrum ? 160.0 : 120.0);
+  const double direct = kind == SurfKind::kSum ? 26.0 : (kind == SurfKind::kSpectrum ? 130.0 : 109.0);
+  const double surf = nodes_x * nodes_y * natoms * node + 25.0 * (nx * ny * nodes_y + nx * nodes_x * nodes_y);
+  return surf < 0.8 * direct * nx * ny * natoms;
 }
 
 __host__ __device__ inline bool smooth(const SurfMol &m, float s2max) {
@@ -454,10 +457,27 @@ struct PlanArgs {
   int slots;       // resident workgroups of the node sums
   int slot_cap;    // partial slots that fit
   int max_nx, max_ny;  // nodes that fit the workspace
-  bool spectrum;
+  SurfKind kind;
   double scale, spread;  // of a spectrum: largest s_k, largest |s_k / sc - 1|
   SurfJob *out;
+  // adjoint: pixel values 2 g F e^{2 pi i q.r0} from the list, F and g
+  const float *hkl;
+  const float2 *F;
+  const float *gI;
+  float2 *pixels;
 };
+
+__device__ __forceinline__ void prepare_pixels(const PlanArgs &a, const SurfJob &jb, int first, int step) {
+  for (int p = first; p < jb.nx * jb.ny; p += step) {
+    const double t = __builtin_fma((double)a.hkl[3 * p + 2], jb.r0[2],
+                                   __builtin_fma((double)a.hkl[3 * p + 1], jb.r0[1], (double)a.hkl[3 * p] * jb.r0[0]));
+    double sn, cs;
+    sincospi(2.0 * __builtin_amdgcn_fract(t), &sn, &cs);
+    const float2 f = a.F[p];
+    const double g = 2.0 * (double)a.gI[p];
+    a.pixels[p] = make_float2((float)(g * (f.x * cs - f.y * sn)), (float)(g * (f.x * sn + f.y * cs)));
+  }
+}
 
 // Interpolation weights of one axis (node-major [n][npix]), one wave per
 // pixel: barycentric formula in s = cos t, whose weights at the Chebyshev
@@ -582,7 +602,7 @@ __global__ __launch_bounds__(kT) void surface_plan_kernel(PlanArgs a) {
   // G is taken at the spectrum's centre scale, so it is off by the spread
   const bool ok = smooth(mol, a.fit->s2max) && 2.0 * kPi * mol.radius * mol.dev * a.spread <= kMaxSpreadDev &&
                   nx <= a.max_nx && ny <= a.max_ny &&
-                  worth(nx, ny, a.job.nx, a.job.ny, a.job.natoms, a.spectrum);
+                  worth(nx, ny, a.job.nx, a.job.ny, a.job.natoms, a.kind);
   if (!ok) {
     if (blockIdx.x == 0 && blockIdx.y == 0 && t == 0) a.out->ok = 0;
     return;
@@ -627,7 +647,13 @@ __global__ __launch_bounds__(kT) void surface_plan_kernel(PlanArgs a) {
   }
   __syncthreads();
   build(blockIdx.y, a.fit, job.sh, job.nx, job.ny, snx, wnx, sny, wny);
-  if (blockIdx.y == 2) prepare_atoms(job, a.has_b, (int)(blockIdx.x * kT) + t, (int)gridDim.x * kT);
+  if (blockIdx.y == 2) {
+    const int first = (int)(blockIdx.x * kT) + t, step = (int)gridDim.x * kT;
+    if (a.kind == SurfKind::kAdjoint)
+      prepare_pixels(a, job, first, step);
+    else
+      prepare_atoms(job, a.has_b, first, step);
+  }
 }
 
 __global__ __launch_bounds__(kT) void surface_tables_kernel(const SurfFit *fit, SurfShape sh, int nx, int ny) {
@@ -987,7 +1013,243 @@ __global__ __launch_bounds__(kT) void surface_cols_kernel(const SurfJob *jobs, i
     }
 }
 
+// ---- adjoint ---------------------------------------------------------------------
+//
+// The gradients of a loss with dL/dI_p = g_p given need, per atom j,
+//   S_j = sum_p A_p h_j(q_p),  A_p = 2 g_p F_p,  h_j(q) = f(|q|) e^{-B_j s^2} e^{2 pi i q.r_j},
+// with dL/dr_j = -2 pi w_j Im sum_p q_p A_p h_j and dL/dB_j = -w_j Re sum_p s_p^2 A_p h_j
+// (adjoint.hip). h_j is as smooth over the detector as F, so the transposed
+// interpolation carries the pixels' values to the nodes,
+//   a_v = sum_p L_v(p) A_p,  b_v = sum_p L_v(p) A_p d_p   (d: the list's deviation),
+// two dense products again (FP64 for a, FP32 for b), and every atom sums
+// nodes instead of pixels: S_j = sum_v h_j(q_v) Z_v, Z_v = a_v + 2 pi i r_j.b_v.
+
+constexpr int kGatherNodes = 8;  // nodes of a row per wave of the second product
+
+// First product: t[split][k][x] = sum over the split's rows of ty[k][y] A(y, x);
+// 16 node rows x 16 columns per wave, blockIdx.z: rows of the list.
+__global__ __launch_bounds__(kT) void surface_gather_rows_kernel(const SurfJob *job, const float2 *__restrict__ pixels,
+                                                                 const float *__restrict__ dev) {
+  const SurfJob &jb = *job;
+  if (!jb.ok) return;
+  const int nyn = jb.sh.ay.n, nx = jb.nx, ny = jb.ny;
+  const int l = threadIdx.x & 63, m = l & 15, gq = l >> 4;
+  const int k0 = (int)blockIdx.y * 16, x = (int)blockIdx.x * 64 + (int)(threadIdx.x / 64) * 16 + m;
+  if (k0 >= nyn || x - m >= nx) return;
+  const int steps = (ny + 3) / 4, splits = gridDim.z;
+  const int y0 = 4 * (int)((long long)steps * blockIdx.z / splits);
+  const int y1 = 4 * (int)((long long)steps * (blockIdx.z + 1) / splits);
+  const int xc = min(x, nx - 1);
+  const double *w = jb.sh.ty + (size_t)min(k0 + m, nyn - 1) * ny;
+  const double *wp = jb.sh.ty + (size_t)min(k0 + prow(m), nyn - 1) * ny;
+  Fields acc;
+  clear(acc);
+#pragma unroll 4
+  for (int y = y0; y < y1; y += 4) {
+    const int yy = min(y + gq, ny - 1);
+    const bool in = y + gq < ny;  // rows past the end weigh nothing
+    const double a = in ? w[yy] : 0.0;
+    const float a32 = in ? (float)wp[yy] : 0.0f;
+    const size_t p = (size_t)yy * nx + xc;
+    const float2 v = pixels[p];
+    const float d[3] = {dev[3 * p], dev[3 * p + 1], dev[3 * p + 2]};
+    acc.re = __builtin_amdgcn_mfma_f64_16x16x4f64(a, (double)v.x, acc.re, 0, 0, 0);
+    acc.im = __builtin_amdgcn_mfma_f64_16x16x4f64(a, (double)v.y, acc.im, 0, 0, 0);
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+      acc.g[2 * c] = __builtin_amdgcn_mfma_f32_16x16x4f32(a32, v.x * d[c], acc.g[2 * c], 0, 0, 0);
+      acc.g[2 * c + 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(a32, v.y * d[c], acc.g[2 * c + 1], 0, 0, 0);
+    }
+  }
+  if (x >= nx) return;
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    const int k = k0 + gq + 4 * r;
+    if (k >= nyn) continue;
+    const size_t o = ((size_t)blockIdx.z * nyn + k) * nx + x;
+    jb.t64[o] = make_double2(acc.re[r], acc.im[r]);
+    float2 *t = (float2 *)jb.t32 + 3 * o;
+#pragma unroll
+    for (int c = 0; c < 3; ++c) t[c] = make_float2(acc.g[2 * c][r], acc.g[2 * c + 1][r]);
+  }
+}
+
+// Second product, with the splits added: f, g of node (i, k) = sum_x tx[i][x] t[k][x].
+// One wave per node row k and 8 nodes i: the lanes share the columns.
+__global__ __launch_bounds__(kT) void surface_gather_nodes_kernel(const SurfJob *job, int splits) {
+  const SurfJob &jb = *job;
+  if (!jb.ok) return;
+  const int nyn = jb.sh.ay.n, nxn = jb.sh.ax.n, nx = jb.nx;
+  const int k = blockIdx.y, i0 = ((int)blockIdx.x * (kT / 64) + (int)(threadIdx.x / 64)) * kGatherNodes;
+  if (k >= nyn || i0 >= nxn) return;
+  const int lane = threadIdx.x & 63;
+  double re[kGatherNodes], im[kGatherNodes];
+  float g[kGatherNodes][6];
+#pragma unroll
+  for (int i = 0; i < kGatherNodes; ++i) {
+    re[i] = im[i] = 0.0;
+#pragma unroll
+    for (int c = 0; c < 6; ++c) g[i][c] = 0.0f;
+  }
+  for (int x = lane; x < nx; x += 64) {
+    double tr = 0.0, ti = 0.0;
+    float tg[6] = {0, 0, 0, 0, 0, 0};
+#pragma unroll 8
+    for (int s = 0; s < splits; ++s) {
+      const size_t o = ((size_t)s * nyn + k) * nx + x;
+      const double2 v = jb.t64[o];
+      const float2 *t = (const float2 *)jb.t32 + 3 * o;
+      tr += v.x;
+      ti += v.y;
+#pragma unroll
+      for (int c = 0; c < 3; ++c) {
+        tg[2 * c] += t[c].x;
+        tg[2 * c + 1] += t[c].y;
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < kGatherNodes; ++i) {
+      const double w = jb.sh.tx[(size_t)min(i0 + i, nxn - 1) * nx + x];
+      re[i] = __builtin_fma(w, tr, re[i]);
+      im[i] = __builtin_fma(w, ti, im[i]);
+#pragma unroll
+      for (int c = 0; c < 6; ++c) g[i][c] = __builtin_fmaf((float)w, tg[c], g[i][c]);
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < kGatherNodes; ++i) {
+    for (int o = 32; o > 0; o >>= 1) {
+      re[i] += __shfl_xor(re[i], o);
+      im[i] += __shfl_xor(im[i], o);
+#pragma unroll
+      for (int c = 0; c < 6; ++c) g[i][c] += __shfl_xor(g[i][c], o);
+    }
+    if (lane == 0 && i0 + i < nxn) {
+      const size_t node = (size_t)(i0 + i) * nyn + k;
+      jb.f[node] = make_double2(re[i], im[i]);
+      for (int c = 0; c < 6; ++c) jb.g[6 * node + c] = g[i][c];
+    }
+  }
+}
+
+// A node as every atom of one species reads it: f(|q|) Z's parts, b times 2 pi.
+struct __align__(16) AdjNode {
+  double qx, qy, qz;
+  float ar, ai;
+  float br[3], bi[3];
+  float qxf, qyf, qzf;
+  float s2, nl2, pad;
+};
+static_assert(sizeof(AdjNode) == 80, "adjoint node record");
+
+// Per atom: U = Im sum q h Z and V = Re sum s^2 h Z over a range of nodes; one
+// tile of 512 atoms of one species per workgroup (2 per lane), the nodes
+// staged in LDS 128 at a time. FP32 sums over a chunk, FP64 across chunks.
+template <bool HAS_B, bool WANT_B>
+__global__ __launch_bounds__(kT) void surface_adjoint_kernel(const SurfJob *job, const SurfAtomTile *tiles,
+                                                             const float *__restrict__ ff, float b_global,
+                                                             double4 *__restrict__ partial) {
+  constexpr int KA = kSurfAtomsPerLane, kChunk = 128;
+  __shared__ AdjNode sm[kChunk];
+  const SurfJob &jb = *job;
+  if (!jb.ok) return;
+  const SurfAtomTile tile = tiles[blockIdx.x];
+  const int nodes = jb.sh.ax.n * jb.sh.ay.n, split = blockIdx.y, nsplit = gridDim.y;
+  const int n_begin = (int)((long long)nodes * split / nsplit), n_end = (int)((long long)nodes * (split + 1) / nsplit);
+  const float Bs = tile.species == SPSIM_HIP_UNIT_SPECIES ? 0.0f : b_global;
+  const float *c = ff + tile.species * SPSIM_HIP_FF_STRIDE;
+  double rx[KA], ry[KA], rz[KA], Ux[KA], Uy[KA], Uz[KA], V[KA];
+  float xf[KA], yf[KA], zf[KA], bj[KA];
+#pragma unroll
+  for (int k = 0; k < KA; ++k) {
+    const int i = threadIdx.x + k * kT;
+    const bool ok = i < tile.count;
+    const spsim_hip_atom at = ok ? jb.atoms[tile.start + i] : spsim_hip_atom{0.f, 0.f, 0.f, 0.f};
+    rx[k] = ok ? at.x - jb.r0[0] : 0.0;
+    ry[k] = ok ? at.y - jb.r0[1] : 0.0;
+    rz[k] = ok ? at.z - jb.r0[2] : 0.0;
+    xf[k] = (float)rx[k];
+    yf[k] = (float)ry[k];
+    zf[k] = (float)rz[k];
+    bj[k] = (HAS_B && ok) ? jb.atom_b[tile.start + i] : 0.0f;
+    Ux[k] = Uy[k] = Uz[k] = V[k] = 0.0;
+  }
+  for (int n0 = n_begin; n0 < n_end; n0 += kChunk) {
+    const int n = min(kChunk, n_end - n0);
+    __syncthreads();
+    if ((int)threadIdx.x < n) {
+      const size_t node = n0 + threadIdx.x;
+      const double *q = jb.sh.nodes + 3 * node;
+      AdjNode r;
+      r.qx = q[0];
+      r.qy = q[1];
+      r.qz = q[2];
+      r.qxf = (float)q[0];
+      r.qyf = (float)q[1];
+      r.qzf = (float)q[2];
+      const double s2 = (q[0] * q[0] + q[1] * q[1] + q[2] * q[2]) * 2.5e-21;
+      const double f = form_factor64(c, s2, Bs);
+      const double2 a = jb.f[node];
+      r.ar = (float)(f * a.x);
+      r.ai = (float)(f * a.y);
+      const float f2 = (float)(2.0 * kPi * f);
+      for (int i = 0; i < 3; ++i) {
+        r.br[i] = f2 * jb.g[6 * node + 2 * i];
+        r.bi[i] = f2 * jb.g[6 * node + 2 * i + 1];
+      }
+      r.s2 = (float)s2;
+      r.nl2 = (float)(-s2 * kLog2e);
+      r.pad = 0.0f;
+      sm[threadIdx.x] = r;
+    }
+    __syncthreads();
+    float ux[KA], uy[KA], uz[KA], v[KA];
+#pragma unroll
+    for (int k = 0; k < KA; ++k) ux[k] = uy[k] = uz[k] = v[k] = 0.0f;
+    for (int i = 0; i < n; ++i) {
+      const AdjNode r = sm[i];
+#pragma unroll
+      for (int k = 0; k < KA; ++k) {
+        const double t = __builtin_fma(r.qz, rz[k], __builtin_fma(r.qy, ry[k], r.qx * rx[k]));
+        const float ph = (float)__builtin_amdgcn_fract(t);
+        float cs = __builtin_amdgcn_cosf(ph), sn = __builtin_amdgcn_sinf(ph);
+        if constexpr (HAS_B) {
+          const float e = __builtin_amdgcn_exp2f(bj[k] * r.nl2);
+          cs *= e;
+          sn *= e;
+        }
+        // Z = a + i (2 pi r.b)
+        const float zr = __builtin_fmaf(
+            -zf[k], r.bi[2], __builtin_fmaf(-yf[k], r.bi[1], __builtin_fmaf(-xf[k], r.bi[0], r.ar)));
+        const float zi = __builtin_fmaf(
+            zf[k], r.br[2], __builtin_fmaf(yf[k], r.br[1], __builtin_fmaf(xf[k], r.br[0], r.ai)));
+        const float u = __builtin_fmaf(cs, zi, sn * zr);
+        ux[k] = __builtin_fmaf(u, r.qxf, ux[k]);
+        uy[k] = __builtin_fmaf(u, r.qyf, uy[k]);
+        uz[k] = __builtin_fmaf(u, r.qzf, uz[k]);
+        if constexpr (WANT_B) v[k] = __builtin_fmaf(r.s2, __builtin_fmaf(cs, zr, -(sn * zi)), v[k]);
+      }
+    }
+#pragma unroll
+    for (int k = 0; k < KA; ++k) {
+      Ux[k] += ux[k];
+      Uy[k] += uy[k];
+      Uz[k] += uz[k];
+      V[k] += v[k];
+    }
+  }
+#pragma unroll
+  for (int k = 0; k < KA; ++k) {
+    const int i = threadIdx.x + k * kT;
+    if (i < tile.count)
+      partial[(size_t)split * jb.natoms + tile.start + i] = make_double4(Ux[k], Uy[k], Uz[k], V[k]);
+  }
+}
+
 size_t align_up(size_t n) { return (n + 255) / 256 * 256; }
+
+// Row ranges of the adjoint's first product: enough waves for the chip.
+int gather_splits(int nx) { return std::max(2, std::min(16, 8192 / nx)); }
 
 // Workspace of one pattern: the nodes of an axis are limited to what can pay
 // (worth() needs n_x n_y below about a third of the pixels).
@@ -996,7 +1258,7 @@ struct SingleLayout {
   size_t fit, records, centres, job, dev, nodes, tx, ty, prep, f, g, slots, t64, t32, total;
 };
 
-SingleLayout single_layout(int nx, int ny, int natoms) {
+SingleLayout single_layout(int nx, int ny, int natoms, bool adjoint) {
   SingleLayout l;
   auto cap = [](int n) { return std::max(kSurfMinNodes, std::min(kSurfMaxNodes, (int)(0.6 * n) / 4 * 4)); };
   l.max_nx = cap(nx);
@@ -1017,12 +1279,13 @@ SingleLayout single_layout(int nx, int ny, int natoms) {
   l.nodes = take(sizeof(double) * 3 * nodes);
   l.tx = take(sizeof(double) * (size_t)l.max_nx * nx);
   l.ty = take(sizeof(double) * (size_t)l.max_ny * ny);
-  l.prep = take(sizeof(NodeAtom) * (size_t)natoms);
+  l.prep = adjoint ? take(sizeof(float2) * npix) : take(sizeof(NodeAtom) * (size_t)natoms);
   l.f = take(sizeof(double2) * nodes);
   l.g = take(sizeof(float) * 6 * nodes);
-  l.slots = take(sizeof(NodeSlot) * (size_t)l.slot_cap);
-  l.t64 = take(sizeof(double2) * (size_t)l.max_ny * nx);
-  l.t32 = take(sizeof(float) * 6 * (size_t)l.max_ny * nx);
+  const size_t rows = (size_t)l.max_ny * nx * (adjoint ? gather_splits(nx) : 1);
+  l.slots = adjoint ? at : take(sizeof(NodeSlot) * (size_t)l.slot_cap);
+  l.t64 = take(sizeof(double2) * rows);
+  l.t32 = take(sizeof(float) * 6 * rows);
   l.total = at;
   return l;
 }
@@ -1063,14 +1326,13 @@ bool surf_worth(long long nx, long long ny, long long natoms, long long min_term
   return nx >= kSurfMinSide && ny >= kSurfMinSide && nx * ny * natoms >= min_terms;
 }
 
-size_t surf_single_bytes(int nx, int ny, int natoms) { return single_layout(nx, ny, natoms).total; }
+size_t surf_single_bytes(int nx, int ny, int natoms) { return single_layout(nx, ny, natoms, false).total; }
 
-int launch_surface(const PatternLaunch &a, int nx, int ny, const Spectrum *sp, int cus, void *ws, const int **ok_flag,
-                   hipStream_t s) {
-  const SingleLayout l = single_layout(nx, ny, a.natoms);
-  char *w = (char *)ws;
-  const bool has_b = a.atom_b != nullptr;
-  const int slots = resident_slots(nodes_kernel(has_b, sp != nullptr), cus);
+namespace {
+
+// Scan and plan of one pattern; the job is left at the workspace's start.
+int launch_plan(const PatternLaunch &a, int nx, int ny, const Spectrum *sp, SurfKind kind, const float *gI,
+                const SingleLayout &l, char *w, int slots, int cus, hipStream_t s) {
   PlanArgs p{};
   p.job.nx = nx;
   p.job.ny = ny;
@@ -1096,12 +1358,12 @@ int launch_surface(const PatternLaunch &a, int nx, int ny, const Spectrum *sp, i
   p.centres = (const double *)(w + l.centres);
   p.ff = a.ff;
   p.b_global = a.b_global;
-  p.has_b = has_b;
+  p.has_b = a.atom_b != nullptr;
   p.slots = slots;
   p.slot_cap = l.slot_cap;
   p.max_nx = l.max_nx;
   p.max_ny = l.max_ny;
-  p.spectrum = sp != nullptr;
+  p.kind = kind;
   p.scale = 1.0;
   if (sp) {
     p.scale = 0.0;
@@ -1111,14 +1373,72 @@ int launch_surface(const PatternLaunch &a, int nx, int ny, const Spectrum *sp, i
     }
   }
   p.out = (SurfJob *)(w + l.job);
-  const SurfJob *job = p.out;
-  ScanArgs sc{a.hkl,    nx, ny, p.list_blocks, a.atoms, a.atom_b, nullptr, a.natoms, !sp, (SurfFit *)(w + l.fit),
-              (float *)(w + l.dev), (SurfRecord *)(w + l.records), (double *)(w + l.centres)};
+  if (kind == SurfKind::kAdjoint) {
+    p.hkl = a.hkl;
+    p.F = a.F;
+    p.gI = gI;
+    p.pixels = (float2 *)(w + l.prep);
+  }
+  const ScanArgs sc{a.hkl,
+                    nx,
+                    ny,
+                    p.list_blocks,
+                    a.atoms,
+                    a.atom_b,
+                    nullptr,
+                    a.natoms,
+                    !sp,
+                    (SurfFit *)(w + l.fit),
+                    (float *)(w + l.dev),
+                    (SurfRecord *)(w + l.records),
+                    (double *)(w + l.centres)};
   hipLaunchKernelGGL(surface_scan_kernel, dim3(p.list_blocks + kSurfAtomBlocks), dim3(kT), 0, s, sc);
   hipLaunchKernelGGL(surface_plan_kernel, dim3(std::max(1, 2 * cus / 3), 3), dim3(kT), 0, s, p);
-  SPSIM_TRY(launch_nodes(job, nullptr, 0, slots, a.ff, a.b_global, has_b, sp, s));
-  launch_interpolation(job, 0, 1, nx, ny, l.max_nx * l.max_ny, l.max_ny, (const float *)(w + l.dev), a.hkl, a.F, a.I, s);
   SPSIM_HIP_TRY(hipGetLastError());
+  return SPSIM_HIP_OK;
+}
+
+}  // namespace
+
+int launch_surface(const PatternLaunch &a, int nx, int ny, const Spectrum *sp, int cus, void *ws, const int **ok_flag,
+                   hipStream_t s) {
+  const SingleLayout l = single_layout(nx, ny, a.natoms, false);
+  char *w = (char *)ws;
+  const SurfJob *job = (const SurfJob *)(w + l.job);
+  const bool has_b = a.atom_b != nullptr;
+  const int slots = resident_slots(nodes_kernel(has_b, sp != nullptr), cus);
+  SPSIM_TRY(launch_plan(a, nx, ny, sp, sp ? SurfKind::kSpectrum : SurfKind::kSum, nullptr, l, w, slots, cus, s));
+  SPSIM_TRY(launch_nodes(job, nullptr, 0, slots, a.ff, a.b_global, has_b, sp, s));
+  launch_interpolation(job, 0, 1, nx, ny, l.max_nx * l.max_ny, l.max_ny, (const float *)(w + l.dev), a.hkl, a.F, a.I,
+                       s);
+  SPSIM_HIP_TRY(hipGetLastError());
+  *ok_flag = &job->ok;
+  return SPSIM_HIP_OK;
+}
+
+size_t surf_adjoint_bytes(int nx, int ny, int natoms) { return single_layout(nx, ny, natoms, true).total; }
+
+int launch_surface_adjoint(const PatternLaunch &a, const float *gI, int nx, int ny, const SurfAtomTile *tiles,
+                           int ntiles, int splits, bool want_b, double4 *partial, int cus, void *ws,
+                           const int **ok_flag, hipStream_t s) {
+  const SingleLayout l = single_layout(nx, ny, a.natoms, true);
+  char *w = (char *)ws;
+  const SurfJob *job = (const SurfJob *)(w + l.job);
+  SPSIM_TRY(launch_plan(a, nx, ny, nullptr, SurfKind::kAdjoint, gI, l, w, cus, cus, s));
+  const int gs = gather_splits(nx), per_block = kGatherNodes * (kT / 64);
+  hipLaunchKernelGGL(surface_gather_rows_kernel, dim3((nx + 63) / 64, (l.max_ny + 15) / 16, gs), dim3(kT), 0, s, job,
+                     (const float2 *)(w + l.prep), (const float *)(w + l.dev));
+  hipLaunchKernelGGL(surface_gather_nodes_kernel, dim3((l.max_nx + per_block - 1) / per_block, l.max_ny), dim3(kT), 0, s,
+                     job, gs);
+  const bool hb = a.atom_b != nullptr;
+  const void *k = hb ? (want_b ? (const void *)&surface_adjoint_kernel<true, true>
+                               : (const void *)&surface_adjoint_kernel<true, false>)
+                     : (want_b ? (const void *)&surface_adjoint_kernel<false, true>
+                               : (const void *)&surface_adjoint_kernel<false, false>);
+  const float *ff = a.ff;
+  float bg = a.b_global;
+  void *params[] = {(void *)&job, (void *)&tiles, (void *)&ff, (void *)&bg, (void *)&partial};
+  SPSIM_HIP_TRY(hipLaunchKernel(k, dim3(ntiles, splits), dim3(kT), params, 0, s));
   *ok_flag = &job->ok;
   return SPSIM_HIP_OK;
 }
@@ -1165,7 +1485,7 @@ bool choose(const SurfFit &fit, const SurfMol &mol, int nx, int ny, int natoms, 
     *out[k] = SurfAxis{n, axis_stretch(n), 0.0};
     out[k]->asin_a = std::asin(out[k]->a);
   }
-  return worth(ax->n, ay->n, nx, ny, natoms, false);
+  return worth(ax->n, ay->n, nx, ny, natoms, SurfKind::kSum);
 }
 
 // Lays the job's buffers out in a workspace from `at` on; returns the end.

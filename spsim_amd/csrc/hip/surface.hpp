@@ -97,6 +97,23 @@ size_t surf_single_bytes(int nx, int ny, int natoms);
 int launch_surface(const PatternLaunch &a, int nx, int ny, const Spectrum *sp, int cus, void *ws, const int **ok_flag,
                    hipStream_t s);
 
+// ---- adjoint (adjoint.hip) ----
+
+constexpr int kSurfAtomsPerLane = 2;
+
+// A run of packed atoms of one species, at most 256 kSurfAtomsPerLane.
+struct SurfAtomTile {
+  int start, count, species, pad;
+};
+
+// Sums of the gradients over the detector a.hkl with the forward's a.F and
+// g = dL/dI, by way of the nodes: partial[split][atom] as adjoint_kernel leaves
+// them, `splits` node ranges per tile. *ok_flag as for launch_surface.
+size_t surf_adjoint_bytes(int nx, int ny, int natoms);
+int launch_surface_adjoint(const PatternLaunch &a, const float *gI, int nx, int ny, const SurfAtomTile *tiles,
+                           int ntiles, int splits, bool want_b, double4 *partial, int cus, void *ws,
+                           const int **ok_flag, hipStream_t s);
+
 // ---- plans that decide on the host (batch.hip) ----
 
 struct SurfPlan;

@@ -223,21 +223,68 @@ def test_interpolated_spectrum_vs_f64(gpu, bandwidth, samples, with_b):
     assert np.linalg.norm(Fh[:, 0] + 1j * Fh[:, 1] - F_ref) / np.linalg.norm(F_ref) < TOL
 
 
-def test_flat_lists_of_square_length(gpu):
-    """A flat list of n^2 vectors is tried as a detector: a detector's list is
-    interpolated, a 64^3 volume's (512^2 vectors) is not and gives the direct
-    kernel's bits."""
+def test_flat_volume_keeps_the_direct_spectrum(gpu):
+    """A flat list of n^2 vectors that is no detector (a 64^3 volume's 512^2)
+    gives the direct kernel's bits."""
     import torch
 
     rng = np.random.default_rng(3)
-    ff = dv.form_factor_table(device=gpu)
-    Z, pos, _ = wl.random_molecule(2_500, 4e-9, rng)
-    atoms = dv.DeviceAtoms(dv.pack_atoms(Z, pos), gpu)
-    flat = torch.from_numpy(_list(512, 512)).to(gpu)
+    Z, pos, _ = wl.random_molecule(1_000, 4e-9, rng)
+    atoms, ff = dv.DeviceAtoms(dv.pack_atoms(Z, pos), gpu), dv.form_factor_table(device=gpu)
     volume = dv.hkl_detector_3d(64, 64, 64, 5e-3, 5e-3, 5e-3, 0.1, 0.2e-9, device=gpu)
-    for q, smooth in ((flat, True), (volume, False)):
-        _, I = dv.structure_factor(q, atoms, ff)
-        _, Id = dv.structure_factor(q, atoms, ff, tile=dv.make_tile(2, 256, 0))
-        torch.cuda.synchronize()
-        assert torch.equal(I, Id) != smooth
-        assert rel_l2(I.cpu().numpy(), Id.cpu().numpy()) < 2 * TOL
+    sc, w = dv.spectrum_samples(0.2e-9, 0.02, 5)
+    _, I = dv.structure_factor_spectrum(volume, atoms, ff, sc, w)
+    _, Id = dv.structure_factor_spectrum(volume, atoms, ff, sc, w, tile=dv.make_tile(2, 256, 0))
+    torch.cuda.synchronize()
+    assert torch.equal(I, Id)
+
+
+@pytest.mark.parametrize("n,natoms,radius,with_b,want_b,listing", [
+    (150, 25_000, 6e-9, True, True, "detector"),
+    (257, 9_000, 5e-9, False, False, "detector"),
+    (200, 13_000, 5e-9, True, False, "off centre"),
+    (131, 30_000, 4e-9, False, True, "detector"),
+    (512, 2_000, 4e-9, True, True, "volume"),
+])
+def test_adjoint_by_nodes_vs_f64(gpu, n, natoms, radius, with_b, want_b, listing):
+    """Gradients of a loss with random dL/dI on square detectors, given F,
+    against FP64 sums; a 64^3 volume of 512^2 vectors takes the direct kernel.
+    The sums are FP32 (1e-7 of each term); 2e-6 allows for their cancellation."""
+    import ctypes as C
+
+    import torch
+
+    from spsim_amd import _lib
+
+    rng = np.random.default_rng(n)
+    Z, pos, b = wl.random_molecule(natoms, radius, rng, atom_b_range=(5.0, 40.0))
+    pos = (pos + np.array([2e-9, -1e-9, 1e-9])).astype(np.float32)
+    if listing == "volume":
+        hkl = oracle.hkl_3d(64, 64, 64, 5e-3, 5e-3, 5e-3, 0.1, 0.2e-9)
+    else:
+        hkl = _list(n, n, pixel=1.5e-4, cx=2e-3 if listing == "off centre" else 0.0)
+    npix = n * n
+    packed = dv.pack_atoms(Z, pos, atom_b=b if with_b else None)
+    atoms = dv.DeviceAtoms(packed, gpu)
+    q, ff = torch.from_numpy(hkl).to(gpu), dv.form_factor_table(device=gpu)
+    F, _ = dv.structure_factor(q, atoms, ff, B=3.0)
+    g = rng.normal(size=npix).astype(np.float32)
+    gI = torch.from_numpy(g).to(gpu)
+    gp = torch.full((natoms, 3), float("nan"), device=gpu)
+    gb = torch.full((natoms,), float("nan"), device=gpu) if want_b else None
+    vp = lambda t: None if t is None else C.c_void_p(t.data_ptr())
+    segs = np.ascontiguousarray(packed.segs)
+    _lib.check(_lib.load().spsim_hip_sf_adjoint(vp(q), npix, vp(atoms.atoms), vp(atoms.b),
+                                                segs.ctypes.data_as(C.c_void_p), atoms.nsegs, natoms, vp(ff), 3.0,
+                                                vp(F), vp(gI), vp(gp), vp(gb), None), "adjoint")
+    Fh = F.cpu().numpy().astype(np.float64)
+    some = np.sort(rng.choice(natoms, 24, replace=False))
+    rp, rb = oracle.sf_grad_given_f_f64(hkl, Fh[:, 0] + 1j * Fh[:, 1], Z, pos, g, some, atom_b=b if with_b else None,
+                                        B=3.0, threads=oracle_threads())
+    at = {int(o): i for i, o in enumerate(packed.perm)}
+    rows = [at[int(j)] for j in some]
+    e = rel_l2(gp.cpu().numpy()[rows], rp)
+    print(f"adjoint {n}: positions {e:.2e}", flush=True)
+    assert e < 2e-6
+    if want_b:
+        assert rel_l2(gb.cpu().numpy()[rows], rb) < 2e-6
