@@ -22,6 +22,8 @@ int ensure_device(int *cus);
 int workspace(size_t bytes, void **ptr);
 bool workspace_holds(size_t bytes);  // workspace(bytes) would not have to grow it
 void workspace_release();
+// Frees the idle buffers and streams of the host-array bridge on the current device.
+void bridge_release();
 
 // Streams the library forks independent work onto, kHelperStreams per device,
 // created at the first call at the default priority and kept until the process

@@ -158,6 +158,7 @@ int spsim_hip_default_form_factors(float *out) {
 
 int spsim_hip_release(void) {
   spsim::workspace_release();
+  spsim::bridge_release();
   return SPSIM_HIP_OK;
 }
 

@@ -63,6 +63,15 @@ int spsim_bridge_detector_chain(const spsim_hip_detector *det, const float *I, u
                                 float *thomson, float *solid_angle, float *photons, float *count, float *electrons,
                                 float *real_output, float *noiseless_output);
 
+/* A whole shot of a 2-D detector in one trip: q list, its rotation (hkl receives
+   the rotated list), structure factor by the grid kernels, detector chain. The
+   kernels and results are those of the separate calls above. */
+int spsim_bridge_shot(const spsim_hip_detector *det, const double *rot9, const spsim_hip_atom *atoms,
+                      const spsim_hip_segment *segs, int nsegs, int natoms, const float *ff, float b_global,
+                      uint64_t seed, uint64_t pattern, float *hkl, Complex *F, float *I, float *thomson,
+                      float *solid_angle, float *photons, float *count, float *electrons, float *real_output,
+                      float *noiseless_output);
+
 #ifdef __cplusplus
 }
 #endif

@@ -119,20 +119,23 @@ float *get_HKL_list_for_3d_detector(CCD *det, Experiment *exp, int *HKL_list_siz
   return list;
 }
 
-SpRotation *apply_orientation_to_HKL_list(float **HKL_list, int *HKL_list_size, Options *opts) {
-  SpRotation *rot;
+SpRotation *spsim_orientation(const Options *opts) {
+  if (opts->random_orientation) return sp_rot_uniform();
+  /* intrinsic rotation: the coordinate system is rotated, not the sample */
+  return sp_rot_euler(opts->euler_orientation[0], opts->euler_orientation[1], opts->euler_orientation[2]);
+}
+
+void spsim_rotate_list(float *list, int size, const SpRotation *rot) {
   double R[9];
-  if (!HKL_list || !HKL_list_size || !opts) return NULL;
-  if (opts->random_orientation) {
-    rot = sp_rot_uniform();
-  } else {
-    /* intrinsic rotation: the coordinate system is rotated, not the sample */
-    rot = sp_rot_euler(opts->euler_orientation[0], opts->euler_orientation[1], opts->euler_orientation[2]);
-  }
-  if (!rot) return NULL;
   for (int i = 0; i < 9; ++i) R[i] = (double)rot->data[i];
-  int rc = spsim_bridge_rotate_hkl(*HKL_list, *HKL_list_size, R);
+  int rc = spsim_bridge_rotate_hkl(list, size, R);
   if (rc != SPSIM_HIP_OK) spsim_report("apply_orientation_to_HKL_list", rc);
+}
+
+SpRotation *apply_orientation_to_HKL_list(float **HKL_list, int *HKL_list_size, Options *opts) {
+  if (!HKL_list || !HKL_list_size || !opts) return NULL;
+  SpRotation *rot = spsim_orientation(opts);
+  if (rot) spsim_rotate_list(*HKL_list, *HKL_list_size, rot);
   return rot;
 }
 
@@ -159,6 +162,16 @@ static void grid_dims(int size, const Options *opts, int *nx, int *ny) {
   if ((long long)n * n == size) *nx = *ny = n;
 }
 
+/* Amplitudes of the beam's illumination at every atom. */
+static void atom_amplitudes(const Molecule *mol, const Experiment *exp, int mode, float *amp) {
+  for (int j = 0; j < mol->natoms; ++j) {
+    const double il = illumination_function(exp, &mol->pos[3 * j]);
+    /* plain path: sqrt(illumination) (src/diffraction.c:834); the vector path
+       stores sqrt(illumination) and takes sqrt again (:886, :919-922). */
+    amp[j] = (mode == SPSIM_HIP_PACK_VECTOR) ? (float)sqrt((float)sqrt(il)) : (float)sqrt((float)il);
+  }
+}
+
 /* nsamples > 0 selects the wavelength-spectrum kernel with the given phase
    scales and weights (delta_atoms is then ignored, as the reference's spectrum
    kernel ignores it). */
@@ -182,12 +195,7 @@ static Diffraction_Pattern *compute_pattern(Molecule *mol, float *HKL_list, int 
   res->HKL_list_size = HKL_list_size;
   res->rot = NULL;
 
-  for (int j = 0; j < N; ++j) {
-    const double il = illumination_function(exp, &mol->pos[3 * j]);
-    /* plain path: sqrt(illumination) (src/diffraction.c:834); the vector path
-       stores sqrt(illumination) and takes sqrt again (:886, :919-922). */
-    amp[j] = (mode == SPSIM_HIP_PACK_VECTOR) ? (float)sqrt((float)sqrt(il)) : (float)sqrt((float)il);
-  }
+  atom_amplitudes(mol, exp, mode, amp);
   int natoms = 0, nsegs = 0;
   int rc = spsim_hip_pack_atoms(mol->atomic_number, mol->pos, amp, NULL, N, delta, mode, atoms, NULL, NULL, segs,
                                 &natoms, &nsegs);
@@ -296,6 +304,52 @@ fail:
   }
   free(atoms);
   return NULL;
+}
+
+Diffraction_Pattern *spsim_shot_pattern(const Molecule *mol, const Options *opts, const SpRotation *rot, int mode,
+                                        const spsim_hip_detector *p, uint64_t seed, uint64_t pattern,
+                                        float *const out[7]) {
+  const double t0 = now_seconds();
+  double R[9];
+  for (int i = 0; i < 9; ++i) R[i] = (double)rot->data[i];
+  const int N = mol->natoms, npix = p->nx * p->ny;
+  if (N < 0 || npix <= 0) return NULL;
+  Diffraction_Pattern *res = (Diffraction_Pattern *)calloc(1, sizeof(Diffraction_Pattern));
+  float *amp = (float *)malloc(sizeof(float) * (N > 0 ? N : 1));
+  spsim_hip_atom *atoms = (spsim_hip_atom *)malloc(sizeof(spsim_hip_atom) * (N > 0 ? N : 1));
+  spsim_hip_segment segs[SPSIM_HIP_NSPECIES];
+  int natoms = 0, nsegs = 0, rc = SPSIM_HIP_ERR_NOMEM;
+  if (res && amp && atoms) {
+    res->F = (Complex *)malloc(sizeof(Complex) * (size_t)npix + 1);
+    res->ints = (float *)malloc(sizeof(float) * (size_t)npix + 1);
+    res->HKL_list = (float *)malloc(sizeof(float) * 3 * (size_t)npix + 1);
+    res->HKL_list_size = npix;
+    if (res->F && res->ints && res->HKL_list) {
+      atom_amplitudes(mol, opts->experiment, mode, amp);
+      rc = spsim_hip_pack_atoms(mol->atomic_number, mol->pos, amp, NULL, N, opts->delta_atoms, mode, atoms, NULL, NULL,
+                                segs, &natoms, &nsegs);
+    }
+  }
+  if (rc == SPSIM_HIP_OK)
+    rc = spsim_bridge_shot(p, R, atoms, segs, nsegs, natoms, spsim_form_factor_table(), opts->b_factor, seed,
+                           pattern, res->HKL_list, res->F, res->ints, out[0], out[1], out[2], out[3], out[4], out[5],
+                           out[6]);
+  free(amp);
+  free(atoms);
+  if (rc != SPSIM_HIP_OK) {
+    if (res) {
+      free(res->F);
+      free(res->ints);
+      free(res->HKL_list);
+      free(res);
+    }
+    return NULL;
+  }
+  if (opts->verbosity_level > 0) {
+    const double dt = now_seconds() - t0;
+    printf("%g atoms.pixel/s\n", (double)npix * N / (dt > 0 ? dt : 1e-9));
+  }
+  return res;
 }
 
 void spsim_detector_params(const CCD *det, const Experiment *exp, spsim_hip_detector *p) {

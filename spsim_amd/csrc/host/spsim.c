@@ -2,7 +2,8 @@
  * Drop-in pipeline driver (reference src/spsim.c:84-371).
  *
  * simulate_shot keeps the reference's order (q list, orientation, structure
- * factor, detector chain) and fills the same CCD arrays, but runs the whole
+ * factor, detector chain) and fills the same CCD arrays, but runs a shot of a
+ * 2-D detector in one trip to the device (spsim_bridge_shot), and the whole
  * detector chain as one fused GPU pass (spsim_hip_detector_chain) that is
  * bit-identical to calling the stages one by one with the same noise counters.
  * As in the reference, the previous shot's CCD arrays are replaced without
@@ -138,50 +139,69 @@ Diffraction_Pattern *simulate_shot(Molecule *mol, Options *opts) {
     fprintf(stderr, "spsim: simulate_shot: loading patterns from sf_filename is not supported\n");
     return NULL;
   }
-  float *HKL_list = get_HKL_list(opts, &HKL_list_size);
-  if (!HKL_list) return NULL;
-  SpRotation *rot = apply_orientation_to_HKL_list(&HKL_list, &HKL_list_size, opts);
-  Diffraction_Pattern *pattern = compute_sf(mol, HKL_list, HKL_list_size, opts);
-  free(HKL_list);
-  if (!pattern) {
-    free(rot);
-    return NULL;
-  }
-  pattern->rot = rot;
-  gaussian_blur_pattern(opts, pattern);
-
   CCD *det = opts->detector;
   spsim_hip_detector p;
   spsim_detector_params(det, opts->experiment, &p);
   const int nz = p.nz > 0 ? p.nz : 1, bz = p.bin_z > 0 ? p.bin_z : 1;
-  const size_t n = (size_t)det->nx * det->ny * nz;
+  const size_t n = (size_t)(det->nx > 0 ? det->nx : 0) * (det->ny > 0 ? det->ny : 0) * nz;
   const size_t nb = (size_t)(det->nx / p.bin_x) * (det->ny / p.bin_y) * (nz / bz);
-  float *th = (float *)malloc(sizeof(float) * n + 1), *om = (float *)malloc(sizeof(float) * n + 1);
-  float *ph = (float *)malloc(sizeof(float) * n + 1), *cnt = (float *)malloc(sizeof(float) * n + 1);
-  float *el = (float *)malloc(sizeof(float) * n + 1);
-  float *real = (float *)malloc(sizeof(float) * nb + 1), *nl = (float *)malloc(sizeof(float) * nb + 1);
-  int rc = SPSIM_HIP_ERR_NOMEM;
-  if (th && om && ph && cnt && el && real && nl)
-    rc = spsim_bridge_detector_chain(&p, pattern->ints, spsim_noise_seed(), spsim_next_shot_pattern(), th, om, ph, cnt,
-                                     el, real, nl);
-  if (rc != SPSIM_HIP_OK) {
-    spsim_report("simulate_shot (detector chain)", rc);
-    free(th);
-    free(om);
-    free(ph);
-    free(cnt);
-    free(el);
-    free(real);
-    free(nl);
-    return pattern;
+  float *out[7]; /* thomson, solid angle, photons, count, electrons, real, noiseless */
+  int allocated = 1;
+  for (int i = 0; i < 7; ++i) {
+    out[i] = (float *)malloc(sizeof(float) * (i < 5 ? n : nb) + 1);
+    allocated = allocated && out[i];
   }
-  det->thomson_correction = th;
-  det->solid_angle = om;
-  det->photons_per_pixel = ph;
-  det->photon_count = cnt;
-  det->electrons_per_pixel = el;
-  det->real_output = real;
-  det->noiseless_output = nl;
+
+  /* The common shot, a direct structure factor on a 2-D detector, makes one trip
+     to the device. Everything else, and whatever that cannot run, goes stage by
+     stage, which reports its errors. */
+  Diffraction_Pattern *pattern = NULL;
+  SpRotation *rot = NULL;
+  uint64_t shot = 0;
+  int have_shot = 0;
+  const int spectrum = opts->use_cuda && opts->experiment->bandwidth != 0 && opts->wavelength_samples > 1;
+  if (allocated && n > 0 && nz == 1 && !opts->use_fft_for_sf && !opts->use_nfft_for_sf && !spectrum) {
+    rot = spsim_orientation(opts);
+    if (rot) {
+      const int mode = opts->vectorize && !opts->use_cuda ? SPSIM_HIP_PACK_VECTOR : SPSIM_HIP_PACK_PLAIN;
+      shot = spsim_next_shot_pattern();
+      have_shot = 1;
+      pattern = spsim_shot_pattern(mol, opts, rot, mode, &p, spsim_noise_seed(), shot, out);
+    }
+  }
+  int rc = SPSIM_HIP_OK;
+  if (!pattern) {
+    float *HKL_list = get_HKL_list(opts, &HKL_list_size);
+    if (HKL_list && !rot)
+      rot = apply_orientation_to_HKL_list(&HKL_list, &HKL_list_size, opts);
+    else if (HKL_list)
+      spsim_rotate_list(HKL_list, HKL_list_size, rot);
+    if (HKL_list) pattern = compute_sf(mol, HKL_list, HKL_list_size, opts);
+    free(HKL_list);
+    if (pattern && !have_shot) shot = spsim_next_shot_pattern();
+    if (pattern)
+      rc = allocated ? spsim_bridge_detector_chain(&p, pattern->ints, spsim_noise_seed(), shot, out[0], out[1], out[2],
+                                                   out[3], out[4], out[5], out[6])
+                     : SPSIM_HIP_ERR_NOMEM;
+  }
+  if (!pattern || rc != SPSIM_HIP_OK) {
+    if (pattern) spsim_report("simulate_shot (detector chain)", rc);
+    for (int i = 0; i < 7; ++i) free(out[i]);
+    if (!pattern) {
+      free(rot);
+      return NULL;
+    }
+  }
+  pattern->rot = rot;
+  gaussian_blur_pattern(opts, pattern);
+  if (rc != SPSIM_HIP_OK) return pattern;
+  det->thomson_correction = out[0];
+  det->solid_angle = out[1];
+  det->photons_per_pixel = out[2];
+  det->photon_count = out[3];
+  det->electrons_per_pixel = out[4];
+  det->real_output = out[5];
+  det->noiseless_output = out[6];
   return pattern;
 }
 

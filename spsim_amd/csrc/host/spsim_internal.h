@@ -5,6 +5,8 @@
 #include <stdint.h>
 
 #include "config.h"
+#include "diffraction.h"
+#include "molecule.h"
 #include "spsim_hip.h"
 
 #ifdef __cplusplus
@@ -21,6 +23,15 @@ uint64_t spsim_next_shot_pattern(void);
 const float *spsim_form_factor_table(void);
 /* Fills the detector-chain parameters from the reference structs; exp may be NULL. */
 void spsim_detector_params(const CCD *det, const Experiment *exp, spsim_hip_detector *p);
+/* The orientation that opts ask for, and its application to a q list. */
+SpRotation *spsim_orientation(const Options *opts);
+void spsim_rotate_list(float *list, int size, const SpRotation *rot);
+/* One shot in one device trip (spsim_bridge_shot): the pattern (rot unset) with
+   the detector chain's outputs in out[7] (thomson .. noiseless, arrays of the
+   caller). Null, without a report, when it cannot be run that way. */
+Diffraction_Pattern *spsim_shot_pattern(const Molecule *mol, const Options *opts, const SpRotation *rot, int mode,
+                                        const spsim_hip_detector *p, uint64_t seed, uint64_t pattern,
+                                        float *const out[7]);
 /* Reports a failed device call on stderr (the reference API has no status codes). */
 void spsim_report(const char *what, int rc);
 

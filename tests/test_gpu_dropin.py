@@ -269,3 +269,87 @@ def test_atomsf_lib_override_intensity(gpu, tmp_path):
     assert rel_l2(I, I_ref) < 1e-5
     _, I_builtin = oracle.sf_f64(q, Z, pos, B=2.5)
     assert rel_l2(I_builtin, I_ref) > 1e-2  # the override changes the pattern
+
+
+@pytest.mark.parametrize("nx,ny,binning,cx,cuda", [(48, 48, 1, 0.0, 1), (37, 52, 2, 1e-3, 0), (300, 290, 2, 0.0, 1)])
+def test_one_trip_shot_equals_the_stages(gpu, nx, ny, binning, cx, cuda):
+    """simulate_shot (one device trip; staged and, at 300 x 290, separate copies)
+    gives the bits of the calls it stands for, made one by one, shot after shot."""
+    opts = make_opts(48)
+    d, e = opts.detector, opts.experiment
+    d.nx, d.ny, d.center_x = nx, ny, cx
+    d.width, d.height = float(np.float32(nx * 2e-4)), float(np.float32(ny * 2e-4))
+    d.binning_x = d.binning_y = binning
+    e.beam_intensity, e.polarization = 1e25, 3
+    d.quantum_efficiency, d.readout_noise = 0.5, 2.0
+    opts.random_orientation, opts.use_cuda = 1, cuda
+    Z, pos, mol = molecule(700, seed=4)
+    n, nb = nx * ny, (nx // binning) * (ny // binning)
+    spsim.sp_srand(5)
+    shots = []
+    for _ in range(2):
+        pat = spsim.simulate_shot(mol, opts)
+        shots.append([spsim.float_array(pat.HKL_list, 3 * n), spsim.float_array(pat.ints, n),
+                      spsim.complex_array(pat.F, n), spsim.float_array(d.photon_count, n),
+                      spsim.float_array(d.electrons_per_pixel, n), spsim.float_array(d.real_output, nb),
+                      spsim.float_array(d.noiseless_output, nb), [pat.rot.data[i] for i in range(9)]])
+        spsim.free_diffraction_pattern(pat)
+        spsim.free_output_in_options(opts)
+    spsim.sp_srand(5)
+    for shot in shots:
+        ptr, size, _ = hkl_of(opts)
+        pp, nn = C.pointer(ptr), C.c_int(size)
+        rot = spsim.apply_orientation_to_HKL_list(pp, C.byref(nn), opts)
+        pat = spsim.compute_sf(mol, ptr, size, opts)
+        spsim.calculate_photons_per_pixel(pat, opts)
+        spsim.generate_poisson_noise(d)
+        spsim.calculate_electrons_per_pixel(d, e)
+        spsim.calculate_real_detector_output(d, e)
+        spsim.calculate_noiseless_detector_output(d, e)
+        staged = [spsim.float_array(pat.HKL_list, 3 * n), spsim.float_array(pat.ints, n),
+                  spsim.complex_array(pat.F, n), spsim.float_array(d.photon_count, n),
+                  spsim.float_array(d.electrons_per_pixel, n), spsim.float_array(d.real_output, nb),
+                  spsim.float_array(d.noiseless_output, nb), [rot.data[i] for i in range(9)]]
+        for a, b in zip(shot, staged):
+            np.testing.assert_array_equal(a, b)
+        spsim.free_diffraction_pattern(pat)
+        spsim.free_output_in_options(opts)
+
+
+def test_threads_share_the_bridge(gpu):
+    """Drop-in calls of several threads, each with its own sizes, give what they
+    give one after another; releasing the library's buffers between them changes
+    nothing."""
+    import threading
+
+    from spsim_amd import _lib
+
+    def chain(n, seed):
+        p = _lib.DetectorParams(nx=n, ny=n, bin_x=1, bin_y=1, width=n * 2e-4, height=n * 2e-4, distance=0.1,
+                                pixel_width=2e-4, pixel_height=2e-4, beam_intensity=1e24, quantum_efficiency=0.5,
+                                wavelength=2e-10, nz=1, bin_z=1)
+        I = np.random.default_rng(seed).exponential(1e4, n * n).astype(np.float32)
+        out = [np.zeros(n * n, np.float32) for _ in range(7)]
+        fp = C.POINTER(C.c_float)
+        rc = _lib.load().spsim_bridge_detector_chain(C.byref(p), I.ctypes.data_as(fp), C.c_uint64(seed), C.c_uint64(1),
+                                                     *[o.ctypes.data_as(fp) for o in out])
+        assert rc == 0
+        return out
+
+    sizes = [(40, 1), (333, 2), (64, 3), (700, 4), (91, 5), (128, 6)]
+    want = [chain(*s) for s in sizes]
+    _lib.load().spsim_hip_release()
+    got = [None] * len(sizes)
+
+    def work(i):
+        for _ in range(3):
+            got[i] = chain(*sizes[i])
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(len(sizes))]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    for a, b in zip(want, got):
+        for x, y in zip(a, b):
+            np.testing.assert_array_equal(x, y)
