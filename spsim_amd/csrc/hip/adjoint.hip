@@ -265,7 +265,8 @@ extern "C" int spsim_hip_sf_adjoint(const float *d_hkl, int npix, const spsim_hi
   const int side = (int)std::lround(std::sqrt((double)npix));
   const bool smooth = (long long)side * side == npix && surf_worth(side, side, natoms, 500000000LL);
   const size_t segs_bytes = (((size_t)nsegs * sizeof(spsim_hip_segment) + 255) / 256) * 256;
-  const int node_splits = (int)std::max<long long>(1, std::min<long long>(32, (4LL * cus + tiles.size() - 1) / (long long)tiles.size()));
+  // one round of the node sums' workgroups (four resident per CU)
+  const int node_splits = (int)std::max<long long>(1, std::min<long long>(32, 4LL * cus / (long long)tiles.size()));
   const size_t partial_bytes = sizeof(double4) * (size_t)nsplit * natoms;
   const size_t node_bytes = smooth ? sizeof(double4) * (size_t)node_splits * natoms : 0;
   const size_t head = tiles_bytes + segs_bytes + partial_bytes + node_bytes;

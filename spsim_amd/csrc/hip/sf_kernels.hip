@@ -947,8 +947,8 @@ PatternLaunch make_launch(const float *d_hkl, int npix, const spsim_hip_atom *d_
 // decides on the device, without a host round trip), and by the direct kernel
 // `kind` otherwise, which is launched behind it and finds the outputs written.
 // Both use the library workspace, the direct sums' partials past the flag.
-// The interpolation's eight launches take about 60 us, the direct sums that from
-// about min_terms on.
+// The interpolation's launches take about 70 us, the direct sums that from about
+// min_terms on.
 int launch_smooth(Kind kind, const PatternLaunch &a, int nx, int ny, const spsim_hip_tile &t, int splits, int cus,
                   long long min_terms, const Spectrum *spec, hipStream_t s) {
   if (!surf_worth(nx, ny, a.natoms, min_terms)) return launch_single(kind, a, nx, ny, t, splits, s, spec);

@@ -10,8 +10,10 @@
 //
 //  1. Surface. q(x, y) is replaced by the polynomial qs(u, v) through 16 x 16
 //     of its pixels (Chebyshev form, FP64). What the list has beyond it,
-//     d = q - qs, is the FP32 rounding of the list and must be small:
-//     2 pi R |d| <= 2e-4 at every pixel, otherwise the list is not taken.
+//     d = q - qs, is the FP32 rounding of the list, resolved along the surface's
+//     tangents and a fixed normal n, d = alpha dqs/du + beta dqs/dv + gamma n.
+//     It must be small, 2 pi R |d| <= 2e-4 at every pixel, otherwise the list is
+//     not taken.
 //  2. Nodes. u_i = asin(a cos t_i) / asin(a), t_i = (2 i + 1) pi / (2 n), the
 //     Chebyshev points stretched towards even spacing (Kosloff & Tal-Ezer,
 //     J. Comput. Phys. 104 (1993) 457), with a = 1 / cosh(20.7 / n), so that
@@ -19,17 +21,20 @@
 //     exp(i theta u) fall off like Bessel functions beyond theta:
 //     n = theta + 4 theta^(1/3) + 8 leaves 1e-9..1e-8 of |F| (measured against
 //     FP64 sums), a tenth of the FP32 sums' own error.
-//  3. Node sums. F and its gradient G = dF/dq at the nodes, by the arithmetic
+//  3. Node sums. F and its derivative N = n.dF/dq at the nodes, by the arithmetic
 //     of the direct kernels (FP64 phase reduced to turns, FP32 sine and
-//     cosine, FP32 sums over 64 atoms folded into FP64).
+//     cosine, FP32 sums over 64 atoms folded into FP64). On a square detector
+//     centred on the beam the nodes come in octants, as its pixels do in the
+//     octant kernel (sf_kernels.hip).
 //  4. Interpolation along the rows, then along the columns: two small dense
-//     products with FP64 weights for F (FP32 for G), then per pixel
-//     F(q) = e^{-2 pi i q.r0} (F(qs) + d.G(qs)),
+//     products with FP64 weights for F (FP32 for N and for the derivatives of F,
+//     whose weights are the derivatives of F's), then per pixel
+//     F(q) = e^{-2 pi i q.r0} (F + alpha dF/du + beta dF/dv + gamma N)(u, v),
 //     which takes the list's rounding into account to first order (second
 //     order: (2 pi R |d|)^2 / 2 <= 2e-8).
 //
-// The cost is n_x n_y natoms terms instead of npix natoms: 35 times fewer on
-// 100,000 atoms x 1024^2 at 0.15 nm (n = 160). The interpolation weights add
+// The cost is n_x n_y natoms terms instead of npix natoms: 30 times fewer on
+// 100,000 atoms x 1024^2 at 0.15 nm (n = 188). The interpolation weights add
 // no error of their own: the sum of their squares is 1 at every pixel.
 #include "surface.hpp"
 
@@ -50,7 +55,11 @@ constexpr double kPi = 3.14159265358979323846;
 constexpr float kStretch = 20.7f;       // -ln of the node map's own error
 constexpr double kMaxPhaseDev = 2e-4;   // largest 2 pi R |q - surface|
 constexpr double kMaxSpreadDev = 3e-7;  // the same times the spectrum's largest |s_k / sc - 1|
-constexpr float kMinWeakest = 0.02f;    // see surf_terms
+constexpr float kMinWeakest = 0.02f;    // see species_terms
+// v_cos_f32 and v_sin_f32 round towards zero: |e^{-i phi}| is short by 3.22e-8 on
+// average over the phases (2^26 random ones against FP64), coherently where the
+// atoms scatter in phase, so the form factors make up for it.
+constexpr double kTrigBias = 3.22e-8;
 constexpr float kMaxGauss = 60.0f;      // largest exponent B s^2 over the detector
 
 // a-th of the kSurfDeg sample pixels of an axis: the pixel nearest to the
@@ -61,14 +70,14 @@ __device__ __forceinline__ int sample_pixel(int a, int n) {
 __device__ __forceinline__ double pixel_u(int x, int n) { return (2.0 * x - (n - 1)) / (double)(n - 1); }
 
 // Largest (sum for SUM) of N values over the workgroup, given to every thread.
-template <int N, bool SUM = false>
-__device__ __forceinline__ void block_reduce(double (&v)[N]) {
-  __shared__ double part[kT / 64][N];
+template <int N, bool SUM = false, class T = double>
+__device__ __forceinline__ void block_reduce(T (&v)[N]) {
+  __shared__ T part[kT / 64][N];
 #pragma unroll
   for (int i = 0; i < N; ++i)
     for (int o = 32; o > 0; o >>= 1) {
-      const double w = __shfl_xor(v[i], o);
-      v[i] = SUM ? v[i] + w : fmax(v[i], w);
+      const T w = __shfl_xor(v[i], o);
+      v[i] = SUM ? v[i] + w : (v[i] < w ? w : v[i]);
     }
   __syncthreads();
   if ((threadIdx.x & 63) == 0)
@@ -77,7 +86,7 @@ __device__ __forceinline__ void block_reduce(double (&v)[N]) {
 #pragma unroll
   for (int i = 0; i < N; ++i) {
     v[i] = part[0][i];
-    for (int w = 1; w < kT / 64; ++w) v[i] = SUM ? v[i] + part[w][i] : fmax(v[i], part[w][i]);
+    for (int w = 1; w < kT / 64; ++w) v[i] = SUM ? v[i] + part[w][i] : (v[i] < part[w][i] ? part[w][i] : v[i]);
   }
 }
 
@@ -121,7 +130,7 @@ __device__ void sample_to_chebyshev(const double *us, const double *cosines, dou
 __device__ __forceinline__ void clenshaw3(const double (*c)[3], double u, double out[3]) {
   double b1[3] = {0, 0, 0}, b2[3] = {0, 0, 0};
   const double u2 = 2.0 * u;
-#pragma unroll
+#pragma unroll 5
   for (int m = D - 1; m >= 1; --m) {
 #pragma unroll
     for (int k = 0; k < 3; ++k) {
@@ -134,8 +143,8 @@ __device__ __forceinline__ void clenshaw3(const double (*c)[3], double u, double
   for (int k = 0; k < 3; ++k) out[k] = __builtin_fma(u, b1[k], c[0][k] - b2[k]);
 }
 
-// Coefficients along u of the surface's line v (or of its derivative in v):
-// row[m][k] = sum_n T_n(v) coef[n][m][k]. Threads 0..47.
+// Coefficients along u of the surface's line v: row[m][k] = sum_n T_n(v) coef[n][m][k].
+// Threads 0..47.
 __device__ __forceinline__ void surface_row(const double (*coef)[D][3], double v, double (*row)[3]) {
   if (threadIdx.x < 3 * D) {
     const int m = threadIdx.x / 3, k = threadIdx.x % 3;
@@ -148,6 +157,92 @@ __device__ __forceinline__ void surface_row(const double (*coef)[D][3], double v
     }
     row[m][k] = s;
   }
+}
+
+// The same of dq/dv: sum_n n U_{n-1}(v) coef[n][m][k]. Threads 64..111.
+__device__ __forceinline__ void surface_row_dv(const double (*coef)[D][3], double v, float (*row)[3]) {
+  const int t = (int)threadIdx.x - 64;
+  if (t >= 0 && t < 3 * D) {
+    const int m = t / 3, k = t % 3;
+    double u0 = 0.0, u1 = 1.0, s = 0.0;
+    for (int n = 1; n < D; ++n) {
+      s = __builtin_fma(n * u1, coef[n][m][k], s);
+      const double u2 = __builtin_fma(2.0 * v, u1, -u0);
+      u0 = u1;
+      u1 = u2;
+    }
+    row[m][k] = (float)s;
+  }
+}
+
+// The tangents at u of a line (coefficients c of q, cv of dq/dv), in FP32.
+__device__ __forceinline__ void tangents(const double (*c)[3], const float (*cv)[3], float u, float qu[3],
+                                         float qv[3]) {
+  float a1[3] = {0, 0, 0}, a2[3] = {0, 0, 0}, b1[3] = {0, 0, 0}, b2[3] = {0, 0, 0};
+  const float u2 = 2.0f * u;
+#pragma unroll 3
+  for (int m = D - 1; m >= 1; --m) {
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+      const float a = __builtin_fmaf(u2, a1[k], (float)m * (float)c[m][k] - a2[k]);  // sum m c_m U_{m-1}
+      a2[k] = a1[k];
+      a1[k] = a;
+      const float b = __builtin_fmaf(u2, b1[k], cv[m][k] - b2[k]);
+      b2[k] = b1[k];
+      b1[k] = b;
+    }
+  }
+#pragma unroll
+  for (int k = 0; k < 3; ++k) {
+    qu[k] = a1[k];
+    qv[k] = __builtin_fmaf(u, b1[k], cv[0][k] - b2[k]);
+  }
+}
+
+__device__ __forceinline__ void cross(const float a[3], const float b[3], float c[3]) {
+  c[0] = a[1] * b[2] - a[2] * b[1];
+  c[1] = a[2] * b[0] - a[0] * b[2];
+  c[2] = a[0] * b[1] - a[1] * b[0];
+}
+__device__ __forceinline__ float dot(const float a[3], const float b[3]) { return a[0] * b[0] + a[1] * b[1] + a[2] * b[2]; }
+
+// Makes the surface of a detector centred on the beam exactly symmetric: q_x
+// odd in u and even in v, q_y even and odd, q_z even in both; and, on a square
+// one, q_x(u, v) = q_y(v, u). Coefficients that break it by their rounding
+// alone are dropped (what they stood for moves to the deviations). Returns 2,
+// 1 (no transposed symmetry) or 0 (none). The normal is that of the middle.
+__device__ int symmetrise(double (*Q)[D][3], bool square, float normal[3]) {
+  const int n = threadIdx.x / D, m = threadIdx.x % D;  // T_n(v) T_m(u)
+  const double x = Q[n][m][0], y = Q[n][m][1], z = Q[n][m][2];
+  const bool om = m & 1, on = n & 1;
+  // dq/du and dq/dv at u = v = 0 (T_n(0) = cos(n pi / 2), U_{m-1}(0) = sin(m pi / 2)),
+  // the coefficients that mirrors and the transposition forbid, all coefficients
+  const double au = om && !on ? ((m / 2 + n / 2) & 1 ? -m : m) : 0.0;
+  const double av = on && !om ? ((m / 2 + n / 2) & 1 ? -n : n) : 0.0;
+  float v[9] = {(float)(au * x),
+                (float)(au * y),
+                (float)(au * z),
+                (float)(av * x),
+                (float)(av * y),
+                (float)(av * z),
+                (float)((om && !on ? 0.0 : fabs(x)) + (on && !om ? 0.0 : fabs(y)) + (om || on ? fabs(z) : 0.0)),
+                (float)(fabs(x - Q[m][n][1]) + fabs(z - Q[m][n][2])),
+                (float)(fabs(x) + fabs(y) + fabs(z))};
+  block_reduce<9, true>(v);
+  const int sym = v[6] <= 1e-6f * v[8] ? (square && v[7] <= 1e-6f * v[8] ? 2 : 1) : 0;
+  const double xt = Q[m][n][1], yt = Q[m][n][0], zt = Q[m][n][2];
+  __syncthreads();
+  if (sym > 0) {
+    Q[n][m][0] = om && !on ? (sym == 2 ? 0.5 * (x + xt) : x) : 0.0;
+    Q[n][m][1] = on && !om ? (sym == 2 ? 0.5 * (y + yt) : y) : 0.0;
+    Q[n][m][2] = om || on ? 0.0 : (sym == 2 ? 0.5 * (z + zt) : z);
+  }
+  __syncthreads();
+  cross(v, v + 3, normal);
+  if (sym > 0) normal[0] = normal[1] = 0.0f;
+  const float len = sqrtf(dot(normal, normal));
+  for (int k = 0; k < 3; ++k) normal[k] /= len;
+  return sym;
 }
 
 struct ScanArgs {
@@ -168,6 +263,7 @@ struct ScanArgs {
 __device__ void scan_list(const ScanArgs &a) {
   __shared__ double C[2][D][D], tmp[D][D], Q[D][D][3], P[D][D][3], row[D][3], us[2][D], cosines[2 * D + 1];
   __shared__ int px[2][D];
+  __shared__ float row_v[D][3];
   const int t = threadIdx.x, b = t / D, i = t % D;
   if (t < 2 * D) {
     const int n = b ? a.ny : a.nx;
@@ -200,6 +296,8 @@ __device__ void scan_list(const ScanArgs &a) {
     Q[b][i][k] = s;
   }
   __syncthreads();
+  float normal[3];
+  const int sym = symmetrise(Q, a.nx == a.ny, normal);
   const int rows = a.list_blocks - 2;  // workgroups that take the list's rows
   if ((int)blockIdx.x >= rows) {
     // slopes along one axis on the kLines x kLines Lobatto points: T_m and
@@ -242,33 +340,47 @@ __device__ void scan_list(const ScanArgs &a) {
     }
     __syncthreads();
     if (t < kLines) (along_y ? a.fit->slope_y : a.fit->slope_x)[t] = __uint_as_float(smax[t]);
-    if (t == 0) a.records[blockIdx.x] = SurfRecord{{0, 0, 0}, 0.0, 0.0f, 0.0f, 0, 0};
+    if (t == 0) a.records[blockIdx.x] = SurfRecord{0.0, 0.0, 0.0f, 0.0f, 0, 0};
     if (!along_y) {
-      if (t == 0) a.fit->s2max = (float)s2[0];
+      if (t == 0) {
+        a.fit->s2max = (float)s2[0];
+        a.fit->sym = sym;
+        for (int k = 0; k < 3; ++k) a.fit->normal[k] = normal[k];
+      }
       for (int c = t; c < D * D * 3; c += kT) (&a.fit->coef[0][0][0])[c] = (&Q[0][0][0])[c];
     }
     return;
   }
-  double m[4] = {0, 0, 0, 0};
+  double m[2] = {0, 0};
   for (int y = blockIdx.x; y < a.ny; y += rows) {
     __syncthreads();
     surface_row(Q, pixel_u(y, a.ny), row);
+    surface_row_dv(Q, pixel_u(y, a.ny), row_v);
     __syncthreads();
     for (int x = t; x < a.nx; x += kT) {
       double s[3];
-      clenshaw3(row, pixel_u(x, a.nx), s);
+      float qu[3], qv[3], d[3], uv[3], vn[3], nu[3];
+      const double u = pixel_u(x, a.nx);
+      clenshaw3(row, u, s);
+      tangents(row, row_v, (float)u, qu, qv);
       const size_t p = 3 * ((size_t)y * a.nx + x);
 #pragma unroll
-      for (int k = 0; k < 3; ++k) {
-        const double d = (double)a.hkl[p + k] - s[k];
-        a.dev[p + k] = (float)d;
-        if (!(fabs(d) < 1e30)) m[3] = 1.0;
-        m[k] = fmax(m[k], fabs(d));
-      }
+      for (int k = 0; k < 3; ++k) d[k] = (float)((double)a.hkl[p + k] - s[k]);
+      cross(qu, qv, uv);
+      cross(qv, normal, vn);
+      cross(normal, qu, nu);
+      const float inv = 1.0f / dot(qu, vn);
+      const float al = dot(d, vn) * inv, be = dot(d, nu) * inv, ga = dot(d, uv) * inv;
+      a.dev[p] = al;
+      a.dev[p + 1] = be;
+      a.dev[p + 2] = ga;
+      const float size = fabsf(al) * sqrtf(dot(qu, qu)) + fabsf(be) * sqrtf(dot(qv, qv)) + fabsf(ga);
+      if (!(size < 1e30f)) m[1] = 1.0;
+      m[0] = fmax(m[0], (double)size);
     }
   }
   block_reduce(m);
-  if (t == 0) a.records[blockIdx.x] = SurfRecord{{m[0], m[1], m[2]}, 0.0, 0.0f, 0.0f, m[3] > 0.0, 0};
+  if (t == 0) a.records[blockIdx.x] = SurfRecord{m[0], 0.0, 0.0f, 0.0f, m[1] > 0.0, 0};
 }
 
 // The molecule's centre is the mean of 1024 evenly spaced atoms: any point near
@@ -309,10 +421,10 @@ __device__ void scan_atoms(const ScanArgs &a) {
   }
   block_reduce(m);
   if (t == 0)
-    a.records[blockIdx.x] = SurfRecord{{0, 0, 0}, m[0], (float)-m[1], (float)m[2], m[3] > 0.0, 0};
+    a.records[blockIdx.x] = SurfRecord{0.0, m[0], (float)-m[1], (float)m[2], m[3] > 0.0, 0};
 }
 
-__global__ __launch_bounds__(kT) void surface_scan_kernel(ScanArgs a) {
+__global__ __launch_bounds__(kT, 3) void surface_scan_kernel(ScanArgs a) {
   if ((int)blockIdx.x < a.list_blocks)
     scan_list(a);
   else
@@ -351,10 +463,10 @@ enum class SurfKind { kSum, kSpectrum, kAdjoint };
 
 __host__ __device__ inline bool worth(double nodes_x, double nodes_y, double nx, double ny, double natoms,
                                       SurfKind kind) {
-  // Issue cycles per lane: a term of the node sums 80 (160 with a spectrum, 120
+  // Issue cycles per lane: a term of the node sums 60 (140 with a spectrum, 100
   // in the adjoint), of the direct sums 26 to 45 (130, 109); the interpolation
   // 25 per node row and pixel. Measured on the MI355X.
-  const double node = kind == SurfKind::kSum ? 80.0 : (kind == SurfKind::kSpectrum ? 160.0 : 120.0);
+  const double node = kind == SurfKind::kSum ? 60.0 : (kind == SurfKind::kSpectrum ? 140.0 : 100.0);
   const double direct = kind == SurfKind::kSum ? 26.0 : (kind == SurfKind::kSpectrum ? 130.0 : 109.0);
   const double surf = nodes_x * nodes_y * natoms * node + 25.0 * (nx * ny * nodes_y + nx * nodes_x * nodes_y);
   return surf < 0.8 * direct * nx * ny * natoms;
@@ -384,12 +496,12 @@ __host__ __device__ inline void species_terms(const float *c, float Bs, float bm
   *weakest = ratio < *weakest || !(ratio < 1e30f) ? (ratio < 1e30f ? ratio : 0.0f) : *weakest;
 }
 
-// Atom records of the node sums: position relative
-// to the centre, rotated (FP64), and the amplitude with its products with the
-// position; with per-atom B, v holds log2 of the amplitude, B and the position.
+// Atom records of the node sums: position relative to the centre, rotated
+// (FP64), the amplitude w and its product with n.r; with per-atom B, log2 of the
+// amplitude, n.r and B.
 struct __align__(16) NodeAtom {
   double x, y, z;
-  float v[6];
+  float w, n, b, pad;
 };
 static_assert(sizeof(NodeAtom) == 48, "node-sum atom record");
 
@@ -409,31 +521,64 @@ __device__ __forceinline__ void prepare_atoms(const SurfJob &jb, bool has_b, int
       r.y = y;
       r.z = z;
     }
-    const float xf = (float)r.x, yf = (float)r.y, zf = (float)r.z;
-    if (has_b) {
-      r.v[0] = log2f(at.w);
-      r.v[1] = xf;
-      r.v[2] = yf;
-      r.v[3] = zf;
-      r.v[4] = jb.atom_b[j];
-    } else {
-      r.v[0] = at.w;
-      r.v[1] = at.w * xf;
-      r.v[2] = at.w * yf;
-      r.v[3] = at.w * zf;
-      r.v[4] = 0.0f;
-    }
-    r.v[5] = 0.0f;
+    const float n = jb.normal[0] * (float)r.x + jb.normal[1] * (float)r.y + jb.normal[2] * (float)r.z;
+    r.w = has_b ? log2f(at.w) : at.w;
+    r.n = has_b ? n : at.w * n;
+    r.b = has_b ? jb.atom_b[j] : 0.0f;
+    r.pad = 0.0f;
     out[j] = r;
   }
 }
 
-// Nodes per lane of the node sums: four share an atom's LDS read (2.27 ms
-// against 2.42 ms for two on 35,344 nodes x 100,000 atoms); fewer make more work
-// items (two: 17.6 us against 24 us on 1024 nodes x 5,000 atoms).
-__host__ __device__ inline int surf_per_lane(long long nodes, long long natoms) {
-  const long long terms = nodes * natoms;
-  return terms >= 1LL << 28 ? 4 : (terms >= 1LL << 25 ? 2 : 1);
+// Octants of an n x n node grid (n even).
+__host__ __device__ inline int node_octants(int n) { return n / 2 * (n / 2 + 1) / 2; }
+
+// Nodes per lane of the node sums and tiles of 256 lanes. An octant (8 nodes)
+// shares phases between its nodes: 321 issue cycles per atom against 57 per
+// node alone; four nodes per lane share an atom's LDS read (one: 75). The tiling
+// with the least work; on few terms one node per lane, for the most work items
+// (on 1024 nodes x 5,000 atoms, 13 us against 24 us with four).
+__host__ __device__ inline void node_tiling(int nx, int ny, bool octants, long long natoms, int *per_lane, int *tiles) {
+  const int nodes = nx * ny;
+  if (nodes * natoms < 1LL << 25) {
+    *per_lane = 1;
+    *tiles = (nodes + kT - 1) / kT;
+    return;
+  }
+  const int t2 = (nodes + 2 * kT - 1) / (2 * kT), t4 = (nodes + 4 * kT - 1) / (4 * kT);
+  const int t8 = (node_octants(nx) + kT - 1) / kT;
+  *per_lane = t4 * 228 <= t2 * 120 ? 4 : 2;
+  *tiles = *per_lane == 4 ? t4 : t2;
+  if (octants && t8 * 321 < *tiles * (*per_lane == 4 ? 228 : 120)) {
+    *per_lane = 8;
+    *tiles = t8;
+  }
+}
+
+// Node e of a lane, of a work item's tile: its index, or -1 where there is none.
+// Octant t stands for the node (x, y), x <= y = the row of t in the triangle,
+// its mirrors, and the transposed node with its mirrors.
+__device__ __forceinline__ void octant_node(int t, int &x, int &y) {
+  int yy = (int)((sqrtf(8.0f * (float)t + 1.0f) - 1.0f) * 0.5f);
+  while ((yy + 1) * (yy + 2) / 2 <= t) ++yy;
+  while (yy * (yy + 1) / 2 > t) --yy;
+  y = yy;
+  x = t - yy * (yy + 1) / 2;
+}
+__device__ __forceinline__ int node_index(const SurfJob &jb, int tile, int e, int lane) {
+  const int nyn = jb.sh.ay.n;
+  if (jb.per_lane == 8) {
+    const int t = tile * kT + lane;
+    if (t >= node_octants(nyn)) return -1;
+    int x, y;
+    octant_node(t, x, y);
+    if (e >= 4 && x == y) return -1;  // on the diagonal both quads are the same nodes: one writes them
+    const int m = nyn - 1;
+    const int i = e < 4 ? x : y, k = e < 4 ? y : x;  // mirrored in x for odd e, in y for e & 2
+    return ((e & 1) ? m - i : i) * nyn + ((e & 2) ? m - k : k);
+  }
+  const int node = tile * jb.per_lane * kT + e * kT + lane;
+  return node < jb.sh.ax.n * nyn ? node : -1;
 }
 
 // Time of the node sums in atoms per lane with s atom ranges per tile: rounds
@@ -479,29 +624,46 @@ __device__ __forceinline__ void prepare_pixels(const PlanArgs &a, const SurfJob 
   }
 }
 
-// Interpolation weights of one axis (node-major [n][npix]), one wave per
-// pixel: barycentric formula in s = cos t, whose weights at the Chebyshev
-// points are (-1)^i sin t_i.
+// Interpolation weights of one axis, and in FP32 with their derivatives in u
+// (node-major [n][npix]), one wave per pixel: barycentric formula in s = cos t, whose
+// weights at the Chebyshev points are (-1)^i sin t_i. With r_i = w_i / (s - s_i):
+// l_i = r_i / sum r, dl_i/ds = l_i (sum r_j / (s - s_j) / sum r - 1 / (s - s_i)).
 __device__ __forceinline__ void weight_column(const SurfAxis &ax, int x, int npix, const double *sn, const double *wn,
-                                              double *__restrict__ out) {
+                                              double *__restrict__ out, float2 *__restrict__ out32) {
   const int lane = threadIdx.x & 63;
-  const double s = sinpi(pixel_u(x, npix) * (ax.asin_a / kPi)) / ax.a;
-  double sum = 0.0;
+  double sx, cx;
+  sincospi(pixel_u(x, npix) * (ax.asin_a / kPi), &sx, &cx);
+  const double s = sx / ax.a, ds = ax.asin_a * cx / ax.a;
+  double sum = 0.0, sum2 = 0.0;
   int hit = -1;
   for (int i = lane; i < ax.n; i += 64) {
     const double d = s - sn[i];
-    if (d == 0.0)
+    if (fabs(d) < 1e-13) {
       hit = i;
-    else
-      sum += wn[i] / d;
+    } else {
+      const double r = wn[i] / d;
+      sum += r;
+      sum2 += r / d;
+    }
   }
   for (int o = 32; o > 0; o >>= 1) {
     sum += __shfl_xor(sum, o);
+    sum2 += __shfl_xor(sum2, o);
     hit = max(hit, __shfl_xor(hit, o));
   }
+  // on a node h: l is its unit vector, dl_i/ds = w_i / w_h / (s_h - s_i), and
+  // minus their sum at h itself
   for (int i = lane; i < ax.n; i += 64) {
-    const double d = s - sn[i];
-    out[(size_t)i * npix + x] = hit >= 0 ? (i == hit ? 1.0 : 0.0) : (wn[i] / d) / sum;
+    const double d = s - sn[i], r = wn[i] / d;
+    const size_t o = (size_t)i * npix + x;
+    if (hit >= 0) {
+      out[o] = i == hit ? 1.0 : 0.0;
+      out32[o] = make_float2(i == hit ? 1.0f : 0.0f, (float)(ds * (i == hit ? -sum / wn[hit] : r / wn[hit])));
+    } else {
+      const double l = r / sum;
+      out[o] = l;
+      out32[o] = make_float2((float)l, (float)(ds * l * (sum2 / sum - 1.0 / d)));
+    }
   }
 }
 
@@ -527,9 +689,9 @@ __device__ void build(int part, const SurfFit *fit, const SurfShape &sh, int nx,
     const int waves = kT / 64, wave = t / 64;
     for (int r = (int)blockIdx.x * waves + wave; r < nx + ny; r += (int)gridDim.x * waves) {
       if (r < nx)
-        weight_column(sh.ax, r, nx, snx, wnx, sh.tx);
+        weight_column(sh.ax, r, nx, snx, wnx, sh.tx, sh.tx32);
       else
-        weight_column(sh.ay, r - nx, ny, sny, wny, sh.ty);
+        weight_column(sh.ay, r - nx, ny, sny, wny, sh.ty, sh.ty32);
     }
   } else if (part == 1) {
     for (int i = t; i < D * D * 3; i += kT) (&coef[0][0][0])[i] = (&fit->coef[0][0][0])[i];
@@ -560,16 +722,16 @@ __global__ __launch_bounds__(kT) void surface_plan_kernel(PlanArgs a) {
   __shared__ int best[2], split[1];
   __shared__ SurfJob job;
   const int t = threadIdx.x;
-  double m[7] = {0, 0, 0, 0, -3.4e38, -3.4e38, 0};  // dev, r2, -B, B, not finite
+  double m[5] = {0, 0, -3.4e38, -3.4e38, 0};  // dev, r2, -B, B, not finite
   for (int i = t; i < a.list_blocks + kSurfAtomBlocks; i += kT) {
     const SurfRecord r = a.records[i];
-    for (int k = 0; k < 3; ++k) m[k] = fmax(m[k], r.dev[k]);
-    m[3] = fmax(m[3], r.r2);
+    m[0] = fmax(m[0], r.dev);
+    m[1] = fmax(m[1], r.r2);
     if (i >= a.list_blocks) {
-      m[4] = fmax(m[4], -(double)r.bmin);
-      m[5] = fmax(m[5], (double)r.bmax);
+      m[2] = fmax(m[2], -(double)r.bmin);
+      m[3] = fmax(m[3], (double)r.bmax);
     }
-    if (r.bad) m[6] = 1.0;
+    if (r.bad) m[4] = 1.0;
   }
   block_reduce(m);
   // every form-factor row that is used, one thread each
@@ -577,16 +739,16 @@ __global__ __launch_bounds__(kT) void surface_plan_kernel(PlanArgs a) {
   for (int i = t; i < a.job.nsegs; i += kT) {
     const int sp = a.job.segs[i].species;
     species_terms(a.ff + sp * SPSIM_HIP_FF_STRIDE, sp == SPSIM_HIP_UNIT_SPECIES ? 0.0f : a.b_global,
-                  a.has_b ? (float)-m[4] : 0.0f, a.has_b ? (float)m[5] : 0.0f, a.fit->s2max, &bs, &weak);
+                  a.has_b ? (float)-m[2] : 0.0f, a.has_b ? (float)m[3] : 0.0f, a.fit->s2max, &bs, &weak);
   }
   double e[2] = {(double)bs, -(double)weak};
   block_reduce(e);
   if (t == 0) {
-    mol.radius = sqrt(m[3]) * a.scale;
-    mol.dev = sqrt(m[0] * m[0] + m[1] * m[1] + m[2] * m[2]);
+    mol.radius = sqrt(m[1]) * a.scale;
+    mol.dev = m[0];
     mol.b_smooth = (float)e[0];
     mol.weakest = (float)-e[1];
-    mol.bad = m[6] > 0.0;
+    mol.bad = m[4] > 0.0;
     best[0] = best[1] = 1 << 30;
   }
   __syncthreads();
@@ -599,7 +761,7 @@ __global__ __launch_bounds__(kT) void surface_plan_kernel(PlanArgs a) {
   }
   __syncthreads();
   const int nx = best[0], ny = best[1];
-  // G is taken at the spectrum's centre scale, so it is off by the spread
+  // N is taken at the spectrum's centre scale, so it is off by the spread
   const bool ok = smooth(mol, a.fit->s2max) && 2.0 * kPi * mol.radius * mol.dev * a.spread <= kMaxSpreadDev &&
                   nx <= a.max_nx && ny <= a.max_ny &&
                   worth(nx, ny, a.job.nx, a.job.ny, a.job.natoms, a.kind);
@@ -607,8 +769,9 @@ __global__ __launch_bounds__(kT) void surface_plan_kernel(PlanArgs a) {
     if (blockIdx.x == 0 && blockIdx.y == 0 && t == 0) a.out->ok = 0;
     return;
   }
-  const int per_lane = surf_per_lane((long long)nx * ny, a.job.natoms), tile = per_lane * kT;
-  const int tiles = (nx * ny + tile - 1) / tile;
+  int per_lane, tiles;
+  node_tiling(nx, ny, a.fit->sym == 2 && nx == ny && a.kind == SurfKind::kSum, a.job.natoms, &per_lane, &tiles);
+  const int tile = per_lane * kT;
   if (t < 64) {  // the cheapest number of atom ranges, two candidates per lane
     float c = 3.0e38f;
     int n = 1;
@@ -638,7 +801,10 @@ __global__ __launch_bounds__(kT) void surface_plan_kernel(PlanArgs a) {
     job.sh.ay.asin_a = asin(job.sh.ay.a);
     job.per_lane = per_lane;
     job.tiles = tiles;
-    for (int k = 0; k < 3; ++k) job.r0[k] = a.centres[k];
+    for (int k = 0; k < 3; ++k) {
+      job.r0[k] = a.centres[k];
+      job.normal[k] = a.fit->normal[k];
+    }
   }
   __syncthreads();
   if (t == 0) {
@@ -663,11 +829,13 @@ __global__ __launch_bounds__(kT) void surface_tables_kernel(const SurfFit *fit, 
 
 // ---- 3. node sums ---------------------------------------------------------------
 //
-// One work item: one, two or four nodes per lane x one atom range, whose records are
-// staged in LDS 256 at a time; every lane reads the same record, and its terms
-// share the read (surf_per_lane). Per node and atom: 3 FP64 FMAs, a fraction and a
-// conversion, a sine and cosine, 8 FP32 FMAs (F and the three components of G):
-// 62 issue cycles. (The records through scalar loads instead, one node per
+// One work item: a tile of nodes (node_tiling) x one atom range, whose records
+// are staged in LDS 256 at a time; every lane reads the same record, and its
+// terms share the read. Per node and atom: 3 FP64 FMAs, a fraction and a
+// conversion, a sine and cosine, 4 FP32 FMAs (F and N): 57 issue cycles; an
+// octant's 8 nodes share 9 FP64 operations, 5 fractions, conversions, sines and
+// cosines: 40 per node (100,000 atoms with B, 188^2 nodes: 1.14 ms, two nodes
+// per lane 1.9 ms with three gradient sums instead of N). (The records through scalar loads instead, one node per
 // lane: 128 cycles; the waves drift apart and miss the scalar cache.) A tile's
 // atom ranges leave partial sums, which surface_reduce_kernel adds in range
 // order (added by the tile's last workgroup instead, 64 ranges took 30 us: one
@@ -676,11 +844,6 @@ __global__ __launch_bounds__(kT) void surface_tables_kernel(const SurfFit *fit, 
 
 constexpr int kNodeChunk = 256;  // atoms staged at once
 constexpr int kNodeFold = 64;  // atoms per FP32 partial sum
-
-struct __align__(16) NodeSlot {
-  double fc, fs;
-  float g[8];  // sin, cos of x, y, z; 2 unused
-};
 
 __device__ __forceinline__ double form_factor64(const float *__restrict__ c, double s2, float B) {
   double f = c[8] * exp(-(double)B * s2);
@@ -700,51 +863,74 @@ struct SpectrumArg<true> {
   using type = Spectrum;
 };
 
-// SPEC: a wavelength spectrum, the sample sum in place of the sine and cosine
-// (spectrum_term), and the gradient at the centre scale.
-template <int K, bool HAS_B, bool SPEC>
-__device__ __forceinline__ void node_item(const SurfJob &jb, int tile, int split, const float *__restrict__ ff,
-                                          float b_global, const typename SpectrumArg<SPEC>::type &sp, NodeAtom *sm) {
-  constexpr int kTile = K * kT, kUnroll = K == 1 ? 4 : (K == 2 ? 2 : 1);
-  const int nodes = jb.sh.ax.n * jb.sh.ay.n;
+// A lane's sums of node e: a partial sum, or F and N = -2 pi i sum w f n.r e^{-i phi}.
+__device__ __forceinline__ void store_node(const SurfJob &jb, int tile, int split, int e, double fc, double fs, float nc,
+                                           float ns) {
+  if (jb.splits > 1) {
+    const size_t o = ((size_t)tile * jb.splits + split) * jb.per_lane * kT + e * kT + threadIdx.x;
+    jb.slot_f[o] = make_double2(fc, fs);
+    jb.slot_n[o] = make_float2(nc, ns);
+    return;
+  }
+  const int node = node_index(jb, tile, e, threadIdx.x);
+  if (node < 0) return;
+  jb.f[node] = make_double2(fc, -fs);
+  jb.n[node] = make_float2(-2.0f * (float)kPi * ns, -2.0f * (float)kPi * nc);
+}
+
+// Runs body(first, count, f64) over the LDS chunks of a work item's atoms, at
+// most kNodeFold atoms at a time; form(species) is called once per species.
+template <class Form, class Body>
+__device__ __forceinline__ void over_atoms(const SurfJob &jb, int split, NodeAtom *sm, Form form, Body body) {
   const int a_begin = (int)((long long)jb.natoms * split / jb.splits);
   const int a_end = (int)((long long)jb.natoms * (split + 1) / jb.splits);
-  double qx[K], qy[K], qz[K], s2[K], Fc[K], Fs[K];
-  float nl2[K], gc[K][3], gs[K][3];
-#pragma unroll
-  for (int k = 0; k < K; ++k) {
-    const double *q = jb.sh.nodes + 3 * (size_t)min(tile * kTile + k * kT + (int)threadIdx.x, nodes - 1);
-    qx[k] = q[0];
-    qy[k] = q[1];
-    qz[k] = q[2];
-    s2[k] = (qx[k] * qx[k] + qy[k] * qy[k] + qz[k] * qz[k]) * 2.5e-21;
-    nl2[k] = (float)(-s2[k] * kLog2e);
-    Fc[k] = Fs[k] = 0.0;
-#pragma unroll
-    for (int i = 0; i < 3; ++i) gc[k][i] = gs[k][i] = 0.0f;
-  }
   const NodeAtom *atoms = (const NodeAtom *)jb.prep;
   for (int sg = 0; sg < jb.nsegs; ++sg) {
     const spsim_hip_segment seg = jb.segs[sg];
     const int lo = max(seg.start, a_begin), hi = min(seg.start + seg.count, a_end);
     if (lo >= hi) continue;
-    double f[K];
-#pragma unroll
-    for (int k = 0; k < K; ++k)
-      f[k] = form_factor64(ff + seg.species * SPSIM_HIP_FF_STRIDE, s2[k],
-                           seg.species == SPSIM_HIP_UNIT_SPECIES ? 0.0f : b_global);
+    form(seg.species);
     for (int c0 = lo; c0 < hi; c0 += kNodeChunk) {
       const int n = min(kNodeChunk, hi - c0);
       __syncthreads();
       if ((int)threadIdx.x < n) sm[threadIdx.x] = atoms[c0 + threadIdx.x];
       __syncthreads();
-      for (int j0 = 0; j0 < n; j0 += kNodeFold) {
-        const int j1 = min(n, j0 + kNodeFold);
-        float c[K][4], s[K][4];
+      for (int j0 = 0; j0 < n; j0 += kNodeFold) body(j0, min(n, j0 + kNodeFold));
+    }
+  }
+}
+
+// K nodes per lane. SPEC: a wavelength spectrum, the sample sum in place of the
+// sine and cosine (spectrum_term), and N at the centre scale.
+template <int K, bool HAS_B, bool SPEC>
+__device__ __forceinline__ void node_item(const SurfJob &jb, int tile, int split, const float *__restrict__ ff,
+                                          float b_global, const typename SpectrumArg<SPEC>::type &sp, NodeAtom *sm) {
+  constexpr int kUnroll = K == 1 ? 4 : (K == 2 ? 2 : 1);
+  double qx[K], qy[K], qz[K], s2[K], f[K], Fc[K], Fs[K];
+  float nl2[K], Nc[K], Ns[K];
+#pragma unroll
+  for (int k = 0; k < K; ++k) {
+    const double *q = jb.sh.nodes + 3 * (size_t)max(0, node_index(jb, tile, k, threadIdx.x));
+    qx[k] = q[0];
+    qy[k] = q[1];
+    qz[k] = q[2];
+    s2[k] = (qx[k] * qx[k] + qy[k] * qy[k] + qz[k] * qz[k]) * 2.5e-21;
+    nl2[k] = (float)(-s2[k] * kLog2e);
+    f[k] = Fc[k] = Fs[k] = 0.0;
+    Nc[k] = Ns[k] = 0.0f;
+  }
+  over_atoms(
+      jb, split, sm,
+      [&](int species) {
 #pragma unroll
         for (int k = 0; k < K; ++k)
+          f[k] = (1.0 + kTrigBias) * form_factor64(ff + species * SPSIM_HIP_FF_STRIDE, s2[k],
+                                                   species == SPSIM_HIP_UNIT_SPECIES ? 0.0f : b_global);
+      },
+      [&](int j0, int j1) {
+        float c[K][2], s[K][2];
 #pragma unroll
-          for (int i = 0; i < 4; ++i) c[k][i] = s[k][i] = 0.0f;
+        for (int k = 0; k < K; ++k) c[k][0] = c[k][1] = s[k][0] = s[k][1] = 0.0f;
 #pragma unroll kUnroll
         for (int j = j0; j < j1; ++j) {
           const NodeAtom at = sm[j];
@@ -760,56 +946,118 @@ __device__ __forceinline__ void node_item(const SurfJob &jb, int tile, int split
               sn = __builtin_amdgcn_sinf(ph);
             }
             if constexpr (HAS_B) {
-              const float w = __builtin_amdgcn_exp2f(__builtin_fmaf(at.v[4], nl2[k], at.v[0]));
+              const float w = __builtin_amdgcn_exp2f(__builtin_fmaf(at.b, nl2[k], at.w));
               cs *= w;
               sn *= w;
               c[k][0] += cs;
               s[k][0] += sn;
             } else {
-              c[k][0] = __builtin_fmaf(at.v[0], cs, c[k][0]);
-              s[k][0] = __builtin_fmaf(at.v[0], sn, s[k][0]);
+              c[k][0] = __builtin_fmaf(at.w, cs, c[k][0]);
+              s[k][0] = __builtin_fmaf(at.w, sn, s[k][0]);
             }
-#pragma unroll
-            for (int i = 1; i < 4; ++i) {
-              c[k][i] = __builtin_fmaf(at.v[i], cs, c[k][i]);
-              s[k][i] = __builtin_fmaf(at.v[i], sn, s[k][i]);
-            }
+            c[k][1] = __builtin_fmaf(at.n, cs, c[k][1]);
+            s[k][1] = __builtin_fmaf(at.n, sn, s[k][1]);
           }
         }
 #pragma unroll
         for (int k = 0; k < K; ++k) {
           Fc[k] = __builtin_fma(f[k], (double)c[k][0], Fc[k]);
           Fs[k] = __builtin_fma(f[k], (double)s[k][0], Fs[k]);
-          const float f32 = (float)f[k];
-#pragma unroll
-          for (int i = 0; i < 3; ++i) {
-            gc[k][i] = __builtin_fmaf(f32, c[k][i + 1], gc[k][i]);
-            gs[k][i] = __builtin_fmaf(f32, s[k][i + 1], gs[k][i]);
-          }
+          Nc[k] = __builtin_fmaf((float)f[k], c[k][1], Nc[k]);
+          Ns[k] = __builtin_fmaf((float)f[k], s[k][1], Ns[k]);
         }
-      }
-    }
-  }
+      });
 #pragma unroll
   for (int k = 0; k < K; ++k) {
-    const int l = k * kT + threadIdx.x, node = tile * kTile + l;
-    if constexpr (SPEC)
-      for (int i = 0; i < 3; ++i) {
-        gc[k][i] *= (float)sp.sc;
-        gs[k][i] *= (float)sp.sc;
-      }
-    if (jb.splits > 1) {
-      ((NodeSlot *)jb.slots)[((size_t)tile * jb.splits + split) * kTile + l] =
-          NodeSlot{Fc[k], Fs[k], {gs[k][0], gc[k][0], gs[k][1], gc[k][1], gs[k][2], gc[k][2], 0.0f, 0.0f}};
-    } else if (node < nodes) {
-      // G = dF/dq = -2 pi i sum w f r e^{-i phi}: (re, im) = -2 pi (gs, gc)
-      jb.f[node] = make_double2(Fc[k], -Fs[k]);
-      float2 *g = (float2 *)(jb.g + 6 * (size_t)node);
-#pragma unroll
-      for (int i = 0; i < 3; ++i)
-        g[i] = make_float2(-2.0f * (float)kPi * gs[k][i], -2.0f * (float)kPi * gc[k][i]);
-    }
+    float scale = 1.0f;
+    if constexpr (SPEC) scale = (float)sp.sc;
+    store_node(jb, tile, split, k, Fc[k], Fs[k], scale * Nc[k], scale * Ns[k]);
   }
+}
+
+// One octant per lane: the phases a + b, a - b of the node (x, y) and of its
+// transposed node with a = q_x r_x, b = q_y r_y, c = q_z r_z, and from their sines and
+// cosines the four real sums P, Q per angle, as in octant_sum (sf_kernels.hip),
+// once weighted by w e^{-2 pi i c} (F) and once by n.r times that (N).
+template <bool HAS_B>
+__device__ __forceinline__ void octant_item(const SurfJob &jb, int tile, int split, const float *__restrict__ ff,
+                                            float b_global, NodeAtom *sm) {
+  const double *q = jb.sh.nodes + 3 * (size_t)max(0, node_index(jb, tile, 0, threadIdx.x));
+  const double qx = q[0], qy = q[1], qz = q[2];
+  const double s2 = (qx * qx + qy * qy + qz * qz) * 2.5e-21;
+  const float nl2 = (float)(-s2 * kLog2e);
+  double f = 0.0, Fc[8], Fs[8];
+  float Nc[8], Ns[8];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    Fc[i] = Fs[i] = 0.0;
+    Nc[i] = Ns[i] = 0.0f;
+  }
+  over_atoms(
+      jb, split, sm,
+      [&](int species) {
+        f = (1.0 + 2.0 * kTrigBias) * form_factor64(ff + species * SPSIM_HIP_FF_STRIDE, s2,
+                                                    species == SPSIM_HIP_UNIT_SPECIES ? 0.0f : b_global);
+      },
+      [&](int j0, int j1) {
+        // [half][F, N][P, Q over a + b, P, Q over a - b][by cos c, by sin c]
+        float S[2][2][4][2];
+#pragma unroll
+        for (int i = 0; i < 32; ++i) (&S[0][0][0][0])[i] = 0.0f;
+        for (int j = j0; j < j1; ++j) {
+          const NodeAtom at = sm[j];
+          const double tc = qz * at.z;
+          const double ta[2] = {qx * at.x, qy * at.x}, tb[2] = {qy * at.y, qx * at.y};
+          const float fc = (float)__builtin_amdgcn_fract(tc);
+          float u[2][2];  // [F, N][cos c, sin c]
+          u[0][0] = __builtin_amdgcn_cosf(fc);
+          u[0][1] = __builtin_amdgcn_sinf(fc);
+          if constexpr (HAS_B) {
+            const float w = __builtin_amdgcn_exp2f(__builtin_fmaf(at.b, nl2, at.w));
+            u[0][0] *= w;
+            u[0][1] *= w;
+            u[1][0] = at.n * u[0][0];
+            u[1][1] = at.n * u[0][1];
+          } else {
+            u[1][0] = at.n * u[0][0];
+            u[1][1] = at.n * u[0][1];
+            u[0][0] *= at.w;
+            u[0][1] *= at.w;
+          }
+#pragma unroll
+          for (int h = 0; h < 2; ++h) {
+            const float fs = (float)__builtin_amdgcn_fract(ta[h] + tb[h]);
+            const float fd = (float)__builtin_amdgcn_fract(ta[h] - tb[h]);
+            const float v[4] = {__builtin_amdgcn_cosf(fs), __builtin_amdgcn_sinf(fs), __builtin_amdgcn_cosf(fd),
+                                __builtin_amdgcn_sinf(fd)};
+#pragma unroll
+            for (int w = 0; w < 2; ++w)
+#pragma unroll
+              for (int i = 0; i < 4; ++i)
+#pragma unroll
+                for (int k = 0; k < 2; ++k) S[h][w][i][k] = __builtin_fmaf(u[w][k], v[i], S[h][w][i][k]);
+          }
+        }
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+#pragma unroll
+          for (int e = 0; e < 4; ++e) {
+            // c + (a + b), c - (a - b), c + (a - b), c - (a + b): cosine sums P cos c
+            // -/+ Q sin c, sine sums P sin c +/- Q cos c
+            const int i = e == 0 || e == 3 ? 0 : 2;
+            const bool minus = e == 1 || e == 3;  // the angle enters with a minus
+            const float(*F)[2] = S[h][0], (*N)[2] = S[h][1];
+            const double pf = F[i][0], ps = F[i][1], qf = F[i + 1][0], qs = F[i + 1][1];
+            Fc[4 * h + e] = __builtin_fma(f, minus ? pf + qs : pf - qs, Fc[4 * h + e]);
+            Fs[4 * h + e] = __builtin_fma(f, minus ? ps - qf : ps + qf, Fs[4 * h + e]);
+            const float f32 = (float)f;
+            Nc[4 * h + e] = __builtin_fmaf(f32, minus ? N[i][0] + N[i + 1][1] : N[i][0] - N[i + 1][1], Nc[4 * h + e]);
+            Ns[4 * h + e] = __builtin_fmaf(f32, minus ? N[i][1] - N[i + 1][0] : N[i][1] + N[i + 1][0], Ns[4 * h + e]);
+          }
+        }
+      });
+#pragma unroll
+  for (int e = 0; e < 8; ++e) store_node(jb, tile, split, e, Fc[e], Fs[e], Nc[e], Ns[e]);
 }
 
 template <bool HAS_B, bool SPEC>
@@ -824,6 +1072,12 @@ __global__ __launch_bounds__(kT) void surface_nodes_kernel(const SurfJob *jobs, 
   for (int it = blockIdx.x; it < nitems; it += gridDim.x) {
     const SurfItem m = items ? items[it] : SurfItem{0, it % jobs->tiles, it / jobs->tiles, 0};
     const SurfJob &jb = jobs[m.job];
+    if constexpr (!SPEC) {
+      if (jb.per_lane == 8) {
+        octant_item<HAS_B>(jb, m.tile, m.split, ff, b_global, sm);
+        continue;
+      }
+    }
     if (jb.per_lane == 4)
       node_item<4, HAS_B, SPEC>(jb, m.tile, m.split, ff, b_global, sp, sm);
     else if (jb.per_lane == 2)
@@ -833,73 +1087,77 @@ __global__ __launch_bounds__(kT) void surface_nodes_kernel(const SurfJob *jobs, 
   }
 }
 
-// Adds the atom ranges of every node: one lane per third of a node's slot, so
-// that a wave reads contiguous 16-byte parts and keeps 16 ranges in flight.
+// Adds the atom ranges of every node: one lane per node for F (blockIdx.y = 0)
+// and one for N, 16 ranges in flight.
 __global__ __launch_bounds__(kT) void surface_reduce_kernel(const SurfJob *jobs, int first) {
   const SurfJob &jb = jobs[first + blockIdx.z];
   if (!jb.ok || jb.splits == 1) return;
-  const int nodes = jb.sh.ax.n * jb.sh.ay.n;
-  const int id = (int)blockIdx.x * kT + threadIdx.x, node = id / 3, part = id % 3;
-  if (node >= nodes) return;
-  const int size = jb.per_lane * kT, tile = node / size, lane = node % size, splits = jb.splits;
-  const char *slot = (const char *)((const NodeSlot *)jb.slots + (size_t)tile * splits * size + lane) + 16 * part;
-  const size_t step = sizeof(NodeSlot) * size;
-  if (part == 0) {
+  const int id = (int)blockIdx.x * kT + threadIdx.x, size = jb.per_lane * kT;
+  const int tile = id / size, splits = jb.splits;
+  if (tile >= jb.tiles) return;
+  const int node = node_index(jb, tile, id % size / kT, id % kT);
+  if (node < 0) return;
+  const size_t at = (size_t)tile * splits * size + id % size;
+  if (blockIdx.y == 0) {
     double c = 0.0, s = 0.0;
 #pragma unroll 16
     for (int i = 0; i < splits; ++i) {
-      const double2 v = *(const double2 *)(slot + i * step);
+      const double2 v = jb.slot_f[at + (size_t)i * size];
       c += v.x;
       s += v.y;
     }
     jb.f[node] = make_double2(c, -s);
   } else {
-    float4 a = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    float c = 0.0f, s = 0.0f;
 #pragma unroll 16
     for (int i = 0; i < splits; ++i) {
-      const float4 v = *(const float4 *)(slot + i * step);
-      a.x += v.x;
-      a.y += v.y;
-      a.z += v.z;
-      a.w += v.w;
+      const float2 v = jb.slot_n[at + (size_t)i * size];
+      c += v.x;
+      s += v.y;
     }
-    const float k = -2.0f * (float)kPi;
-    float2 *g = (float2 *)(jb.g + 6 * (size_t)node) + 2 * (part - 1);
-    g[0] = make_float2(k * a.x, k * a.y);
-    if (part == 1) g[1] = make_float2(k * a.z, k * a.w);
+    jb.n[node] = make_float2(-2.0f * (float)kPi * s, -2.0f * (float)kPi * c);
   }
 }
 
 // ---- 4. interpolation -----------------------------------------------------------
 //
-// Both products run on the matrix units, in FP64 for F and FP32 for G
-// (16 x 16 x 4 products; 105 and 40 cycles each, as fast as the vector FMAs
-// they replace: 76 and 42). The second product's waves make two 16 x 16
-// tiles that share the operand with the most fields. Lane l of an FP64 product holds rows
+// Both products run on the matrix units, in FP64 for F and FP32 for N and
+// the derivatives (16 x 16 x 4 products; 105 and 40 cycles each, as fast as the vector FMAs
+// they replace: 76 and 42). Lane l of an FP64 product holds rows
 // l / 16 + 4 r (r = 0..3) of column l % 16, of an FP32 product rows
 // 4 (l / 16) + r: the FP32 products take their rows in the order `prow`, so
-// that a lane's F and G belong to the same pixels. (Scalar operands and vector
+// that a lane's F, N and derivatives belong to the same pixels. (Scalar operands and vector
 // FMAs instead: 18 us for the rows of a 256 x 256 detector at 28 nodes, where
 // each step waits for its scalar loads.)
 
 typedef double double4v __attribute__((ext_vector_type(4)));
 typedef float float4v __attribute__((ext_vector_type(4)));
 
+template <int G>
 struct Fields {
   double4v re, im;
-  float4v g[6];
+  float4v g[G];
 };
 
-__device__ __forceinline__ void clear(Fields &a) {
+template <int G>
+__device__ __forceinline__ void clear(Fields<G> &a) {
   a.re = a.im = double4v{0, 0, 0, 0};
 #pragma unroll
-  for (int c = 0; c < 6; ++c) a.g[c] = float4v{0, 0, 0, 0};
+  for (int c = 0; c < G; ++c) a.g[c] = float4v{0, 0, 0, 0};
+}
+
+__device__ __forceinline__ float4v mfma32(float a, float b, float4v c) {
+  return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+}
+__device__ __forceinline__ double4v mfma64(double a, double b, double4v c) {
+  return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
 }
 
 // Row of an FP32 product that puts a lane's results on its FP64 rows.
 __device__ __forceinline__ int prow(int m) { return m / 4 + 4 * (m % 4); }
 
-// t[k][x] = sum_i node[i][k] tx[i][x]: 16 node rows x 16 columns per wave;
+// Along the rows, t[k][x] = sum_i node[i][k] tx[i][x] of F (FP64), of F with the
+// weights' derivatives and of N: 16 node rows x 16 columns per wave;
 // blockIdx.x: 64 columns, blockIdx.y: 16 node rows, blockIdx.z: pattern.
 __global__ __launch_bounds__(kT) void surface_rows_kernel(const SurfJob *jobs, int first) {
   const SurfJob &jb = jobs[first + blockIdx.z];
@@ -909,21 +1167,25 @@ __global__ __launch_bounds__(kT) void surface_rows_kernel(const SurfJob *jobs, i
   const int k0 = (int)blockIdx.y * 16, x = (int)blockIdx.x * 64 + (int)(threadIdx.x / 64) * 16 + m;
   if (k0 >= nyn || x - m >= nx) return;
   // rows and columns past the end repeat the last one and are not stored
-  const double2 *f = jb.f + (size_t)gq * nyn + min(k0 + m, nyn - 1);
-  const float2 *g = (const float2 *)jb.g + 3 * ((size_t)gq * nyn + min(k0 + prow(m), nyn - 1));
+  const size_t row = (size_t)gq * nyn + min(k0 + m, nyn - 1), prow_ = (size_t)gq * nyn + min(k0 + prow(m), nyn - 1);
+  const double2 *f = jb.f + row, *fp = jb.f + prow_;
+  const float2 *n = jb.n + prow_;
   const double *tx = jb.sh.tx + (size_t)gq * nx + min(x, nx - 1);
-  Fields acc;
+  const float2 *tx32 = jb.sh.tx32 + (size_t)gq * nx + min(x, nx - 1);
+  Fields<4> acc;
   clear(acc);
 #pragma unroll 4
   for (int i = 0; i < nxn; i += 4) {
-    const double2 fv = f[(size_t)i * nyn];
-    const float2 g0 = g[3 * (size_t)i * nyn], g1 = g[3 * (size_t)i * nyn + 1], g2 = g[3 * (size_t)i * nyn + 2];
+    const double2 fv = f[(size_t)i * nyn], fq = fp[(size_t)i * nyn];
+    const float2 nv = n[(size_t)i * nyn];
     const double b = tx[(size_t)i * nx];
-    const float gv[6] = {g0.x, g0.y, g1.x, g1.y, g2.x, g2.y};
-    acc.re = __builtin_amdgcn_mfma_f64_16x16x4f64(fv.x, b, acc.re, 0, 0, 0);
-    acc.im = __builtin_amdgcn_mfma_f64_16x16x4f64(fv.y, b, acc.im, 0, 0, 0);
-#pragma unroll
-    for (int c = 0; c < 6; ++c) acc.g[c] = __builtin_amdgcn_mfma_f32_16x16x4f32(gv[c], (float)b, acc.g[c], 0, 0, 0);
+    const float2 b32 = tx32[(size_t)i * nx];
+    acc.re = mfma64(fv.x, b, acc.re);
+    acc.im = mfma64(fv.y, b, acc.im);
+    acc.g[0] = mfma32((float)fq.x, b32.y, acc.g[0]);
+    acc.g[1] = mfma32((float)fq.y, b32.y, acc.g[1]);
+    acc.g[2] = mfma32(nv.x, b32.x, acc.g[2]);
+    acc.g[3] = mfma32(nv.y, b32.x, acc.g[3]);
   }
   if (x >= nx) return;
 #pragma unroll
@@ -932,17 +1194,15 @@ __global__ __launch_bounds__(kT) void surface_rows_kernel(const SurfJob *jobs, i
     if (k >= nyn) continue;
     const size_t o = (size_t)k * nx + x;
     jb.t64[o] = make_double2(acc.re[r], acc.im[r]);
-    float2 *t = (float2 *)jb.t32 + 3 * o;
-#pragma unroll
-    for (int c = 0; c < 3; ++c) t[c] = make_float2(acc.g[2 * c][r], acc.g[2 * c + 1][r]);
+    jb.t32[o] = make_float4(acc.g[0][r], acc.g[1][r], acc.g[2][r], acc.g[3][r]);
   }
 }
 
-// F(y, x) = sum_k ty[k][y] t[k][x], the list's deviation, the centre's phase
-// and the intensity: J tiles of 16 x 16 pixels per wave (one above the other),
-// 2 x 2 waves per workgroup. One tile where two would leave SIMDs without a
-// wave (a 256 x 256 detector has 256 tiles).
-template <int J>
+// Along the columns, F(y, x) = sum_k ty[k][y] t[k][x] and its derivatives, then the
+// list's deviation, the centre's phase and the intensity: 16 x 16 pixels per
+// wave, 2 x 2 waves per workgroup. (Two tiles per wave, which share the operand t,
+// keep two waves per SIMD instead of four: 82 us against 57 us on 1024^2 pixels
+// and 188 nodes.)
 __global__ __launch_bounds__(kT) void surface_cols_kernel(const SurfJob *jobs, int first, const float *__restrict__ dev,
                                                           const float *__restrict__ hkl, float2 *__restrict__ F,
                                                           float *__restrict__ I) {
@@ -950,34 +1210,29 @@ __global__ __launch_bounds__(kT) void surface_cols_kernel(const SurfJob *jobs, i
   if (!jb.ok) return;
   const int nyn = jb.sh.ay.n, nx = jb.nx, ny = jb.ny;
   const int wave = threadIdx.x / 64, l = threadIdx.x & 63, m = l & 15, gq = l >> 4;
-  const int x = (int)blockIdx.x * 32 + (wave & 1) * 16 + m, y0 = ((int)blockIdx.y * 2 + (wave >> 1)) * 16 * J;
+  const int x = (int)blockIdx.x * 32 + (wave & 1) * 16 + m, y0 = ((int)blockIdx.y * 2 + (wave >> 1)) * 16;
   if (x - m >= nx || y0 >= ny) return;
   const size_t xc = (size_t)gq * nx + min(x, nx - 1);
   const double2 *t64 = jb.t64 + xc;
-  const float2 *t32 = (const float2 *)jb.t32 + 3 * xc;
-  const double *w[J], *wp[J];
-#pragma unroll
-  for (int j = 0; j < J; ++j) {
-    w[j] = jb.sh.ty + (size_t)gq * ny + min(y0 + 16 * j + m, ny - 1);
-    wp[j] = jb.sh.ty + (size_t)gq * ny + min(y0 + 16 * j + prow(m), ny - 1);
-  }
-  Fields acc[J];
-#pragma unroll
-  for (int j = 0; j < J; ++j) clear(acc[j]);
+  const float4 *t32 = jb.t32 + xc;
+  const double *w = jb.sh.ty + (size_t)gq * ny + min(y0 + m, ny - 1);
+  const float2 *w32 = jb.sh.ty32 + (size_t)gq * ny + min(y0 + prow(m), ny - 1);
+  Fields<6> acc;  // F; dF/du, N, dF/dv
+  clear(acc);
 #pragma unroll 4
   for (int k = 0; k < nyn; k += 4) {
     const double2 v = t64[(size_t)k * nx];
-    const float2 g0 = t32[3 * (size_t)k * nx], g1 = t32[3 * (size_t)k * nx + 1], g2 = t32[3 * (size_t)k * nx + 2];
-    const float gv[6] = {g0.x, g0.y, g1.x, g1.y, g2.x, g2.y};
-#pragma unroll
-    for (int j = 0; j < J; ++j) {
-      const double a = w[j][(size_t)k * ny];
-      const float a32 = (float)wp[j][(size_t)k * ny];
-      acc[j].re = __builtin_amdgcn_mfma_f64_16x16x4f64(a, v.x, acc[j].re, 0, 0, 0);
-      acc[j].im = __builtin_amdgcn_mfma_f64_16x16x4f64(a, v.y, acc[j].im, 0, 0, 0);
-#pragma unroll
-      for (int c = 0; c < 6; ++c) acc[j].g[c] = __builtin_amdgcn_mfma_f32_16x16x4f32(a32, gv[c], acc[j].g[c], 0, 0, 0);
-    }
+    const float4 g = t32[(size_t)k * nx];
+    const double a = w[(size_t)k * ny];
+    const float2 a32 = w32[(size_t)k * ny];
+    acc.re = mfma64(a, v.x, acc.re);
+    acc.im = mfma64(a, v.y, acc.im);
+    acc.g[0] = mfma32(a32.x, g.x, acc.g[0]);
+    acc.g[1] = mfma32(a32.x, g.y, acc.g[1]);
+    acc.g[2] = mfma32(a32.x, g.z, acc.g[2]);
+    acc.g[3] = mfma32(a32.x, g.w, acc.g[3]);
+    acc.g[4] = mfma32(a32.y, (float)v.x, acc.g[4]);
+    acc.g[5] = mfma32(a32.y, (float)v.y, acc.g[5]);
   }
   if (x >= nx) return;
   double cx = jb.r0[0], cy = jb.r0[1], cz = jb.r0[2];
@@ -990,27 +1245,24 @@ __global__ __launch_bounds__(kT) void surface_cols_kernel(const SurfJob *jobs, i
   }
   const size_t out = (size_t)jb.pattern * ((size_t)nx * ny);
 #pragma unroll
-  for (int j = 0; j < J; ++j)
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int y = y0 + 16 * j + gq + 4 * r;
-      if (y >= ny) continue;
-      const size_t p = (size_t)y * nx + x;
-      const float dx = dev[3 * p], dy = dev[3 * p + 1], dz = dev[3 * p + 2];
-      const Fields &v = acc[j];
-      const double re =
-          v.re[r] + (double)__builtin_fmaf(dz, v.g[4][r], __builtin_fmaf(dy, v.g[2][r], dx * v.g[0][r]));
-      const double im =
-          v.im[r] + (double)__builtin_fmaf(dz, v.g[5][r], __builtin_fmaf(dy, v.g[3][r], dx * v.g[1][r]));
-      if (I) I[out + p] = (float)(re * re + im * im);
-      if (F) {
-        const double t = __builtin_fma((double)hkl[3 * p + 2], cz,
-                                       __builtin_fma((double)hkl[3 * p + 1], cy, (double)hkl[3 * p] * cx));
-        double sn, cs;
-        sincospi(2.0 * __builtin_amdgcn_fract(t), &sn, &cs);
-        F[out + p] = make_float2((float)(re * cs + im * sn), (float)(im * cs - re * sn));
-      }
+  for (int r = 0; r < 4; ++r) {
+    const int y = y0 + gq + 4 * r;
+    if (y >= ny) continue;
+    const size_t p = (size_t)y * nx + x;
+    const float al = dev[3 * p], be = dev[3 * p + 1], ga = dev[3 * p + 2];
+    const double re =
+        acc.re[r] + (double)__builtin_fmaf(ga, acc.g[2][r], __builtin_fmaf(be, acc.g[4][r], al * acc.g[0][r]));
+    const double im =
+        acc.im[r] + (double)__builtin_fmaf(ga, acc.g[3][r], __builtin_fmaf(be, acc.g[5][r], al * acc.g[1][r]));
+    if (I) I[out + p] = (float)(re * re + im * im);
+    if (F) {
+      const double t = __builtin_fma((double)hkl[3 * p + 2], cz,
+                                     __builtin_fma((double)hkl[3 * p + 1], cy, (double)hkl[3 * p] * cx));
+      double sn, cs;
+      sincospi(2.0 * __builtin_amdgcn_fract(t), &sn, &cs);
+      F[out + p] = make_float2((float)(re * cs + im * sn), (float)(im * cs - re * sn));
     }
+  }
 }
 
 // ---- adjoint ---------------------------------------------------------------------
@@ -1020,13 +1272,12 @@ __global__ __launch_bounds__(kT) void surface_cols_kernel(const SurfJob *jobs, i
 // with dL/dr_j = -2 pi w_j Im sum_p q_p A_p h_j and dL/dB_j = -w_j Re sum_p s_p^2 A_p h_j
 // (adjoint.hip). h_j is as smooth over the detector as F, so the transposed
 // interpolation carries the pixels' values to the nodes,
-//   a_v = sum_p L_v(p) A_p,  b_v = sum_p L_v(p) A_p d_p   (d: the list's deviation),
-// two dense products again (FP64 for a, FP32 for b), and every atom sums
-// nodes instead of pixels: S_j = sum_v h_j(q_v) Z_v, Z_v = a_v + 2 pi i r_j.b_v.
+//   a_v = sum_p A_p (L_v + alpha_p dL_v/du + beta_p dL_v/dv),  b_v = sum_p gamma_p A_p L_v,
+// two dense products again (FP64 for A_p L_v, FP32 for the rest), and every atom
+// sums nodes instead of pixels: S_j = sum_v h_j(q_v) Z_v, Z_v = a_v + 2 pi i n.r_j b_v.
 
-constexpr int kGatherNodes = 8;  // nodes of a row per wave of the second product
-
-// First product: t[split][k][x] = sum over the split's rows of ty[k][y] A(y, x);
+// First product: t[split][k][x], sums over the split's list rows of
+// ty[k][y] A + dty[k][y] beta A (t64), ty[k][y] alpha A and ty[k][y] gamma A (t32);
 // 16 node rows x 16 columns per wave, blockIdx.z: rows of the list.
 __global__ __launch_bounds__(kT) void surface_gather_rows_kernel(const SurfJob *job, const float2 *__restrict__ pixels,
                                                                  const float *__restrict__ dev) {
@@ -1040,26 +1291,28 @@ __global__ __launch_bounds__(kT) void surface_gather_rows_kernel(const SurfJob *
   const int y0 = 4 * (int)((long long)steps * blockIdx.z / splits);
   const int y1 = 4 * (int)((long long)steps * (blockIdx.z + 1) / splits);
   const int xc = min(x, nx - 1);
-  const double *w = jb.sh.ty + (size_t)min(k0 + m, nyn - 1) * ny;
-  const double *wp = jb.sh.ty + (size_t)min(k0 + prow(m), nyn - 1) * ny;
-  Fields acc;
+  const size_t row = (size_t)min(k0 + m, nyn - 1) * ny, prow_ = (size_t)min(k0 + prow(m), nyn - 1) * ny;
+  const double *w = jb.sh.ty + row;
+  const float2 *w32 = jb.sh.ty32 + prow_;
+  Fields<6> acc;
   clear(acc);
 #pragma unroll 4
   for (int y = y0; y < y1; y += 4) {
     const int yy = min(y + gq, ny - 1);
     const bool in = y + gq < ny;  // rows past the end weigh nothing
     const double a = in ? w[yy] : 0.0;
-    const float a32 = in ? (float)wp[yy] : 0.0f;
+    const float2 a32 = in ? w32[yy] : make_float2(0.0f, 0.0f);
     const size_t p = (size_t)yy * nx + xc;
     const float2 v = pixels[p];
-    const float d[3] = {dev[3 * p], dev[3 * p + 1], dev[3 * p + 2]};
-    acc.re = __builtin_amdgcn_mfma_f64_16x16x4f64(a, (double)v.x, acc.re, 0, 0, 0);
-    acc.im = __builtin_amdgcn_mfma_f64_16x16x4f64(a, (double)v.y, acc.im, 0, 0, 0);
-#pragma unroll
-    for (int c = 0; c < 3; ++c) {
-      acc.g[2 * c] = __builtin_amdgcn_mfma_f32_16x16x4f32(a32, v.x * d[c], acc.g[2 * c], 0, 0, 0);
-      acc.g[2 * c + 1] = __builtin_amdgcn_mfma_f32_16x16x4f32(a32, v.y * d[c], acc.g[2 * c + 1], 0, 0, 0);
-    }
+    const float al = dev[3 * p], be = dev[3 * p + 1], ga = dev[3 * p + 2];
+    acc.re = mfma64(a, (double)v.x, acc.re);
+    acc.im = mfma64(a, (double)v.y, acc.im);
+    acc.g[0] = mfma32(a32.y, be * v.x, acc.g[0]);
+    acc.g[1] = mfma32(a32.y, be * v.y, acc.g[1]);
+    acc.g[2] = mfma32(a32.x, al * v.x, acc.g[2]);
+    acc.g[3] = mfma32(a32.x, al * v.y, acc.g[3]);
+    acc.g[4] = mfma32(a32.x, ga * v.x, acc.g[4]);
+    acc.g[5] = mfma32(a32.x, ga * v.y, acc.g[5]);
   }
   if (x >= nx) return;
 #pragma unroll
@@ -1067,84 +1320,103 @@ __global__ __launch_bounds__(kT) void surface_gather_rows_kernel(const SurfJob *
     const int k = k0 + gq + 4 * r;
     if (k >= nyn) continue;
     const size_t o = ((size_t)blockIdx.z * nyn + k) * nx + x;
-    jb.t64[o] = make_double2(acc.re[r], acc.im[r]);
-    float2 *t = (float2 *)jb.t32 + 3 * o;
-#pragma unroll
-    for (int c = 0; c < 3; ++c) t[c] = make_float2(acc.g[2 * c][r], acc.g[2 * c + 1][r]);
+    jb.t64[o] = make_double2(acc.re[r] + (double)acc.g[0][r], acc.im[r] + (double)acc.g[1][r]);
+    jb.t32[o] = make_float4(acc.g[2][r], acc.g[3][r], acc.g[4][r], acc.g[5][r]);
   }
 }
 
-// Second product, with the splits added: f, g of node (i, k) = sum_x tx[i][x] t[k][x].
-// One wave per node row k and 8 nodes i: the lanes share the columns.
+// Second product: a (jb.f) and b (jb.n) of the nodes (i, k) of one node row k.
+// The workgroup adds the splits of 256 columns into LDS at a time; each wave then
+// takes every fourth of its part's nodes, the lanes sharing the columns.
+constexpr int kGatherParts = 4;  // workgroups per node row
+
 __global__ __launch_bounds__(kT) void surface_gather_nodes_kernel(const SurfJob *job, int splits) {
   const SurfJob &jb = *job;
   if (!jb.ok) return;
   const int nyn = jb.sh.ay.n, nxn = jb.sh.ax.n, nx = jb.nx;
-  const int k = blockIdx.y, i0 = ((int)blockIdx.x * (kT / 64) + (int)(threadIdx.x / 64)) * kGatherNodes;
-  if (k >= nyn || i0 >= nxn) return;
-  const int lane = threadIdx.x & 63;
-  double re[kGatherNodes], im[kGatherNodes];
-  float g[kGatherNodes][6];
-#pragma unroll
-  for (int i = 0; i < kGatherNodes; ++i) {
-    re[i] = im[i] = 0.0;
-#pragma unroll
-    for (int c = 0; c < 6; ++c) g[i][c] = 0.0f;
-  }
-  for (int x = lane; x < nx; x += 64) {
-    double tr = 0.0, ti = 0.0;
-    float tg[6] = {0, 0, 0, 0, 0, 0};
+  const int k = blockIdx.y, part = blockIdx.x;
+  if (k >= nyn) return;
+  __shared__ double2 t64[kT];
+  __shared__ float4 t32[kT];
+  __shared__ double2 sum_a[kSurfMaxNodes / kGatherParts + 4];
+  __shared__ float2 sum_b[kSurfMaxNodes / kGatherParts + 4];
+  const int i0 = nxn * part / kGatherParts, i1 = nxn * (part + 1) / kGatherParts;
+  const int t = threadIdx.x, lane = t & 63, wave = t / 64;
+  for (int x0 = 0; x0 < nx; x0 += kT) {
+    double2 a = make_double2(0.0, 0.0);
+    float4 g = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    if (x0 + t < nx) {
 #pragma unroll 8
-    for (int s = 0; s < splits; ++s) {
-      const size_t o = ((size_t)s * nyn + k) * nx + x;
-      const double2 v = jb.t64[o];
-      const float2 *t = (const float2 *)jb.t32 + 3 * o;
-      tr += v.x;
-      ti += v.y;
-#pragma unroll
-      for (int c = 0; c < 3; ++c) {
-        tg[2 * c] += t[c].x;
-        tg[2 * c + 1] += t[c].y;
+      for (int s = 0; s < splits; ++s) {
+        const size_t o = ((size_t)s * nyn + k) * nx + x0 + t;
+        const double2 v = jb.t64[o];
+        const float4 h = jb.t32[o];
+        a.x += v.x;
+        a.y += v.y;
+        g.x += h.x;
+        g.y += h.y;
+        g.z += h.z;
+        g.w += h.w;
       }
     }
+    __syncthreads();
+    t64[t] = a;
+    t32[t] = g;
+    __syncthreads();
+    for (int i = i0 + wave; i < i1; i += kT / 64) {
+      double re = 0.0, im = 0.0;
+      float br = 0.0f, bi = 0.0f;
 #pragma unroll
-    for (int i = 0; i < kGatherNodes; ++i) {
-      const double w = jb.sh.tx[(size_t)min(i0 + i, nxn - 1) * nx + x];
-      re[i] = __builtin_fma(w, tr, re[i]);
-      im[i] = __builtin_fma(w, ti, im[i]);
-#pragma unroll
-      for (int c = 0; c < 6; ++c) g[i][c] = __builtin_fmaf((float)w, tg[c], g[i][c]);
+      for (int c = 0; c < kT / 64; ++c) {
+        const int xl = c * 64 + lane, x = min(x0 + xl, nx - 1);  // columns past the end hold zeros
+        const double w = jb.sh.tx[(size_t)i * nx + x];
+        const float2 w32 = jb.sh.tx32[(size_t)i * nx + x];
+        const double2 v = t64[xl];
+        const float4 h = t32[xl];
+        re = __builtin_fma(w, v.x, re + (double)(w32.y * h.x));
+        im = __builtin_fma(w, v.y, im + (double)(w32.y * h.y));
+        br = __builtin_fmaf(w32.x, h.z, br);
+        bi = __builtin_fmaf(w32.x, h.w, bi);
+      }
+      for (int o = 32; o > 0; o >>= 1) {
+        re += __shfl_xor(re, o);
+        im += __shfl_xor(im, o);
+        br += __shfl_xor(br, o);
+        bi += __shfl_xor(bi, o);
+      }
+      if (lane == 0) {
+        if (x0 == 0) {
+          sum_a[i - i0] = make_double2(re, im);
+          sum_b[i - i0] = make_float2(br, bi);
+        } else {
+          sum_a[i - i0].x += re;
+          sum_a[i - i0].y += im;
+          sum_b[i - i0].x += br;
+          sum_b[i - i0].y += bi;
+        }
+      }
     }
   }
-#pragma unroll
-  for (int i = 0; i < kGatherNodes; ++i) {
-    for (int o = 32; o > 0; o >>= 1) {
-      re[i] += __shfl_xor(re[i], o);
-      im[i] += __shfl_xor(im[i], o);
-#pragma unroll
-      for (int c = 0; c < 6; ++c) g[i][c] += __shfl_xor(g[i][c], o);
-    }
-    if (lane == 0 && i0 + i < nxn) {
-      const size_t node = (size_t)(i0 + i) * nyn + k;
-      jb.f[node] = make_double2(re[i], im[i]);
-      for (int c = 0; c < 6; ++c) jb.g[6 * node + c] = g[i][c];
-    }
+  __syncthreads();
+  for (int i = i0 + t; i < i1; i += kT) {
+    jb.f[(size_t)i * nyn + k] = sum_a[i - i0];
+    jb.n[(size_t)i * nyn + k] = sum_b[i - i0];
   }
 }
 
-// A node as every atom of one species reads it: f(|q|) Z's parts, b times 2 pi.
+// A node as every atom of one species reads it: f(|q|) a, 2 pi f(|q|) b.
 struct __align__(16) AdjNode {
   double qx, qy, qz;
-  float ar, ai;
-  float br[3], bi[3];
+  float ar, ai, br, bi;
   float qxf, qyf, qzf;
   float s2, nl2, pad;
 };
-static_assert(sizeof(AdjNode) == 80, "adjoint node record");
+static_assert(sizeof(AdjNode) == 64, "adjoint node record");
 
 // Per atom: U = Im sum q h Z and V = Re sum s^2 h Z over a range of nodes; one
 // tile of 512 atoms of one species per workgroup (2 per lane), the nodes
-// staged in LDS 128 at a time. FP32 sums over a chunk, FP64 across chunks.
+// staged in LDS 128 at a time. Per term 3 FP64 FMAs, a fraction and a conversion,
+// a sine and cosine, and 8 FP32 FMAs (with B an exponential and 2 more). FP32 sums over a chunk, FP64 across chunks.
 template <bool HAS_B, bool WANT_B>
 __global__ __launch_bounds__(kT) void surface_adjoint_kernel(const SurfJob *job, const SurfAtomTile *tiles,
                                                              const float *__restrict__ ff, float b_global,
@@ -1159,7 +1431,7 @@ __global__ __launch_bounds__(kT) void surface_adjoint_kernel(const SurfJob *job,
   const float Bs = tile.species == SPSIM_HIP_UNIT_SPECIES ? 0.0f : b_global;
   const float *c = ff + tile.species * SPSIM_HIP_FF_STRIDE;
   double rx[KA], ry[KA], rz[KA], Ux[KA], Uy[KA], Uz[KA], V[KA];
-  float xf[KA], yf[KA], zf[KA], bj[KA];
+  float nr[KA], bj[KA];
 #pragma unroll
   for (int k = 0; k < KA; ++k) {
     const int i = threadIdx.x + k * kT;
@@ -1168,9 +1440,7 @@ __global__ __launch_bounds__(kT) void surface_adjoint_kernel(const SurfJob *job,
     rx[k] = ok ? at.x - jb.r0[0] : 0.0;
     ry[k] = ok ? at.y - jb.r0[1] : 0.0;
     rz[k] = ok ? at.z - jb.r0[2] : 0.0;
-    xf[k] = (float)rx[k];
-    yf[k] = (float)ry[k];
-    zf[k] = (float)rz[k];
+    nr[k] = jb.normal[0] * (float)rx[k] + jb.normal[1] * (float)ry[k] + jb.normal[2] * (float)rz[k];
     bj[k] = (HAS_B && ok) ? jb.atom_b[tile.start + i] : 0.0f;
     Ux[k] = Uy[k] = Uz[k] = V[k] = 0.0;
   }
@@ -1188,15 +1458,13 @@ __global__ __launch_bounds__(kT) void surface_adjoint_kernel(const SurfJob *job,
       r.qyf = (float)q[1];
       r.qzf = (float)q[2];
       const double s2 = (q[0] * q[0] + q[1] * q[1] + q[2] * q[2]) * 2.5e-21;
-      const double f = form_factor64(c, s2, Bs);
+      const double f = (1.0 + kTrigBias) * form_factor64(c, s2, Bs);
       const double2 a = jb.f[node];
       r.ar = (float)(f * a.x);
       r.ai = (float)(f * a.y);
-      const float f2 = (float)(2.0 * kPi * f);
-      for (int i = 0; i < 3; ++i) {
-        r.br[i] = f2 * jb.g[6 * node + 2 * i];
-        r.bi[i] = f2 * jb.g[6 * node + 2 * i + 1];
-      }
+      const float2 b = jb.n[node];
+      r.br = (float)(2.0 * kPi * f) * b.x;
+      r.bi = (float)(2.0 * kPi * f) * b.y;
       r.s2 = (float)s2;
       r.nl2 = (float)(-s2 * kLog2e);
       r.pad = 0.0f;
@@ -1218,11 +1486,9 @@ __global__ __launch_bounds__(kT) void surface_adjoint_kernel(const SurfJob *job,
           cs *= e;
           sn *= e;
         }
-        // Z = a + i (2 pi r.b)
-        const float zr = __builtin_fmaf(
-            -zf[k], r.bi[2], __builtin_fmaf(-yf[k], r.bi[1], __builtin_fmaf(-xf[k], r.bi[0], r.ar)));
-        const float zi = __builtin_fmaf(
-            zf[k], r.br[2], __builtin_fmaf(yf[k], r.br[1], __builtin_fmaf(xf[k], r.br[0], r.ai)));
+        // Z = a + i (2 pi n.r b)
+        const float zr = __builtin_fmaf(-nr[k], r.bi, r.ar);
+        const float zi = __builtin_fmaf(nr[k], r.br, r.ai);
         const float u = __builtin_fmaf(cs, zi, sn * zr);
         ux[k] = __builtin_fmaf(u, r.qxf, ux[k]);
         uy[k] = __builtin_fmaf(u, r.qyf, uy[k]);
@@ -1249,13 +1515,16 @@ __global__ __launch_bounds__(kT) void surface_adjoint_kernel(const SurfJob *job,
 size_t align_up(size_t n) { return (n + 255) / 256 * 256; }
 
 // Row ranges of the adjoint's first product: enough waves for the chip.
-int gather_splits(int nx) { return std::max(2, std::min(16, 8192 / nx)); }
+int gather_splits(int nx) { return std::max(2, std::min(8, 4096 / nx)); }
+
+// A tiling's slots beyond the nodes: an octant grid's diagonals and its last tile.
+constexpr int kSlotSlack = 2 * kSurfMaxNodes + 8 * kT;
 
 // Workspace of one pattern: the nodes of an axis are limited to what can pay
 // (worth() needs n_x n_y below about a third of the pixels).
 struct SingleLayout {
   int max_nx, max_ny, slot_cap;
-  size_t fit, records, centres, job, dev, nodes, tx, ty, prep, f, g, slots, t64, t32, total;
+  size_t fit, records, centres, job, dev, nodes, tx, ty, tx32, ty32, prep, f, n, slot_f, slot_n, t64, t32, total;
 };
 
 SingleLayout single_layout(int nx, int ny, int natoms, bool adjoint) {
@@ -1264,7 +1533,7 @@ SingleLayout single_layout(int nx, int ny, int natoms, bool adjoint) {
   l.max_nx = cap(nx);
   l.max_ny = cap(ny);
   const size_t nodes = (size_t)l.max_nx * l.max_ny, npix = (size_t)nx * ny;
-  l.slot_cap = std::max(1 << 20, (int)(nodes + 4 * kT));
+  l.slot_cap = std::max(1 << 20, (int)nodes + kSlotSlack);
   size_t at = 0;
   auto take = [&](size_t bytes) {
     const size_t o = at;
@@ -1279,13 +1548,16 @@ SingleLayout single_layout(int nx, int ny, int natoms, bool adjoint) {
   l.nodes = take(sizeof(double) * 3 * nodes);
   l.tx = take(sizeof(double) * (size_t)l.max_nx * nx);
   l.ty = take(sizeof(double) * (size_t)l.max_ny * ny);
+  l.tx32 = take(sizeof(float2) * (size_t)l.max_nx * nx);
+  l.ty32 = take(sizeof(float2) * (size_t)l.max_ny * ny);
   l.prep = adjoint ? take(sizeof(float2) * npix) : take(sizeof(NodeAtom) * (size_t)natoms);
   l.f = take(sizeof(double2) * nodes);
-  l.g = take(sizeof(float) * 6 * nodes);
+  l.n = take(sizeof(float2) * nodes);
   const size_t rows = (size_t)l.max_ny * nx * (adjoint ? gather_splits(nx) : 1);
-  l.slots = adjoint ? at : take(sizeof(NodeSlot) * (size_t)l.slot_cap);
+  l.slot_f = take(adjoint ? 0 : sizeof(double2) * (size_t)l.slot_cap);
+  l.slot_n = take(adjoint ? 0 : sizeof(float2) * (size_t)l.slot_cap);
   l.t64 = take(sizeof(double2) * rows);
-  l.t32 = take(sizeof(float) * 6 * rows);
+  l.t32 = take(sizeof(float4) * rows);
   l.total = at;
   return l;
 }
@@ -1293,16 +1565,12 @@ SingleLayout single_layout(int nx, int ny, int natoms, bool adjoint) {
 void launch_interpolation(const SurfJob *jobs, int first, int count, int nx, int ny, int max_nodes, int max_ny,
                           const float *dev, const float *hkl, float2 *F, float *I, hipStream_t s) {
   if (max_nodes > 0)  // some pattern's atoms are split
-    hipLaunchKernelGGL(surface_reduce_kernel, dim3((3 * max_nodes + kT - 1) / kT, 1, count), dim3(kT), 0, s, jobs,
-                       first);
+    hipLaunchKernelGGL(surface_reduce_kernel, dim3((max_nodes + kSlotSlack + kT - 1) / kT, 2, count), dim3(kT), 0, s,
+                       jobs, first);
   hipLaunchKernelGGL(surface_rows_kernel, dim3((nx + 63) / 64, (max_ny + 15) / 16, count), dim3(kT), 0, s, jobs,
                      first);
-  if ((long long)nx * ny * count >= 1 << 20)  // at least two waves of two tiles per SIMD
-    hipLaunchKernelGGL(surface_cols_kernel<2>, dim3((nx + 31) / 32, (ny + 63) / 64, count), dim3(kT), 0, s, jobs, first,
-                       dev, hkl, F, I);
-  else
-    hipLaunchKernelGGL(surface_cols_kernel<1>, dim3((nx + 31) / 32, (ny + 31) / 32, count), dim3(kT), 0, s, jobs, first,
-                       dev, hkl, F, I);
+  hipLaunchKernelGGL(surface_cols_kernel, dim3((nx + 31) / 32, (ny + 31) / 32, count), dim3(kT), 0, s, jobs, first, dev,
+                     hkl, F, I);
 }
 
 const void *nodes_kernel(bool has_b, bool spec) {
@@ -1339,6 +1607,8 @@ int launch_plan(const PatternLaunch &a, int nx, int ny, const Spectrum *sp, Surf
   p.job.sh.nodes = (double *)(w + l.nodes);
   p.job.sh.tx = (double *)(w + l.tx);
   p.job.sh.ty = (double *)(w + l.ty);
+  p.job.sh.tx32 = (float2 *)(w + l.tx32);
+  p.job.sh.ty32 = (float2 *)(w + l.ty32);
   p.job.atoms = a.atoms;
   p.job.atom_b = a.atom_b;
   p.job.segs = a.segs;
@@ -1347,11 +1617,12 @@ int launch_plan(const PatternLaunch &a, int nx, int ny, const Spectrum *sp, Surf
   p.job.has_rot = a.has_rot;
   std::copy(a.rot.r, a.rot.r + 9, p.job.rot);
   p.job.f = (double2 *)(w + l.f);
-  p.job.g = (float *)(w + l.g);
-  p.job.slots = w + l.slots;
+  p.job.n = (float2 *)(w + l.n);
+  p.job.slot_f = (double2 *)(w + l.slot_f);
+  p.job.slot_n = (float2 *)(w + l.slot_n);
   p.job.prep = w + l.prep;
   p.job.t64 = (double2 *)(w + l.t64);
-  p.job.t32 = (float *)(w + l.t32);
+  p.job.t32 = (float4 *)(w + l.t32);
   p.fit = (const SurfFit *)(w + l.fit);
   p.records = (const SurfRecord *)(w + l.records);
   p.list_blocks = std::min(kSurfListBlocks, ny + 2);
@@ -1425,11 +1696,10 @@ int launch_surface_adjoint(const PatternLaunch &a, const float *gI, int nx, int 
   char *w = (char *)ws;
   const SurfJob *job = (const SurfJob *)(w + l.job);
   SPSIM_TRY(launch_plan(a, nx, ny, nullptr, SurfKind::kAdjoint, gI, l, w, cus, cus, s));
-  const int gs = gather_splits(nx), per_block = kGatherNodes * (kT / 64);
+  const int gs = gather_splits(nx);
   hipLaunchKernelGGL(surface_gather_rows_kernel, dim3((nx + 63) / 64, (l.max_ny + 15) / 16, gs), dim3(kT), 0, s, job,
                      (const float2 *)(w + l.prep), (const float *)(w + l.dev));
-  hipLaunchKernelGGL(surface_gather_nodes_kernel, dim3((l.max_nx + per_block - 1) / per_block, l.max_ny), dim3(kT), 0, s,
-                     job, gs);
+  hipLaunchKernelGGL(surface_gather_nodes_kernel, dim3(kGatherParts, l.max_ny), dim3(kT), 0, s, job, gs);
   const bool hb = a.atom_b != nullptr;
   const void *k = hb ? (want_b ? (const void *)&surface_adjoint_kernel<true, true>
                                : (const void *)&surface_adjoint_kernel<true, false>)
@@ -1498,37 +1768,35 @@ size_t place(SurfJob *j, int nx, char *ws, size_t at) {
   };
   j->prep = take(sizeof(NodeAtom) * (size_t)j->natoms);
   j->f = (double2 *)take(sizeof(double2) * nodes);
-  j->g = (float *)take(sizeof(float) * 6 * nodes);
-  j->slots = take(j->splits > 1 ? sizeof(NodeSlot) * (size_t)j->tiles * j->per_lane * kT * j->splits : 0);
+  j->n = (float2 *)take(sizeof(float2) * nodes);
+  const size_t slots = j->splits > 1 ? (size_t)j->tiles * j->per_lane * kT * j->splits : 0;
+  j->slot_f = (double2 *)take(sizeof(double2) * slots);
+  j->slot_n = (float2 *)take(sizeof(float2) * slots);
   j->t64 = (double2 *)take(sizeof(double2) * (size_t)j->sh.ay.n * nx);
-  j->t32 = (float *)take(sizeof(float) * 6 * (size_t)j->sh.ay.n * nx);
+  j->t32 = (float4 *)take(sizeof(float4) * (size_t)j->sh.ay.n * nx);
   return at;
 }
+
+// Issue cycles of one atom in a lane's nodes (node_tiling).
+double lane_cost(int per_lane) { return per_lane == 8 ? 321.0 : (per_lane == 1 ? 75.0 : 57.0 * per_lane); }
 
 // Splits a group's atoms so that its work items number about four per resident
 // workgroup, and appends the items, largest first.
 void split_group(std::vector<SurfJob> &jobs, int first, int count, int slots, std::vector<SurfItem> *items) {
   double work = 0.0;
-  for (int i = first; i < first + count; ++i) {
-    SurfJob &j = jobs[i];
-    const int nodes = j.sh.ax.n * j.sh.ay.n;
-    // four nodes per lane, unless two leave much less of the last tile empty
-    const int pad4 = (nodes + 4 * kT - 1) / (4 * kT) * 4 * kT, pad2 = (nodes + 2 * kT - 1) / (2 * kT) * 2 * kT;
-    j.per_lane = pad4 > 1.1 * pad2 ? 2 : 4;
-    j.tiles = (nodes + j.per_lane * kT - 1) / (j.per_lane * kT);
-    work += (double)j.tiles * j.per_lane * j.natoms;
-  }
-  const double share = std::max(work / (4.0 * slots), 512.0);  // nodes per lane x atoms
+  for (int i = first; i < first + count; ++i)
+    work += (double)jobs[i].tiles * lane_cost(jobs[i].per_lane) * jobs[i].natoms;
+  const double share = std::max(work / (4.0 * slots), 128.0 * lane_cost(4));
   const size_t begin = items->size();
   for (int i = first; i < first + count; ++i) {
     SurfJob &j = jobs[i];
-    j.splits = std::max(1, std::min(kSurfMaxSplits, (int)std::ceil(j.per_lane * (double)j.natoms / share)));
+    j.splits = std::max(1, std::min(kSurfMaxSplits, (int)std::ceil(lane_cost(j.per_lane) * j.natoms / share)));
     for (int t = 0; t < j.tiles; ++t)
       for (int k = 0; k < j.splits; ++k) items->push_back(SurfItem{i, t, k, 0});
   }
   std::stable_sort(items->begin() + begin, items->end(), [&](const SurfItem &a, const SurfItem &b) {
     const SurfJob &x = jobs[a.job], &y = jobs[b.job];
-    return (double)x.per_lane * x.natoms / x.splits > (double)y.per_lane * y.natoms / y.splits;
+    return lane_cost(x.per_lane) * x.natoms / x.splits > lane_cost(y.per_lane) * y.natoms / y.splits;
   });
 }
 
@@ -1573,19 +1841,17 @@ int build_plan(SurfPlan *p, const spsim_hip_atom *atoms, const float *atom_b, co
     SPSIM_TRY(rc);
     if (e != hipSuccess) return hip_fail(e, "surface scan");
   }
-  double d2 = 0.0;
+  double dev_max = 0.0;
   bool bad = false;
-  for (int k = 0; k < 3; ++k) {
-    double d = 0.0;
-    for (int i = 0; i < lb; ++i) d = std::max(d, rec[i].dev[k]);
-    d2 += d * d;
+  for (int i = 0; i < lb; ++i) {
+    dev_max = std::max(dev_max, rec[i].dev);
+    bad = bad || rec[i].bad;
   }
-  for (int i = 0; i < lb; ++i) bad = bad || rec[i].bad;
   std::vector<SurfShape> shapes;
   std::vector<int> shape_of(nmol, -1);
   for (int m = 0; m < nmol; ++m) {
     const MolInfo &mi = h_mols[m];
-    SurfMol mol{0.0, std::sqrt(d2), 0.0f, 1.0f, bad};
+    SurfMol mol{0.0, dev_max, 0.0f, 1.0f, bad};
     float lo = 3.4e38f, hi = -3.4e38f;
     for (int i = 0; i < kSurfAtomBlocks; ++i) {
       const SurfRecord &r = rec[lb + (size_t)m * kSurfAtomBlocks + i];
@@ -1607,6 +1873,8 @@ int build_plan(SurfPlan *p, const spsim_hip_atom *atoms, const float *atom_b, co
     SPSIM_TRY(own(p, &sh.nodes, 3 * (size_t)sh.ax.n * sh.ay.n));
     SPSIM_TRY(own(p, &sh.tx, (size_t)sh.ax.n * p->nx));
     SPSIM_TRY(own(p, &sh.ty, (size_t)sh.ay.n * p->ny));
+    SPSIM_TRY(own(p, &sh.tx32, (size_t)sh.ax.n * p->nx));
+    SPSIM_TRY(own(p, &sh.ty32, (size_t)sh.ay.n * p->ny));
     hipLaunchKernelGGL(surface_tables_kernel, dim3(256, 2), dim3(kT), 0, nullptr, (const SurfFit *)d_fit, sh, p->nx,
                        p->ny);
     SPSIM_HIP_TRY(hipGetLastError());
@@ -1632,6 +1900,9 @@ int build_plan(SurfPlan *p, const spsim_hip_atom *atoms, const float *atom_b, co
     j.has_rot = 1;
     std::copy(rot9 + 9 * (size_t)i, rot9 + 9 * (size_t)(i + 1), j.rot);
     std::copy(&centres[3 * (size_t)m], &centres[3 * (size_t)m] + 3, j.r0);
+    std::copy(fit.normal, fit.normal + 3, j.normal);
+    // a group has work enough for every tiling: the one of the least work
+    node_tiling(j.sh.ax.n, j.sh.ay.n, fit.sym == 2 && j.sh.ax.n == j.sh.ay.n, 1LL << 25, &j.per_lane, &j.tiles);
     j.pattern = i;
     jobs.push_back(j);
   }
@@ -1648,8 +1919,6 @@ int build_plan(SurfPlan *p, const spsim_hip_atom *atoms, const float *atom_b, co
     size_t at = 0;
     while (first + g.count < (int)jobs.size() && g.count < 4096) {
       SurfJob probe = jobs[first + g.count];
-      probe.per_lane = 4;
-      probe.tiles = (probe.sh.ax.n * probe.sh.ay.n + 4 * kT - 1) / (4 * kT);
       probe.splits = 4;  // a typical group's; only the group's size depends on it
       const size_t end = place(&probe, p->nx, nullptr, at);
       if (g.count > 0 && end > kGroupBytes) break;

@@ -15,10 +15,10 @@ constexpr int kSurfMaxSplits = 128;  // atom ranges per node tile
 constexpr int kSurfListBlocks = 448;  // with the atom blocks, two workgroups per CU
 constexpr int kSurfAtomBlocks = 64;  // per molecule
 
-// What one workgroup of the scan saw: the largest |q - surface| per component
-// (list blocks), or the largest |r - r0|^2 and the range of B (atom blocks).
+// What one workgroup of the scan saw: the largest |q - surface| (list blocks), or
+// the largest |r - r0|^2 and the range of B (atom blocks).
 struct SurfRecord {
-  double dev[3];
+  double dev;
   double r2;
   float bmin, bmax;
   int bad;  // some value was not finite
@@ -33,6 +33,8 @@ struct SurfFit {
   double coef[kSurfDeg][kSurfDeg][3];
   float slope_x[kSurfLines], slope_y[kSurfLines];
   float s2max;  // largest s^2 = (|q| 1e-10 / 2)^2 seen
+  float normal[3];  // unit normal of the surface's middle
+  int sym;          // 2: mirror- and transpose-symmetric, 1: mirror-symmetric, 0
 };
 
 // Nodes of one axis: u_i = asin(a cos t_i) / asin(a), t_i = (2 i + 1) pi / (2 n);
@@ -42,15 +44,17 @@ struct SurfAxis {
   double a, asin_a;
 };
 
-// One detector shape at one node count: node q [ay.n][ax.n][3] and the
-// interpolation weights, node-major (tx [ax.n][nx], ty [ay.n][ny]).
+// One detector shape at one node count: node q [ax.n][ay.n][3], the
+// interpolation weights, node-major (tx [ax.n][nx], ty [ay.n][ny]), and the same in
+// FP32 with their derivatives in u and v.
 struct SurfShape {
   SurfAxis ax, ay;
   double *nodes, *tx, *ty;
+  float2 *tx32, *ty32;
 };
 
-// One pattern. The node sums f (F) and g (its gradient in q, 3 complex) are
-// [ay.n][ax.n]; t64 and t32 are the same fields along the detector's rows,
+// One pattern. The node sums f (F) and n (its derivative along the normal) are
+// [ax.n][ay.n]; t64 (F) and t32 (dF/du, n) are fields along the detector's rows,
 // [ay.n][nx].
 struct SurfJob {
   int ok;
@@ -63,13 +67,15 @@ struct SurfJob {
   int has_rot;
   double rot[9];
   double r0[3];  // subtracted from every atom
-  int per_lane, tiles, splits;  // node tiles of 256 per_lane nodes, atom ranges per tile
+  float normal[3];
+  int per_lane, tiles, splits;  // node tiles of 256 per_lane nodes (8: octants), atom ranges per tile
   double2 *f;
-  float *g;
-  void *prep;   // atom records of the node sums [natoms]
-  void *slots;  // partial sums [tile * splits + split][256 per_lane]
+  float2 *n;
+  void *prep;  // atom records of the node sums [natoms]
+  double2 *slot_f;  // partial sums [tile * splits + split][256 per_lane]
+  float2 *slot_n;
   double2 *t64;
-  float *t32;
+  float4 *t32;
   long long pattern;  // index of the outputs
 };
 
