@@ -1573,6 +1573,20 @@ void launch_interpolation(const SurfJob *jobs, int first, int count, int nx, int
                      hkl, F, I);
 }
 
+// Bound on how much a matrix lengthens a vector: the root of the largest
+// absolute row sum of R^T R (Gershgorin). 1 for a rotation, but callers may
+// pass any matrix; infinite where an element is not finite.
+double rotation_norm(const double *R) {
+  double most = 0.0;
+  for (int i = 0; i < 3; ++i) {
+    double row = 0.0;
+    for (int j = 0; j < 3; ++j) row += std::fabs(R[i] * R[j] + R[3 + i] * R[3 + j] + R[6 + i] * R[6 + j]);
+    if (!std::isfinite(row)) return INFINITY;
+    most = std::max(most, row);
+  }
+  return std::sqrt(most);
+}
+
 const void *nodes_kernel(bool has_b, bool spec) {
   if (spec)
     return has_b ? (const void *)&surface_nodes_kernel<true, true> : (const void *)&surface_nodes_kernel<false, true>;
@@ -1635,11 +1649,12 @@ int launch_plan(const PatternLaunch &a, int nx, int ny, const Spectrum *sp, Surf
   p.max_nx = l.max_nx;
   p.max_ny = l.max_ny;
   p.kind = kind;
-  p.scale = 1.0;
+  const double norm = a.has_rot ? rotation_norm(a.rot.r) : 1.0;
+  p.scale = norm;
   if (sp) {
     p.scale = 0.0;
     for (int k = 0; k < sp->n; ++k) {
-      p.scale = std::max(p.scale, std::fabs(sp->s[k]));
+      p.scale = std::max(p.scale, norm * std::fabs(sp->s[k]));
       p.spread = std::max(p.spread, std::fabs(sp->s[k] / sp->sc - 1.0));
     }
   }
@@ -1849,6 +1864,11 @@ int build_plan(SurfPlan *p, const spsim_hip_atom *atoms, const float *atom_b, co
   }
   std::vector<SurfShape> shapes;
   std::vector<int> shape_of(nmol, -1);
+  std::vector<double> norm(nmol, 0.0);  // of the matrices a molecule is shown under
+  for (int i = 0; i < npatterns; ++i) {
+    double &n = norm[pattern_mol[i]];
+    n = std::max(n, rotation_norm(rot9 + 9 * (size_t)i));
+  }
   for (int m = 0; m < nmol; ++m) {
     const MolInfo &mi = h_mols[m];
     SurfMol mol{0.0, dev_max, 0.0f, 1.0f, bad};
@@ -1860,6 +1880,7 @@ int build_plan(SurfPlan *p, const spsim_hip_atom *atoms, const float *atom_b, co
       hi = std::max(hi, r.bmax);
       mol.bad |= r.bad;
     }
+    mol.radius *= norm[m];
     for (int i = 0; i < mi.nseg; ++i) {
       const int sp = h_segs[mi.seg_begin + i].species;
       species_terms(h_ff + sp * SPSIM_HIP_FF_STRIDE, sp == SPSIM_HIP_UNIT_SPECIES ? 0.0f : p->b_global,

@@ -71,6 +71,42 @@ def test_interpolated_pattern_vs_f64_and_direct(gpu, nx, ny, natoms, radius, geo
     assert np.linalg.norm(F - Fd) / np.linalg.norm(Fd) < 2 * TOL
 
 
+@pytest.mark.parametrize("scale", [0.3, 1.0, 2.5, (2.0, 0.5, 1.0), np.nan])
+def test_matrices_that_are_not_rotations(gpu, scale):
+    """q' = R q for any matrix: the node counts follow its length, in single
+    patterns and plans, and a non-finite one gives the direct kernel's bits."""
+    import ctypes as C
+
+    import torch
+
+    from spsim_amd import _lib
+    from tests.test_gpu_batch import make_plan
+
+    rng = np.random.default_rng(21)
+    n, natoms = 256, 6_000
+    Z, pos, _ = wl.random_molecule(natoms, 4e-9, rng)
+    R = wl.uniform_rotations(1, rng)[0] @ np.diag(np.broadcast_to(scale, 3).astype(np.float64))
+    hkl = _list(n, n)
+    F, I = _run(gpu, hkl, n, n, Z, pos, R=R)
+    Fd, Id = _run(gpu, hkl, n, n, Z, pos, R=R, tile=dv.make_tile(1, 256, 0))
+    if not np.isfinite(R).all():
+        assert np.array_equal(I, Id, equal_nan=True)
+        return
+    print(f"scale {scale}: {rel_l2(I, Id):.2e}", flush=True)
+    assert not np.array_equal(I, Id) and rel_l2(I, Id) < 2 * TOL
+    # the same molecule in a plan, once more unrotated: one node count serves both
+    plan, *_ = make_plan([(Z, pos)], np.stack([np.eye(3), R]), np.zeros(2, np.int32), hkl, n, n)
+    try:
+        Ip = torch.empty((2, n * n), dtype=torch.float32, device=gpu)
+        _lib.check(_lib.load().spsim_hip_batch_run(plan, None, C.c_void_p(Ip.data_ptr()), 0, None), "run")
+        torch.cuda.synchronize()
+    finally:
+        _lib.load().spsim_hip_batch_destroy(plan)
+    _, I_one = _run(gpu, hkl, n, n, Z, pos)
+    assert rel_l2(Ip[1].cpu().numpy(), Id) < 2 * TOL
+    assert rel_l2(Ip[0].cpu().numpy(), I_one) < 2 * TOL
+
+
 @pytest.mark.parametrize("what", ["pixel", "noise", "nan pixel", "wide B", "infinite weight", "huge molecule"])
 def test_rough_inputs_keep_the_direct_sum(gpu, what):
     """Lists and molecules that do not vary smoothly over the detector give
