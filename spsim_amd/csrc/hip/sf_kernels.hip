@@ -182,6 +182,7 @@ __device__ __forceinline__ void spectrum_sum(const double (&qx)[K], const double
                                              int a_end, const float *__restrict__ ff, float b_global, const double *R,
                                              const Spectrum &sp, AtomLds *__restrict__ sm, double (&Fr)[K],
                                              double (&Fi)[K]) {
+  const int ns = sp.n;
   float nl2[K];
 #pragma unroll
   for (int k = 0; k < K; ++k) {
@@ -216,7 +217,7 @@ __device__ __forceinline__ void spectrum_sum(const double (&qx)[K], const double
         for (int k = 0; k < K; ++k) {
           const double t = __builtin_fma(qz[k], a.z, __builtin_fma(qy[k], a.y, qx[k] * a.x));
           float ur, ui;
-          spectrum_term(sp, t, ur, ui);
+          spectrum_term(sp, ns, t, ur, ui);
           float wt;
           if constexpr (HAS_B) {
             wt = __builtin_amdgcn_exp2f(__builtin_fmaf(a.b, nl2[k], a.w));

@@ -939,7 +939,7 @@ __device__ __forceinline__ void node_item(const SurfJob &jb, int tile, int split
             const double t = __builtin_fma(qz[k], at.z, __builtin_fma(qy[k], at.y, qx[k] * at.x));
             float cs, sn;
             if constexpr (SPEC) {
-              spectrum_term(sp, t, cs, sn);
+              spectrum_term(sp, sp.n, t, cs, sn);
             } else {
               const float ph = (float)__builtin_amdgcn_fract(t);
               cs = __builtin_amdgcn_cosf(ph);
