@@ -244,7 +244,11 @@ int spsim_hip_sf_nfft(const float *d_hkl, int npix, const spsim_hip_atom *d_atom
    to the interval-arithmetic range of R_p over the q box, and every pattern
    only interpolates from it, so the spread and FFT run once.
    The grids are larger than a single pattern's when q does not fill that ball
-   (a flat detector's Ewald cap). Returns after the last pattern is written
+   (a flat detector's Ewald cap). On a square list that is a smooth detector's
+   and where it costs less (spsim_hip_sf_grid says when), the patterns are
+   interpolated over the detector's surface instead, to the direct sums' accuracy;
+   the grids are planned all the same: info describes them, and what they reject
+   is rejected. Returns after the last pattern is written
    (it synchronises `stream`). Other arguments as spsim_hip_sf_nfft. */
 int spsim_hip_sf_nfft_batch(const float *d_hkl, int npix, const spsim_hip_atom *d_atoms, const float *d_atom_b,
                             const spsim_hip_segment *d_segs, int nsegs, int natoms, const float *d_ff, float b_global,
@@ -283,7 +287,9 @@ int spsim_hip_sf_spectrum_nfft(const float *d_hkl, int npix, const spsim_hip_ato
    after every pattern), each stream with its own slice of the library
    workspace. Calls
    that overlap on one device race, as for every entry point sharing the
-   workspace. Same grids and accuracy as spsim_hip_sf_nfft. */
+   workspace. Same grids and accuracy as spsim_hip_sf_nfft; molecules that
+   are cheaper by interpolation over a square detector's surface go that way,
+   as in spsim_hip_sf_nfft_batch. */
 int spsim_hip_sf_nfft_molecules(const float *d_hkl, int npix, int nmol, const spsim_hip_atom *d_atoms,
                                 const float *d_atom_b, const int *atom_offsets, const spsim_hip_segment *d_segs,
                                 const int *seg_offsets, const float *d_ff, float b_global, const double *rot9s,

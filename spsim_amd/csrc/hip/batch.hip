@@ -350,9 +350,9 @@ int spsim_hip_batch_create(const float *hkl, int nx, int ny, int nmol, const int
     return rc;
   }
   if (tile) b->direct = true;
-  if (!tile && (rc = surf_plan_create(b->hkl, nx, ny, b->atoms, b->atom_b, b->segs, b->mols, b->h_mols.data(), nmol,
-                                      h_segs.data(), npatterns, pattern_mol, rot9, b->ff, ffh, b_global, cus,
-                                      &b->surf)) != SPSIM_HIP_OK) {
+  const SurfInput surf{b->hkl, nx,        ny,          b->atoms, b->atom_b, b->segs,  b->mols, b->h_mols.data(),
+                       nmol,   npatterns, pattern_mol, rot9,     b->ff,     b_global, cus,     nullptr};
+  if (!tile && (rc = surf_plan_create(surf, &b->surf)) != SPSIM_HIP_OK) {
     free_batch(b);
     return rc;
   }

@@ -41,6 +41,7 @@
 // The spread sums each grid cell's atoms in registers without FP atomics, in
 // an order fixed by the input (a stable sort bins the atoms by index; the
 // candidates of a block are taken in lane order), so F repeats bit for bit.
+#include <algorithm>
 #include <array>
 #include <cmath>
 #include <mutex>
@@ -51,6 +52,7 @@
 
 #include "common.hpp"
 #include "form_factor.hpp"
+#include "surface.hpp"
 
 namespace spsim {
 namespace {
@@ -173,6 +175,7 @@ __device__ __forceinline__ double nan_max(double a, double b) { return (a != a |
 // NaN propagates.
 constexpr int kNb = 15;
 constexpr int kBoundBlocks = 256;  // workgroups of bounds_partial (records folded on the host)
+constexpr long long kSurfaceMinTerms = 50000000;  // terms below which a list's surface is not looked at
 
 __device__ __forceinline__ double bound_combine(int v, double a, double b) {
   return v < 6 ? nan_min(a, b) : nan_max(a, b);
@@ -2120,10 +2123,61 @@ void fold_bounds(const double *hpart, int nblk, double *hb) {
   }
 }
 
+// Workspace and cost (issue cycles over all lanes) of an evaluation.
+struct NufftNeed {
+  size_t bytes;
+  double cost;
+};
+
 int nufft_run(double *hb, const float *d_hkl, int npix, const spsim_hip_atom *d_atoms, const float *d_atom_b,
               const spsim_hip_segment *d_segs, int nsegs, int natoms, const float *d_ff, float b_global,
               const AtomRot &R, int npat, const double *rots, int W, double eps, float *d_F, float *d_I, int *info,
-              hipStream_t s, size_t *need = nullptr, void *ws_in = nullptr);
+              hipStream_t s, NufftNeed *need = nullptr, void *ws_in = nullptr);
+
+// Side of a square list of npix q on which `terms` = atoms x patterns atoms are
+// worth a look at interpolation over the detector surface (surface.hip), or 0.
+int surface_side(int npix, long long terms) {
+  const int n = (int)llround(sqrt((double)npix));
+  return (long long)n * n == npix && surf_worth(n, n, terms, kSurfaceMinTerms) ? n : 0;
+}
+
+// Whether R^T R is the identity: a batch takes the Debye-Waller factors of
+// Gaussian-spread atoms at R q, sums over the atoms take them at q.
+bool is_rotation(const double *R) {
+  for (int i = 0; i < 3; ++i)
+    for (int j = 0; j < 3; ++j)
+      if (!(fabs(R[i] * R[j] + R[3 + i] * R[3 + j] + R[6 + i] * R[6 + j] - (i == j ? 1.0 : 0.0)) < 1e-6)) return false;
+  return true;
+}
+
+// Every pattern of `in` by interpolation over the detector surface, when all are
+// smooth enough and cheaper so than in.limit: *done. The scan's digest is in
+// h_digest and, on the device, at the workspace's start; the scan itself lies
+// `head` bytes on. A workspace without the memory leaves the patterns to the
+// grids.
+int surface_patterns(const SurfInput &in, const char *h_digest, size_t head, float *d_F, float *d_I, hipStream_t s,
+                     bool *done) {
+  *done = false;
+  SurfPlan *plan = surf_plan_choose(in, h_digest);
+  if (!plan) return SPSIM_HIP_OK;
+  bool all = true;
+  for (int p = 0; p < in.npatterns; ++p) all = all && surf_plan_takes(plan, p);
+  int rc = SPSIM_HIP_OK;
+  if (all) {
+    const size_t at = head + align256(surf_scan_bytes(in.nx, in.ny, in.nmol)), total = at + surf_plan_bytes(plan);
+    const bool grows = !workspace_holds(total);
+    void *ws = nullptr;
+    if (workspace(total, &ws) == SPSIM_HIP_OK) {
+      char *w = (char *)ws;
+      if (grows) rc = surf_scan(in, w + head, w, s);  // the scan went with the smaller workspace
+      if (rc == SPSIM_HIP_OK) rc = surf_plan_bind(plan, w + head, w + at, s);
+      if (rc == SPSIM_HIP_OK) rc = surf_plan_run(plan, (float2 *)d_F, d_I, s);
+      *done = rc == SPSIM_HIP_OK;
+    }
+  }
+  surf_plan_destroy(plan);
+  return rc;
+}
 
 int nufft_impl(const float *d_hkl, int npix, const spsim_hip_atom *d_atoms, const float *d_atom_b,
                const spsim_hip_segment *d_segs, int nsegs, int natoms, const float *d_ff, float b_global,
@@ -2161,32 +2215,63 @@ int nufft_impl(const float *d_hkl, int npix, const spsim_hip_atom *d_atoms, cons
   }
 
   // 1. Bounds of the atoms and of q: per-workgroup records, folded on the host
-  // after the call's one synchronisation.
+  // after the call's one synchronisation; and the look at the list's surface.
+  // A single pattern stays on the grids: 100,000 atoms on 1024^2 take 0.69 ms
+  // there, 1.2 ms by the surface's node sums.
+  int side = npat > 0 ? surface_side(npix, (long long)natoms * nout) : 0;
+  for (int p = 0; p < npat && d_atom_b; ++p)
+    if (!is_rotation(rots + 9 * (size_t)p)) side = 0;
   const int most = natoms > npix ? natoms : npix;
   int nblk = (most + kThreads - 1) / kThreads;
   if (nblk > kBoundBlocks) nblk = kBoundBlocks;
+  constexpr size_t kDigest = (surf_digest_bytes(1) + 255) / 256 * 256;
+  const size_t b_part = align256(sizeof(double) * kNb * nblk), head = kDigest + b_part;
+  int cus = 0;
+  SPSIM_TRY(ensure_device(&cus));
+  const MolInfo mol{0, natoms, 0, nsegs};
+  SurfInput in{d_hkl, side, side, d_atoms, d_atom_b, d_segs, nullptr, &mol, 1, nout, nullptr,
+               npat > 0 ? rots : rot9, d_ff, b_global, cus, nullptr};
   void *ws = nullptr;
-  SPSIM_TRY(workspace(align256(sizeof(double) * kNb * nblk), &ws));
-  double *part = (double *)ws;
+  SPSIM_TRY(workspace(head + (side ? surf_scan_bytes(side, side, 1) : 0), &ws));
   hipLaunchKernelGGL(bounds_partial, dim3(nblk), dim3(kThreads), 0, s, d_atoms, d_atom_b, natoms, d_hkl, npix, R,
-                     part);
+                     (double *)((char *)ws + kDigest));
   SPSIM_HIP_TRY(hipGetLastError());
-  double hpart[kNb * kBoundBlocks], hb[kNb];
-  SPSIM_HIP_TRY(hipMemcpyAsync(hpart, part, sizeof(double) * kNb * nblk, hipMemcpyDeviceToHost, s));
+  if (side) SPSIM_TRY(surf_scan(in, (char *)ws + head, ws, s));
+  alignas(16) char h[kDigest + sizeof(double) * kNb * kBoundBlocks];
+  double hb[kNb];
+  const size_t from = side ? 0 : kDigest;
+  SPSIM_HIP_TRY(hipMemcpyAsync(h + from, (char *)ws + from, kDigest + sizeof(double) * kNb * nblk - from,
+                               hipMemcpyDeviceToHost, s));
   SPSIM_HIP_TRY(hipStreamSynchronize(s));
-  fold_bounds(hpart, nblk, hb);
+  fold_bounds((const double *)(h + kDigest), nblk, hb);
+  if (side) {
+    double hcopy[kNb];
+    std::copy(hb, hb + kNb, hcopy);
+    NufftNeed need{};
+    // planned all the same: info describes the grids, and what they refuse is refused
+    SPSIM_TRY(nufft_run(hcopy, d_hkl, npix, d_atoms, d_atom_b, d_segs, nsegs, natoms, d_ff, b_global, R, npat, rots, W,
+                        eps, nullptr, nullptr, info, s, &need));
+    const double limit = need.cost / nout;
+    in.limit = &limit;
+    bool done = false;
+    SPSIM_TRY(surface_patterns(in, h, head, d_F, d_I, s, &done));
+    if (done) {
+      if (npat > 0) SPSIM_HIP_TRY(hipStreamSynchronize(s));
+      return SPSIM_HIP_OK;
+    }
+  }
   return nufft_run(hb, d_hkl, npix, d_atoms, d_atom_b, d_segs, nsegs, natoms, d_ff, b_global, R, npat, rots, W, eps,
                    d_F, d_I, info, s);
 }
 
 // Plans the grids from the folded bounds hb and enqueues every stage after the
 // bounds on s (a batch synchronises at the end for its rotations' host buffer).
-// With need set it only plans and stores the workspace bytes the stages take;
+// With need set it only plans and stores what the stages take;
 // with ws_in set the stages use that buffer instead of the library workspace.
 int nufft_run(double *hb, const float *d_hkl, int npix, const spsim_hip_atom *d_atoms, const float *d_atom_b,
               const spsim_hip_segment *d_segs, int nsegs, int natoms, const float *d_ff, float b_global,
               const AtomRot &R, int npat, const double *rots, int W, double eps, float *d_F, float *d_I, int *info,
-              hipStream_t s, size_t *need, void *ws_in) {
+              hipStream_t s, NufftNeed *need, void *ws_in) {
   const int nout = npat > 0 ? npat : 1;
   void *ws = nullptr;
   for (int v = 0; v <= 12; ++v)
@@ -2379,7 +2464,9 @@ int nufft_run(double *hb, const float *d_hkl, int npix, const spsim_hip_atom *d_
   const size_t b_all = b_dec + 2 * b_rec + 2 * b_rng + 2 * b_key + 2 * b_key2 + b_sort + 2 * b_cell + 2 * b_scan +
                        b_tw + b_rot + b1 + b2 + b_part;
   if (need) {
-    *need = b_all;
+    // plan_cost's gather takes about 22 cycles, a spread's grid point 300
+    *need = NufftNeed{b_all, 22.0 * (double)nch * plan_cost(g.d, W2, (double)nout * npix) +
+                                 300.0 * natoms * (double)Wsp * Wsp * Wsp};
     return SPSIM_HIP_OK;
   }
   if (ws_in)
@@ -2567,32 +2654,44 @@ extern "C" int spsim_hip_sf_nfft_molecules(const float *d_hkl, int npix, int nmo
   SPSIM_TRY(ensure_device(nullptr));
   const int W = width_for(eps);
   // 1. Bounds: the q list's once (every molecule shares it) and every
-  // molecule's atoms in one launch, read with one synchronisation.
+  // molecule's atoms in one launch, and the look at the list's surface, read
+  // with one synchronisation.
   constexpr int kMolBlocks = 64;
   if (nmol > 65535) return fail(SPSIM_HIP_ERR_INVALID, "at most 65535 molecules per call (%d)", nmol);
+  const int total_atoms = atom_offsets[nmol];
+  const int side = surface_side(npix, total_atoms);
   const int qblk = (npix + kThreads - 1) / kThreads < kBoundBlocks ? (npix + kThreads - 1) / kThreads : kBoundBlocks;
+  const size_t b_dig = side ? align256(surf_digest_bytes(nmol)) : 0;
   const size_t b_q = align256(sizeof(double) * kNb * qblk);
   const size_t b_part = align256(sizeof(double) * kNb * kMolBlocks * (size_t)nmol);
   const size_t b_off = align256(sizeof(int) * ((size_t)nmol + 1));
   const size_t b_rot = rot9s ? align256(sizeof(double) * 9 * (size_t)nmol) : 0;
+  const size_t b_mols = side ? align256(sizeof(MolInfo) * (size_t)nmol) : 0;
+  const size_t at_part = b_dig + b_q, at_off = at_part + b_part, at_rot = at_off + b_off, at_mols = at_rot + b_rot;
+  const size_t head = at_mols + b_mols, b_scan = side ? align256(surf_scan_bytes(side, side, nmol)) : 0;
+  int cus = 0;
+  SPSIM_TRY(ensure_device(&cus));
   void *ws = nullptr;
-  SPSIM_TRY(workspace(b_q + b_part + b_off + b_rot, &ws));
-  double *qpart = (double *)ws;
-  double *part = (double *)((char *)ws + b_q);
-  int *d_off = (int *)((char *)ws + b_q + b_part);
-  double *d_rot = rot9s ? (double *)((char *)ws + b_q + b_part + b_off) : nullptr;
+  SPSIM_TRY(workspace(head + b_scan, &ws));
+  char *w = (char *)ws;
+  double *qpart = (double *)(w + b_dig);
+  double *part = (double *)(w + at_part);
+  int *d_off = (int *)(w + at_off);
+  double *d_rot = rot9s ? (double *)(w + at_rot) : nullptr;
   std::vector<AtomRot> Rs(nmol);
+  std::vector<MolInfo> mols(nmol);
   for (int m = 0; m < nmol; ++m) {
     Rs[m] = AtomRot{};
     if (rot9s) {
       Rs[m].on = 1;
       for (int i = 0; i < 9; ++i) Rs[m].r[i] = rot9s[9 * (size_t)m + i];
     }
+    mols[m] = MolInfo{atom_offsets[m], atom_offsets[m + 1], seg_offsets[m], seg_offsets[m + 1] - seg_offsets[m]};
   }
   hipLaunchKernelGGL(bounds_partial, dim3(qblk), dim3(kThreads), 0, s, nullptr, nullptr, 0, d_hkl, npix, AtomRot{},
                      qpart);
   SPSIM_HIP_TRY(hipGetLastError());
-  if (atom_offsets[nmol] > 0) {
+  if (total_atoms > 0) {
     // pageable sources: both copies have completed by the synchronisation below
     SPSIM_HIP_TRY(hipMemcpyAsync(d_off, atom_offsets, sizeof(int) * ((size_t)nmol + 1), hipMemcpyHostToDevice, s));
     if (rot9s)
@@ -2601,52 +2700,89 @@ extern "C" int spsim_hip_sf_nfft_molecules(const float *d_hkl, int npix, int nmo
                        d_off, d_rot, part);
     SPSIM_HIP_TRY(hipGetLastError());
   }
-  std::vector<double> hq((size_t)qblk * kNb), hpart((size_t)nmol * kMolBlocks * kNb);
-  SPSIM_HIP_TRY(hipMemcpyAsync(hq.data(), qpart, sizeof(double) * hq.size(), hipMemcpyDeviceToHost, s));
-  if (atom_offsets[nmol] > 0)
-    SPSIM_HIP_TRY(hipMemcpyAsync(hpart.data(), part, sizeof(double) * hpart.size(), hipMemcpyDeviceToHost, s));
+  SurfInput in{d_hkl, side, side, d_atoms, d_atom_b, d_segs, nullptr, mols.data(), nmol, nmol, nullptr,
+               rot9s, d_ff, b_global, cus, nullptr};
+  auto scan_surface = [&](char *base) -> int {
+    in.d_mols = (const MolInfo *)(base + at_mols);
+    SPSIM_HIP_TRY(hipMemcpyAsync(base + at_mols, mols.data(), sizeof(MolInfo) * mols.size(), hipMemcpyHostToDevice, s));
+    return surf_scan(in, base + head, base, s);
+  };
+  if (side) SPSIM_TRY(scan_surface(w));
+  std::vector<char> h(at_off);
+  SPSIM_HIP_TRY(hipMemcpyAsync(h.data(), w, total_atoms > 0 ? at_off : at_part, hipMemcpyDeviceToHost, s));
   SPSIM_HIP_TRY(hipStreamSynchronize(s));
+  const double *hpart = (const double *)(h.data() + at_part);
   double hbq[kNb];
-  fold_bounds(hq.data(), qblk, hbq);
-  // 2. Every molecule's grids planned on the host (workspace bytes only), then
-  // the stages enqueued back to back on kWorkers streams: the kHelperStreams
-  // streams forked from s, and s itself. Molecule m goes to worker
-  // m mod kWorkers, each worker with a workspace slice as large as its largest
-  // molecule's. Small molecules' kernels fill few CUs, so the streams overlap
-  // them; s then waits for the helpers.
-  std::vector<double> hbs((size_t)nmol * kNb);
-  std::vector<size_t> need(nmol, 0);
+  fold_bounds((const double *)(h.data() + b_dig), qblk, hbq);
+  // 2. Every molecule's grids planned on the host (sizes and refusals only).
+  std::vector<double> hbs((size_t)nmol * kNb), limit(nmol, 0.0);
+  std::vector<NufftNeed> need(nmol, NufftNeed{0, 0.0});
   for (int m = 0; m < nmol; ++m) {
     const int na = atom_offsets[m + 1] - atom_offsets[m], ns = seg_offsets[m + 1] - seg_offsets[m];
     if (na == 0) continue;
     double *hb = hbs.data() + (size_t)m * kNb;
-    fold_bounds(hpart.data() + (size_t)m * kMolBlocks * kNb, kMolBlocks, hb);
+    fold_bounds(hpart + (size_t)m * kMolBlocks * kNb, kMolBlocks, hb);
     for (int v : {3, 4, 5, 9, 10, 11, 12}) hb[v] = hbq[v];
     double hcopy[kNb];
     for (int v = 0; v < kNb; ++v) hcopy[v] = hb[v];
     SPSIM_TRY(nufft_run(hcopy, d_hkl, npix, d_atoms + atom_offsets[m], d_atom_b ? d_atom_b + atom_offsets[m] : nullptr,
                         d_segs + seg_offsets[m], ns, na, d_ff, b_global, Rs[m], 0, nullptr, W, eps, nullptr, nullptr,
                         nullptr, s, &need[m]));
+    limit[m] = need[m].cost;
   }
+  in.limit = limit.data();
+  struct PlanOwner {
+    SurfPlan *p;
+    ~PlanOwner() { surf_plan_destroy(p); }
+  } plan{side ? surf_plan_choose(in, h.data()) : nullptr};
+  // 3. The molecules that the plan leaves, their stages enqueued back to back
+  // on kWorkers streams: the kHelperStreams streams forked from s, and s
+  // itself. The i-th goes to worker i mod kWorkers, each worker with a
+  // workspace slice as large as its largest molecule's. Small molecules'
+  // kernels fill few CUs, so the streams overlap them; s then waits for the
+  // helpers.
   constexpr int kWorkers = kHelperStreams + 1;
-  size_t slice[kWorkers] = {}, off[kWorkers] = {}, total = 0;
-  for (int m = 0; m < nmol; ++m)
-    if (need[m] > slice[m % kWorkers]) slice[m % kWorkers] = need[m];
-  for (int k = 0; k < kWorkers; ++k) {
-    off[k] = total;
-    total += align256(slice[k]);
+  std::vector<int> rest;
+  size_t off[kWorkers] = {};
+  bool grows = false;
+  for (;;) {
+    rest.clear();
+    for (int m = 0; m < nmol; ++m)
+      if (!surf_plan_takes(plan.p, m)) rest.push_back(m);
+    size_t slice[kWorkers] = {};
+    for (size_t i = 0; i < rest.size(); ++i)
+      slice[i % kWorkers] = std::max(slice[i % kWorkers], need[rest[i]].bytes);
+    // the bounds' records are on the host already; the plan's scan stays in use
+    size_t total = plan.p ? head + b_scan + align256(surf_plan_bytes(plan.p)) : 0;
+    for (int k = 0; k < kWorkers; ++k) {
+      off[k] = total;
+      total += align256(slice[k]);
+    }
+    grows = !workspace_holds(total);
+    const int rc = workspace(total > 0 ? total : 256, &ws);
+    if (rc == SPSIM_HIP_OK) break;
+    if (!plan.p) return rc;
+    surf_plan_destroy(plan.p);  // no memory for both: the grids alone, as far as they go
+    plan.p = nullptr;
   }
-  SPSIM_TRY(workspace(total > 0 ? total : 256, &ws));  // the bounds' records are on the host already
+  w = (char *)ws;
   hipStream_t hs[kWorkers];
   hipEvent_t ev[kHelperStreams + 1];
-  SPSIM_TRY(helper_streams(hs, ev));
+  const int helpers = rest.empty() ? 0 : kHelperStreams;
+  if (helpers > 0) SPSIM_TRY(helper_streams(hs, ev));
   hs[kHelperStreams] = s;
-  SPSIM_HIP_TRY(hipEventRecord(ev[kHelperStreams], s));
-  for (int k = 0; k < kHelperStreams; ++k) SPSIM_HIP_TRY(hipStreamWaitEvent(hs[k], ev[kHelperStreams], 0));
+  if (helpers > 0) SPSIM_HIP_TRY(hipEventRecord(ev[kHelperStreams], s));
+  for (int k = 0; k < helpers; ++k) SPSIM_HIP_TRY(hipStreamWaitEvent(hs[k], ev[kHelperStreams], 0));
   int rc = SPSIM_HIP_OK;
-  for (int m = 0; m < nmol && rc == SPSIM_HIP_OK; ++m) {
+  if (plan.p) {
+    if (grows) rc = scan_surface(w);  // the scan went with the smaller workspace
+    if (rc == SPSIM_HIP_OK) rc = surf_plan_bind(plan.p, w + head, w + head + b_scan, s);
+    if (rc == SPSIM_HIP_OK) rc = surf_plan_run(plan.p, (float2 *)d_F, d_I, s);
+  }
+  for (size_t i = 0; i < rest.size() && rc == SPSIM_HIP_OK; ++i) {
+    const int m = rest[i];
     const int na = atom_offsets[m + 1] - atom_offsets[m], ns = seg_offsets[m + 1] - seg_offsets[m];
-    const int k = m % kWorkers;
+    const int k = (int)(i % kWorkers);
     float *F = d_F ? d_F + (size_t)m * npix * 2 : nullptr;
     float *I = d_I ? d_I + (size_t)m * npix : nullptr;
     if (na == 0) {
@@ -2659,10 +2795,10 @@ extern "C" int spsim_hip_sf_nfft_molecules(const float *d_hkl, int npix, int nmo
     }
     rc = nufft_run(hbs.data() + (size_t)m * kNb, d_hkl, npix, d_atoms + atom_offsets[m],
                    d_atom_b ? d_atom_b + atom_offsets[m] : nullptr, d_segs + seg_offsets[m], ns, na, d_ff, b_global,
-                   Rs[m], 0, nullptr, W, eps, F, I, nullptr, hs[k], nullptr, (char *)ws + off[k]);
+                   Rs[m], 0, nullptr, W, eps, F, I, nullptr, hs[k], nullptr, w + off[k]);
   }
   // join even after a failure, so that s orders after whatever was enqueued
-  for (int k = 0; k < kHelperStreams; ++k) {
+  for (int k = 0; k < helpers; ++k) {
     SPSIM_HIP_TRY(hipEventRecord(ev[k], hs[k]));
     SPSIM_HIP_TRY(hipStreamWaitEvent(s, ev[k], 0));
   }

@@ -251,8 +251,8 @@ struct ScanArgs {
   int list_blocks;  // the last two measure the slopes
   const spsim_hip_atom *atoms;
   const float *atom_b;
-  const MolInfo *mols;  // null: one molecule of natoms atoms
-  int natoms;
+  const MolInfo *mols;  // null: the one molecule
+  MolInfo one;
   bool centre;  // false: the molecules' centres are the origin
   SurfFit *fit;
   float *dev;
@@ -389,8 +389,8 @@ __device__ void scan_atoms(const ScanArgs &a) {
   const int t = threadIdx.x;
   const int mol = ((int)blockIdx.x - a.list_blocks) / kSurfAtomBlocks;
   const int part = ((int)blockIdx.x - a.list_blocks) % kSurfAtomBlocks;
-  const int begin = a.mols ? a.mols[mol].atom_begin : 0;
-  const int n = a.mols ? a.mols[mol].atom_end - begin : a.natoms;
+  const MolInfo mi = a.mols ? a.mols[mol] : a.one;
+  const int begin = mi.atom_begin, n = mi.atom_end - begin;
   const spsim_hip_atom *atoms = a.atoms + begin;
   double c[3] = {0, 0, 0};
   if (n > 0 && a.centre)
@@ -716,18 +716,16 @@ __device__ void build(int part, const SurfFit *fit, const SurfShape &sh, int nx,
   }
 }
 
-__global__ __launch_bounds__(kT) void surface_plan_kernel(PlanArgs a) {
-  __shared__ double snx[kSurfMaxNodes], wnx[kSurfMaxNodes], sny[kSurfMaxNodes], wny[kSurfMaxNodes];
-  __shared__ SurfMol mol;
-  __shared__ int best[2], split[1];
-  __shared__ SurfJob job;
+// What the scan found about a molecule on its list, in *out (thread 0).
+__device__ void fold_records(const SurfRecord *list, int nlist, const SurfRecord *atoms, const spsim_hip_segment *segs,
+                             int nsegs, const float *ff, float b_global, bool has_b, float s2max, SurfMol *out) {
   const int t = threadIdx.x;
   double m[5] = {0, 0, -3.4e38, -3.4e38, 0};  // dev, r2, -B, B, not finite
-  for (int i = t; i < a.list_blocks + kSurfAtomBlocks; i += kT) {
-    const SurfRecord r = a.records[i];
+  for (int i = t; i < nlist + kSurfAtomBlocks; i += kT) {
+    const SurfRecord r = i < nlist ? list[i] : atoms[i - nlist];
     m[0] = fmax(m[0], r.dev);
     m[1] = fmax(m[1], r.r2);
-    if (i >= a.list_blocks) {
+    if (i >= nlist) {
       m[2] = fmax(m[2], -(double)r.bmin);
       m[3] = fmax(m[3], (double)r.bmax);
     }
@@ -736,19 +734,64 @@ __global__ __launch_bounds__(kT) void surface_plan_kernel(PlanArgs a) {
   block_reduce(m);
   // every form-factor row that is used, one thread each
   float bs = 0.0f, weak = 1.0f;
-  for (int i = t; i < a.job.nsegs; i += kT) {
-    const int sp = a.job.segs[i].species;
-    species_terms(a.ff + sp * SPSIM_HIP_FF_STRIDE, sp == SPSIM_HIP_UNIT_SPECIES ? 0.0f : a.b_global,
-                  a.has_b ? (float)-m[2] : 0.0f, a.has_b ? (float)m[3] : 0.0f, a.fit->s2max, &bs, &weak);
+  for (int i = t; i < nsegs; i += kT) {
+    const int sp = segs[i].species;
+    species_terms(ff + sp * SPSIM_HIP_FF_STRIDE, sp == SPSIM_HIP_UNIT_SPECIES ? 0.0f : b_global,
+                  has_b ? (float)-m[2] : 0.0f, has_b ? (float)m[3] : 0.0f, s2max, &bs, &weak);
   }
   double e[2] = {(double)bs, -(double)weak};
   block_reduce(e);
+  if (t == 0) *out = SurfMol{sqrt(m[1]), m[0], (float)e[0], (float)-e[1], m[4] > 0.0};
+}
+
+// One workgroup per molecule.
+struct DigestArgs {
+  const SurfFit *fit;
+  const SurfRecord *records;
+  int list_blocks;
+  const MolInfo *mols;
+  MolInfo one;
+  const spsim_hip_segment *segs;
+  const float *ff;
+  float b_global;
+  bool has_b;
+  const double *centres;
+  SurfHead *head;
+  SurfDigest *out;
+};
+
+__global__ __launch_bounds__(kT) void surface_digest_kernel(DigestArgs a) {
+  const int m = blockIdx.x, t = threadIdx.x;
+  const MolInfo mi = a.mols ? a.mols[m] : a.one;
+  SurfDigest d;
+  fold_records(a.records, a.list_blocks, a.records + a.list_blocks + (size_t)m * kSurfAtomBlocks, a.segs + mi.seg_begin,
+               mi.nseg, a.ff, a.b_global, a.has_b, a.fit->s2max, &d.mol);
   if (t == 0) {
-    mol.radius = sqrt(m[1]) * a.scale;
-    mol.dev = m[0];
-    mol.b_smooth = (float)e[0];
-    mol.weakest = (float)-e[1];
-    mol.bad = m[4] > 0.0;
+    for (int k = 0; k < 3; ++k) d.centre[k] = a.centres[3 * m + k];
+    a.out[m] = d;
+  }
+  if (m > 0) return;
+  if (t < kLines) {
+    a.head->slope_x[t] = a.fit->slope_x[t];
+    a.head->slope_y[t] = a.fit->slope_y[t];
+  }
+  if (t == 0) {
+    a.head->s2max = a.fit->s2max;
+    for (int k = 0; k < 3; ++k) a.head->normal[k] = a.fit->normal[k];
+    a.head->sym = a.fit->sym;
+  }
+}
+
+__global__ __launch_bounds__(kT) void surface_plan_kernel(PlanArgs a) {
+  __shared__ double snx[kSurfMaxNodes], wnx[kSurfMaxNodes], sny[kSurfMaxNodes], wny[kSurfMaxNodes];
+  __shared__ SurfMol mol;
+  __shared__ int best[2], split[1];
+  __shared__ SurfJob job;
+  const int t = threadIdx.x;
+  fold_records(a.records, a.list_blocks, a.records + a.list_blocks, a.job.segs, a.job.nsegs, a.ff, a.b_global, a.has_b,
+               a.fit->s2max, &mol);
+  if (t == 0) {
+    mol.radius *= a.scale;
     best[0] = best[1] = 1 << 30;
   }
   __syncthreads();
@@ -822,9 +865,9 @@ __global__ __launch_bounds__(kT) void surface_plan_kernel(PlanArgs a) {
   }
 }
 
-__global__ __launch_bounds__(kT) void surface_tables_kernel(const SurfFit *fit, SurfShape sh, int nx, int ny) {
+__global__ __launch_bounds__(kT) void surface_tables_kernel(const SurfFit *fit, const SurfShape *shapes, int nx, int ny) {
   __shared__ double snx[kSurfMaxNodes], wnx[kSurfMaxNodes], sny[kSurfMaxNodes], wny[kSurfMaxNodes];
-  build(blockIdx.y, fit, sh, nx, ny, snx, wnx, sny, wny);
+  build(blockIdx.y, fit, shapes[blockIdx.z], nx, ny, snx, wnx, sny, wny);
 }
 
 // ---- 3. node sums ---------------------------------------------------------------
@@ -1672,7 +1715,7 @@ int launch_plan(const PatternLaunch &a, int nx, int ny, const Spectrum *sp, Surf
                     a.atoms,
                     a.atom_b,
                     nullptr,
-                    a.natoms,
+                    MolInfo{0, a.natoms, 0, a.nsegs},
                     !sp,
                     (SurfFit *)(w + l.fit),
                     (float *)(w + l.dev),
@@ -1736,16 +1779,18 @@ struct SurfPlan {
     int first, count, item_first, nitems, max_nodes, max_ny;
     bool split;
   };
-  int nx = 0, ny = 0, cus = 0;
-  bool has_b = false;
-  float b_global = 0.0f;
-  const float *hkl = nullptr, *ff = nullptr;
+  SurfInput in{};
   std::vector<char> takes;
   std::vector<Group> groups;
-  std::vector<void *> owned;  // device memory
-  const SurfJob *jobs = nullptr;
-  const SurfItem *items = nullptr;
+  std::vector<SurfShape> shapes;
+  std::vector<SurfJob> jobs;
+  std::vector<SurfItem> items;
+  // device memory: shapes, jobs and items (one upload), the shapes' tables, the workspace
+  size_t at_jobs = 0, at_items = 0, at_tables = 0, at_ws = 0, bytes = 0;
+  const SurfJob *d_jobs = nullptr;
+  const SurfItem *d_items = nullptr;
   const float *dev = nullptr;
+  std::vector<void *> owned;
 };
 
 namespace {
@@ -1754,23 +1799,6 @@ constexpr size_t kGroupBytes = (size_t)256 << 20;  // workspace of a group: abou
 
 __global__ __launch_bounds__(kT) void surface_prepare_kernel(const SurfJob *jobs, int first, bool has_b) {
   prepare_atoms(jobs[first + blockIdx.y], has_b, (int)(blockIdx.x * kT + threadIdx.x), (int)gridDim.x * kT);
-}
-
-bool choose(const SurfFit &fit, const SurfMol &mol, int nx, int ny, int natoms, SurfAxis *ax, SurfAxis *ay) {
-  if (!smooth(mol, fit.s2max)) return false;
-  SurfAxis *out[2] = {ax, ay};
-  for (int k = 0; k < 2; ++k) {
-    const float *slope = k ? fit.slope_y : fit.slope_x;
-    int n = kSurfMinNodes;
-    // steps of 8 from 64 nodes on: molecules of similar size share their tables
-    while (n <= kSurfMaxNodes &&
-           !(axis_need(slope, (float)mol.radius, mol.b_smooth * fit.s2max, axis_stretch(n)) <= (float)n))
-      n += n < 64 ? 4 : 8;
-    if (n > kSurfMaxNodes) return false;
-    *out[k] = SurfAxis{n, axis_stretch(n), 0.0};
-    out[k]->asin_a = std::asin(out[k]->a);
-  }
-  return worth(ax->n, ay->n, nx, ny, natoms, SurfKind::kSum);
 }
 
 // Lays the job's buffers out in a workspace from `at` on; returns the end.
@@ -1792,8 +1820,29 @@ size_t place(SurfJob *j, int nx, char *ws, size_t at) {
   return at;
 }
 
+// The same for a shape's node positions and weights.
+size_t place_tables(SurfShape *sh, int nx, int ny, char *mem, size_t at) {
+  auto take = [&](size_t bytes) {
+    char *p = mem + at;
+    at += align_up(bytes);
+    return p;
+  };
+  const size_t wx = (size_t)sh->ax.n * nx, wy = (size_t)sh->ay.n * ny;
+  sh->nodes = (double *)take(sizeof(double) * 3 * sh->ax.n * sh->ay.n);
+  sh->tx = (double *)take(sizeof(double) * wx);
+  sh->ty = (double *)take(sizeof(double) * wy);
+  sh->tx32 = (float2 *)take(sizeof(float2) * wx);
+  sh->ty32 = (float2 *)take(sizeof(float2) * wy);
+  return at;
+}
+
 // Issue cycles of one atom in a lane's nodes (node_tiling).
 double lane_cost(int per_lane) { return per_lane == 8 ? 321.0 : (per_lane == 1 ? 75.0 : 57.0 * per_lane); }
+
+// Issue cycles of a pattern's interpolation: 85 us on 1024^2 pixels at 188 nodes.
+double interpolation_cost(double nodes_x, double nodes_y, double nx, double ny) {
+  return 57.0 * (nx * ny * nodes_y + nx * nodes_x * nodes_y);
+}
 
 // Splits a group's atoms so that its work items number about four per resident
 // workgroup, and appends the items, largest first.
@@ -1815,186 +1864,254 @@ void split_group(std::vector<SurfJob> &jobs, int first, int count, int slots, st
   });
 }
 
-template <class T>
-int own(SurfPlan *p, T **out, size_t n) {
-  *out = nullptr;
-  hipError_t e = hipMalloc((void **)out, std::max<size_t>(1, n) * sizeof(T));
-  if (e != hipSuccess) return fail(SPSIM_HIP_ERR_NOMEM, "hipMalloc(%zu) failed: %s", n * sizeof(T), hipGetErrorString(e));
-  p->owned.push_back(*out);
+// Scan memory, within a block of surf_scan_bytes.
+struct ScanLayout {
+  size_t fit, dev, records, centres, total;
+  int list_blocks;
+};
+ScanLayout scan_layout(int nx, int ny, int nmol) {
+  ScanLayout l{};
+  l.list_blocks = std::min(kSurfListBlocks, ny + 2);
+  size_t at = 0;
+  auto take = [&](size_t bytes) {
+    const size_t o = at;
+    at += align_up(bytes);
+    return o;
+  };
+  l.fit = take(sizeof(SurfFit));
+  l.dev = take(sizeof(float) * 3 * (size_t)nx * ny);
+  l.records = take(sizeof(SurfRecord) * (l.list_blocks + (size_t)nmol * kSurfAtomBlocks));
+  l.centres = take(sizeof(double) * 3 * (size_t)nmol);
+  l.total = at;
+  return l;
+}
+
+// Node counts of an axis: multiples of 4 up to 64 and of 8 from there on, so
+// that molecules of similar size share their tables; the need falls as the
+// count grows and the stretch with it.
+int axis_count(int k) { return k <= 12 ? kSurfMinNodes + 4 * k : 64 + 8 * (k - 12); }
+
+int axis_nodes(const float *slope, double radius, float gauss) {
+  auto enough = [&](int n) { return axis_need(slope, (float)radius, gauss, axis_stretch(n)) <= (float)n; };
+  int lo = -1, hi = 12 + (kSurfMaxNodes - 64) / 8;
+  if (!enough(axis_count(hi))) return 0;
+  while (hi - lo > 1) {
+    const int mid = (lo + hi) / 2;
+    (enough(axis_count(mid)) ? hi : lo) = mid;
+  }
+  return axis_count(hi);
+}
+
+// Nodes of a pattern; false when it is left to its other path.
+bool choose(const SurfHead &head, SurfMol mol, double norm, int nx, int ny, int natoms, const double *limit,
+            SurfAxis *ax, SurfAxis *ay) {
+  mol.radius *= norm;
+  if (natoms <= 0 || !smooth(mol, head.s2max)) return false;
+  SurfAxis *out[2] = {ax, ay};
+  for (int k = 0; k < 2; ++k) {
+    const int n = axis_nodes(k ? head.slope_y : head.slope_x, mol.radius, mol.b_smooth * head.s2max);
+    if (n == 0) return false;
+    *out[k] = SurfAxis{n, axis_stretch(n), 0.0};
+    out[k]->asin_a = std::asin(out[k]->a);
+  }
+  if (!limit) return worth(ax->n, ay->n, nx, ny, natoms, SurfKind::kSum);
+  int per_lane, tiles;
+  node_tiling(ax->n, ay->n, head.sym == 2 && ax->n == ay->n, 1LL << 25, &per_lane, &tiles);
+  return (double)tiles * kT * lane_cost(per_lane) * natoms + interpolation_cost(ax->n, ay->n, nx, ny) < *limit;
+}
+
+}  // namespace
+
+size_t surf_scan_bytes(int nx, int ny, int nmol) { return scan_layout(nx, ny, nmol).total; }
+
+int surf_scan(const SurfInput &in, void *scan, void *digest, hipStream_t s) {
+  const ScanLayout l = scan_layout(in.nx, in.ny, in.nmol);
+  char *w = (char *)scan;
+  const MolInfo one = in.d_mols ? MolInfo{} : in.h_mols[0];
+  const ScanArgs sc{in.hkl,
+                    in.nx,
+                    in.ny,
+                    l.list_blocks,
+                    in.atoms,
+                    in.atom_b,
+                    in.d_mols,
+                    one,
+                    true,
+                    (SurfFit *)(w + l.fit),
+                    (float *)(w + l.dev),
+                    (SurfRecord *)(w + l.records),
+                    (double *)(w + l.centres)};
+  hipLaunchKernelGGL(surface_scan_kernel, dim3(l.list_blocks + in.nmol * kSurfAtomBlocks), dim3(kT), 0, s, sc);
+  const DigestArgs d{sc.fit, sc.records,  l.list_blocks,        in.d_mols,  one,
+                     in.segs, in.ff,      in.b_global,          in.atom_b != nullptr, sc.centres,
+                     (SurfHead *)digest,  (SurfDigest *)((char *)digest + sizeof(SurfHead))};
+  hipLaunchKernelGGL(surface_digest_kernel, dim3(in.nmol), dim3(kT), 0, s, d);
+  SPSIM_HIP_TRY(hipGetLastError());
   return SPSIM_HIP_OK;
 }
 
-int build_plan(SurfPlan *p, const spsim_hip_atom *atoms, const float *atom_b, const spsim_hip_segment *segs,
-               const MolInfo *d_mols, const MolInfo *h_mols, int nmol, const spsim_hip_segment *h_segs, int npatterns,
-               const int *pattern_mol, const double *rot9, const float *h_ff) {
-  const int lb = std::min(kSurfListBlocks, p->ny + 2);
-  SurfFit *d_fit = nullptr;
-  float *dev = nullptr;
-  SPSIM_TRY(own(p, &d_fit, 1));
-  SPSIM_TRY(own(p, &dev, 3 * (size_t)p->nx * p->ny));
-  p->dev = dev;
-  SurfFit fit;
-  std::vector<SurfRecord> rec(lb + (size_t)nmol * kSurfAtomBlocks);
-  std::vector<double> centres(3 * (size_t)nmol);
-  {
-    SurfPlan scratch;  // released below
-    SurfRecord *d_rec = nullptr;
-    double *d_centres = nullptr;
-    int rc = own(&scratch, &d_rec, rec.size());
-    if (rc == SPSIM_HIP_OK) rc = own(&scratch, &d_centres, centres.size());
-    hipError_t e = hipSuccess;
-    if (rc == SPSIM_HIP_OK) {
-      const ScanArgs sc{p->hkl, p->nx, p->ny, lb, atoms, atom_b, d_mols, 0, true, d_fit, dev, d_rec, d_centres};
-      hipLaunchKernelGGL(surface_scan_kernel, dim3(lb + nmol * kSurfAtomBlocks), dim3(kT), 0, nullptr, sc);
-      e = hipGetLastError();
-      if (e == hipSuccess) e = hipMemcpy(&fit, d_fit, sizeof fit, hipMemcpyDeviceToHost);
-      if (e == hipSuccess) e = hipMemcpy(rec.data(), d_rec, rec.size() * sizeof(SurfRecord), hipMemcpyDeviceToHost);
-      if (e == hipSuccess)
-        e = hipMemcpy(centres.data(), d_centres, centres.size() * sizeof(double), hipMemcpyDeviceToHost);
+SurfPlan *surf_plan_choose(const SurfInput &in, const void *digest) {
+  const SurfHead &head = *(const SurfHead *)digest;
+  const SurfDigest *mols = (const SurfDigest *)((const char *)digest + sizeof(SurfHead));
+  SurfPlan *p = new SurfPlan;
+  p->in = in;
+  p->takes.assign(in.npatterns, 0);
+  struct Choice {
+    double norm;
+    int shape;  // -1: not taken
+  };
+  std::vector<Choice> last(in.nmol, Choice{-1.0, -1});  // of a molecule's last pattern
+  std::vector<SurfJob> &jobs = p->jobs;
+  for (int i = 0; i < in.npatterns; ++i) {
+    const int m = in.pattern_mol ? in.pattern_mol[i] : (in.nmol == 1 ? 0 : i);
+    const int natoms = in.h_mols[m].atom_end - in.h_mols[m].atom_begin;
+    // rotations differ from 1 by rounding: one node count serves them
+    double norm = in.rot9 ? rotation_norm(in.rot9 + 9 * (size_t)i) : 1.0;
+    if (std::fabs(norm - 1.0) < 1e-6) norm = 1.0;
+    if (last[m].norm != norm) {
+      last[m] = Choice{norm, -1};
+      SurfShape sh{};
+      if (choose(head, mols[m].mol, norm, in.nx, in.ny, natoms, in.limit ? in.limit + m : nullptr, &sh.ax, &sh.ay)) {
+        for (size_t k = 0; k < p->shapes.size(); ++k)
+          if (p->shapes[k].ax.n == sh.ax.n && p->shapes[k].ay.n == sh.ay.n) last[m].shape = (int)k;
+        if (last[m].shape < 0) {
+          last[m].shape = (int)p->shapes.size();
+          p->shapes.push_back(sh);
+        }
+      }
     }
-    for (void *m : scratch.owned) (void)hipFree(m);
-    SPSIM_TRY(rc);
-    if (e != hipSuccess) return hip_fail(e, "surface scan");
-  }
-  double dev_max = 0.0;
-  bool bad = false;
-  for (int i = 0; i < lb; ++i) {
-    dev_max = std::max(dev_max, rec[i].dev);
-    bad = bad || rec[i].bad;
-  }
-  std::vector<SurfShape> shapes;
-  std::vector<int> shape_of(nmol, -1);
-  std::vector<double> norm(nmol, 0.0);  // of the matrices a molecule is shown under
-  for (int i = 0; i < npatterns; ++i) {
-    double &n = norm[pattern_mol[i]];
-    n = std::max(n, rotation_norm(rot9 + 9 * (size_t)i));
-  }
-  for (int m = 0; m < nmol; ++m) {
-    const MolInfo &mi = h_mols[m];
-    SurfMol mol{0.0, dev_max, 0.0f, 1.0f, bad};
-    float lo = 3.4e38f, hi = -3.4e38f;
-    for (int i = 0; i < kSurfAtomBlocks; ++i) {
-      const SurfRecord &r = rec[lb + (size_t)m * kSurfAtomBlocks + i];
-      mol.radius = std::max(mol.radius, std::sqrt(r.r2));
-      lo = std::min(lo, r.bmin);
-      hi = std::max(hi, r.bmax);
-      mol.bad |= r.bad;
-    }
-    mol.radius *= norm[m];
-    for (int i = 0; i < mi.nseg; ++i) {
-      const int sp = h_segs[mi.seg_begin + i].species;
-      species_terms(h_ff + sp * SPSIM_HIP_FF_STRIDE, sp == SPSIM_HIP_UNIT_SPECIES ? 0.0f : p->b_global,
-                    p->has_b ? lo : 0.0f, p->has_b ? hi : 0.0f, fit.s2max, &mol.b_smooth, &mol.weakest);
-    }
-    SurfShape sh{};
-    if (!choose(fit, mol, p->nx, p->ny, mi.atom_end - mi.atom_begin, &sh.ax, &sh.ay)) continue;
-    for (size_t i = 0; i < shapes.size(); ++i)
-      if (shapes[i].ax.n == sh.ax.n && shapes[i].ay.n == sh.ay.n) shape_of[m] = (int)i;
-    if (shape_of[m] >= 0) continue;
-    SPSIM_TRY(own(p, &sh.nodes, 3 * (size_t)sh.ax.n * sh.ay.n));
-    SPSIM_TRY(own(p, &sh.tx, (size_t)sh.ax.n * p->nx));
-    SPSIM_TRY(own(p, &sh.ty, (size_t)sh.ay.n * p->ny));
-    SPSIM_TRY(own(p, &sh.tx32, (size_t)sh.ax.n * p->nx));
-    SPSIM_TRY(own(p, &sh.ty32, (size_t)sh.ay.n * p->ny));
-    hipLaunchKernelGGL(surface_tables_kernel, dim3(256, 2), dim3(kT), 0, nullptr, (const SurfFit *)d_fit, sh, p->nx,
-                       p->ny);
-    SPSIM_HIP_TRY(hipGetLastError());
-    shape_of[m] = (int)shapes.size();
-    shapes.push_back(sh);
-  }
-  std::vector<SurfJob> jobs;
-  p->takes.assign(npatterns, 0);
-  for (int i = 0; i < npatterns; ++i) {
-    const int m = pattern_mol[i];
-    if (shape_of[m] < 0) continue;
+    if (last[m].shape < 0) continue;
     p->takes[i] = 1;
     SurfJob j{};
     j.ok = 1;
-    j.nx = p->nx;
-    j.ny = p->ny;
-    j.sh = shapes[shape_of[m]];
-    j.atoms = atoms + h_mols[m].atom_begin;
-    j.atom_b = p->has_b ? atom_b + h_mols[m].atom_begin : nullptr;
-    j.segs = segs + h_mols[m].seg_begin;
-    j.nsegs = h_mols[m].nseg;
-    j.natoms = h_mols[m].atom_end - h_mols[m].atom_begin;
-    j.has_rot = 1;
-    std::copy(rot9 + 9 * (size_t)i, rot9 + 9 * (size_t)(i + 1), j.rot);
-    std::copy(&centres[3 * (size_t)m], &centres[3 * (size_t)m] + 3, j.r0);
-    std::copy(fit.normal, fit.normal + 3, j.normal);
+    j.nx = in.nx;
+    j.ny = in.ny;
+    j.sh = p->shapes[last[m].shape];
+    j.shape = last[m].shape;
+    j.atoms = in.atoms + in.h_mols[m].atom_begin;
+    j.atom_b = in.atom_b ? in.atom_b + in.h_mols[m].atom_begin : nullptr;
+    j.segs = in.segs + in.h_mols[m].seg_begin;
+    j.nsegs = in.h_mols[m].nseg;
+    j.natoms = natoms;
+    j.has_rot = in.rot9 != nullptr;
+    if (in.rot9) std::copy(in.rot9 + 9 * (size_t)i, in.rot9 + 9 * (size_t)(i + 1), j.rot);
+    std::copy(mols[m].centre, mols[m].centre + 3, j.r0);
+    std::copy(head.normal, head.normal + 3, j.normal);
     // a group has work enough for every tiling: the one of the least work
-    node_tiling(j.sh.ax.n, j.sh.ay.n, fit.sym == 2 && j.sh.ax.n == j.sh.ay.n, 1LL << 25, &j.per_lane, &j.tiles);
+    node_tiling(j.sh.ax.n, j.sh.ay.n, head.sym == 2 && j.sh.ax.n == j.sh.ay.n, 1LL << 25, &j.per_lane, &j.tiles);
     j.pattern = i;
     jobs.push_back(j);
   }
-  if (jobs.empty()) return SPSIM_HIP_OK;
+  if (jobs.empty()) {
+    delete p;
+    return nullptr;
+  }
   // largest first, so that a group's patterns need similar grids
   std::stable_sort(jobs.begin(), jobs.end(), [](const SurfJob &a, const SurfJob &b) {
     return (double)a.sh.ax.n * a.sh.ay.n * a.natoms > (double)b.sh.ax.n * b.sh.ay.n * b.natoms;
   });
-  const int slots = resident_slots(nodes_kernel(p->has_b, false), p->cus);
-  std::vector<SurfItem> items;
+  const int slots = resident_slots(nodes_kernel(in.atom_b != nullptr, false), in.cus);
   size_t ws_bytes = 0;
   for (int first = 0; first < (int)jobs.size();) {
-    SurfPlan::Group g{first, 0, (int)items.size(), 0, 0, 0, false};
+    SurfPlan::Group g{first, 0, (int)p->items.size(), 0, 0, 0, false};
     size_t at = 0;
     while (first + g.count < (int)jobs.size() && g.count < 4096) {
       SurfJob probe = jobs[first + g.count];
       probe.splits = 4;  // a typical group's; only the group's size depends on it
-      const size_t end = place(&probe, p->nx, nullptr, at);
+      const size_t end = place(&probe, in.nx, nullptr, at);
       if (g.count > 0 && end > kGroupBytes) break;
       at = end;
       g.max_nodes = std::max(g.max_nodes, probe.sh.ax.n * probe.sh.ay.n);
       g.max_ny = std::max(g.max_ny, probe.sh.ay.n);
       ++g.count;
     }
-    split_group(jobs, first, g.count, slots, &items);
-    g.nitems = (int)items.size() - g.item_first;
+    split_group(jobs, first, g.count, slots, &p->items);
+    g.nitems = (int)p->items.size() - g.item_first;
     at = 0;
     for (int i = first; i < first + g.count; ++i) {
-      at = place(&jobs[i], p->nx, nullptr, at);
+      at = place(&jobs[i], in.nx, nullptr, at);
       g.split = g.split || jobs[i].splits > 1;
     }
     ws_bytes = std::max(ws_bytes, at);
     p->groups.push_back(g);
     first += g.count;
   }
-  char *ws = nullptr;
-  SurfJob *d_jobs = nullptr;
-  SurfItem *d_items = nullptr;
-  SPSIM_TRY(own(p, &ws, ws_bytes));
+  p->in.h_mols = nullptr;  // the caller's arrays
+  p->in.pattern_mol = nullptr;
+  p->in.rot9 = nullptr;
+  p->in.limit = nullptr;
+  p->at_jobs = align_up(sizeof(SurfShape) * p->shapes.size());
+  p->at_items = p->at_jobs + align_up(sizeof(SurfJob) * jobs.size());
+  p->at_tables = p->at_items + align_up(sizeof(SurfItem) * p->items.size());
+  size_t at = p->at_tables;
+  for (SurfShape &sh : p->shapes) at = place_tables(&sh, in.nx, in.ny, nullptr, at);
+  p->at_ws = at;
+  p->bytes = at + ws_bytes;
+  return p;
+}
+
+size_t surf_plan_bytes(const SurfPlan *p) { return p->bytes; }
+
+int surf_plan_bind(SurfPlan *p, const void *scan, void *mem, hipStream_t s) {
+  const SurfInput &in = p->in;
+  const ScanLayout l = scan_layout(in.nx, in.ny, in.nmol);
+  char *w = (char *)mem;
+  size_t at = p->at_tables;
+  for (SurfShape &sh : p->shapes) at = place_tables(&sh, in.nx, in.ny, w, at);
   for (const SurfPlan::Group &g : p->groups) {
-    size_t at = 0;
-    for (int i = g.first; i < g.first + g.count; ++i) at = place(&jobs[i], p->nx, ws, at);
+    at = p->at_ws;
+    for (int i = g.first; i < g.first + g.count; ++i) {
+      p->jobs[i].sh = p->shapes[p->jobs[i].shape];
+      at = place(&p->jobs[i], in.nx, w, at);
+    }
   }
-  SPSIM_TRY(own(p, &d_jobs, jobs.size()));
-  SPSIM_TRY(own(p, &d_items, items.size()));
-  SPSIM_HIP_TRY(hipMemcpy(d_jobs, jobs.data(), jobs.size() * sizeof(SurfJob), hipMemcpyHostToDevice));
-  SPSIM_HIP_TRY(hipMemcpy(d_items, items.data(), items.size() * sizeof(SurfItem), hipMemcpyHostToDevice));
-  SPSIM_HIP_TRY(hipStreamSynchronize(nullptr));  // the tables
-  p->jobs = d_jobs;
-  p->items = d_items;
+  std::vector<char> image(p->at_tables);
+  std::copy(p->shapes.begin(), p->shapes.end(), (SurfShape *)image.data());
+  std::copy(p->jobs.begin(), p->jobs.end(), (SurfJob *)(image.data() + p->at_jobs));
+  std::copy(p->items.begin(), p->items.end(), (SurfItem *)(image.data() + p->at_items));
+  SPSIM_HIP_TRY(hipMemcpyAsync(w, image.data(), image.size(), hipMemcpyHostToDevice, s));
+  const int nshapes = (int)p->shapes.size();
+  for (int first = 0; first < nshapes; first += 4096)
+    hipLaunchKernelGGL(surface_tables_kernel, dim3(256, 2, std::min(4096, nshapes - first)), dim3(kT), 0, s,
+                       (const SurfFit *)((const char *)scan + l.fit), (const SurfShape *)w + first, in.nx, in.ny);
+  SPSIM_HIP_TRY(hipGetLastError());
+  SPSIM_HIP_TRY(hipStreamSynchronize(s));  // the copy reads image
+  p->dev = (const float *)((const char *)scan + l.dev);
+  p->d_jobs = (const SurfJob *)(w + p->at_jobs);
+  p->d_items = (const SurfItem *)(w + p->at_items);
   return SPSIM_HIP_OK;
 }
 
-}  // namespace
-
-int surf_plan_create(const float *hkl, int nx, int ny, const spsim_hip_atom *atoms, const float *atom_b,
-                     const spsim_hip_segment *segs, const MolInfo *d_mols, const MolInfo *h_mols, int nmol,
-                     const spsim_hip_segment *h_segs, int npatterns, const int *pattern_mol, const double *rot9,
-                     const float *d_ff, const float *h_ff, float b_global, int cus, SurfPlan **out) {
+int surf_plan_create(const SurfInput &in, SurfPlan **out) {
   *out = nullptr;
-  if (nx < kSurfMinSide || ny < kSurfMinSide) return SPSIM_HIP_OK;
-  SurfPlan *p = new SurfPlan;
-  p->nx = nx;
-  p->ny = ny;
-  p->cus = cus;
-  p->has_b = atom_b != nullptr;
-  p->b_global = b_global;
-  p->hkl = hkl;
-  p->ff = d_ff;
-  const int rc = build_plan(p, atoms, atom_b, segs, d_mols, h_mols, nmol, h_segs, npatterns, pattern_mol, rot9, h_ff);
-  if (rc != SPSIM_HIP_OK || p->groups.empty()) {
+  if (in.nx < kSurfMinSide || in.ny < kSurfMinSide) return SPSIM_HIP_OK;
+  const size_t scan_bytes = surf_scan_bytes(in.nx, in.ny, in.nmol), digest_bytes = surf_digest_bytes(in.nmol);
+  auto alloc = [](void **m, size_t bytes) {
+    const hipError_t e = hipMalloc(m, bytes);
+    return e == hipSuccess ? SPSIM_HIP_OK
+                           : fail(SPSIM_HIP_ERR_NOMEM, "hipMalloc(%zu) failed: %s", bytes, hipGetErrorString(e));
+  };
+  void *scan = nullptr, *mem = nullptr;
+  SPSIM_TRY(alloc(&scan, scan_bytes + digest_bytes));
+  void *digest = (char *)scan + scan_bytes;
+  std::vector<char> h(digest_bytes);
+  int rc = surf_scan(in, scan, digest, nullptr);
+  if (rc == SPSIM_HIP_OK) {
+    const hipError_t e = hipMemcpy(h.data(), digest, digest_bytes, hipMemcpyDeviceToHost);
+    if (e != hipSuccess) rc = hip_fail(e, "surface scan");
+  }
+  SurfPlan *p = rc == SPSIM_HIP_OK ? surf_plan_choose(in, h.data()) : nullptr;
+  if (!p) {
+    (void)hipFree(scan);
+    return rc;
+  }
+  p->owned.push_back(scan);
+  rc = alloc(&mem, p->bytes);
+  if (rc == SPSIM_HIP_OK) {
+    p->owned.push_back(mem);
+    rc = surf_plan_bind(p, scan, mem, nullptr);
+  }
+  if (rc != SPSIM_HIP_OK) {
     surf_plan_destroy(p);
     return rc;
   }
@@ -2005,13 +2122,15 @@ int surf_plan_create(const float *hkl, int nx, int ny, const spsim_hip_atom *ato
 bool surf_plan_takes(const SurfPlan *p, int pattern) { return p && p->takes[pattern]; }
 
 int surf_plan_run(const SurfPlan *p, float2 *F, float *I, hipStream_t s) {
-  const int slots = resident_slots(nodes_kernel(p->has_b, false), p->cus);
+  const SurfInput &in = p->in;
+  const bool has_b = in.atom_b != nullptr;
+  const int slots = resident_slots(nodes_kernel(has_b, false), in.cus);
   for (const SurfPlan::Group &g : p->groups) {
-    hipLaunchKernelGGL(surface_prepare_kernel, dim3(16, g.count), dim3(kT), 0, s, p->jobs, g.first, p->has_b);
-    const SurfItem *items = p->items + g.item_first;
+    hipLaunchKernelGGL(surface_prepare_kernel, dim3(16, g.count), dim3(kT), 0, s, p->d_jobs, g.first, has_b);
+    const SurfItem *items = p->d_items + g.item_first;
     const int blocks = std::min(g.nitems, slots);
-    SPSIM_TRY(launch_nodes(p->jobs, items, g.nitems, blocks, p->ff, p->b_global, p->has_b, nullptr, s));
-    launch_interpolation(p->jobs, g.first, g.count, p->nx, p->ny, g.split ? g.max_nodes : 0, g.max_ny, p->dev, p->hkl,
+    SPSIM_TRY(launch_nodes(p->d_jobs, items, g.nitems, blocks, in.ff, in.b_global, has_b, nullptr, s));
+    launch_interpolation(p->d_jobs, g.first, g.count, in.nx, in.ny, g.split ? g.max_nodes : 0, g.max_ny, p->dev, in.hkl,
                          F, I, s);
   }
   SPSIM_HIP_TRY(hipGetLastError());

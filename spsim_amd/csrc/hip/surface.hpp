@@ -77,6 +77,7 @@ struct SurfJob {
   double2 *t64;
   float4 *t32;
   long long pattern;  // index of the outputs
+  int shape;          // of a plan
 };
 
 struct SurfItem {
@@ -120,17 +121,58 @@ int launch_surface_adjoint(const PatternLaunch &a, const float *gI, int nx, int 
                            int ntiles, int splits, bool want_b, double4 *partial, int cus, void *ws,
                            const int **ok_flag, hipStream_t s);
 
-// ---- plans that decide on the host (batch.hip) ----
+// ---- plans that decide on the host (batch.hip, nufft.hip) ----
+
+// What the host reads of a list, and of a molecule seen on it.
+struct SurfHead {
+  float slope_x[kSurfLines], slope_y[kSurfLines];
+  float s2max, normal[3];
+  int sym, pad;
+};
+struct SurfDigest {
+  SurfMol mol;
+  double centre[3];
+};
+
+// A list and its patterns. Pattern p shows molecule pattern_mol[p] (null:
+// molecule p, or 0 when there is only one) under the matrix rot9 + 9 p (null:
+// none). All pointers but h_mols, pattern_mol, rot9 and limit are device memory;
+// d_mols is null for one molecule h_mols[0].
+struct SurfInput {
+  const float *hkl;
+  int nx, ny;
+  const spsim_hip_atom *atoms;
+  const float *atom_b;
+  const spsim_hip_segment *segs;
+  const MolInfo *d_mols, *h_mols;
+  int nmol, npatterns;
+  const int *pattern_mol;
+  const double *rot9;
+  const float *ff;
+  float b_global;
+  int cus;
+  const double *limit;  // per molecule, cost above which its patterns are left; null: of the direct sum
+};
+
+// The scan's device memory (which a plan keeps using) and its digest: a SurfHead
+// and a SurfDigest per molecule, for the host to copy.
+size_t surf_scan_bytes(int nx, int ny, int nmol);
+constexpr size_t surf_digest_bytes(int nmol) { return sizeof(SurfHead) + sizeof(SurfDigest) * (size_t)nmol; }
+int surf_scan(const SurfInput &in, void *scan, void *digest, hipStream_t s);
 
 struct SurfPlan;
 
-// Looks at a plan's list and molecules (all in device memory; pattern p shows
-// molecule pattern_mol[p] rotated by rot9 + 9 p) and prepares the patterns that
-// are smooth enough. *out is null when there is none. Synchronises.
-int surf_plan_create(const float *hkl, int nx, int ny, const spsim_hip_atom *atoms, const float *atom_b,
-                     const spsim_hip_segment *segs, const MolInfo *d_mols, const MolInfo *h_mols, int nmol,
-                     const spsim_hip_segment *h_segs, int npatterns, const int *pattern_mol, const double *rot9,
-                     const float *d_ff, const float *h_ff, float b_global, int cus, SurfPlan **out);
+// The patterns that are smooth enough and cheaper than in.limit, from the host
+// copy of a digest; null when there is none. No device work.
+SurfPlan *surf_plan_choose(const SurfInput &in, const void *digest);
+// Device memory of its own that the plan needs, and the upload of its tables
+// there. The host copy may go when surf_plan_bind returns (it waits for s).
+size_t surf_plan_bytes(const SurfPlan *p);
+int surf_plan_bind(SurfPlan *p, const void *scan, void *mem, hipStream_t s);
+
+// All of it, in device memory that the plan owns. *out is null when no pattern
+// is taken. Synchronises.
+int surf_plan_create(const SurfInput &in, SurfPlan **out);
 // Whether the plan takes pattern p.
 bool surf_plan_takes(const SurfPlan *p, int pattern);
 // Writes the outputs of the patterns it takes.

@@ -324,3 +324,88 @@ def test_adjoint_by_nodes_vs_f64(gpu, n, natoms, radius, with_b, want_b, listing
     assert e < 2e-6
     if want_b:
         assert rel_l2(gb.cpu().numpy()[rows], rb) < 2e-6
+
+
+def _nfft_both(gpu, q, Z, pos, b, rots, ff):
+    """Orientations through the NUFFT entry point on a square list, and on the
+    same list with one vector more, which only the grids take."""
+    import torch
+
+    atoms = dv.DeviceAtoms(dv.pack_atoms(Z, pos, atom_b=b), gpu)
+    longer = np.concatenate([q, q[-1:]])
+    F, I, info = dv.structure_factor_nfft_batch(torch.from_numpy(q).to(gpu), atoms, ff, rots, B=2.0)
+    _, Ig, info_g = dv.structure_factor_nfft_batch(torch.from_numpy(longer).to(gpu), atoms, ff, rots, B=2.0)
+    assert {k: info[k] for k in info if k != "staged"} == {k: info_g[k] for k in info_g if k != "staged"}
+    return F.cpu().numpy(), I.cpu().numpy(), Ig.cpu().numpy()[:, :-1]
+
+
+@pytest.mark.parametrize("with_b", [False, True])
+def test_nfft_orientations_by_the_surface(gpu, with_b):
+    """Orientations of one molecule through the NUFFT's entry point on a square
+    list are interpolated, with the error of direct sums; the grids' sizes are
+    reported all the same."""
+    rng = np.random.default_rng(31)
+    n, natoms = 320, 400
+    Z, pos, b = wl.random_molecule(natoms, 4e-9, rng, atom_b_range=(5.0, 10.0))
+    pos = (pos + np.array([2e-9, 0, -1e-9])).astype(np.float32)
+    b = b if with_b else None
+    q = _list(n, n)
+    rots = wl.uniform_rotations(3, rng)
+    F, I, Ig = _nfft_both(gpu, q, Z, pos, b, rots, dv.form_factor_table(device=gpu))
+    for p in range(3):
+        Fr, Ir = oracle.sf_f64(q, Z, pos, atom_b=b, B=2.0, R=rots[p], threads=oracle_threads())
+        assert rel_l2(I[p], Ir) < TOL, p
+        assert np.linalg.norm(F[p, :, 0] + 1j * F[p, :, 1] - Fr) / np.linalg.norm(Fr) < TOL, p
+        assert 1e-7 < rel_l2(Ig[p], I[p]) < 2e-5
+
+
+@pytest.mark.parametrize("what", ["scaled B", "rough", "small"])
+def test_nfft_orientations_that_keep_the_grids(gpu, what):
+    """Scaled matrices with per-atom B (whose factors the grids take at R q),
+    rough lists and few terms: the grids' values."""
+    rng = np.random.default_rng(32)
+    n, natoms = (64, 300) if what == "small" else (320, 400)
+    Z, pos, b = wl.random_molecule(natoms, 4e-9, rng, atom_b_range=(5.0, 10.0))
+    q = _list(n, n)
+    rots = wl.uniform_rotations(2, rng)
+    if what == "scaled B":
+        rots = 0.9 * rots
+    if what == "rough":
+        q = (q * (1.0 - 1e-4 * rng.uniform(size=q.shape))).astype(np.float32)
+    _, I, Ig = _nfft_both(gpu, q, Z, pos, b if what == "scaled B" else None, rots, dv.form_factor_table(device=gpu))
+    assert rel_l2(I, Ig) < 1e-7
+
+
+@pytest.mark.parametrize("with_b,rotated", [(False, True), (True, False)])
+def test_nfft_molecules_split_between_surface_and_grids(gpu, with_b, rotated):
+    """Molecules in one call: two that are interpolated, one too wide for it (the
+    grids) and an empty one; twice, the second time in a workspace that holds
+    everything."""
+    import torch
+
+    rng = np.random.default_rng(33)
+    n = 256
+    q = _list(n, n)
+    mols = []
+    for natoms, radius in ((900, 3e-9), (200, 2.5e-7), (0, 0.0), (1500, 5e-9)):
+        mols.append(wl.random_molecule(natoms, radius, rng, atom_b_range=(5.0, 10.0)) if natoms else
+                    (np.zeros(0, np.int32), np.zeros((0, 3), np.float32), np.zeros(0, np.float32)))
+    rots = wl.uniform_rotations(len(mols), rng) if rotated else None
+    dm = dv.DeviceMolecules([dv.pack_atoms(Z, pos, atom_b=b if with_b else None) for Z, pos, b in mols], gpu)
+    ff = dv.form_factor_table(device=gpu)
+    qs = torch.from_numpy(q).to(gpu)
+    out = []
+    for _ in range(2):
+        F, I = dv.structure_factor_nfft_molecules(qs, dm, ff, rots, B=1.0)
+        torch.cuda.synchronize()
+        out.append(I.cpu().numpy())
+    assert np.array_equal(out[0], out[1])
+    for m, (Z, pos, b) in enumerate(mols):
+        if not len(Z):
+            assert not out[0][m].any()
+            continue
+        _, Ir = oracle.sf_f64(q, Z, pos, atom_b=b if with_b else None, B=1.0, R=rots[m] if rotated else None,
+                              threads=oracle_threads())
+        e = rel_l2(out[0][m], Ir)
+        print(f"molecule {m}: {e:.2e}", flush=True)
+        assert TOL < e < 2e-5 if m == 1 else e < TOL, m
