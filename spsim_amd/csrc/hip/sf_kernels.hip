@@ -954,7 +954,7 @@ int launch_smooth(Kind kind, const PatternLaunch &a, int nx, int ny, const spsim
                   long long min_terms, const Spectrum *spec, hipStream_t s) {
   if (!surf_worth(nx, ny, a.natoms, min_terms)) return launch_single(kind, a, nx, ny, t, splits, s, spec);
   constexpr size_t kFlag = (sizeof(SurfJob) + 255) / 256 * 256;
-  const size_t bytes = std::max(surf_single_bytes(nx, ny, a.natoms), kFlag + sizeof(double2) * (size_t)splits * a.npix);
+  const size_t bytes = std::max(surf_single_bytes(nx, ny, a.natoms, a.nsegs), kFlag + sizeof(double2) * (size_t)splits * a.npix);
   if (!workspace_holds(bytes)) {
     // A capture cannot grow the workspace: it takes the direct kernel, as long as that one's partials fit.
     hipStreamCaptureStatus st = hipStreamCaptureStatusNone;

@@ -21,7 +21,8 @@
 //     exp(i theta u) fall off like Bessel functions beyond theta:
 //     n = theta + 4 theta^(1/3) + 8 leaves 1e-9..1e-8 of |F| (measured against
 //     FP64 sums), a tenth of the FP32 sums' own error.
-//  3. Node sums. F and its derivative N = n.dF/dq at the nodes, by the arithmetic
+//  3. Node sums. F and its derivative N = n.dF/dq at the nodes, of large molecules
+//     by cells (below), by the arithmetic
 //     of the direct kernels (FP64 phase reduced to turns, FP32 sine and
 //     cosine, FP32 sums over 64 atoms folded into FP64). On a square detector
 //     centred on the beam the nodes come in octants, as its pixels do in the
@@ -304,7 +305,7 @@ __device__ void scan_list(const ScanArgs &a) {
     // m U_{m-1} at the points, then dq/du of every row of coefficients, then the points'
     const bool along_y = (int)blockIdx.x == rows + 1;
     __shared__ double T[D][kLines], U[D][kLines], R[D][kLines][3];
-    __shared__ unsigned smax[kLines];
+    __shared__ unsigned smax[4][kLines];
     if (t < kLines) {
       const double u = cospi((double)t / (kLines - 1));
       double t0 = 1.0, t1 = u, u0 = 0.0, u1 = 1.0;
@@ -317,7 +318,7 @@ __device__ void scan_list(const ScanArgs &a) {
         u0 = u1;
         u1 = un;
       }
-      smax[t] = 0u;
+      for (int k = 0; k < 4; ++k) smax[k][t] = 0u;
     }
     __syncthreads();
     for (int c = t; c < D * kLines; c += kT) {
@@ -336,10 +337,15 @@ __device__ void scan_list(const ScanArgs &a) {
       for (int n = 0; n < D; ++n)
         for (int k = 0; k < 3; ++k) d[k] = __builtin_fma(T[n][across], R[n][line][k], d[k]);
       // non-negative floats order as their bits
-      atomicMax(&smax[line], __float_as_uint((float)sqrt(d[0] * d[0] + d[1] * d[1] + d[2] * d[2])));
+      atomicMax(&smax[3][line], __float_as_uint((float)sqrt(d[0] * d[0] + d[1] * d[1] + d[2] * d[2])));
+      for (int k = 0; k < 3; ++k) atomicMax(&smax[k][line], __float_as_uint((float)fabs(d[k])));
     }
     __syncthreads();
-    if (t < kLines) (along_y ? a.fit->slope_y : a.fit->slope_x)[t] = __uint_as_float(smax[t]);
+    if (t < kLines) {
+      SurfSlopes &out = along_y ? a.fit->slope_y : a.fit->slope_x;
+      out.all[t] = __uint_as_float(smax[3][t]);
+      for (int k = 0; k < 3; ++k) out.part[k][t] = __uint_as_float(smax[k][t]);
+    }
     if (t == 0) a.records[blockIdx.x] = SurfRecord{0.0, 0.0, 0.0f, 0.0f, 0, 0};
     if (!along_y) {
       if (t == 0) {
@@ -433,11 +439,12 @@ __global__ __launch_bounds__(kT, 3) void surface_scan_kernel(ScanArgs a) {
 
 // ---- 2. nodes -------------------------------------------------------------------
 
-// The stretch parameter of n nodes, and the nodes that phases of the given
-// slopes need at that stretch. 2 % are added to the slopes for their sampling.
+// The stretch parameter of n nodes, and the nodes that atoms within `radius` and
+// within a box of half edges h need at that stretch. 2 % are added to the slopes
+// for their sampling.
 __host__ __device__ inline float axis_stretch(int n) { return 1.0f / coshf(kStretch / n); }
 
-__host__ __device__ inline float axis_need(const float *slope, float radius, float gauss, float a) {
+__host__ __device__ inline float axis_need(const SurfSlopes &slope, float radius, const float *h, float gauss, float a) {
   const float as = asinf(a);
   float w = 0.0f;
   for (int k = 0; k < kLines; ++k) {
@@ -453,9 +460,10 @@ __host__ __device__ inline float axis_need(const float *slope, float radius, flo
     const float sx = std::sin(x), cx = std::cos(x);
     const float g = std::sqrt(std::max(0.0f, a * a - sx * sx)) / std::max(cx, 1e-6f);
 #endif
-    w = fmaxf(w, slope[k] * g);
+    const float box = slope.part[0][k] * h[0] + slope.part[1][k] * h[1] + slope.part[2][k] * h[2];
+    w = fmaxf(w, fminf(slope.all[k] * radius, box) * g);
   }
-  const float theta = 1.02f * 2.0f * (float)kPi * radius * w / as;
+  const float theta = 1.02f * 2.0f * (float)kPi * w / as;
   return theta + 4.0f * cbrtf(theta) + 8.0f + 2.0f * sqrtf(fmaxf(gauss, 0.0f));
 }
 
@@ -505,8 +513,14 @@ struct __align__(16) NodeAtom {
 };
 static_assert(sizeof(NodeAtom) == 48, "node-sum atom record");
 
+// Cell index along an axis of g cells over [-extent, extent].
+__device__ __forceinline__ int cell_index(double x, double extent, int g) {
+  return min(g - 1, max(0, (int)((x / extent + 1.0) * 0.5 * g)));
+}
+
 __device__ __forceinline__ void prepare_atoms(const SurfJob &jb, bool has_b, int first, int step) {
   NodeAtom *out = (NodeAtom *)jb.prep;
+  const SurfCells &c = jb.c;
   for (int j = first; j < jb.natoms; j += step) {
     const spsim_hip_atom at = jb.atoms[j];
     const double x = at.x - jb.r0[0], y = at.y - jb.r0[1], z = at.z - jb.r0[2];
@@ -527,6 +541,9 @@ __device__ __forceinline__ void prepare_atoms(const SurfJob &jb, bool has_b, int
     r.b = has_b ? jb.atom_b[j] : 0.0f;
     r.pad = 0.0f;
     out[j] = r;
+    if (c.g > 0)
+      c.id[j] = (unsigned short)((cell_index(r.z, c.extent, c.gz) * c.g + cell_index(r.y, c.extent, c.g)) * c.g +
+                                 cell_index(r.x, c.extent, c.g));
   }
 }
 
@@ -565,10 +582,10 @@ __device__ __forceinline__ void octant_node(int t, int &x, int &y) {
   y = yy;
   x = t - yy * (yy + 1) / 2;
 }
-__device__ __forceinline__ int node_index(const SurfJob &jb, int tile, int e, int lane) {
-  const int nyn = jb.sh.ay.n;
-  if (jb.per_lane == 8) {
-    const int t = tile * kT + lane;
+template <int T = kT>  // lanes per tile
+__device__ __forceinline__ int node_index(int per_lane, int nxn, int nyn, int tile, int e, int lane) {
+  if (per_lane == 8) {
+    const int t = tile * T + lane;
     if (t >= node_octants(nyn)) return -1;
     int x, y;
     octant_node(t, x, y);
@@ -577,8 +594,11 @@ __device__ __forceinline__ int node_index(const SurfJob &jb, int tile, int e, in
     const int i = e < 4 ? x : y, k = e < 4 ? y : x;  // mirrored in x for odd e, in y for e & 2
     return ((e & 1) ? m - i : i) * nyn + ((e & 2) ? m - k : k);
   }
-  const int node = tile * jb.per_lane * kT + e * kT + lane;
-  return node < jb.sh.ax.n * nyn ? node : -1;
+  const int node = tile * per_lane * T + e * T + lane;
+  return node < nxn * nyn ? node : -1;
+}
+__device__ __forceinline__ int node_index(const SurfJob &jb, int tile, int e, int lane) {
+  return node_index(jb.per_lane, jb.sh.ax.n, jb.sh.ay.n, tile, e, lane);
 }
 
 // Time of the node sums in atoms per lane with s atom ranges per tile: rounds
@@ -602,6 +622,8 @@ struct PlanArgs {
   int slots;       // resident workgroups of the node sums
   int slot_cap;    // partial slots that fit
   int max_nx, max_ny;  // nodes that fit the workspace
+  int max_cells;       // 0: no sums by cells
+  long long max_cell_sums, max_cell_rows;
   SurfKind kind;
   double scale, spread;  // of a spectrum: largest s_k, largest |s_k / sc - 1|
   SurfJob *out;
@@ -625,14 +647,15 @@ __device__ __forceinline__ void prepare_pixels(const PlanArgs &a, const SurfJob 
 }
 
 // Interpolation weights of one axis, and in FP32 with their derivatives in u
-// (node-major [n][npix]), one wave per pixel: barycentric formula in s = cos t, whose
+// (DERIV; node-major [n][npix]), one wave per pixel x at u: barycentric formula in s = cos t, whose
 // weights at the Chebyshev points are (-1)^i sin t_i. With r_i = w_i / (s - s_i):
 // l_i = r_i / sum r, dl_i/ds = l_i (sum r_j / (s - s_j) / sum r - 1 / (s - s_i)).
-__device__ __forceinline__ void weight_column(const SurfAxis &ax, int x, int npix, const double *sn, const double *wn,
-                                              double *__restrict__ out, float2 *__restrict__ out32) {
+template <bool DERIV = true>
+__device__ __forceinline__ void weight_column(const SurfAxis &ax, double u, int x, int npix, const double *sn,
+                                              const double *wn, double *__restrict__ out, float2 *__restrict__ out32) {
   const int lane = threadIdx.x & 63;
   double sx, cx;
-  sincospi(pixel_u(x, npix) * (ax.asin_a / kPi), &sx, &cx);
+  sincospi(u * (ax.asin_a / kPi), &sx, &cx);
   const double s = sx / ax.a, ds = ax.asin_a * cx / ax.a;
   double sum = 0.0, sum2 = 0.0;
   int hit = -1;
@@ -658,62 +681,128 @@ __device__ __forceinline__ void weight_column(const SurfAxis &ax, int x, int npi
     const size_t o = (size_t)i * npix + x;
     if (hit >= 0) {
       out[o] = i == hit ? 1.0 : 0.0;
-      out32[o] = make_float2(i == hit ? 1.0f : 0.0f, (float)(ds * (i == hit ? -sum / wn[hit] : r / wn[hit])));
+      if constexpr (DERIV)
+        out32[o] = make_float2(i == hit ? 1.0f : 0.0f, (float)(ds * (i == hit ? -sum / wn[hit] : r / wn[hit])));
     } else {
       const double l = r / sum;
       out[o] = l;
-      out32[o] = make_float2((float)l, (float)(ds * l * (sum2 / sum - 1.0 / d)));
+      if constexpr (DERIV)
+        out32[o] = make_float2((float)l, (float)(ds * l * (sum2 / sum - 1.0 / d)));
+    }
+  }
+}
+
+__device__ __forceinline__ double node_u(const SurfAxis &ax, int i) {
+  return asin(ax.a * cospi((2 * i + 1) / (2.0 * ax.n))) / ax.asin_a;
+}
+
+// LDS arrays of build().
+struct BuildLds {
+  double snx[kSurfMaxNodes], wnx[kSurfMaxNodes], sny[kSurfMaxNodes], wny[kSurfMaxNodes];
+  double coef[D][D][3], row[D][3];
+};
+
+// Barycentric nodes and weights of an axis.
+__device__ __forceinline__ void axis_tables(const SurfAxis &ax, double *sn, double *wn) {
+  for (int i = threadIdx.x; i < ax.n; i += kT) {
+    const double ph = (2 * i + 1) / (2.0 * ax.n);
+    sn[i] = cospi(ph);
+    wn[i] = (i & 1) ? -sinpi(ph) : sinpi(ph);
+  }
+}
+
+// q at the nodes ax x ay, node (i, k) -> index i ay.n + k: a row of 16 nodes is
+// contiguous for the first product.
+__device__ void build_nodes(const SurfFit *fit, const SurfAxis &ax, const SurfAxis &ay, double *out, BuildLds &l) {
+  const int t = threadIdx.x;
+  for (int i = t; i < D * D * 3; i += kT) (&l.coef[0][0][0])[i] = (&fit->coef[0][0][0])[i];
+  for (int i = t; i < ax.n; i += kT) l.snx[i] = node_u(ax, i);
+  for (int i = t; i < ay.n; i += kT) l.sny[i] = node_u(ay, i);
+  for (int k = blockIdx.x; k < ay.n; k += gridDim.x) {
+    __syncthreads();
+    surface_row(l.coef, l.sny[k], l.row);
+    __syncthreads();
+    for (int i = t; i < ax.n; i += kT) {
+      double q[3];
+      clenshaw3(l.row, l.snx[i], q);
+      double *o = out + 3 * ((size_t)i * ay.n + k);
+      o[0] = q[0];
+      o[1] = q[1];
+      o[2] = q[2];
     }
   }
 }
 
 // Part 0: the weights of both axes, part 1: the node q of a shape, spread over
-// gridDim.x workgroups. Called by every thread; sn* and wn* are LDS arrays of
-// kSurfMaxNodes.
-__device__ void build(int part, const SurfFit *fit, const SurfShape &sh, int nx, int ny, double *snx, double *wnx,
-                      double *sny, double *wny) {
-  __shared__ double coef[D][D][3], row[D][3];
-  const int t = threadIdx.x;
-  if (part == 0) {
-    for (int i = t; i < sh.ax.n; i += kT) {
-      const double ph = (2 * i + 1) / (2.0 * sh.ax.n);
-      snx[i] = cospi(ph);
-      wnx[i] = (i & 1) ? -sinpi(ph) : sinpi(ph);
-    }
-    for (int i = t; i < sh.ay.n; i += kT) {
-      const double ph = (2 * i + 1) / (2.0 * sh.ay.n);
-      sny[i] = cospi(ph);
-      wny[i] = (i & 1) ? -sinpi(ph) : sinpi(ph);
-    }
-    __syncthreads();
-    const int waves = kT / 64, wave = t / 64;
-    for (int r = (int)blockIdx.x * waves + wave; r < nx + ny; r += (int)gridDim.x * waves) {
-      if (r < nx)
-        weight_column(sh.ax, r, nx, snx, wnx, sh.tx, sh.tx32);
-      else
-        weight_column(sh.ay, r - nx, ny, sny, wny, sh.ty, sh.ty32);
-    }
-  } else if (part == 1) {
-    for (int i = t; i < D * D * 3; i += kT) (&coef[0][0][0])[i] = (&fit->coef[0][0][0])[i];
-    for (int i = t; i < sh.ax.n; i += kT)
-      snx[i] = asin(sh.ax.a * cospi((2 * i + 1) / (2.0 * sh.ax.n))) / sh.ax.asin_a;
-    for (int i = t; i < sh.ay.n; i += kT)
-      sny[i] = asin(sh.ay.a * cospi((2 * i + 1) / (2.0 * sh.ay.n))) / sh.ay.asin_a;
-    // node (i, k) -> index i ay.n + k: a row of 16 nodes is contiguous for the first product
-    for (int k = blockIdx.x; k < sh.ay.n; k += gridDim.x) {
-      __syncthreads();
-      surface_row(coef, sny[k], row);
-      __syncthreads();
-      for (int i = t; i < sh.ax.n; i += kT) {
-        double q[3];
-        clenshaw3(row, snx[i], q);
-        double *o = sh.nodes + 3 * ((size_t)i * sh.ay.n + k);
-        o[0] = q[0];
-        o[1] = q[1];
-        o[2] = q[2];
-      }
-    }
+// gridDim.x workgroups. Called by every thread.
+__device__ void build(int part, const SurfFit *fit, const SurfShape &sh, int nx, int ny, BuildLds &l) {
+  if (part == 1) build_nodes(fit, sh.ax, sh.ay, sh.nodes, l);
+  if (part != 0) return;
+  axis_tables(sh.ax, l.snx, l.wnx);
+  axis_tables(sh.ay, l.sny, l.wny);
+  __syncthreads();
+  const int waves = kT / 64, wave = threadIdx.x / 64;
+  for (int r = (int)blockIdx.x * waves + wave; r < nx + ny; r += (int)gridDim.x * waves) {
+    if (r < nx)
+      weight_column(sh.ax, pixel_u(r, nx), r, nx, l.snx, l.wnx, sh.tx, sh.tx32);
+    else
+      weight_column(sh.ay, pixel_u(r - nx, ny), r - nx, ny, l.sny, l.wny, sh.ty, sh.ty32);
   }
+}
+
+// The same for the coarse nodes of a molecule's cells, onto the pattern's nodes.
+__device__ void build_coarse(int part, const SurfFit *fit, const SurfCoarse &co, BuildLds &l) {
+  if (part == 1) build_nodes(fit, co.ax, co.ay, co.nodes, l);
+  if (part != 0) return;
+  axis_tables(co.ax, l.snx, l.wnx);
+  axis_tables(co.ay, l.sny, l.wny);
+  __syncthreads();
+  const int waves = kT / 64, wave = threadIdx.x / 64, nx = co.fx.n, ny = co.fy.n;
+  for (int r = (int)blockIdx.x * waves + wave; r < nx + ny; r += (int)gridDim.x * waves) {
+    if (r < nx)
+      weight_column<false>(co.ax, node_u(co.fx, r), r, nx, l.snx, l.wnx, co.wx, nullptr);
+    else
+      weight_column<false>(co.ay, node_u(co.fy, r - nx), r - nx, ny, l.sny, l.wny, co.wy, nullptr);
+  }
+}
+
+// Box grids that are tried: cells across the beam and along it.
+constexpr int kCellGrids = 4, kMaxCells = 512;
+// Most atoms per work item of a cell's sums: at most 512 ranges besides one
+// of every cell.
+__host__ __device__ inline int cell_range(int natoms) { return 256 * (natoms / (256 * 512) + 1); }
+__host__ __device__ inline void cell_grid(int k, int *g, int *gz) {
+  *g = k == 0 ? 4 : (k == 1 ? 6 : 8);
+  *gz = k == 0 ? 2 : (k == 1 ? 3 : (k == 2 ? 4 : 8));
+}
+constexpr int kCellMinNodes = 16, kCellMaxNodes = 128;  // of a cell's sums, per axis
+
+// The same for the nodes of a cell, in tiles of 64 lanes.
+__host__ __device__ inline void cell_tiling(int nx, int ny, bool octants, int *per_lane, int *tiles) {
+  const int nodes = nx * ny, t2 = (nodes + 127) / 128, t4 = (nodes + 255) / 256, t8 = (node_octants(nx) + 63) / 64;
+  *per_lane = t4 * 228 <= t2 * 120 ? 4 : 2;
+  *tiles = *per_lane == 4 ? t4 : t2;
+  if (octants && t8 * 321 < *tiles * (*per_lane == 4 ? 228 : 120)) {
+    *per_lane = 8;
+    *tiles = t8;
+  }
+}
+
+// Issue cycles over all lanes of a pattern's node sums (nx x ny nodes), and of
+// the same by cells with mx x my nodes each: the sums, the two products
+// (290 cycles per 16 x 16 x 4 block, an FP64 sine and cosine per node and cell)
+// and the products' memory (about 33 cycles a byte).
+__host__ __device__ inline double sums_cost(int nx, int ny, bool octants, double natoms, int *per_lane, int *tiles) {
+  node_tiling(nx, ny, octants, 1LL << 25, per_lane, tiles);
+  return (double)*tiles * kT * (*per_lane == 8 ? 321.0 : 57.0 * *per_lane) * natoms;
+}
+__host__ __device__ inline double cells_cost(int nx, int ny, int mx, int my, int ncells, bool octants, double natoms) {
+  int per_lane, tiles;
+  cell_tiling(mx, my, octants, &per_lane, &tiles);
+  const double sums = tiles * 64.0 * (per_lane == 8 ? 321.0 : 57.0 * per_lane) * natoms;
+  auto up = [](int n) { return (n + 15) / 16; };
+  const double rows = 290.0 * up(nx) * up(my) * (mx / 4), cols = up(nx) * up(ny) * (290.0 * (my / 4) + 2000.0);
+  return 1.2 * sums + 0.6 * ncells * (64.0 * (rows + cols) + 33.0 * 48.0 * my * nx);
 }
 
 // What the scan found about a molecule on its list, in *out (thread 0).
@@ -734,14 +823,17 @@ __device__ void fold_records(const SurfRecord *list, int nlist, const SurfRecord
   block_reduce(m);
   // every form-factor row that is used, one thread each
   float bs = 0.0f, weak = 1.0f;
+  double e[3] = {0.0, 0.0, 0.0};  // Gaussian, -weakest, out of order
   for (int i = t; i < nsegs; i += kT) {
+    if (segs[i].count < 0 || (i > 0 && segs[i].start < segs[i - 1].start + segs[i - 1].count)) e[2] = 1.0;
     const int sp = segs[i].species;
     species_terms(ff + sp * SPSIM_HIP_FF_STRIDE, sp == SPSIM_HIP_UNIT_SPECIES ? 0.0f : b_global,
                   has_b ? (float)-m[2] : 0.0f, has_b ? (float)m[3] : 0.0f, s2max, &bs, &weak);
   }
-  double e[2] = {(double)bs, -(double)weak};
+  e[0] = bs;
+  e[1] = -(double)weak;
   block_reduce(e);
-  if (t == 0) *out = SurfMol{sqrt(m[1]), m[0], (float)e[0], (float)-e[1], m[4] > 0.0};
+  if (t == 0) *out = SurfMol{sqrt(m[1]), m[0], (float)e[0], (float)-e[1], m[4] > 0.0, e[2] == 0.0};
 }
 
 // One workgroup per molecule.
@@ -771,9 +863,9 @@ __global__ __launch_bounds__(kT) void surface_digest_kernel(DigestArgs a) {
     a.out[m] = d;
   }
   if (m > 0) return;
-  if (t < kLines) {
-    a.head->slope_x[t] = a.fit->slope_x[t];
-    a.head->slope_y[t] = a.fit->slope_y[t];
+  for (int i = t; i < (int)(sizeof(SurfSlopes) / sizeof(float)); i += kT) {
+    ((float *)&a.head->slope_x)[i] = ((const float *)&a.fit->slope_x)[i];
+    ((float *)&a.head->slope_y)[i] = ((const float *)&a.fit->slope_y)[i];
   }
   if (t == 0) {
     a.head->s2max = a.fit->s2max;
@@ -782,10 +874,50 @@ __global__ __launch_bounds__(kT) void surface_digest_kernel(DigestArgs a) {
   }
 }
 
+// Partial sums over the cells, for about 1024 workgroups of the second product.
+__host__ __device__ inline int cell_splits(int nx, int ny, int count, long long slot_cap) {
+  const int wgs = ((nx + 31) / 32) * ((ny + 31) / 32) * count;
+  int s = 1024 / wgs;
+  const long long nodes = ((long long)nx * ny + kT - 1) / kT * kT;
+  s = s < 1 ? 1 : (s > 32 ? 32 : s);
+  while (s > 1 && nodes * s > slot_cap) --s;
+  return s;
+}
+
+// *out = *in by the workgroup (one lane would take a struct through scratch).
+template <class T>
+__device__ __forceinline__ void copy_words(T *out, const T *in) {
+  static_assert(sizeof(T) % 4 == 0, "whole words");
+  for (int i = threadIdx.x; i < (int)(sizeof(T) / 4); i += kT) ((unsigned *)out)[i] = ((const unsigned *)in)[i];
+}
+
+// The grid of boxes that costs least, or -1 when the plain sums do. max_*: what
+// the workspace holds.
+__device__ int choose_cells(const PlanArgs &a, int nx, int ny, bool octants, const int (*n)[2]) {
+  __shared__ float cost[kCellGrids + 1];
+  const int k = threadIdx.x;
+  int per_lane, tiles;
+  if (k < kCellGrids) {  // one grid per lane
+    int g, gz;
+    cell_grid(k, &g, &gz);
+    const int mx = n[k][0], my = n[k][1], ncells = g * g * gz;
+    const bool fits = mx <= kCellMaxNodes && my <= kCellMaxNodes && ncells <= a.max_cells &&
+                      (long long)(a.job.natoms / cell_range(a.job.natoms) + ncells) * mx * my <= a.max_cell_sums &&
+                      (long long)ncells * my * nx <= a.max_cell_rows;
+    cost[k] = fits ? (float)cells_cost(nx, ny, mx, my, ncells, octants && mx == my, a.job.natoms) : 3e38f;
+  } else if (k == kCellGrids) {
+    cost[k] = (float)(0.7 * sums_cost(nx, ny, octants, a.job.natoms, &per_lane, &tiles) - 4e9);
+  }
+  __syncthreads();
+  int best = kCellGrids;
+  for (int i = 0; i < kCellGrids; ++i) best = cost[i] < cost[best] ? i : best;
+  return best < kCellGrids ? best : -1;
+}
+
 __global__ __launch_bounds__(kT) void surface_plan_kernel(PlanArgs a) {
-  __shared__ double snx[kSurfMaxNodes], wnx[kSurfMaxNodes], sny[kSurfMaxNodes], wny[kSurfMaxNodes];
+  __shared__ BuildLds lds;
   __shared__ SurfMol mol;
-  __shared__ int best[2], split[1];
+  __shared__ int best[2], split[1], cell_best[kCellGrids][2];
   __shared__ SurfJob job;
   const int t = threadIdx.x;
   fold_records(a.records, a.list_blocks, a.records + a.list_blocks, a.job.segs, a.job.nsegs, a.ff, a.b_global, a.has_b,
@@ -793,15 +925,27 @@ __global__ __launch_bounds__(kT) void surface_plan_kernel(PlanArgs a) {
   if (t == 0) {
     mol.radius *= a.scale;
     best[0] = best[1] = 1 << 30;
+    for (int k = 0; k < kCellGrids; ++k) cell_best[k][0] = cell_best[k][1] = 1 << 30;
   }
   __syncthreads();
   {  // smallest sufficient node count of each axis, one candidate per thread
     const int axis = t / 128, n = kSurfMinNodes + 4 * (t % 128);
-    const float *slope = axis ? a.fit->slope_y : a.fit->slope_x;
-    if (n <= kSurfMaxNodes &&
-        axis_need(slope, (float)mol.radius, mol.b_smooth * a.fit->s2max, axis_stretch(n)) <= (float)n)
+    const SurfSlopes &slope = axis ? a.fit->slope_y : a.fit->slope_x;
+    const float r = (float)mol.radius, h[3] = {r, r, r};
+    if (n <= kSurfMaxNodes && axis_need(slope, r, h, mol.b_smooth * a.fit->s2max, axis_stretch(n)) <= (float)n)
       atomicMin(&best[axis], n);
   }
+  if (a.max_cells > 0)  // and of the cells of every grid of boxes
+    for (int i = t; i < kCellGrids * 2 * 32; i += kT) {
+      const int k = i / 64, axis = i / 32 % 2, n = kCellMinNodes + 4 * (i % 32);
+      int g, gz;
+      cell_grid(k, &g, &gz);
+      const SurfSlopes &slope = axis ? a.fit->slope_y : a.fit->slope_x;
+      const float r = (float)mol.radius, h[3] = {r / g, r / g, r / gz};
+      if (n <= kCellMaxNodes && axis_need(slope, sqrtf(h[0] * h[0] + h[1] * h[1] + h[2] * h[2]), h,
+                                          mol.b_smooth * a.fit->s2max, axis_stretch(n)) <= (float)n)
+        atomicMin(&cell_best[k][axis], n);
+    }
   __syncthreads();
   const int nx = best[0], ny = best[1];
   // N is taken at the spectrum's centre scale, so it is off by the spread
@@ -812,8 +956,16 @@ __global__ __launch_bounds__(kT) void surface_plan_kernel(PlanArgs a) {
     if (blockIdx.x == 0 && blockIdx.y == 0 && t == 0) a.out->ok = 0;
     return;
   }
-  int per_lane, tiles;
-  node_tiling(nx, ny, a.fit->sym == 2 && nx == ny && a.kind == SurfKind::kSum, a.job.natoms, &per_lane, &tiles);
+  int per_lane, tiles, grid = -1;
+  const bool octants = a.fit->sym == 2 && nx == ny && a.kind == SurfKind::kSum;
+  if (a.max_cells > 0 && mol.ordered) grid = choose_cells(a, nx, ny, octants, cell_best);
+  node_tiling(nx, ny, octants, a.job.natoms, &per_lane, &tiles);
+  copy_words(&job, &a.job);
+  __syncthreads();
+  if (grid >= 0) {  // F and N come as partial sums over cells, node by node
+    per_lane = 1;
+    tiles = (nx * ny + kT - 1) / kT;
+  }
   const int tile = per_lane * kT;
   if (t < 64) {  // the cheapest number of atom ranges, two candidates per lane
     float c = 3.0e38f;
@@ -834,9 +986,8 @@ __global__ __launch_bounds__(kT) void surface_plan_kernel(PlanArgs a) {
         n = n2;
       }
     }
-    if (t == 0) split[0] = n;
+    if (t == 0) split[0] = grid >= 0 ? cell_splits(nx, ny, 1, a.slot_cap) : n;
   } else if (t == 64) {
-    job = a.job;
     job.ok = 1;
     job.sh.ax = SurfAxis{nx, axis_stretch(nx), 0.0};
     job.sh.ay = SurfAxis{ny, axis_stretch(ny), 0.0};
@@ -844,18 +995,30 @@ __global__ __launch_bounds__(kT) void surface_plan_kernel(PlanArgs a) {
     job.sh.ay.asin_a = asin(job.sh.ay.a);
     job.per_lane = per_lane;
     job.tiles = tiles;
+    job.c.g = 0;
+    if (grid >= 0) {
+      SurfCells &c = job.c;
+      cell_grid(grid, &c.g, &c.gz);
+      c.extent = mol.radius;
+      c.co.ax = SurfAxis{cell_best[grid][0], axis_stretch(cell_best[grid][0]), 0.0};
+      c.co.ay = SurfAxis{cell_best[grid][1], axis_stretch(cell_best[grid][1]), 0.0};
+      c.co.ax.asin_a = asin(c.co.ax.a);
+      c.co.ay.asin_a = asin(c.co.ay.a);
+      c.co.fx = job.sh.ax;
+      c.co.fy = job.sh.ay;
+      cell_tiling(c.co.ax.n, c.co.ay.n, octants && c.co.ax.n == c.co.ay.n, &c.per_lane, &c.tiles);
+    }
     for (int k = 0; k < 3; ++k) {
       job.r0[k] = a.centres[k];
       job.normal[k] = a.fit->normal[k];
     }
   }
   __syncthreads();
-  if (t == 0) {
-    job.splits = split[0];
-    if (blockIdx.x == 0 && blockIdx.y == 0) *a.out = job;
-  }
+  if (t == 0) job.splits = split[0];
   __syncthreads();
-  build(blockIdx.y, a.fit, job.sh, job.nx, job.ny, snx, wnx, sny, wny);
+  if (blockIdx.x == 0 && blockIdx.y == 0) copy_words(a.out, &job);
+  build(blockIdx.y, a.fit, job.sh, job.nx, job.ny, lds);
+  if (job.c.g > 0) build_coarse((int)blockIdx.y - 3, a.fit, job.c.co, lds);
   if (blockIdx.y == 2) {
     const int first = (int)(blockIdx.x * kT) + t, step = (int)gridDim.x * kT;
     if (a.kind == SurfKind::kAdjoint)
@@ -866,8 +1029,8 @@ __global__ __launch_bounds__(kT) void surface_plan_kernel(PlanArgs a) {
 }
 
 __global__ __launch_bounds__(kT) void surface_tables_kernel(const SurfFit *fit, const SurfShape *shapes, int nx, int ny) {
-  __shared__ double snx[kSurfMaxNodes], wnx[kSurfMaxNodes], sny[kSurfMaxNodes], wny[kSurfMaxNodes];
-  build(blockIdx.y, fit, shapes[blockIdx.z], nx, ny, snx, wnx, sny, wny);
+  __shared__ BuildLds lds;
+  build(blockIdx.y, fit, shapes[blockIdx.z], nx, ny, lds);
 }
 
 // ---- 3. node sums ---------------------------------------------------------------
@@ -921,23 +1084,38 @@ __device__ __forceinline__ void store_node(const SurfJob &jb, int tile, int spli
   jb.n[node] = make_float2(-2.0f * (float)kPi * ns, -2.0f * (float)kPi * nc);
 }
 
-// Runs body(first, count, f64) over the LDS chunks of a work item's atoms, at
-// most kNodeFold atoms at a time; form(species) is called once per species.
-template <class Form, class Body>
-__device__ __forceinline__ void over_atoms(const SurfJob &jb, int split, NodeAtom *sm, Form form, Body body) {
-  const int a_begin = (int)((long long)jb.natoms * split / jb.splits);
-  const int a_end = (int)((long long)jb.natoms * (split + 1) / jb.splits);
-  const NodeAtom *atoms = (const NodeAtom *)jb.prep;
+// The nodes of a grid and the atoms [a_begin, a_end) of a work item.
+struct NodeWork {
+  const double *nodes;
+  int nxn, nyn, per_lane;
+  const NodeAtom *atoms;
+  const spsim_hip_segment *segs;
+  int nsegs, a_begin, a_end;
+};
+
+// Lanes of a wave see the LDS writes of the others.
+__device__ __forceinline__ void wave_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
+// Runs body(first, count) over the LDS chunks of a work item's atoms, at most
+// kNodeFold atoms at a time; form(species) is called once per species. WAVE: the
+// item is one wave's, with an sm of its own for 64 atoms.
+template <bool WAVE, class Form, class Body>
+__device__ __forceinline__ void over_atoms(const NodeWork &jb, NodeAtom *sm, Form form, Body body) {
   for (int sg = 0; sg < jb.nsegs; ++sg) {
     const spsim_hip_segment seg = jb.segs[sg];
-    const int lo = max(seg.start, a_begin), hi = min(seg.start + seg.count, a_end);
+    const int lo = max(seg.start, jb.a_begin), hi = min(seg.start + seg.count, jb.a_end);
     if (lo >= hi) continue;
     form(seg.species);
-    for (int c0 = lo; c0 < hi; c0 += kNodeChunk) {
-      const int n = min(kNodeChunk, hi - c0);
-      __syncthreads();
-      if ((int)threadIdx.x < n) sm[threadIdx.x] = atoms[c0 + threadIdx.x];
-      __syncthreads();
+    constexpr int kChunk = WAVE ? 64 : kNodeChunk;
+    const int t = WAVE ? threadIdx.x & 63 : threadIdx.x;
+    for (int c0 = lo; c0 < hi; c0 += kChunk) {
+      const int n = min(kChunk, hi - c0);
+      WAVE ? wave_sync() : __syncthreads();
+      if (t < n) sm[t] = jb.atoms[c0 + t];
+      WAVE ? wave_sync() : __syncthreads();
       for (int j0 = 0; j0 < n; j0 += kNodeFold) body(j0, min(n, j0 + kNodeFold));
     }
   }
@@ -945,15 +1123,16 @@ __device__ __forceinline__ void over_atoms(const SurfJob &jb, int split, NodeAto
 
 // K nodes per lane. SPEC: a wavelength spectrum, the sample sum in place of the
 // sine and cosine (spectrum_term), and N at the centre scale.
-template <int K, bool HAS_B, bool SPEC>
-__device__ __forceinline__ void node_item(const SurfJob &jb, int tile, int split, const float *__restrict__ ff,
-                                          float b_global, const typename SpectrumArg<SPEC>::type &sp, NodeAtom *sm) {
+template <int K, bool HAS_B, bool SPEC, bool WAVE, class Store>
+__device__ __forceinline__ void node_item(const NodeWork &jb, int tile, const float *__restrict__ ff, float b_global,
+                                          const typename SpectrumArg<SPEC>::type &sp, NodeAtom *sm, Store store) {
   constexpr int kUnroll = K == 1 ? 4 : (K == 2 ? 2 : 1);
+  const int lane = WAVE ? threadIdx.x & 63 : threadIdx.x;
   double qx[K], qy[K], qz[K], s2[K], f[K], Fc[K], Fs[K];
   float nl2[K], Nc[K], Ns[K];
 #pragma unroll
   for (int k = 0; k < K; ++k) {
-    const double *q = jb.sh.nodes + 3 * (size_t)max(0, node_index(jb, tile, k, threadIdx.x));
+    const double *q = jb.nodes + 3 * (size_t)max(0, node_index<WAVE ? 64 : kT>(K, jb.nxn, jb.nyn, tile, k, lane));
     qx[k] = q[0];
     qy[k] = q[1];
     qz[k] = q[2];
@@ -962,8 +1141,8 @@ __device__ __forceinline__ void node_item(const SurfJob &jb, int tile, int split
     f[k] = Fc[k] = Fs[k] = 0.0;
     Nc[k] = Ns[k] = 0.0f;
   }
-  over_atoms(
-      jb, split, sm,
+  over_atoms<WAVE>(
+      jb, sm,
       [&](int species) {
 #pragma unroll
         for (int k = 0; k < K; ++k)
@@ -1014,7 +1193,7 @@ __device__ __forceinline__ void node_item(const SurfJob &jb, int tile, int split
   for (int k = 0; k < K; ++k) {
     float scale = 1.0f;
     if constexpr (SPEC) scale = (float)sp.sc;
-    store_node(jb, tile, split, k, Fc[k], Fs[k], scale * Nc[k], scale * Ns[k]);
+    store(k, Fc[k], Fs[k], scale * Nc[k], scale * Ns[k]);
   }
 }
 
@@ -1022,10 +1201,11 @@ __device__ __forceinline__ void node_item(const SurfJob &jb, int tile, int split
 // transposed node with a = q_x r_x, b = q_y r_y, c = q_z r_z, and from their sines and
 // cosines the four real sums P, Q per angle, as in octant_sum (sf_kernels.hip),
 // once weighted by w e^{-2 pi i c} (F) and once by n.r times that (N).
-template <bool HAS_B>
-__device__ __forceinline__ void octant_item(const SurfJob &jb, int tile, int split, const float *__restrict__ ff,
-                                            float b_global, NodeAtom *sm) {
-  const double *q = jb.sh.nodes + 3 * (size_t)max(0, node_index(jb, tile, 0, threadIdx.x));
+template <bool HAS_B, bool WAVE, class Store>
+__device__ __forceinline__ void octant_item(const NodeWork &jb, int tile, const float *__restrict__ ff, float b_global,
+                                            NodeAtom *sm, Store store) {
+  const int lane = WAVE ? threadIdx.x & 63 : threadIdx.x;
+  const double *q = jb.nodes + 3 * (size_t)max(0, node_index<WAVE ? 64 : kT>(8, jb.nxn, jb.nyn, tile, 0, lane));
   const double qx = q[0], qy = q[1], qz = q[2];
   const double s2 = (qx * qx + qy * qy + qz * qz) * 2.5e-21;
   const float nl2 = (float)(-s2 * kLog2e);
@@ -1036,8 +1216,8 @@ __device__ __forceinline__ void octant_item(const SurfJob &jb, int tile, int spl
     Fc[i] = Fs[i] = 0.0;
     Nc[i] = Ns[i] = 0.0f;
   }
-  over_atoms(
-      jb, split, sm,
+  over_atoms<WAVE>(
+      jb, sm,
       [&](int species) {
         f = (1.0 + 2.0 * kTrigBias) * form_factor64(ff + species * SPSIM_HIP_FF_STRIDE, s2,
                                                     species == SPSIM_HIP_UNIT_SPECIES ? 0.0f : b_global);
@@ -1100,7 +1280,24 @@ __device__ __forceinline__ void octant_item(const SurfJob &jb, int tile, int spl
         }
       });
 #pragma unroll
-  for (int e = 0; e < 8; ++e) store_node(jb, tile, split, e, Fc[e], Fs[e], Nc[e], Ns[e]);
+  for (int e = 0; e < 8; ++e) store(e, Fc[e], Fs[e], Nc[e], Ns[e]);
+}
+
+template <bool HAS_B, bool SPEC, bool WAVE, class Store>
+__device__ __forceinline__ void any_item(const NodeWork &w, int tile, const float *__restrict__ ff, float b_global,
+                                         const typename SpectrumArg<SPEC>::type &sp, NodeAtom *sm, Store store) {
+  if constexpr (!SPEC) {
+    if (w.per_lane == 8) {
+      octant_item<HAS_B, WAVE>(w, tile, ff, b_global, sm, store);
+      return;
+    }
+  }
+  if (w.per_lane == 4)
+    node_item<4, HAS_B, SPEC, WAVE>(w, tile, ff, b_global, sp, sm, store);
+  else if (w.per_lane == 2)
+    node_item<2, HAS_B, SPEC, WAVE>(w, tile, ff, b_global, sp, sm, store);
+  else
+    node_item<1, HAS_B, SPEC, WAVE>(w, tile, ff, b_global, sp, sm, store);
 }
 
 template <bool HAS_B, bool SPEC>
@@ -1109,24 +1306,226 @@ __global__ __launch_bounds__(kT) void surface_nodes_kernel(const SurfJob *jobs, 
                                                            typename SpectrumArg<SPEC>::type sp) {
   __shared__ NodeAtom sm[kNodeChunk];
   if (!items) {  // one pattern: every (tile, range) of job 0
-    if (!jobs->ok) return;
+    if (!jobs->ok || jobs->c.g > 0) return;
     nitems = jobs->tiles * jobs->splits;
   }
   for (int it = blockIdx.x; it < nitems; it += gridDim.x) {
     const SurfItem m = items ? items[it] : SurfItem{0, it % jobs->tiles, it / jobs->tiles, 0};
     const SurfJob &jb = jobs[m.job];
-    if constexpr (!SPEC) {
-      if (jb.per_lane == 8) {
-        octant_item<HAS_B>(jb, m.tile, m.split, ff, b_global, sm);
-        continue;
+    const NodeWork w{jb.sh.nodes,
+                     jb.sh.ax.n,
+                     jb.sh.ay.n,
+                     jb.per_lane,
+                     (const NodeAtom *)jb.prep,
+                     jb.segs,
+                     jb.nsegs,
+                     (int)((long long)jb.natoms * m.split / jb.splits),
+                     (int)((long long)jb.natoms * (m.split + 1) / jb.splits)};
+    any_item<HAS_B, SPEC, false>(w, m.tile, ff, b_global, sp, sm, [&](int e, double fc, double fs, float nc, float ns) {
+      store_node(jb, m.tile, m.split, e, fc, fs, nc, ns);
+    });
+  }
+}
+
+// ---- 3b. node sums by cells -------------------------------------------------------
+//
+// On many nodes the atoms are summed by cells: g x g x gz boxes, each of whose
+// sums about the box's centre varies 1 / g as fast over the detector and
+// needs that many fewer nodes per axis; its values there are interpolated to the
+// pattern's nodes like the pattern's to the pixels (FP64 products for F, FP32 for
+// N), turned by the centre's phase and added up. Terms fall with the square of
+// the coarse nodes, the interpolation grows with the cells: cells_cost. On
+// 100,000 atoms with B and 188^2 nodes, 108 cells of 64^2 nodes: 33 us for the
+// sort, 161 us for the sums, 73 and 84 us for the products, against 1140 us for
+// the plain sums.
+
+// The records of one cell (blockIdx.x), in their order, which is that of the
+// species: every wave goes over one section of the atoms' cell indexes, 512 at a
+// time, counts its atoms in this cell and in lower ones, and copies its own behind
+// those of the waves before it. The cell's ranges are numbered from
+// start / range length + cell, which leaves each room enough.
+constexpr int kSortT = 1024;
+
+__global__ __launch_bounds__(kSortT) void surface_sort_kernel(const SurfJob *jobs, int first) {
+  const SurfJob &jb = jobs[first + blockIdx.z];
+  const SurfCells &c = jb.c;
+  const int cell = blockIdx.x, t = threadIdx.x, lane = t & 63, wave = t / 64;
+  if (!jb.ok || cell >= c.g * c.g * c.gz) return;
+  constexpr int kWaves = kSortT / 64;
+  __shared__ int counts[kWaves][2], seg_count[SPSIM_HIP_NSPECIES];
+  const int n = jb.natoms, len = cell_range(n);
+  const int section = (n + 512 * kWaves - 1) / (512 * kWaves) * 512;
+  const int lo = min(n, section * wave), hi = min(n, section * (wave + 1));
+  // the 8 indexes from j on: a mask of those in this cell, and the number of lower ones
+  auto look = [&](int j, int *lower) {
+    unsigned in = 0;
+    if (j < hi) {
+      const uint4 v = *(const uint4 *)(c.id + j);  // the buffer ends on a multiple of 8
+      const unsigned w[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+      for (int k = 0; k < 8; ++k) {
+        const int id = (w[k / 2] >> (16 * (k & 1))) & 0xffff;
+        if (j + k < hi) {
+          in |= id == cell ? 1u << k : 0u;
+          *lower += id < cell;
+        }
       }
     }
-    if (jb.per_lane == 4)
-      node_item<4, HAS_B, SPEC>(jb, m.tile, m.split, ff, b_global, sp, sm);
-    else if (jb.per_lane == 2)
-      node_item<2, HAS_B, SPEC>(jb, m.tile, m.split, ff, b_global, sp, sm);
-    else
-      node_item<1, HAS_B, SPEC>(jb, m.tile, m.split, ff, b_global, sp, sm);
+    return in;
+  };
+  int lower = 0, own = 0;
+#pragma unroll 4
+  for (int j = lo; j < hi; j += 512) own += __popc(look(j + 8 * lane, &lower));
+  for (int o = 32; o > 0; o >>= 1) {
+    lower += __shfl_xor(lower, o);
+    own += __shfl_xor(own, o);
+  }
+  if (lane == 0) {
+    counts[wave][0] = lower;
+    counts[wave][1] = own;
+  }
+  if (t < jb.nsegs) seg_count[t] = 0;
+  __syncthreads();
+  int start = 0, total = 0, at = 0;
+  for (int i = 0; i < kWaves; ++i) {
+    start += counts[i][0];
+    at += i < wave ? counts[i][1] : 0;
+    total += counts[i][1];
+  }
+  at += start;
+  for (int j = lo; j < hi && own > 0; j += 512) {
+    unsigned mask = look(j + 8 * lane, &lower);
+    if (__ballot(mask != 0) == 0) continue;
+    int before = __popc(mask);  // of the lanes below: inclusive scan, less its own
+    const int mine = before;
+    for (int o = 1; o < 64; o <<= 1) {
+      const int v = __shfl_up(before, o);
+      before += lane >= o ? v : 0;
+    }
+    int to = at + before - mine;
+    at += __shfl(before, 63);
+    own -= __shfl(before, 63);
+    for (; mask; mask &= mask - 1) c.order[to++] = j + 8 * lane + __ffs(mask) - 1;
+  }
+  const int ix[3] = {cell % c.g, cell / c.g % c.g, cell / (c.g * c.g)};
+  double centre[3];
+#pragma unroll
+  for (int k = 0; k < 3; ++k) centre[k] = c.extent * ((2 * ix[k] + 1) / (double)(k < 2 ? c.g : c.gz) - 1.0);
+  __threadfence_block();
+  __syncthreads();
+  for (int i = start + t; i < start + total; i += kSortT) {
+    const int a = c.order[i];
+    NodeAtom r = ((const NodeAtom *)jb.prep)[a];
+    int sg = 0;
+    while (sg < jb.nsegs - 1 && a >= jb.segs[sg].start + jb.segs[sg].count) ++sg;
+    r.x -= centre[0];
+    r.y -= centre[1];
+    r.z -= centre[2];
+    if (a < jb.segs[sg].start || a >= jb.segs[sg].start + jb.segs[sg].count) {  // of no species: not summed
+      r.w = jb.atom_b ? -INFINITY : 0.0f;
+      r.n = 0.0f;
+    }
+    ((NodeAtom *)c.sorted)[i] = r;
+    atomicAdd(&seg_count[sg], 1);
+  }
+  __syncthreads();
+  if (t == 0) {
+    spsim_hip_segment *segs = c.segs + (size_t)cell * jb.nsegs;
+    int s = start;
+    for (int i = 0; i < jb.nsegs; ++i) {
+      segs[i].start = s;
+      segs[i].count = seg_count[i];
+      segs[i].species = jb.segs[i].species;
+      s += seg_count[i];
+    }
+    SurfCell out_cell;
+#pragma unroll
+    for (int k = 0; k < 3; ++k) out_cell.centre[k] = centre[k];
+    out_cell.start = start;
+    out_cell.count = total;
+    out_cell.range0 = start / len + cell;
+    out_cell.ranges = (total + len - 1) / len;
+    c.cells[cell] = out_cell;
+  }
+  const int r0 = start / len + cell, used = (total + len - 1) / len;
+  const int r1 = (start + total) / len + cell + 1;
+  for (int r = r0 + t; r < r1; r += kSortT) c.range_cell[r] = r < r0 + used ? cell : -1;
+}
+
+// One (range, tile of 64 lanes) per workgroup at a time, of pattern
+// first + blockIdx.y: every wave sums a quarter of the range's atoms, and the first
+// one adds them up. Bound by the issue of the sums (58 % of it; ranges of 1024
+// atoms take 204 us for 161 us, their last ones run alone).
+template <bool HAS_B>
+__global__ __launch_bounds__(kT, 4) void surface_cell_nodes_kernel(const SurfJob *jobs, int first,
+                                                                   const float *__restrict__ ff, float b_global) {
+  constexpr int kWaves = kT / 64;
+  __shared__ union {
+    NodeAtom sm[kWaves][64];
+    struct {
+      double f[kWaves - 1][2][8][64];
+      float n[kWaves - 1][2][8][64];
+    } part;
+  } lds;
+  const SurfJob &jb = jobs[first + blockIdx.y];
+  const SurfCells &c = jb.c;
+  if (!jb.ok || c.g == 0) return;
+  const int len = cell_range(jb.natoms), items = (jb.natoms / len + c.g * c.g * c.gz) * c.tiles;
+  for (int it = blockIdx.x; it < items; it += gridDim.x) {
+    const int range = it / c.tiles, tile = it % c.tiles, id = c.range_cell[range];
+    if (id < 0) continue;
+    const SurfCell cell = c.cells[id];
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64), lane = threadIdx.x & 63;
+    const int r = range - cell.range0;
+    const int begin = cell.start + cell.count * r / cell.ranges;
+    const int count = cell.start + cell.count * (r + 1) / cell.ranges - begin;
+    const int nxn = c.co.ax.n, nyn = c.co.ay.n;
+    const NodeWork w{c.co.nodes,
+                     nxn,
+                     nyn,
+                     c.per_lane,
+                     (const NodeAtom *)c.sorted,
+                     c.segs + (size_t)id * jb.nsegs,
+                     jb.nsegs,
+                     begin + count * wave / kWaves,
+                     begin + count * (wave + 1) / kWaves};
+    NoSpectrum none;
+    double fc[8] = {}, fs[8] = {};
+    float nc[8] = {}, ns[8] = {};
+    any_item<HAS_B, false, true>(w, tile, ff, b_global, none, lds.sm[wave],
+                                 [&](int e, double c0, double s0, float c1, float s1) {
+                                   fc[e] = c0;
+                                   fs[e] = s0;
+                                   nc[e] = c1;
+                                   ns[e] = s1;
+                                 });
+    __syncthreads();
+    if (wave > 0)
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        lds.part.f[wave - 1][0][e][lane] = fc[e];
+        lds.part.f[wave - 1][1][e][lane] = fs[e];
+        lds.part.n[wave - 1][0][e][lane] = nc[e];
+        lds.part.n[wave - 1][1][e][lane] = ns[e];
+      }
+    __syncthreads();
+    double2 *f = c.f + (size_t)range * nxn * nyn;
+    float2 *n = c.n + (size_t)range * nxn * nyn;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      if (wave > 0 || e >= c.per_lane) break;
+      for (int k = 0; k < kWaves - 1; ++k) {
+        fc[e] += lds.part.f[k][0][e][lane];
+        fs[e] += lds.part.f[k][1][e][lane];
+        nc[e] += lds.part.n[k][0][e][lane];
+        ns[e] += lds.part.n[k][1][e][lane];
+      }
+      const int node = node_index<64>(c.per_lane, nxn, nyn, tile, e, lane);
+      if (node < 0) continue;
+      f[node] = make_double2(fc[e], -fs[e]);
+      n[node] = make_float2(-2.0f * (float)kPi * ns[e], -2.0f * (float)kPi * nc[e]);
+    }
+    __syncthreads();
   }
 }
 
@@ -1198,6 +1597,141 @@ __device__ __forceinline__ double4v mfma64(double a, double b, double4v c) {
 
 // Row of an FP32 product that puts a lane's results on its FP64 rows.
 __device__ __forceinline__ int prow(int m) { return m / 4 + 4 * (m % 4); }
+
+// A cell's sums onto the pattern's node columns: tf[cell][k][x] =
+// sum_i f[i][k] wx[i][x] over the cell's ranges. 16 coarse rows x 64 columns of a
+// cell per workgroup at a time, 16 columns per wave; blockIdx.y: pattern.
+__global__ __launch_bounds__(kT) void surface_cell_rows_kernel(const SurfJob *jobs, int first) {
+  const SurfJob &jb = jobs[first + blockIdx.y];
+  const SurfCells &c = jb.c;
+  if (!jb.ok || c.g == 0) return;
+  const int mxn = c.co.ax.n, myn = c.co.ay.n, nxn = c.co.fx.n;
+  const int l = threadIdx.x & 63, m = l & 15, gq = l >> 4;
+  const int tiles_x = (nxn + 63) / 64, tiles_k = (myn + 15) / 16, items = tiles_x * tiles_k * c.g * c.g * c.gz;
+  for (int it = blockIdx.x; it < items; it += gridDim.x) {
+    const int id = it / (tiles_x * tiles_k), k0 = it / tiles_x % tiles_k * 16;
+    const int x = it % tiles_x * 64 + (int)(threadIdx.x / 64) * 16 + m;
+    const SurfCell cell = c.cells[id];
+    if (cell.count == 0 || x - m >= nxn) continue;
+    // rows and columns past the end repeat the last one and are not stored
+    const size_t base = (size_t)cell.range0 * mxn * myn, step = (size_t)mxn * myn;
+    const double2 *f = c.f + base + (size_t)gq * myn + min(k0 + m, myn - 1);
+    const float2 *n = c.n + base + (size_t)gq * myn + min(k0 + prow(m), myn - 1);
+    const double *wx = c.co.wx + (size_t)gq * nxn + min(x, nxn - 1);
+    Fields<2> acc;
+    clear(acc);
+    // the ranges' products are added rather than their values: no load waits for another
+    for (int r = 0; r < cell.ranges; ++r, f += step, n += step)
+#pragma unroll 4
+      for (int i = 0; i < mxn; i += 4) {
+        const double2 fv = f[(size_t)i * myn];
+        const float2 nv = n[(size_t)i * myn];
+        const double b = wx[(size_t)i * nxn];
+        acc.re = mfma64(fv.x, b, acc.re);
+        acc.im = mfma64(fv.y, b, acc.im);
+        acc.g[0] = mfma32(nv.x, (float)b, acc.g[0]);
+        acc.g[1] = mfma32(nv.y, (float)b, acc.g[1]);
+      }
+    if (x >= nxn) continue;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int k = k0 + gq + 4 * r;
+      if (k >= myn) continue;
+      const size_t o = ((size_t)id * myn + k) * nxn + x;
+      c.tf[o] = make_double2(acc.re[r], acc.im[r]);
+      c.tn[o] = make_float2(acc.g[0][r], acc.g[1][r]);
+    }
+  }
+}
+
+// And onto its rows, F(x, y) = sum_cells e^{-2 pi i q.c} sum_k wy[k][y] tf[cell][k][x] at
+// the pattern's nodes: 16 x 16 nodes per wave, 2 x 2 waves per workgroup;
+// blockIdx.y: every splits-th cell, whose partial sums the reduction adds.
+// e^{2 pi i t} from a table of 64 angles (LDS) and the series of what is left,
+// |x| <= pi / 64: 1e-15, a quarter of sincospi's time.
+__device__ __forceinline__ void turn(double t, const double2 *table, double &cs, double &sn) {
+  const double k = rint(t * 64.0);
+  const double x = __builtin_fma(k, -1.0 / 64.0, t) * (2.0 * kPi), x2 = x * x;
+  const double2 e = table[(int)(long long)k & 63];
+  const double s =
+      x * __builtin_fma(x2, __builtin_fma(x2, __builtin_fma(x2, -1.0 / 5040.0, 1.0 / 120.0), -1.0 / 6.0), 1.0);
+  const double c = __builtin_fma(
+      x2, __builtin_fma(x2, __builtin_fma(x2, __builtin_fma(x2, 1.0 / 40320.0, -1.0 / 720.0), 1.0 / 24.0), -0.5), 1.0);
+  cs = e.x * c - e.y * s;
+  sn = e.y * c + e.x * s;
+}
+
+__global__ __launch_bounds__(kT, 4) void surface_cell_cols_kernel(const SurfJob *jobs, int first) {
+  __shared__ double wy[kCellMaxNodes][32];
+  __shared__ double2 table[64];
+  const SurfJob &jb = jobs[first + blockIdx.z];
+  const SurfCells &c = jb.c;
+  if (!jb.ok || c.g == 0 || (int)blockIdx.y >= jb.splits) return;
+  const int nxn = c.co.fx.n, nyn = c.co.fy.n, myn = c.co.ay.n;
+  const int tiles_x = (nxn + 31) / 32, bx = (int)blockIdx.x % tiles_x, by = (int)blockIdx.x / tiles_x;
+  const int wave = threadIdx.x / 64, l = threadIdx.x & 63, m = l & 15, gq = l >> 4;
+  const int x = bx * 32 + (wave & 1) * 16 + m, y0 = (by * 2 + (wave >> 1)) * 16;
+  if (by * 32 >= nyn) return;
+  for (int i = threadIdx.x; i < myn * 32; i += kT)
+    wy[i / 32][i % 32] = c.co.wy[(size_t)(i / 32) * nyn + min(by * 32 + i % 32, nyn - 1)];
+  if (threadIdx.x < 64) sincospi(threadIdx.x / 32.0, &table[threadIdx.x].y, &table[threadIdx.x].x);
+  __syncthreads();
+  if (x - m >= nxn || y0 >= nyn) return;
+  const int xc = min(x, nxn - 1);
+  const double *w = &wy[gq][(wave >> 1) * 16 + m], *w32 = &wy[gq][(wave >> 1) * 16 + prow(m)];
+  double q[4][3], re[4] = {}, im[4] = {};
+  float nr[4] = {}, ni[4] = {};
+#pragma unroll
+  for (int r = 0; r < 4; ++r)
+    for (int k = 0; k < 3; ++k) q[r][k] = jb.sh.nodes[3 * ((size_t)xc * nyn + min(y0 + gq + 4 * r, nyn - 1)) + k];
+  const int ncells = c.g * c.g * c.gz;
+  for (int id = blockIdx.y; id < ncells; id += jb.splits) {
+    const SurfCell &cell = c.cells[id];
+    if (cell.count == 0) continue;
+    const double2 *tf = c.tf + ((size_t)id * myn + gq) * nxn + xc;
+    const float2 *tn = c.tn + ((size_t)id * myn + gq) * nxn + xc;
+    Fields<2> acc;
+    clear(acc);
+#pragma unroll 4
+    for (int k = 0; k < myn; k += 4) {
+      const double2 v = tf[(size_t)k * nxn];
+      const float2 n = tn[(size_t)k * nxn];
+      const double a = w[32 * k];
+      const float a32 = (float)w32[32 * k];
+      acc.re = mfma64(a, v.x, acc.re);
+      acc.im = mfma64(a, v.y, acc.im);
+      acc.g[0] = mfma32(a32, n.x, acc.g[0]);
+      acc.g[1] = mfma32(a32, n.y, acc.g[1]);
+    }
+    const double cx = cell.centre[0], cy = cell.centre[1], cz = cell.centre[2];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const double t = __builtin_fma(q[r][2], cz, __builtin_fma(q[r][1], cy, q[r][0] * cx));
+      double sn, cs;
+      turn(t - rint(t), table, cs, sn);
+      re[r] += acc.re[r] * cs + acc.im[r] * sn;
+      im[r] += acc.im[r] * cs - acc.re[r] * sn;
+      const float cf = (float)cs, sf = (float)sn;
+      nr[r] += acc.g[0][r] * cf + acc.g[1][r] * sf;
+      ni[r] += acc.g[1][r] * cf - acc.g[0][r] * sf;
+    }
+  }
+  if (x >= nxn) return;
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    const int y = y0 + gq + 4 * r;
+    if (y >= nyn) continue;
+    const int node = x * nyn + y;
+    if (jb.splits > 1) {  // as store_node leaves them
+      const size_t o = ((size_t)(node / kT) * jb.splits + blockIdx.y) * kT + node % kT;
+      jb.slot_f[o] = make_double2(re[r], -im[r]);
+      jb.slot_n[o] = make_float2(ni[r] / (-2.0f * (float)kPi), nr[r] / (-2.0f * (float)kPi));
+    } else {
+      jb.f[node] = make_double2(re[r], im[r]);
+      jb.n[node] = make_float2(nr[r], ni[r]);
+    }
+  }
+}
 
 // Along the rows, t[k][x] = sum_i node[i][k] tx[i][x] of F (FP64), of F with the
 // weights' derivatives and of N: 16 node rows x 16 columns per wave;
@@ -1568,9 +2102,19 @@ constexpr int kSlotSlack = 2 * kSurfMaxNodes + 8 * kT;
 struct SingleLayout {
   int max_nx, max_ny, slot_cap;
   size_t fit, records, centres, job, dev, nodes, tx, ty, tx32, ty32, prep, f, n, slot_f, slot_n, t64, t32, total;
+  // sums by cells, for large patterns
+  int cells;
+  long long cell_sums, cell_rows;
+  size_t c_nodes, c_wx, c_wy, c_id, c_sorted, c_cells, c_segs, c_range, c_order, c_f, c_n, c_tf, c_tn;
 };
 
-SingleLayout single_layout(int nx, int ny, int natoms, bool adjoint) {
+// Terms below which no pattern's node sums take long enough for cells (100 us:
+// 50,000 atoms at 80^2 nodes, on 512^2 pixels), so that their launches are left out.
+constexpr long long kCellMinTerms = 10000000000;
+// Ranges and cells hold at most these for one pattern.
+constexpr long long kCellSums = 4 << 20, kCellRows = 4 << 20;
+
+SingleLayout single_layout(int nx, int ny, int natoms, int nsegs, bool adjoint) {
   SingleLayout l;
   auto cap = [](int n) { return std::max(kSurfMinNodes, std::min(kSurfMaxNodes, (int)(0.6 * n) / 4 * 4)); };
   l.max_nx = cap(nx);
@@ -1601,6 +2145,25 @@ SingleLayout single_layout(int nx, int ny, int natoms, bool adjoint) {
   l.slot_n = take(adjoint ? 0 : sizeof(float2) * (size_t)l.slot_cap);
   l.t64 = take(sizeof(double2) * rows);
   l.t32 = take(sizeof(float4) * rows);
+  l.cells = !adjoint && (long long)npix * natoms >= kCellMinTerms ? kMaxCells : 0;
+  l.cell_sums = l.cell_rows = 0;
+  if (l.cells > 0) {
+    l.cell_sums = kCellSums;
+    l.cell_rows = kCellRows;
+    l.c_nodes = take(sizeof(double) * 3 * kCellMaxNodes * kCellMaxNodes);
+    l.c_wx = take(sizeof(double) * kCellMaxNodes * (size_t)l.max_nx);
+    l.c_wy = take(sizeof(double) * kCellMaxNodes * (size_t)l.max_ny);
+    l.c_id = take(sizeof(unsigned short) * ((size_t)natoms + 8));
+    l.c_sorted = take(sizeof(NodeAtom) * (size_t)natoms);
+    l.c_cells = take(sizeof(SurfCell) * kMaxCells);
+    l.c_segs = take(sizeof(spsim_hip_segment) * kMaxCells * (size_t)nsegs);
+    l.c_range = take(sizeof(int) * (512 + kMaxCells + 1));
+    l.c_order = take(sizeof(int) * (size_t)natoms);
+    l.c_f = take(sizeof(double2) * (size_t)l.cell_sums);
+    l.c_n = take(sizeof(float2) * (size_t)l.cell_sums);
+    l.c_tf = take(sizeof(double2) * (size_t)l.cell_rows);
+    l.c_tn = take(sizeof(float2) * (size_t)l.cell_rows);
+  }
   l.total = at;
   return l;
 }
@@ -1614,6 +2177,24 @@ void launch_interpolation(const SurfJob *jobs, int first, int count, int nx, int
                      first);
   hipLaunchKernelGGL(surface_cols_kernel, dim3((nx + 31) / 32, (ny + 31) / 32, count), dim3(kT), 0, s, jobs, first, dev,
                      hkl, F, I);
+}
+
+// Grid sizes for the sums by cells of some patterns.
+struct CellBounds {
+  int cells;        // per pattern
+  long long items;  // (range, tile) pairs
+  int rows;         // workgroups of the first product
+  int nxn, nyn, splits;
+};
+
+void launch_cells(const SurfJob *jobs, int first, int count, const CellBounds &b, const float *ff, float b_global,
+                  bool has_b, hipStream_t s) {
+  hipLaunchKernelGGL(surface_sort_kernel, dim3(b.cells, 1, count), dim3(kSortT), 0, s, jobs, first);
+  hipLaunchKernelGGL(has_b ? surface_cell_nodes_kernel<true> : surface_cell_nodes_kernel<false>,
+                     dim3((unsigned)b.items, count), dim3(kT), 0, s, jobs, first, ff, b_global);
+  hipLaunchKernelGGL(surface_cell_rows_kernel, dim3(b.rows, count), dim3(kT), 0, s, jobs, first);
+  hipLaunchKernelGGL(surface_cell_cols_kernel, dim3(((b.nxn + 31) / 32) * ((b.nyn + 31) / 32), b.splits, count),
+                     dim3(kT), 0, s, jobs, first);
 }
 
 // Bound on how much a matrix lengthens a vector: the root of the largest
@@ -1651,7 +2232,9 @@ bool surf_worth(long long nx, long long ny, long long natoms, long long min_term
   return nx >= kSurfMinSide && ny >= kSurfMinSide && nx * ny * natoms >= min_terms;
 }
 
-size_t surf_single_bytes(int nx, int ny, int natoms) { return single_layout(nx, ny, natoms, false).total; }
+size_t surf_single_bytes(int nx, int ny, int natoms, int nsegs) {
+  return single_layout(nx, ny, natoms, nsegs, false).total;
+}
 
 namespace {
 
@@ -1691,6 +2274,26 @@ int launch_plan(const PatternLaunch &a, int nx, int ny, const Spectrum *sp, Surf
   p.slot_cap = l.slot_cap;
   p.max_nx = l.max_nx;
   p.max_ny = l.max_ny;
+  const bool cells = l.cells > 0 && kind == SurfKind::kSum;
+  if (cells) {
+    p.max_cells = l.cells;
+    p.max_cell_sums = l.cell_sums;
+    p.max_cell_rows = l.cell_rows;
+    SurfCells &c = p.job.c;
+    c.co.nodes = (double *)(w + l.c_nodes);
+    c.co.wx = (double *)(w + l.c_wx);
+    c.co.wy = (double *)(w + l.c_wy);
+    c.id = (unsigned short *)(w + l.c_id);
+    c.sorted = w + l.c_sorted;
+    c.cells = (SurfCell *)(w + l.c_cells);
+    c.segs = (spsim_hip_segment *)(w + l.c_segs);
+    c.range_cell = (int *)(w + l.c_range);
+    c.order = (int *)(w + l.c_order);
+    c.f = (double2 *)(w + l.c_f);
+    c.n = (float2 *)(w + l.c_n);
+    c.tf = (double2 *)(w + l.c_tf);
+    c.tn = (float2 *)(w + l.c_tn);
+  }
   p.kind = kind;
   const double norm = a.has_rot ? rotation_norm(a.rot.r) : 1.0;
   p.scale = norm;
@@ -1722,7 +2325,7 @@ int launch_plan(const PatternLaunch &a, int nx, int ny, const Spectrum *sp, Surf
                     (SurfRecord *)(w + l.records),
                     (double *)(w + l.centres)};
   hipLaunchKernelGGL(surface_scan_kernel, dim3(p.list_blocks + kSurfAtomBlocks), dim3(kT), 0, s, sc);
-  hipLaunchKernelGGL(surface_plan_kernel, dim3(std::max(1, 2 * cus / 3), 3), dim3(kT), 0, s, p);
+  hipLaunchKernelGGL(surface_plan_kernel, dim3(std::max(1, cells ? 3 * cus / 5 : 2 * cus / 3), cells ? 5 : 3), dim3(kT), 0, s, p);
   SPSIM_HIP_TRY(hipGetLastError());
   return SPSIM_HIP_OK;
 }
@@ -1731,13 +2334,24 @@ int launch_plan(const PatternLaunch &a, int nx, int ny, const Spectrum *sp, Surf
 
 int launch_surface(const PatternLaunch &a, int nx, int ny, const Spectrum *sp, int cus, void *ws, const int **ok_flag,
                    hipStream_t s) {
-  const SingleLayout l = single_layout(nx, ny, a.natoms, false);
+  const SingleLayout l = single_layout(nx, ny, a.natoms, a.nsegs, false);
   char *w = (char *)ws;
   const SurfJob *job = (const SurfJob *)(w + l.job);
   const bool has_b = a.atom_b != nullptr;
   const int slots = resident_slots(nodes_kernel(has_b, sp != nullptr), cus);
   SPSIM_TRY(launch_plan(a, nx, ny, sp, sp ? SurfKind::kSpectrum : SurfKind::kSum, nullptr, l, w, slots, cus, s));
   SPSIM_TRY(launch_nodes(job, nullptr, 0, slots, a.ff, a.b_global, has_b, sp, s));
+  if (l.cells > 0 && !sp) {
+    CellBounds b{};
+    b.cells = l.cells;
+    // ranges x ceil(nodes / 128) tiles of at most cell_sums range nodes
+    b.items = std::min(512 + l.cells + l.cell_sums / 128, 16LL * cus);
+    b.rows = 8 * cus;
+    b.nxn = l.max_nx;
+    b.nyn = l.max_ny;
+    b.splits = 32;
+    launch_cells(job, 0, 1, b, a.ff, a.b_global, has_b, s);
+  }
   launch_interpolation(job, 0, 1, nx, ny, l.max_nx * l.max_ny, l.max_ny, (const float *)(w + l.dev), a.hkl, a.F, a.I,
                        s);
   SPSIM_HIP_TRY(hipGetLastError());
@@ -1745,12 +2359,12 @@ int launch_surface(const PatternLaunch &a, int nx, int ny, const Spectrum *sp, i
   return SPSIM_HIP_OK;
 }
 
-size_t surf_adjoint_bytes(int nx, int ny, int natoms) { return single_layout(nx, ny, natoms, true).total; }
+size_t surf_adjoint_bytes(int nx, int ny, int natoms) { return single_layout(nx, ny, natoms, 0, true).total; }
 
 int launch_surface_adjoint(const PatternLaunch &a, const float *gI, int nx, int ny, const SurfAtomTile *tiles,
                            int ntiles, int splits, bool want_b, double4 *partial, int cus, void *ws,
                            const int **ok_flag, hipStream_t s) {
-  const SingleLayout l = single_layout(nx, ny, a.natoms, true);
+  const SingleLayout l = single_layout(nx, ny, a.natoms, 0, true);
   char *w = (char *)ws;
   const SurfJob *job = (const SurfJob *)(w + l.job);
   SPSIM_TRY(launch_plan(a, nx, ny, nullptr, SurfKind::kAdjoint, gI, l, w, cus, cus, s));
@@ -1891,8 +2505,9 @@ ScanLayout scan_layout(int nx, int ny, int nmol) {
 // count grows and the stretch with it.
 int axis_count(int k) { return k <= 12 ? kSurfMinNodes + 4 * k : 64 + 8 * (k - 12); }
 
-int axis_nodes(const float *slope, double radius, float gauss) {
-  auto enough = [&](int n) { return axis_need(slope, (float)radius, gauss, axis_stretch(n)) <= (float)n; };
+int axis_nodes(const SurfSlopes &slope, double radius, float gauss) {
+  const float r = (float)radius, h[3] = {r, r, r};
+  auto enough = [&](int n) { return axis_need(slope, r, h, gauss, axis_stretch(n)) <= (float)n; };
   int lo = -1, hi = 12 + (kSurfMaxNodes - 64) / 8;
   if (!enough(axis_count(hi))) return 0;
   while (hi - lo > 1) {

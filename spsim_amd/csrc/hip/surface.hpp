@@ -25,13 +25,18 @@ struct SurfRecord {
   int pad;
 };
 
+// Steepest slopes of the surface along an axis: the largest |dq/du| and |dq_k/du|
+// on the lines u = cos(pi j / (kSurfLines - 1)).
+struct SurfSlopes {
+  float all[kSurfLines], part[3][kSurfLines];
+};
+
 // The list's surface: Chebyshev coefficients of a polynomial through q at
 // kSurfDeg x kSurfDeg pixels, in the pixel coordinates u, v in [-1, 1]
-// (coef[n][m][k]: T_n(v) T_m(u), component k), and its steepest slopes:
-// slope_x[j] is the largest |dq/du| on the line u = cos(pi j / (kSurfLines - 1)).
+// (coef[n][m][k]: T_n(v) T_m(u), component k), and its slopes.
 struct SurfFit {
   double coef[kSurfDeg][kSurfDeg][3];
-  float slope_x[kSurfLines], slope_y[kSurfLines];
+  SurfSlopes slope_x, slope_y;
   float s2max;  // largest s^2 = (|q| 1e-10 / 2)^2 seen
   float normal[3];  // unit normal of the surface's middle
   int sym;          // 2: mirror- and transpose-symmetric, 1: mirror-symmetric, 0
@@ -51,6 +56,36 @@ struct SurfShape {
   SurfAxis ax, ay;
   double *nodes, *tx, *ty;
   float2 *tx32, *ty32;
+};
+
+// One cell of a molecule that is summed by cells: its atoms are `count` records
+// from `start`, its sums `ranges` partial ones from `range0`.
+struct SurfCell {
+  double centre[3];
+  int start, count, range0, ranges;
+};
+
+// Nodes at which a cell's sums are formed, and the weights that take them to the
+// nodes fx x fy of the whole pattern: wx [ax.n][fx.n], wy [ay.n][fy.n].
+struct SurfCoarse {
+  SurfAxis ax, ay, fx, fy;
+  double *nodes, *wx, *wy;
+};
+
+// A molecule summed by cells: g x g x gz boxes of the cube of half edge
+// `extent` (g = 0: not). f and n are [range][ax.n][ay.n], tf and tn [cell][ay.n][fx.n].
+struct SurfCells {
+  int g, gz, per_lane, tiles;
+  double extent;
+  SurfCoarse co;
+  unsigned short *id;  // of every atom, its cell
+  int *order;          // the atoms by cell
+  void *sorted;        // and their records
+  SurfCell *cells;
+  spsim_hip_segment *segs;  // [cell][nsegs], of the sorted records
+  int *range_cell;          // cell of a range, or -1
+  double2 *f, *tf;
+  float2 *n, *tn;
 };
 
 // One pattern. The node sums f (F) and n (its derivative along the normal) are
@@ -77,7 +112,8 @@ struct SurfJob {
   double2 *t64;
   float4 *t32;
   long long pattern;  // index of the outputs
-  int shape;          // of a plan
+  int shape, coarse;  // of a plan
+  SurfCells c;
 };
 
 struct SurfItem {
@@ -91,6 +127,7 @@ struct SurfMol {
   float b_smooth;    // largest Gaussian coefficient of the terms (form factor + B), A^2
   float weakest;     // smallest ratio of a term's amplitude at s2max to that at 0
   int bad;
+  int ordered;       // the species' segments follow each other
 };
 
 // Host sizes only: is the pattern large enough to look at its list?
@@ -99,7 +136,7 @@ bool surf_worth(long long nx, long long ny, long long natoms, long long min_term
 // One pattern on the device alone (no host decision). On return *ok_flag points
 // to a device int that is non-zero when the outputs were written and zero when
 // the list or molecule is not smooth enough, in which case nothing was.
-size_t surf_single_bytes(int nx, int ny, int natoms);
+size_t surf_single_bytes(int nx, int ny, int natoms, int nsegs);
 // sp: a wavelength spectrum, or null.
 int launch_surface(const PatternLaunch &a, int nx, int ny, const Spectrum *sp, int cus, void *ws, const int **ok_flag,
                    hipStream_t s);
@@ -125,7 +162,7 @@ int launch_surface_adjoint(const PatternLaunch &a, const float *gI, int nx, int 
 
 // What the host reads of a list, and of a molecule seen on it.
 struct SurfHead {
-  float slope_x[kSurfLines], slope_y[kSurfLines];
+  SurfSlopes slope_x, slope_y;
   float s2max, normal[3];
   int sym, pad;
 };

@@ -409,3 +409,54 @@ def test_nfft_molecules_split_between_surface_and_grids(gpu, with_b, rotated):
         e = rel_l2(out[0][m], Ir)
         print(f"molecule {m}: {e:.2e}", flush=True)
         assert TOL < e < 2e-5 if m == 1 else e < TOL, m
+
+
+@pytest.mark.parametrize("shape,n,natoms,geometry,with_b,rotated", [
+    ("ball", (640, 640), 30_011, {}, False, False),
+    ("ball", (700, 610), 30_000, {"cx": 1.1e-3, "wavelength": 0.15e-9}, True, True),
+    ("rod", (800, 800), 20_001, {"pixel": 60e-6}, True, False),
+    ("dense", (720, 720), 24_000, {}, False, True),
+    ("unordered", (640, 640), 30_011, {}, False, False),
+])
+def test_sums_by_cells(gpu, shape, n, natoms, geometry, with_b, rotated):
+    """Large patterns, whose node sums go by cells: octants and plain nodes, atom
+    counts that end within every piece, a rod (empty cells), nearly all atoms
+    in a few cells, and species that are not in order (no cells). The same bits
+    on every call and replay."""
+    import torch
+
+    nx, ny = n
+    rng = np.random.default_rng(natoms)
+    Z, pos, b = wl.random_molecule(natoms, 13e-9, rng, atom_b_range=(5.0, 40.0))
+    if shape == "rod":
+        pos = pos * np.array([1.2, 0.1, 0.1], np.float32)
+    if shape == "dense":
+        pos[: natoms - 200] *= np.float32(0.1)
+    atoms = dv.DeviceAtoms(dv.pack_atoms(Z, pos, atom_b=b if with_b else None), gpu)
+    if shape == "unordered":
+        atoms.segs = torch.flip(atoms.segs.reshape(-1, 4), [0]).contiguous()
+    R = wl.uniform_rotations(1, rng)[0] if rotated else None
+    ff = dv.form_factor_table(device=gpu)
+    q = _list(nx, ny, **geometry)
+    qs = torch.from_numpy(q).to(gpu)
+    run = lambda **kw: dv.structure_factor_grid(qs, nx, ny, atoms, ff, B=1.0, R=R, **kw)
+    F, I = run()
+    _, Id = run(tile=dv.make_tile(1, 256, 0))
+    torch.cuda.synchronize()
+    first, Fh, Id = I.cpu().numpy(), F.cpu().numpy(), Id.cpu().numpy()
+    sub = np.unique(np.concatenate([[0, nx - 1, nx * ny - nx, nx * ny - 1], rng.choice(nx * ny, 400, replace=False)]))
+    Fr, Ir = oracle.sf_f64(q[sub], Z, pos, atom_b=b if with_b else None, B=1.0, R=R, threads=oracle_threads())
+    e, ed = rel_l2(first[sub], Ir), rel_l2(Id[sub], Ir)
+    print(f"{shape}: I {e:.2e} (direct {ed:.2e})", flush=True)
+    assert e < TOL and np.linalg.norm(Fh[sub, 0] + 1j * Fh[sub, 1] - Fr) / np.linalg.norm(Fr) < TOL
+    assert not np.array_equal(first, Id) and rel_l2(first, Id) < 2 * TOL
+    stream = torch.cuda.Stream()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=stream):
+        run(F=F, I=I, stream=torch.cuda.current_stream())
+    for _ in range(2):
+        I.fill_(float("nan"))
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert np.array_equal(I.cpu().numpy(), first)
