@@ -228,8 +228,12 @@ int spsim_hip_sf_spectrum(const float *d_hkl, int npix, const spsim_hip_atom *d_
    1 when the interpolation staged each wave's grid box in LDS (lists whose
    consecutive q are close, such as detector rows), and the Gaussian spread
    window's width (0 without per-atom B). Uses
-   the library workspace; synchronises `stream` once (to read the bounds that
-   size the grids), the rest is stream-ordered. */
+   the library workspace; synchronises `stream` (to read the bounds that size
+   the grids, and for the upload of a plan's tables), the rest is stream-ordered.
+   With eps <= 1e-6, on a square list that is a smooth detector's and where it
+   costs less (spsim_hip_sf_grid says when), the pattern is interpolated over the detector's
+   surface instead, to the direct sums' accuracy; the grids are planned all the
+   same: info describes them, and what they reject is rejected. */
 int spsim_hip_sf_nfft(const float *d_hkl, int npix, const spsim_hip_atom *d_atoms, const float *d_atom_b,
                       const spsim_hip_segment *d_segs, int nsegs, int natoms, const float *d_ff, float b_global,
                       const double *rot9, double eps, float *d_F, float *d_I, int *info, void *stream);
@@ -244,11 +248,8 @@ int spsim_hip_sf_nfft(const float *d_hkl, int npix, const spsim_hip_atom *d_atom
    to the interval-arithmetic range of R_p over the q box, and every pattern
    only interpolates from it, so the spread and FFT run once.
    The grids are larger than a single pattern's when q does not fill that ball
-   (a flat detector's Ewald cap). On a square list that is a smooth detector's
-   and where it costs less (spsim_hip_sf_grid says when), the patterns are
-   interpolated over the detector's surface instead, to the direct sums' accuracy;
-   the grids are planned all the same: info describes them, and what they reject
-   is rejected. Returns after the last pattern is written
+   (a flat detector's Ewald cap). Interpolated over the detector's surface
+   as spsim_hip_sf_nfft is, when every pattern can be. Returns after the last pattern is written
    (it synchronises `stream`). Other arguments as spsim_hip_sf_nfft. */
 int spsim_hip_sf_nfft_batch(const float *d_hkl, int npix, const spsim_hip_atom *d_atoms, const float *d_atom_b,
                             const spsim_hip_segment *d_segs, int nsegs, int natoms, const float *d_ff, float b_global,

@@ -2136,7 +2136,11 @@ int nufft_run(double *hb, const float *d_hkl, int npix, const spsim_hip_atom *d_
 
 // Side of a square list of npix q on which `terms` = atoms x patterns atoms are
 // worth a look at interpolation over the detector surface (surface.hip), or 0.
-int surface_side(int npix, long long terms) {
+// The look costs 40 us, of 250 us and more on the grids from kSurfaceMinTerms
+// on. A coarser eps than 1e-6 (W < 7) keeps the grids: their values are that
+// far from the direct sums', which callers who compare runs would see.
+int surface_side(int npix, long long terms, int W) {
+  if (W < 7) return 0;
   const int n = (int)llround(sqrt((double)npix));
   return (long long)n * n == npix && surf_worth(n, n, terms, kSurfaceMinTerms) ? n : 0;
 }
@@ -2216,9 +2220,7 @@ int nufft_impl(const float *d_hkl, int npix, const spsim_hip_atom *d_atoms, cons
 
   // 1. Bounds of the atoms and of q: per-workgroup records, folded on the host
   // after the call's one synchronisation; and the look at the list's surface.
-  // A single pattern stays on the grids: 100,000 atoms on 1024^2 take 0.69 ms
-  // there, 1.2 ms by the surface's node sums.
-  int side = npat > 0 ? surface_side(npix, (long long)natoms * nout) : 0;
+  int side = surface_side(npix, (long long)natoms * nout, W);
   for (int p = 0; p < npat && d_atom_b; ++p)
     if (!is_rotation(rots + 9 * (size_t)p)) side = 0;
   const int most = natoms > npix ? natoms : npix;
@@ -2659,7 +2661,7 @@ extern "C" int spsim_hip_sf_nfft_molecules(const float *d_hkl, int npix, int nmo
   constexpr int kMolBlocks = 64;
   if (nmol > 65535) return fail(SPSIM_HIP_ERR_INVALID, "at most 65535 molecules per call (%d)", nmol);
   const int total_atoms = atom_offsets[nmol];
-  const int side = surface_side(npix, total_atoms);
+  const int side = surface_side(npix, total_atoms, W);
   const int qblk = (npix + kThreads - 1) / kThreads < kBoundBlocks ? (npix + kThreads - 1) / kThreads : kBoundBlocks;
   const size_t b_dig = side ? align256(surf_digest_bytes(nmol)) : 0;
   const size_t b_q = align256(sizeof(double) * kNb * qblk);

@@ -41,41 +41,6 @@ struct Spectrum {
 // (host code). The polynomial is used from 4 samples on.
 void spectrum_fit(Spectrum &sp);
 
-// One term of a spectrum: U(t) = sum_k W_k e^{-2 pi i s_k t} as (ur, -ui) for
-// the FP64 phase t = q.r in turns, by the polynomials within their range, else
-// by the sample sum with each s_k t reduced to turns in FP64.
-__device__ __forceinline__ void spectrum_term(const Spectrum &sp, int ns, double t, float &ur, float &ui) {
-  const double tc = sp.sc * t;
-  const float tf = (float)tc;
-  if (__builtin_fabsf(tf) <= sp.tlim) {
-    asm volatile("");  // keeps the polynomials under the branch: formed for every atom, 3 samples took 216 us for 165 us
-    const float ph = (float)__builtin_amdgcn_fract(tc);
-    const float cs = __builtin_amdgcn_cosf(ph);
-    const float sn = __builtin_amdgcn_sinf(ph);
-    const float v = tf * sp.inv_tlim;
-    const float u = v * v;
-    float gc = sp.p[kSpectrumDegree], gq = sp.q[kSpectrumDegree];
-#pragma unroll
-    for (int d = kSpectrumDegree - 1; d >= 0; --d) {
-      gc = __builtin_fmaf(gc, u, sp.p[d]);
-      gq = __builtin_fmaf(gq, u, sp.q[d]);
-    }
-    const float gs = v * gq;
-    ur = __builtin_fmaf(cs, gc, -sn * gs);
-    ui = __builtin_fmaf(sn, gc, cs * gs);
-    return;
-  }
-  float sr = 0.0f, si = 0.0f;
-  int m = 0;
-  do {  // at least one sample
-    const float ph = (float)__builtin_amdgcn_fract(sp.s[m] * t);
-    sr = __builtin_fmaf(sp.w[m], __builtin_amdgcn_cosf(ph), sr);
-    si = __builtin_fmaf(sp.w[m], __builtin_amdgcn_sinf(ph), si);
-  } while (++m < ns);
-  ur = sr;
-  ui = si;
-}
-
 struct PatternLaunch {
   const float *hkl;
   int npix;

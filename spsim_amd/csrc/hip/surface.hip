@@ -444,27 +444,37 @@ __global__ __launch_bounds__(kT, 3) void surface_scan_kernel(ScanArgs a) {
 // for their sampling.
 __host__ __device__ inline float axis_stretch(int n) { return 1.0f / coshf(kStretch / n); }
 
-__host__ __device__ inline float axis_need(const SurfSlopes &slope, float radius, const float *h, float gauss, float a) {
-  const float as = asinf(a);
+// On the line u = cos(pi k / (kLines - 1)), x = u asin(a): s = sin(x) / a,
+// |du/dt| = sqrt(1 - s^2) a / (asin(a) cos(x)), here times asin(a). Lines mirrored
+// about the middle share them.
+__host__ __device__ inline float line_density(int k, float a, float as) {
+#ifdef __HIP_DEVICE_COMPILE__
+  const float x = fabsf(__builtin_amdgcn_cosf(0.5f * k / (kLines - 1))) * as;
+  const float sx = __builtin_amdgcn_sinf(x * (float)(0.5 / kPi)), cx = __builtin_amdgcn_cosf(x * (float)(0.5 / kPi));
+  return __builtin_amdgcn_sqrtf(fmaxf(0.0f, a * a - sx * sx)) * __builtin_amdgcn_rcpf(fmaxf(cx, 1e-6f));
+#else
+  const float x = std::fabs(std::cos((float)kPi * k / (kLines - 1))) * as;
+  const float sx = std::sin(x), cx = std::cos(x);
+  return std::sqrt(std::max(0.0f, a * a - sx * sx)) / std::max(cx, 1e-6f);
+#endif
+}
+
+// density(k) as line_density at the stretch whose asin is as.
+template <class Density>
+__host__ __device__ inline float axis_need(const SurfSlopes &slope, float radius, const float *h, float gauss, float as,
+                                           Density density) {
   float w = 0.0f;
   for (int k = 0; k < kLines; ++k) {
-    // On the line u = cos(pi k / (kLines - 1)), x = u asin(a): s = sin(x) / a,
-    // |du/dt| = sqrt(1 - s^2) a / (asin(a) cos(x)). Lines mirrored about the
-    // middle share them.
-#ifdef __HIP_DEVICE_COMPILE__
-    const float x = fabsf(__builtin_amdgcn_cosf(0.5f * k / (kLines - 1))) * as;
-    const float sx = __builtin_amdgcn_sinf(x * (float)(0.5 / kPi)), cx = __builtin_amdgcn_cosf(x * (float)(0.5 / kPi));
-    const float g = __builtin_amdgcn_sqrtf(fmaxf(0.0f, a * a - sx * sx)) * __builtin_amdgcn_rcpf(fmaxf(cx, 1e-6f));
-#else
-    const float x = std::fabs(std::cos((float)kPi * k / (kLines - 1))) * as;
-    const float sx = std::sin(x), cx = std::cos(x);
-    const float g = std::sqrt(std::max(0.0f, a * a - sx * sx)) / std::max(cx, 1e-6f);
-#endif
     const float box = slope.part[0][k] * h[0] + slope.part[1][k] * h[1] + slope.part[2][k] * h[2];
-    w = fmaxf(w, fminf(slope.all[k] * radius, box) * g);
+    w = fmaxf(w, fminf(slope.all[k] * radius, box) * density(k));
   }
   const float theta = 1.02f * 2.0f * (float)kPi * w / as;
   return theta + 4.0f * cbrtf(theta) + 8.0f + 2.0f * sqrtf(fmaxf(gauss, 0.0f));
+}
+
+__device__ __forceinline__ float axis_need(const SurfSlopes &slope, float radius, const float *h, float gauss, float a) {
+  const float as = asinf(a);
+  return axis_need(slope, radius, h, gauss, as, [&](int k) { return line_density(k, a, as); });
 }
 
 enum class SurfKind { kSum, kSpectrum, kAdjoint };
@@ -1033,6 +1043,11 @@ __global__ __launch_bounds__(kT) void surface_tables_kernel(const SurfFit *fit, 
   build(blockIdx.y, fit, shapes[blockIdx.z], nx, ny, lds);
 }
 
+__global__ __launch_bounds__(kT) void surface_coarse_kernel(const SurfFit *fit, const SurfCoarse *coarse) {
+  __shared__ BuildLds lds;
+  build_coarse(blockIdx.y, fit, coarse[blockIdx.z], lds);
+}
+
 // ---- 3. node sums ---------------------------------------------------------------
 //
 // One work item: a tile of nodes (node_tiling) x one atom range, whose records
@@ -1068,6 +1083,42 @@ template <>
 struct SpectrumArg<true> {
   using type = Spectrum;
 };
+
+// One term of a spectrum: U(t) = sum_k W_k e^{-2 pi i s_k t} as (ur, -ui) for
+// the FP64 phase t = q.r in turns, by the polynomials within their range, else
+// by the sample sum with each s_k t reduced to turns in FP64, as in spectrum_sum
+// (sf_kernels.hip).
+__device__ __forceinline__ void spectrum_term(const Spectrum &sp, int ns, double t, float &ur, float &ui) {
+  const double tc = sp.sc * t;
+  const float tf = (float)tc;
+  if (__builtin_fabsf(tf) <= sp.tlim) {
+    asm volatile("");  // keeps the polynomials under the branch, not formed for every atom
+    const float ph = (float)__builtin_amdgcn_fract(tc);
+    const float cs = __builtin_amdgcn_cosf(ph);
+    const float sn = __builtin_amdgcn_sinf(ph);
+    const float v = tf * sp.inv_tlim;
+    const float u = v * v;
+    float gc = sp.p[kSpectrumDegree], gq = sp.q[kSpectrumDegree];
+#pragma unroll
+    for (int d = kSpectrumDegree - 1; d >= 0; --d) {
+      gc = __builtin_fmaf(gc, u, sp.p[d]);
+      gq = __builtin_fmaf(gq, u, sp.q[d]);
+    }
+    const float gs = v * gq;
+    ur = __builtin_fmaf(cs, gc, -sn * gs);
+    ui = __builtin_fmaf(sn, gc, cs * gs);
+    return;
+  }
+  float sr = 0.0f, si = 0.0f;
+  int m = 0;
+  do {  // at least one sample
+    const float ph = (float)__builtin_amdgcn_fract(sp.s[m] * t);
+    sr = __builtin_fmaf(sp.w[m], __builtin_amdgcn_cosf(ph), sr);
+    si = __builtin_fmaf(sp.w[m], __builtin_amdgcn_sinf(ph), si);
+  } while (++m < ns);
+  ur = sr;
+  ui = si;
+}
 
 // A lane's sums of node e: a partial sum, or F and N = -2 pi i sum w f n.r e^{-i phi}.
 __device__ __forceinline__ void store_node(const SurfJob &jb, int tile, int split, int e, double fc, double fs, float nc,
@@ -1336,7 +1387,7 @@ __global__ __launch_bounds__(kT) void surface_nodes_kernel(const SurfJob *jobs, 
 // N), turned by the centre's phase and added up. Terms fall with the square of
 // the coarse nodes, the interpolation grows with the cells: cells_cost. On
 // 100,000 atoms with B and 188^2 nodes, 108 cells of 64^2 nodes: 33 us for the
-// sort, 161 us for the sums, 73 and 84 us for the products, against 1140 us for
+// sort, 161 us for the sums, 36 and 84 us for the products, against 1140 us for
 // the plain sums.
 
 // The records of one cell (blockIdx.x), in their order, which is that of the
@@ -1599,48 +1650,67 @@ __device__ __forceinline__ double4v mfma64(double a, double b, double4v c) {
 __device__ __forceinline__ int prow(int m) { return m / 4 + 4 * (m % 4); }
 
 // A cell's sums onto the pattern's node columns: tf[cell][k][x] =
-// sum_i f[i][k] wx[i][x] over the cell's ranges. 16 coarse rows x 64 columns of a
-// cell per workgroup at a time, 16 columns per wave; blockIdx.y: pattern.
+// sum_i f[i][k] wx[i][x]: 16 coarse rows of a cell per workgroup at a time, whose
+// sums over the ranges it gathers in LDS first, every wave then for every
+// fourth 16 columns; blockIdx.y: pattern. 36 us on 108 cells of 64^2 nodes in
+// 490 ranges, bound by their loads. (Read by every wave as it goes, 16 columns
+// each: 71 us, a chain of loads and products; 32 columns each: 91 us.)
 __global__ __launch_bounds__(kT) void surface_cell_rows_kernel(const SurfJob *jobs, int first) {
+  __shared__ double2 sf[kCellMaxNodes * 16];
+  __shared__ float2 sn[kCellMaxNodes * 16];
   const SurfJob &jb = jobs[first + blockIdx.y];
   const SurfCells &c = jb.c;
   if (!jb.ok || c.g == 0) return;
   const int mxn = c.co.ax.n, myn = c.co.ay.n, nxn = c.co.fx.n;
-  const int l = threadIdx.x & 63, m = l & 15, gq = l >> 4;
-  const int tiles_x = (nxn + 63) / 64, tiles_k = (myn + 15) / 16, items = tiles_x * tiles_k * c.g * c.g * c.gz;
+  const int wave = threadIdx.x / 64, l = threadIdx.x & 63, m = l & 15, gq = l >> 4;
+  const int tiles_k = (myn + 15) / 16, items = tiles_k * c.g * c.g * c.gz;
+  const size_t step = (size_t)mxn * myn;
   for (int it = blockIdx.x; it < items; it += gridDim.x) {
-    const int id = it / (tiles_x * tiles_k), k0 = it / tiles_x % tiles_k * 16;
-    const int x = it % tiles_x * 64 + (int)(threadIdx.x / 64) * 16 + m;
+    const int id = it / tiles_k, k0 = it % tiles_k * 16;
     const SurfCell cell = c.cells[id];
-    if (cell.count == 0 || x - m >= nxn) continue;
+    if (cell.count == 0) continue;
     // rows and columns past the end repeat the last one and are not stored
-    const size_t base = (size_t)cell.range0 * mxn * myn, step = (size_t)mxn * myn;
-    const double2 *f = c.f + base + (size_t)gq * myn + min(k0 + m, myn - 1);
-    const float2 *n = c.n + base + (size_t)gq * myn + min(k0 + prow(m), myn - 1);
-    const double *wx = c.co.wx + (size_t)gq * nxn + min(x, nxn - 1);
-    Fields<2> acc;
-    clear(acc);
-    // the ranges' products are added rather than their values: no load waits for another
-    for (int r = 0; r < cell.ranges; ++r, f += step, n += step)
+    for (int e = threadIdx.x; e < 16 * mxn; e += kT) {
+      const size_t node = cell.range0 * step + (size_t)(e / 16) * myn + min(k0 + e % 16, myn - 1);
+      double re = 0.0, im = 0.0;
+      float nr = 0.0f, ni = 0.0f;
+#pragma unroll 4
+      for (int r = 0; r < cell.ranges; ++r) {
+        const double2 f = c.f[node + r * step];
+        const float2 n = c.n[node + r * step];
+        re += f.x;
+        im += f.y;
+        nr += n.x;
+        ni += n.y;
+      }
+      sf[e] = make_double2(re, im);
+      sn[e] = make_float2(nr, ni);
+    }
+    __syncthreads();
+    for (int x = wave * 16 + m; x - m < nxn; x += kT / 4) {
+      const double *wx = c.co.wx + (size_t)gq * nxn + min(x, nxn - 1);
+      Fields<2> acc;
+      clear(acc);
 #pragma unroll 4
       for (int i = 0; i < mxn; i += 4) {
-        const double2 fv = f[(size_t)i * myn];
-        const float2 nv = n[(size_t)i * myn];
+        const double2 f = sf[16 * (i + gq) + m];
+        const float2 n = sn[16 * (i + gq) + prow(m)];
         const double b = wx[(size_t)i * nxn];
-        acc.re = mfma64(fv.x, b, acc.re);
-        acc.im = mfma64(fv.y, b, acc.im);
-        acc.g[0] = mfma32(nv.x, (float)b, acc.g[0]);
-        acc.g[1] = mfma32(nv.y, (float)b, acc.g[1]);
+        acc.re = mfma64(f.x, b, acc.re);
+        acc.im = mfma64(f.y, b, acc.im);
+        acc.g[0] = mfma32(n.x, (float)b, acc.g[0]);
+        acc.g[1] = mfma32(n.y, (float)b, acc.g[1]);
       }
-    if (x >= nxn) continue;
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int k = k0 + gq + 4 * r;
-      if (k >= myn) continue;
-      const size_t o = ((size_t)id * myn + k) * nxn + x;
-      c.tf[o] = make_double2(acc.re[r], acc.im[r]);
-      c.tn[o] = make_float2(acc.g[0][r], acc.g[1][r]);
+      for (int r = 0; r < 4; ++r) {
+        const int k = k0 + gq + 4 * r;
+        if (k >= myn || x >= nxn) continue;
+        const size_t o = ((size_t)id * myn + k) * nxn + x;
+        c.tf[o] = make_double2(acc.re[r], acc.im[r]);
+        c.tn[o] = make_float2(acc.g[0][r], acc.g[1][r]);
+      }
     }
+    __syncthreads();
   }
 }
 
@@ -2390,17 +2460,20 @@ int launch_surface_adjoint(const PatternLaunch &a, const float *gI, int nx, int 
 struct SurfPlan {
   // Patterns that run together and share the workspace.
   struct Group {
-    int first, count, item_first, nitems, max_nodes, max_ny;
+    int first, count, item_first, nitems, max_nodes, max_ny, max_atoms;
     bool split;
+    int celled;  // the first ones, summed by cells
+    CellBounds cells;
   };
   SurfInput in{};
   std::vector<char> takes;
   std::vector<Group> groups;
   std::vector<SurfShape> shapes;
+  std::vector<SurfCoarse> coarse;
   std::vector<SurfJob> jobs;
   std::vector<SurfItem> items;
-  // device memory: shapes, jobs and items (one upload), the shapes' tables, the workspace
-  size_t at_jobs = 0, at_items = 0, at_tables = 0, at_ws = 0, bytes = 0;
+  // device memory: shapes, coarse nodes, jobs and items (one upload), the tables, the workspace
+  size_t at_coarse = 0, at_jobs = 0, at_items = 0, at_tables = 0, at_ws = 0, bytes = 0;
   const SurfJob *d_jobs = nullptr;
   const SurfItem *d_items = nullptr;
   const float *dev = nullptr;
@@ -2431,6 +2504,21 @@ size_t place(SurfJob *j, int nx, char *ws, size_t at) {
   j->slot_n = (float2 *)take(sizeof(float2) * slots);
   j->t64 = (double2 *)take(sizeof(double2) * (size_t)j->sh.ay.n * nx);
   j->t32 = (float4 *)take(sizeof(float4) * (size_t)j->sh.ay.n * nx);
+  if (j->c.g > 0) {
+    SurfCells &c = j->c;
+    const size_t cells = (size_t)c.g * c.g * c.gz, ranges = j->natoms / cell_range(j->natoms) + cells;
+    const size_t sums = ranges * c.co.ax.n * c.co.ay.n, rows = cells * c.co.ay.n * j->sh.ax.n;
+    c.id = (unsigned short *)take(sizeof(unsigned short) * ((size_t)j->natoms + 8));
+    c.order = (int *)take(sizeof(int) * (size_t)j->natoms);
+    c.sorted = take(sizeof(NodeAtom) * (size_t)j->natoms);
+    c.cells = (SurfCell *)take(sizeof(SurfCell) * cells);
+    c.segs = (spsim_hip_segment *)take(sizeof(spsim_hip_segment) * cells * j->nsegs);
+    c.range_cell = (int *)take(sizeof(int) * ranges);
+    c.f = (double2 *)take(sizeof(double2) * sums);
+    c.n = (float2 *)take(sizeof(float2) * sums);
+    c.tf = (double2 *)take(sizeof(double2) * rows);
+    c.tn = (float2 *)take(sizeof(float2) * rows);
+  }
   return at;
 }
 
@@ -2450,6 +2538,18 @@ size_t place_tables(SurfShape *sh, int nx, int ny, char *mem, size_t at) {
   return at;
 }
 
+size_t place_tables(SurfCoarse *co, char *mem, size_t at) {
+  auto take = [&](size_t bytes) {
+    char *p = mem + at;
+    at += align_up(bytes);
+    return p;
+  };
+  co->nodes = (double *)take(sizeof(double) * 3 * co->ax.n * co->ay.n);
+  co->wx = (double *)take(sizeof(double) * (size_t)co->ax.n * co->fx.n);
+  co->wy = (double *)take(sizeof(double) * (size_t)co->ay.n * co->fy.n);
+  return at;
+}
+
 // Issue cycles of one atom in a lane's nodes (node_tiling).
 double lane_cost(int per_lane) { return per_lane == 8 ? 321.0 : (per_lane == 1 ? 75.0 : 57.0 * per_lane); }
 
@@ -2463,11 +2563,12 @@ double interpolation_cost(double nodes_x, double nodes_y, double nx, double ny) 
 void split_group(std::vector<SurfJob> &jobs, int first, int count, int slots, std::vector<SurfItem> *items) {
   double work = 0.0;
   for (int i = first; i < first + count; ++i)
-    work += (double)jobs[i].tiles * lane_cost(jobs[i].per_lane) * jobs[i].natoms;
+    if (jobs[i].c.g == 0) work += (double)jobs[i].tiles * lane_cost(jobs[i].per_lane) * jobs[i].natoms;
   const double share = std::max(work / (4.0 * slots), 128.0 * lane_cost(4));
   const size_t begin = items->size();
   for (int i = first; i < first + count; ++i) {
     SurfJob &j = jobs[i];
+    if (j.c.g > 0) continue;  // summed by cells
     j.splits = std::max(1, std::min(kSurfMaxSplits, (int)std::ceil(lane_cost(j.per_lane) * j.natoms / share)));
     for (int t = 0; t < j.tiles; ++t)
       for (int k = 0; k < j.splits; ++k) items->push_back(SurfItem{i, t, k, 0});
@@ -2505,34 +2606,97 @@ ScanLayout scan_layout(int nx, int ny, int nmol) {
 // count grows and the stretch with it.
 int axis_count(int k) { return k <= 12 ? kSurfMinNodes + 4 * k : 64 + 8 * (k - 12); }
 
+// Whether n nodes (a multiple of 4) are enough: axis_need() with the densities of
+// every count formed once.
+bool enough_nodes(const SurfSlopes &slope, float radius, const float *h, float gauss, int n) {
+  struct Line {
+    float as, density[kLines];
+  };
+  static const std::vector<Line> lines = [] {
+    std::vector<Line> l(kSurfMaxNodes / 4 + 1);
+    for (int i = 1; i <= kSurfMaxNodes / 4; ++i) {
+      const float a = axis_stretch(4 * i);
+      l[i].as = std::asin(a);
+      for (int k = 0; k < kLines; ++k) l[i].density[k] = line_density(k, a, l[i].as);
+    }
+    return l;
+  }();
+  const Line &l = lines[n / 4];
+  return axis_need(slope, radius, h, gauss, l.as, [&](int k) { return l.density[k]; }) <= (float)n;
+}
+
 int axis_nodes(const SurfSlopes &slope, double radius, float gauss) {
   const float r = (float)radius, h[3] = {r, r, r};
-  auto enough = [&](int n) { return axis_need(slope, r, h, gauss, axis_stretch(n)) <= (float)n; };
   int lo = -1, hi = 12 + (kSurfMaxNodes - 64) / 8;
-  if (!enough(axis_count(hi))) return 0;
+  if (!enough_nodes(slope, r, h, gauss, axis_count(hi))) return 0;
   while (hi - lo > 1) {
     const int mid = (lo + hi) / 2;
-    (enough(axis_count(mid)) ? hi : lo) = mid;
+    (enough_nodes(slope, r, h, gauss, axis_count(mid)) ? hi : lo) = mid;
   }
   return axis_count(hi);
 }
 
-// Nodes of a pattern; false when it is left to its other path.
-bool choose(const SurfHead &head, SurfMol mol, double norm, int nx, int ny, int natoms, const double *limit,
-            SurfAxis *ax, SurfAxis *ay) {
-  mol.radius *= norm;
-  if (natoms <= 0 || !smooth(mol, head.s2max)) return false;
-  SurfAxis *out[2] = {ax, ay};
-  for (int k = 0; k < 2; ++k) {
-    const int n = axis_nodes(k ? head.slope_y : head.slope_x, mol.radius, mol.b_smooth * head.s2max);
-    if (n == 0) return false;
-    *out[k] = SurfAxis{n, axis_stretch(n), 0.0};
-    out[k]->asin_a = std::asin(out[k]->a);
+// The same for a box of half edges h, in multiples of 4 up to kCellMaxNodes.
+int box_nodes(const SurfSlopes &slope, const float *h, float gauss) {
+  const float r = std::sqrt(h[0] * h[0] + h[1] * h[1] + h[2] * h[2]);
+  int lo = -1, hi = (kCellMaxNodes - kCellMinNodes) / 4;
+  if (!enough_nodes(slope, r, h, gauss, kCellMaxNodes)) return 0;
+  while (hi - lo > 1) {
+    const int mid = (lo + hi) / 2;
+    (enough_nodes(slope, r, h, gauss, kCellMinNodes + 4 * mid) ? hi : lo) = mid;
   }
-  if (!limit) return worth(ax->n, ay->n, nx, ny, natoms, SurfKind::kSum);
+  return kCellMinNodes + 4 * hi;
+}
+
+// How a molecule's patterns are evaluated: their nodes and cells, if any.
+struct Choice {
+  double norm = -1.0;  // of the matrices it holds for
+  bool taken = false;
+  SurfAxis ax{}, ay{};
+  int g = 0, gz = 0, mx = 0, my = 0;
+  int shape = -1, coarse = -1;
+};
+
+SurfAxis axis_of(int n) {
+  SurfAxis a{n, axis_stretch(n), 0.0};
+  a.asin_a = std::asin(a.a);
+  return a;
+}
+
+Choice choose(const SurfHead &head, SurfMol mol, double norm, int nx, int ny, int natoms, const double *limit) {
+  Choice c;
+  c.norm = norm;
+  mol.radius *= norm;
+  if (natoms <= 0 || !smooth(mol, head.s2max)) return c;
+  const float gauss = mol.b_smooth * head.s2max;
+  const int n[2] = {axis_nodes(head.slope_x, mol.radius, gauss), axis_nodes(head.slope_y, mol.radius, gauss)};
+  if (n[0] == 0 || n[1] == 0) return c;
+  c.ax = axis_of(n[0]);
+  c.ay = axis_of(n[1]);
+  const bool octants = head.sym == 2 && n[0] == n[1];
   int per_lane, tiles;
-  node_tiling(ax->n, ay->n, head.sym == 2 && ax->n == ay->n, 1LL << 25, &per_lane, &tiles);
-  return (double)tiles * kT * lane_cost(per_lane) * natoms + interpolation_cost(ax->n, ay->n, nx, ny) < *limit;
+  double sums = sums_cost(n[0], n[1], octants, natoms, &per_lane, &tiles);
+  // cells: the launches are shared by a plan's patterns
+  double least = 0.7 * sums - 1e9;
+  for (int k = 0; k < kCellGrids && mol.ordered && least > 0.0; ++k) {
+    int g, gz;
+    cell_grid(k, &g, &gz);
+    const float r = (float)mol.radius, h[3] = {r / g, r / g, r / gz};
+    const int mx = box_nodes(head.slope_x, h, gauss), my = box_nodes(head.slope_y, h, gauss);
+    if (mx == 0 || my == 0 || (long long)(natoms / cell_range(natoms) + g * g * gz) * mx * my > kCellSums ||
+        (long long)g * g * gz * my * n[0] > kCellRows)
+      continue;
+    const double cost = cells_cost(n[0], n[1], mx, my, g * g * gz, octants && mx == my, natoms);
+    if (cost >= least) continue;
+    least = sums = cost;
+    c.g = g;
+    c.gz = gz;
+    c.mx = mx;
+    c.my = my;
+  }
+  const double direct = 0.8 * 26.0 * nx * ny * natoms;  // as worth() takes them
+  c.taken = sums + interpolation_cost(n[0], n[1], nx, ny) < (limit ? *limit : direct);
+  return c;
 }
 
 }  // namespace
@@ -2571,11 +2735,7 @@ SurfPlan *surf_plan_choose(const SurfInput &in, const void *digest) {
   SurfPlan *p = new SurfPlan;
   p->in = in;
   p->takes.assign(in.npatterns, 0);
-  struct Choice {
-    double norm;
-    int shape;  // -1: not taken
-  };
-  std::vector<Choice> last(in.nmol, Choice{-1.0, -1});  // of a molecule's last pattern
+  std::vector<Choice> last(in.nmol);  // of a molecule's last pattern
   std::vector<SurfJob> &jobs = p->jobs;
   for (int i = 0; i < in.npatterns; ++i) {
     const int m = in.pattern_mol ? in.pattern_mol[i] : (in.nmol == 1 ? 0 : i);
@@ -2583,26 +2743,35 @@ SurfPlan *surf_plan_choose(const SurfInput &in, const void *digest) {
     // rotations differ from 1 by rounding: one node count serves them
     double norm = in.rot9 ? rotation_norm(in.rot9 + 9 * (size_t)i) : 1.0;
     if (std::fabs(norm - 1.0) < 1e-6) norm = 1.0;
-    if (last[m].norm != norm) {
-      last[m] = Choice{norm, -1};
-      SurfShape sh{};
-      if (choose(head, mols[m].mol, norm, in.nx, in.ny, natoms, in.limit ? in.limit + m : nullptr, &sh.ax, &sh.ay)) {
-        for (size_t k = 0; k < p->shapes.size(); ++k)
-          if (p->shapes[k].ax.n == sh.ax.n && p->shapes[k].ay.n == sh.ay.n) last[m].shape = (int)k;
-        if (last[m].shape < 0) {
-          last[m].shape = (int)p->shapes.size();
-          p->shapes.push_back(sh);
+    Choice &ch = last[m];
+    if (ch.norm != norm) {
+      ch = choose(head, mols[m].mol, norm, in.nx, in.ny, natoms, in.limit ? in.limit + m : nullptr);
+      if (ch.taken) {
+        auto find = [](auto &list, auto same) {
+          for (size_t k = 0; k < list.size(); ++k)
+            if (same(list[k])) return (int)k;
+          list.emplace_back();
+          return (int)list.size() - 1;
+        };
+        ch.shape = find(p->shapes, [&](const SurfShape &sh) { return sh.ax.n == ch.ax.n && sh.ay.n == ch.ay.n; });
+        p->shapes[ch.shape].ax = ch.ax;
+        p->shapes[ch.shape].ay = ch.ay;
+        if (ch.g > 0) {
+          ch.coarse = find(p->coarse, [&](const SurfCoarse &co) {
+            return co.ax.n == ch.mx && co.ay.n == ch.my && co.fx.n == ch.ax.n && co.fy.n == ch.ay.n;
+          });
+          p->coarse[ch.coarse] = SurfCoarse{axis_of(ch.mx), axis_of(ch.my), ch.ax, ch.ay, nullptr, nullptr, nullptr};
         }
       }
     }
-    if (last[m].shape < 0) continue;
+    if (!ch.taken) continue;
     p->takes[i] = 1;
     SurfJob j{};
     j.ok = 1;
     j.nx = in.nx;
     j.ny = in.ny;
-    j.sh = p->shapes[last[m].shape];
-    j.shape = last[m].shape;
+    j.sh = p->shapes[ch.shape];
+    j.shape = ch.shape;
     j.atoms = in.atoms + in.h_mols[m].atom_begin;
     j.atom_b = in.atom_b ? in.atom_b + in.h_mols[m].atom_begin : nullptr;
     j.segs = in.segs + in.h_mols[m].seg_begin;
@@ -2612,8 +2781,21 @@ SurfPlan *surf_plan_choose(const SurfInput &in, const void *digest) {
     if (in.rot9) std::copy(in.rot9 + 9 * (size_t)i, in.rot9 + 9 * (size_t)(i + 1), j.rot);
     std::copy(mols[m].centre, mols[m].centre + 3, j.r0);
     std::copy(head.normal, head.normal + 3, j.normal);
-    // a group has work enough for every tiling: the one of the least work
-    node_tiling(j.sh.ax.n, j.sh.ay.n, head.sym == 2 && j.sh.ax.n == j.sh.ay.n, 1LL << 25, &j.per_lane, &j.tiles);
+    const bool octants = head.sym == 2 && j.sh.ax.n == j.sh.ay.n;
+    if (ch.g > 0) {
+      SurfCells &c = j.c;
+      c.g = ch.g;
+      c.gz = ch.gz;
+      c.extent = mols[m].mol.radius * norm;
+      c.co = p->coarse[ch.coarse];
+      j.coarse = ch.coarse;
+      cell_tiling(ch.mx, ch.my, octants && ch.mx == ch.my, &c.per_lane, &c.tiles);
+      j.per_lane = 1;
+      j.tiles = (j.sh.ax.n * j.sh.ay.n + kT - 1) / kT;
+    } else {
+      // a group has work enough for every tiling: the one of the least work
+      node_tiling(j.sh.ax.n, j.sh.ay.n, octants, 1LL << 25, &j.per_lane, &j.tiles);
+    }
     j.pattern = i;
     jobs.push_back(j);
   }
@@ -2621,25 +2803,42 @@ SurfPlan *surf_plan_choose(const SurfInput &in, const void *digest) {
     delete p;
     return nullptr;
   }
-  // largest first, so that a group's patterns need similar grids
+  // those with cells first, and largest first, so that a group's patterns need similar grids
   std::stable_sort(jobs.begin(), jobs.end(), [](const SurfJob &a, const SurfJob &b) {
+    if ((a.c.g > 0) != (b.c.g > 0)) return a.c.g > 0;
     return (double)a.sh.ax.n * a.sh.ay.n * a.natoms > (double)b.sh.ax.n * b.sh.ay.n * b.natoms;
   });
   const int slots = resident_slots(nodes_kernel(in.atom_b != nullptr, false), in.cus);
   size_t ws_bytes = 0;
   for (int first = 0; first < (int)jobs.size();) {
-    SurfPlan::Group g{first, 0, (int)p->items.size(), 0, 0, 0, false};
+    SurfPlan::Group g{first, 0, (int)p->items.size(), 0, 0, 0, 0, false, 0, CellBounds{}};
     size_t at = 0;
     while (first + g.count < (int)jobs.size() && g.count < 4096) {
       SurfJob probe = jobs[first + g.count];
       probe.splits = 4;  // a typical group's; only the group's size depends on it
       const size_t end = place(&probe, in.nx, nullptr, at);
-      if (g.count > 0 && end > kGroupBytes) break;
+      if (g.count > 0 && (end > kGroupBytes || (probe.c.g == 0 && g.celled > 0))) break;
       at = end;
+      g.celled += probe.c.g > 0;
       g.max_nodes = std::max(g.max_nodes, probe.sh.ax.n * probe.sh.ay.n);
       g.max_ny = std::max(g.max_ny, probe.sh.ay.n);
+      g.max_atoms = std::max(g.max_atoms, probe.natoms);
       ++g.count;
     }
+    for (int i = first; i < first + g.celled; ++i) {
+      SurfJob &j = jobs[i];
+      const SurfCells &c = j.c;
+      CellBounds &b = g.cells;
+      j.splits = cell_splits(j.sh.ax.n, j.sh.ay.n, g.celled, 1LL << 40);
+      const int cells = c.g * c.g * c.gz;
+      b.cells = std::max(b.cells, cells);
+      b.items = std::max(b.items, (long long)(j.natoms / cell_range(j.natoms) + cells) * c.tiles);
+      b.nxn = std::max(b.nxn, j.sh.ax.n);
+      b.nyn = std::max(b.nyn, j.sh.ay.n);
+      b.splits = std::max(b.splits, j.splits);
+    }
+    g.cells.items = std::min(g.cells.items, std::max(64LL, 32LL * in.cus / std::max(1, g.celled)));
+    g.cells.rows = std::max(64, 8 * in.cus / std::max(1, g.celled));
     split_group(jobs, first, g.count, slots, &p->items);
     g.nitems = (int)p->items.size() - g.item_first;
     at = 0;
@@ -2655,11 +2854,13 @@ SurfPlan *surf_plan_choose(const SurfInput &in, const void *digest) {
   p->in.pattern_mol = nullptr;
   p->in.rot9 = nullptr;
   p->in.limit = nullptr;
-  p->at_jobs = align_up(sizeof(SurfShape) * p->shapes.size());
+  p->at_coarse = align_up(sizeof(SurfShape) * p->shapes.size());
+  p->at_jobs = p->at_coarse + align_up(sizeof(SurfCoarse) * p->coarse.size());
   p->at_items = p->at_jobs + align_up(sizeof(SurfJob) * jobs.size());
   p->at_tables = p->at_items + align_up(sizeof(SurfItem) * p->items.size());
   size_t at = p->at_tables;
   for (SurfShape &sh : p->shapes) at = place_tables(&sh, in.nx, in.ny, nullptr, at);
+  for (SurfCoarse &co : p->coarse) at = place_tables(&co, nullptr, at);
   p->at_ws = at;
   p->bytes = at + ws_bytes;
   return p;
@@ -2673,15 +2874,18 @@ int surf_plan_bind(SurfPlan *p, const void *scan, void *mem, hipStream_t s) {
   char *w = (char *)mem;
   size_t at = p->at_tables;
   for (SurfShape &sh : p->shapes) at = place_tables(&sh, in.nx, in.ny, w, at);
+  for (SurfCoarse &co : p->coarse) at = place_tables(&co, w, at);
   for (const SurfPlan::Group &g : p->groups) {
     at = p->at_ws;
     for (int i = g.first; i < g.first + g.count; ++i) {
       p->jobs[i].sh = p->shapes[p->jobs[i].shape];
+      if (p->jobs[i].c.g > 0) p->jobs[i].c.co = p->coarse[p->jobs[i].coarse];
       at = place(&p->jobs[i], in.nx, w, at);
     }
   }
   std::vector<char> image(p->at_tables);
   std::copy(p->shapes.begin(), p->shapes.end(), (SurfShape *)image.data());
+  std::copy(p->coarse.begin(), p->coarse.end(), (SurfCoarse *)(image.data() + p->at_coarse));
   std::copy(p->jobs.begin(), p->jobs.end(), (SurfJob *)(image.data() + p->at_jobs));
   std::copy(p->items.begin(), p->items.end(), (SurfItem *)(image.data() + p->at_items));
   SPSIM_HIP_TRY(hipMemcpyAsync(w, image.data(), image.size(), hipMemcpyHostToDevice, s));
@@ -2689,6 +2893,10 @@ int surf_plan_bind(SurfPlan *p, const void *scan, void *mem, hipStream_t s) {
   for (int first = 0; first < nshapes; first += 4096)
     hipLaunchKernelGGL(surface_tables_kernel, dim3(256, 2, std::min(4096, nshapes - first)), dim3(kT), 0, s,
                        (const SurfFit *)((const char *)scan + l.fit), (const SurfShape *)w + first, in.nx, in.ny);
+  const int ncoarse = (int)p->coarse.size();
+  for (int first = 0; first < ncoarse; first += 4096)
+    hipLaunchKernelGGL(surface_coarse_kernel, dim3(64, 2, std::min(4096, ncoarse - first)), dim3(kT), 0, s,
+                       (const SurfFit *)((const char *)scan + l.fit), (const SurfCoarse *)(w + p->at_coarse) + first);
   SPSIM_HIP_TRY(hipGetLastError());
   SPSIM_HIP_TRY(hipStreamSynchronize(s));  // the copy reads image
   p->dev = (const float *)((const char *)scan + l.dev);
@@ -2741,10 +2949,12 @@ int surf_plan_run(const SurfPlan *p, float2 *F, float *I, hipStream_t s) {
   const bool has_b = in.atom_b != nullptr;
   const int slots = resident_slots(nodes_kernel(has_b, false), in.cus);
   for (const SurfPlan::Group &g : p->groups) {
-    hipLaunchKernelGGL(surface_prepare_kernel, dim3(16, g.count), dim3(kT), 0, s, p->d_jobs, g.first, has_b);
+    const int wgs = std::max(16, std::min((g.max_atoms + kT - 1) / kT, 4 * in.cus / g.count));
+    hipLaunchKernelGGL(surface_prepare_kernel, dim3(wgs, g.count), dim3(kT), 0, s, p->d_jobs, g.first, has_b);
     const SurfItem *items = p->d_items + g.item_first;
     const int blocks = std::min(g.nitems, slots);
-    SPSIM_TRY(launch_nodes(p->d_jobs, items, g.nitems, blocks, in.ff, in.b_global, has_b, nullptr, s));
+    if (g.nitems > 0) SPSIM_TRY(launch_nodes(p->d_jobs, items, g.nitems, blocks, in.ff, in.b_global, has_b, nullptr, s));
+    if (g.celled > 0) launch_cells(p->d_jobs, g.first, g.celled, g.cells, in.ff, in.b_global, has_b, s);
     launch_interpolation(p->d_jobs, g.first, g.count, in.nx, in.ny, g.split ? g.max_nodes : 0, g.max_ny, p->dev, in.hkl,
                          F, I, s);
   }
