@@ -10,9 +10,12 @@ all 512 patterns, inputs and outputs already in HBM; the tile is chosen by the
 plan's autotuner. Beside it: G pixel-atom terms/s, the plain path (one
 single-pattern launch per pattern with a host synchronisation after each),
 the FP64 error on 4,096 random pixels of 4 patterns, and the roofline of the
-timed kernel.
+timed launch.
 
-Roofline: the structure-factor kernels are bound by VALU issue. `achieved` is
+Roofline: plans without a tile of the caller's interpolate smooth patterns over
+the detector surface, so their terms are not executed one by one; they are
+priced against HBM, by the bytes that every method has to move (atoms and q in,
+intensities out). The direct kernels are bound by VALU issue. `achieved` is
 the VALU wave instructions the timed kernel executes (its inner loop's count
 per wave and atom, read from this build's gfx950 assembly, times the
 wave-atom iterations of the launch), expressed as FP32 flop-equivalents at the
@@ -179,6 +182,20 @@ def executed_roofline(family, has_b, wave_atoms, kernel_ms, terms, kernel_name):
     }
 
 
+def surface_roofline(nbytes, kernel_ms, terms):
+    """Roofline of patterns interpolated over the detector surface: the bytes
+    that every method has to move against the HBM peak."""
+    achieved = nbytes / (kernel_ms * 1e-3) / 1e9
+    return {
+        "bound": "hbm", "achieved": round(achieved, 2), "peak": HBM_PEAK_GBS, "unit": "GB/s",
+        "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": None, "kernel": "surface_nodes_kernel",
+        "work": {"bytes": float(nbytes), "kernel_ms": round(kernel_ms, 4)},
+        "textbook": {"w_eq_per_term": W_TEXTBOOK, "terms_per_launch": terms,
+                     "note": "terms of the direct sum; the sums are formed at a few nodes per detector axis "
+                             "and interpolated to the pixels"},
+    }
+
+
 def recorded_traffic(name, kernel, per_lane, chunk, splits=None):
     """HBM bytes per launch of a kernel from the FETCH_SIZE / WRITE_SIZE counter
     runs recorded in profiles/<name> (each scaled by the same counter's reading
@@ -336,11 +353,15 @@ def headline(args, torch, dv, wl, _lib):
             log("headline: FP64 check on 4 patterns x 4096 pixels")
             res["rel_err"], res["rel_errs"] = fp64_check(I_host, q, mols, rots, pats, 4096, 7)
             res["rel_err_patterns"] = [{"pattern": p, "natoms": int(sizes[p])} for p in pats]
-        wave_atoms = wave_atoms_of(mols, range(npat), st["family"], det.n, det.n, st["per_lane"])
-        roof = executed_roofline(st["family"], False, wave_atoms, kernel_ms, terms, st["kernel"])
-        roof["traffic"] = recorded_traffic("traffic_batched.json", st["kernel"], st["per_lane"], st["chunk_atoms"])
-        roof["algorithmic_bytes_per_launch"] = float(16 * sum(len(m[0]) for m in mols) + 12 * det.npix +
-                                                     4 * det.npix * npat)
+        nbytes = float(16 * sum(len(m[0]) for m in mols) + 12 * det.npix + 4 * det.npix * npat)
+        if args.batch_tile:
+            wave_atoms = wave_atoms_of(mols, range(npat), st["family"], det.n, det.n, st["per_lane"])
+            roof = executed_roofline(st["family"], False, wave_atoms, kernel_ms, terms, st["kernel"])
+            roof["traffic"] = recorded_traffic("traffic_batched.json", st["kernel"], st["per_lane"],
+                                               st["chunk_atoms"])
+        else:
+            roof = surface_roofline(nbytes, kernel_ms, terms)
+        roof["algorithmic_bytes_per_launch"] = nbytes
         res["roofline"] = roof
         res["workload"] = (f"{npat} molecules, N log-uniform in [2e3, 2e5] (mean {res['natoms_mean']:.0f}), C/N/O/S "
                            f"62:17:20:1, radius 5 nm (N/5000)^(1/3), uniform random orientations, "
@@ -375,9 +396,8 @@ def batched_vs_plain(name, det, mols, rots, args, torch, dv, _lib, fp64_patterns
                "patterns_per_s_plain": round(npat / (ms_p * 1e-3), 1),
                "speedup_batched_vs_plain": round(ms_p / ms_b, 3),
                "gterms_per_s_batched": round(terms.value / (ms_b * 1e-3) / 1e9, 1)}
-        wave_atoms = wave_atoms_of(mols, range(npat), st["family"], det.n, det.n, st["per_lane"])
-        out["valu_issue_frac"] = executed_roofline(st["family"], False, wave_atoms, ms_b, terms.value,
-                                                   st["kernel"])["frac"]
+        out["hbm_frac"] = surface_roofline(16 * sum(len(m[0]) for m in mols) + 12 * det.npix + 4 * det.npix * npat,
+                                           ms_b, terms.value)["frac"]
         out["rel_err_vs_fp64"], _ = fp64_check(I_host, q, mols, rots, fp64_patterns, 2048, 11)
         if extra:
             extra(L, plan, I, stream, out)
@@ -470,6 +490,19 @@ def single_pattern(args, torch, dv, wl, _lib):
     hkl = q.cpu().numpy()
     _, I_ref = oracle.sf_f64(hkl[sub], Z, pos, atom_b=B, threads=oracle_threads())
     err = rel_l2(I.cpu().numpy()[sub], I_ref)
+    # the library's own choice (no tile): interpolated over the detector surface
+    auto = lambda: dv.structure_factor_grid(q, det.n, det.n, atoms, ff, I=I, want_F=False)
+    for _ in range(3):
+        auto()
+    torch.cuda.synchronize()
+    ev = [(torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)) for _ in range(reps)]
+    for e0, e1 in ev:
+        e0.record()
+        auto()
+        e1.record()
+    torch.cuda.synchronize()
+    auto_ms = float(np.mean([a.elapsed_time(b) for a, b in ev]))
+    auto_err = rel_l2(I.cpu().numpy()[sub], I_ref)
     family = kernel_family(kind == "grid", tile.pixels_per_lane)
     kname = {"octant": "sf_octant_kernel"}.get(family, "sf_grid_kernel" if kind == "grid" else "sf_pattern_kernel")
     wave_atoms = float(atoms.natoms) * tiles_per_pattern(family, det.n, det.n, tile.pixels_per_lane) * WAVES_PER_TILE
@@ -483,6 +516,9 @@ def single_pattern(args, torch, dv, wl, _lib):
         "tile": {"kernel": kind, "per_lane": tile.pixels_per_lane, "chunk_atoms": tile.chunk_atoms,
                  "atom_splits": tile.atom_splits, "sweep": sweep},
         "roofline": roof, "rel_err_vs_fp64": err, "rel_err_sample": "4096 random pixels",
+        "automatic": {"ms": round(auto_ms, 4), "speedup_vs_direct": round(kernel_ms / auto_ms, 2),
+                      "rel_err_vs_fp64": auto_err,
+                      "roofline": surface_roofline(20 * atoms.natoms + 16 * npix, auto_ms, terms)},
         "Z": Z, "pos": pos, "B": B, "hkl": q, "npix": npix,
     }
 
@@ -554,8 +590,7 @@ def pipeline(args, torch, dv, wl, _lib):
         ms_plain = time_plain(L, _lib, plan, I, stream)
         err, _ = fp64_check(I_host, q, [(Z, pos)] * npat, rots, [0, npat // 2, npat - 1], 4096, 13)
         chain_bytes = npat * (n * n * 4 + 2 * nb * 4)
-        wave_atoms = wave_atoms_of([(Z, pos)], [0] * npat, st["family"], n, n, st["per_lane"])
-        roof = executed_roofline(st["family"], False, wave_atoms, ms_sf, terms.value, st["kernel"])
+        roof = surface_roofline(16 * len(Z) + 12 * n * n + 4 * n * n * npat, ms_sf, terms.value)
         return {
             "workload": f"{npat} orientations of one 50000-atom C/N/O/S molecule (radius 10 nm), 1024x1024 detector "
                         f"20 um at 0.05 m, lambda 1.3 nm, 4x4 binning, QE 0.15, readout 10 e-, dark 0.1, "
