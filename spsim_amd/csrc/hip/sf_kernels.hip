@@ -427,6 +427,62 @@ __device__ __forceinline__ void grid_tile(const float *__restrict__ hkl, int nx,
   }
 }
 
+// The sums of tile_sum for the four mirrored pixels of a quad (quad_pixels), bit
+// for bit: mirroring only changes signs in q.r = q_z z + (q_y y + q_x x), so that
+// the four phases share the inner sums (5 of 12 FP64 operations) and the weights
+// (a quarter of the exponentials).
+template <int CHUNK, bool HAS_B>
+__device__ __forceinline__ void quad_exact_sum(double qx, double qy, double qz, float s2,
+                                               const spsim_hip_atom *__restrict__ atoms,
+                                               const float *__restrict__ atom_b,
+                                               const spsim_hip_segment *__restrict__ segs, int nsegs, int a_begin,
+                                               int a_end, const float *__restrict__ ff, float b_global, const double *R,
+                                               AtomLds *__restrict__ sm, double (&Fr)[4], double (&Fi)[4]) {
+  const float nl2 = -s2 * (float)kLog2e;
+#pragma unroll
+  for (int k = 0; k < 4; ++k) Fr[k] = Fi[k] = 0.0;
+  for (int sg = 0; sg < nsegs; ++sg) {
+    const int s_start = segs[sg].start;
+    const int s_end = s_start + segs[sg].count;
+    const int species = segs[sg].species;
+    const int lo = max(s_start, a_begin);
+    const int hi = min(s_end, a_end);
+    if (lo >= hi) continue;
+    const float Bs = (species == SPSIM_HIP_UNIT_SPECIES) ? 0.0f : b_global;
+    const float f = form_factor(ff + species * SPSIM_HIP_FF_STRIDE, s2, Bs);
+    for (int c0 = lo; c0 < hi; c0 += CHUNK) {
+      const int n = min(CHUNK, hi - c0);
+      stage_chunk<HAS_B>(atoms, atom_b, c0, n, R, sm);
+      float sr[4] = {}, si[4] = {};
+#pragma unroll 2
+      for (int j = 0; j < n; ++j) {
+        const AtomLds a = sm[j];
+        const double px = qx * a.x;
+        const double p = __builtin_fma(qy, a.y, px), m = __builtin_fma(qy, a.y, -px);
+        const double t[4] = {__builtin_fma(qz, a.z, p), __builtin_fma(qz, a.z, m), __builtin_fma(qz, a.z, -m),
+                             __builtin_fma(qz, a.z, -p)};
+        float wt;
+        if constexpr (HAS_B) {
+          wt = __builtin_amdgcn_exp2f(__builtin_fmaf(a.b, nl2, a.w));
+        } else {
+          wt = a.w;
+        }
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          const float ph = (float)__builtin_amdgcn_fract(t[k]);
+          sr[k] = __builtin_fmaf(wt, __builtin_amdgcn_cosf(ph), sr[k]);
+          si[k] = __builtin_fmaf(wt, __builtin_amdgcn_sinf(ph), si[k]);
+        }
+      }
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        Fr[k] = __builtin_fma((double)f, (double)sr[k], Fr[k]);
+        Fi[k] = __builtin_fma((double)f, (double)si[k], Fi[k]);
+      }
+    }
+  }
+}
+
 // ---- Square mirror-symmetric detectors: octants -----------------------------
 //
 // On a square detector centred on the beam with square pixels, the transposed
@@ -618,11 +674,33 @@ __device__ __forceinline__ void octant_tile(const float *__restrict__ hkl, int n
 
 // ---- single-pattern kernels (blockIdx.x = tile, blockIdx.y = atom split) ----
 
+// Whether an n x n list is mirror-symmetric: rough[b] = 0 from every one of
+// kMirrorBlocks workgroups.
+constexpr int kMirrorBlocks = 64;
+__global__ __launch_bounds__(kThreads) void sf_mirror_check_kernel(const float *__restrict__ hkl, int n,
+                                                                   int *__restrict__ rough) {
+  bool sym = true;
+  for (int qd = blockIdx.x * kThreads + threadIdx.x; qd < grid_quads(n, n); qd += kMirrorBlocks * kThreads) {
+    int p0, p1, p2, p3;
+    quad_pixels(qd, n, n, p0, p1, p2, p3);
+    sym = sym && mirrored(hkl, p0, p1, -1.0f, 1.0f) && mirrored(hkl, p0, p2, 1.0f, -1.0f) &&
+          mirrored(hkl, p0, p3, -1.0f, -1.0f);
+  }
+  const int bad = __syncthreads_or(!sym);
+  if (threadIdx.x == 0) rough[blockIdx.x] = bad ? 1 : 0;
+}
+__device__ __forceinline__ bool all_mirrored(const int *__restrict__ rough) {
+  static_assert(kMirrorBlocks == 64, "one lane per workgroup of the check");
+  return __ballot(rough[threadIdx.x & 63] != 0) == 0;
+}
+
 // SKIP: the outputs are already written when *a.skip. A kernel of its own: the test
 // costs the others 0.5 us of 40 us, an argument load to wait for.
 
-template <int K, int CHUNK, bool HAS_B>
+template <int K, int CHUNK, bool HAS_B, bool SKIP>
 __global__ __launch_bounds__(kThreads) void sf_pattern_kernel(PatternLaunch a, double2 *__restrict__ partial) {
+  if constexpr (SKIP)
+    if (all_mirrored(a.skip)) return;
   __shared__ AtomLds sm[CHUNK];
   const int split = blockIdx.y, nsplit = gridDim.y;
   const int a_begin = (int)(((long long)a.natoms * split) / nsplit);
@@ -643,6 +721,33 @@ __global__ __launch_bounds__(kThreads) void sf_pattern_kernel(PatternLaunch a, d
     const int pix = base + k * kThreads;
     if (pix < a.npix) store_pixel(pix, Fr[k], Fi[k], a.npix, split, partial, a.F, a.I);
   }
+}
+
+// sf_pattern_kernel's results, bit for bit, on an n x n list that
+// sf_mirror_check_kernel found mirror-symmetric (otherwise nothing): one quad of
+// mirrored pixels per lane, which share what their symmetry allows
+// (quad_exact_sum). Bound by VALU issue: 20,000 atoms with B on 512^2 1.54 ms,
+// 2.02 ms by sf_pattern_kernel.
+template <int CHUNK, bool HAS_B>
+__global__ __launch_bounds__(kThreads) void sf_pattern_quads_kernel(PatternLaunch a, int n,
+                                                                    double2 *__restrict__ partial) {
+  if (!all_mirrored(a.skip)) return;
+  __shared__ AtomLds sm[CHUNK];
+  const int split = blockIdx.y, nsplit = gridDim.y;
+  const int a_begin = (int)(((long long)a.natoms * split) / nsplit);
+  const int a_end = (int)(((long long)a.natoms * (split + 1)) / nsplit);
+  const int qd = blockIdx.x * kThreads + threadIdx.x;
+  const bool in = qd < grid_quads(n, n);
+  int pix[4];
+  quad_pixels(in ? qd : 0, n, n, pix[0], pix[1], pix[2], pix[3]);
+  double qx, qy, qz, Fr[4], Fi[4];
+  float s2;
+  load_q(a.hkl, pix[0], true, qx, qy, qz, s2);
+  quad_exact_sum<CHUNK, HAS_B>(qx, qy, qz, s2, a.atoms, a.atom_b, a.segs, a.nsegs, a_begin, a_end, a.ff, a.b_global,
+                               a.has_rot ? a.rot.r : nullptr, sm, Fr, Fi);
+  if (!in) return;
+#pragma unroll
+  for (int k = 0; k < 4; ++k) store_pixel(pix[k], Fr[k], Fi[k], a.npix, split, partial, a.F, a.I);
 }
 
 template <int K, int CHUNK, bool HAS_B, bool SKIP>
@@ -889,7 +994,7 @@ const void *single_kernel_ptr(Kind kind, int K, int C) {
 template <bool HAS_B>
 const void *kernel_ptr(Kind kind, int K, int C) {
 #define P(k_, c_) \
-  if (K == k_ && C == c_) return kind == Kind::kPattern ? (const void *)&sf_pattern_kernel<k_, c_, HAS_B> \
+  if (K == k_ && C == c_) return kind == Kind::kPattern ? (const void *)&sf_pattern_kernel<k_, c_, HAS_B, false> \
                                                           : (const void *)&sf_batch_kernel<k_, c_, HAS_B>;
 #define Q(k_, c_) \
   if (K == k_ && C == c_) return (const void *)&sf_batch_grid_kernel<k_, c_, HAS_B>;
@@ -951,6 +1056,26 @@ int launch_single(Kind kind, const PatternLaunch &a, int nx, int ny, const spsim
                        (const double2 *)partial, splits, a.npix, a.skip, a.F, a.I);
     SPSIM_HIP_TRY(hipGetLastError());
   }
+  return SPSIM_HIP_OK;
+}
+
+// A pattern on a flat list of n^2 vectors, by quads where it is mirror-symmetric
+// and by sf_pattern_kernel's K pixels per lane otherwise; the device looks. Both
+// use the workspace ws, past the flags.
+template <bool HAS_B>
+int launch_quads(const PatternLaunch &in, int n, int quad_tiles, int K, int tiles, int splits, void *ws, hipStream_t s) {
+  PatternLaunch a = in;
+  a.skip = (const int *)ws;
+  double2 *partial = splits > 1 ? (double2 *)((char *)ws + sizeof(int) * kMirrorBlocks) : nullptr;
+  hipLaunchKernelGGL(sf_mirror_check_kernel, dim3(kMirrorBlocks), dim3(kThreads), 0, s, a.hkl, n, (int *)ws);
+  hipLaunchKernelGGL((sf_pattern_quads_kernel<256, HAS_B>), dim3(quad_tiles, splits), dim3(kThreads), 0, s, a, n,
+                     partial);
+  hipLaunchKernelGGL((K == 2 ? sf_pattern_kernel<2, 256, HAS_B, true> : sf_pattern_kernel<1, 256, HAS_B, true>),
+                     dim3(tiles, splits), dim3(kThreads), 0, s, a, partial);
+  if (splits > 1)
+    hipLaunchKernelGGL(sf_reduce_kernel<false>, dim3((a.npix + kThreads - 1) / kThreads), dim3(kThreads), 0, s,
+                       (const double2 *)partial, splits, a.npix, (const int *)nullptr, a.F, a.I);
+  SPSIM_HIP_TRY(hipGetLastError());
   return SPSIM_HIP_OK;
 }
 
@@ -1212,6 +1337,27 @@ extern "C" int spsim_hip_sf_pattern(const float *d_hkl, int npix, const spsim_hi
                                        (int)std::min<size_t>(64, kWorkspacePartials / (size_t)npix));
   const PatternLaunch a =
       make_launch(d_hkl, npix, d_atoms, d_atom_b, d_segs, nsegs, natoms, d_ff, b_global, rot9, d_F, d_I);
+  // A list of n^2 vectors may be a square detector's. The same atom ranges keep
+  // the bits; the quads have to fill the chip in so many. A list that is not
+  // mirror-symmetric pays the check and an empty launch, 8 us, of the 1 ms and
+  // more that kQuadMinTerms take.
+  constexpr long long kQuadMinTerms = 2500000000;
+  const int side = (int)std::lround(std::sqrt((double)npix));
+  const int quad_tiles = (grid_quads(side, side) + kThreads - 1) / kThreads;
+  if (!tile && t.chunk_atoms == 256 && t.pixels_per_lane <= 2 && (long long)side * side == npix &&
+      (long long)npix * natoms >= kQuadMinTerms && (long long)quad_tiles * splits >= 2LL * cus) {
+    const size_t bytes = sizeof(int) * kMirrorBlocks + (splits > 1 ? sizeof(double2) * (size_t)splits * npix : 0);
+    // a capture cannot grow the workspace
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    if (workspace_holds(bytes) ||
+        (hipStreamIsCapturing((hipStream_t)stream, &st) == hipSuccess && st == hipStreamCaptureStatusNone)) {
+      void *ws = nullptr;
+      SPSIM_TRY(workspace(bytes, &ws));
+      return d_atom_b ? launch_quads<true>(a, side, quad_tiles, t.pixels_per_lane, tiles, splits, ws, (hipStream_t)stream)
+                      : launch_quads<false>(a, side, quad_tiles, t.pixels_per_lane, tiles, splits, ws,
+                                            (hipStream_t)stream);
+    }
+  }
   return launch_pattern(a, t, splits, (hipStream_t)stream);
 }
 

@@ -460,3 +460,31 @@ def test_sums_by_cells(gpu, shape, n, natoms, geometry, with_b, rotated):
         graph.replay()
         torch.cuda.synchronize()
         assert np.array_equal(I.cpu().numpy(), first)
+
+
+@pytest.mark.parametrize("n,natoms,with_b,rotated,geometry", [
+    (400, 16_000, True, False, {}), (401, 16_000, False, True, {}), (400, 16_001, True, True, {"cx": 1e-3}),
+    (2000, 700, True, False, {})])
+def test_flat_square_list_by_quads_keeps_the_bits(gpu, n, natoms, with_b, rotated, geometry):
+    """A large flat list of n x n vectors, mirror-symmetric (one quad per lane) or not,
+    against the same tile asked for: every bit of F and I, odd sides and one
+    atom range (2000^2) included; and with a NaN among the vectors."""
+    import torch
+
+    rng = np.random.default_rng(n + natoms)
+    Z, pos, b = wl.random_molecule(natoms, 6e-9, rng, atom_b_range=(5.0, 40.0))
+    atoms = dv.DeviceAtoms(dv.pack_atoms(Z, pos, atom_b=b if with_b else None), gpu)
+    ff = dv.form_factor_table(device=gpu)
+    R = wl.uniform_rotations(1, rng)[0] if rotated else None
+    q = _list(n, n, **geometry)
+    tile = dv.make_tile(2 if n * n >= 4 * 256 * 256 else 1, 256, 0)  # the library's default
+    for nan in (False, True):
+        if nan:
+            q = q.copy()
+            q[n * 7 + 5, 1] = np.nan
+        qs = torch.from_numpy(q).to(gpu)
+        F, I = dv.structure_factor(qs, atoms, ff, B=1.0, R=R)
+        Ft, It = dv.structure_factor(qs, atoms, ff, B=1.0, R=R, tile=tile)
+        torch.cuda.synchronize()
+        assert np.array_equal(F.cpu().numpy(), Ft.cpu().numpy(), equal_nan=True)
+        assert np.array_equal(I.cpu().numpy(), It.cpu().numpy(), equal_nan=True)
