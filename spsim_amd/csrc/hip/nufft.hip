@@ -2158,9 +2158,9 @@ bool is_rotation(const double *R) {
 // smooth enough and cheaper so than in.limit: *done. The scan's digest is in
 // h_digest and, on the device, at the workspace's start; the scan itself lies
 // `head` bytes on. A workspace without the memory leaves the patterns to the
-// grids.
+// grids. sync: s is synchronised at the end.
 int surface_patterns(const SurfInput &in, const char *h_digest, size_t head, float *d_F, float *d_I, hipStream_t s,
-                     bool *done) {
+                     bool sync, bool *done) {
   *done = false;
   SurfPlan *plan = surf_plan_choose(in, h_digest);
   if (!plan) return SPSIM_HIP_OK;
@@ -2174,9 +2174,13 @@ int surface_patterns(const SurfInput &in, const char *h_digest, size_t head, flo
     if (workspace(total, &ws) == SPSIM_HIP_OK) {
       char *w = (char *)ws;
       if (grows) rc = surf_scan(in, w + head, w, s);  // the scan went with the smaller workspace
-      if (rc == SPSIM_HIP_OK) rc = surf_plan_bind(plan, w + head, w + at, s);
+      if (rc == SPSIM_HIP_OK) rc = surf_plan_bind(plan, w + head, w + at, s, !sync);
       if (rc == SPSIM_HIP_OK) rc = surf_plan_run(plan, (float2 *)d_F, d_I, s);
       *done = rc == SPSIM_HIP_OK;
+      if (sync) {  // also after a failure: the upload reads the plan
+        const hipError_t e = hipStreamSynchronize(s);
+        if (rc == SPSIM_HIP_OK && e != hipSuccess) rc = hip_fail(e, "surface plan");
+      }
     }
   }
   surf_plan_destroy(plan);
@@ -2256,11 +2260,8 @@ int nufft_impl(const float *d_hkl, int npix, const spsim_hip_atom *d_atoms, cons
     const double limit = need.cost / nout;
     in.limit = &limit;
     bool done = false;
-    SPSIM_TRY(surface_patterns(in, h, head, d_F, d_I, s, &done));
-    if (done) {
-      if (npat > 0) SPSIM_HIP_TRY(hipStreamSynchronize(s));
-      return SPSIM_HIP_OK;
-    }
+    SPSIM_TRY(surface_patterns(in, h, head, d_F, d_I, s, npat > 0, &done));
+    if (done) return SPSIM_HIP_OK;
   }
   return nufft_run(hb, d_hkl, npix, d_atoms, d_atom_b, d_segs, nsegs, natoms, d_ff, b_global, R, npat, rots, W, eps,
                    d_F, d_I, info, s);
@@ -2778,7 +2779,7 @@ extern "C" int spsim_hip_sf_nfft_molecules(const float *d_hkl, int npix, int nmo
   int rc = SPSIM_HIP_OK;
   if (plan.p) {
     if (grows) rc = scan_surface(w);  // the scan went with the smaller workspace
-    if (rc == SPSIM_HIP_OK) rc = surf_plan_bind(plan.p, w + head, w + head + b_scan, s);
+    if (rc == SPSIM_HIP_OK) rc = surf_plan_bind(plan.p, w + head, w + head + b_scan, s, true);
     if (rc == SPSIM_HIP_OK) rc = surf_plan_run(plan.p, (float2 *)d_F, d_I, s);
   }
   for (size_t i = 0; i < rest.size() && rc == SPSIM_HIP_OK; ++i) {

@@ -1339,7 +1339,7 @@ extern "C" int spsim_hip_sf_pattern(const float *d_hkl, int npix, const spsim_hi
       make_launch(d_hkl, npix, d_atoms, d_atom_b, d_segs, nsegs, natoms, d_ff, b_global, rot9, d_F, d_I);
   // A list of n^2 vectors may be a square detector's. The same atom ranges keep
   // the bits; the quads have to fill the chip in so many. A list that is not
-  // mirror-symmetric pays the check and an empty launch, 8 us, of the 1 ms and
+  // mirror-symmetric pays the check and an empty launch, 12 us, of the 1 ms and
   // more that kQuadMinTerms take.
   constexpr long long kQuadMinTerms = 2500000000;
   const int side = (int)std::lround(std::sqrt((double)npix));

@@ -127,7 +127,7 @@ struct SurfMol {
   float b_smooth;    // largest Gaussian coefficient of the terms (form factor + B), A^2
   float weakest;     // smallest ratio of a term's amplitude at s2max to that at 0
   int bad;
-  int ordered;       // the species' segments follow each other
+  int ordered;       // the species' segments follow each other and are no more than species
 };
 
 // Host sizes only: is the pattern large enough to look at its list?
@@ -203,9 +203,10 @@ struct SurfPlan;
 // copy of a digest; null when there is none. No device work.
 SurfPlan *surf_plan_choose(const SurfInput &in, const void *digest);
 // Device memory of its own that the plan needs, and the upload of its tables
-// there. The host copy may go when surf_plan_bind returns (it waits for s).
+// there. The plan has to outlast the upload: wait for s here, or synchronise it
+// before surf_plan_destroy.
 size_t surf_plan_bytes(const SurfPlan *p);
-int surf_plan_bind(SurfPlan *p, const void *scan, void *mem, hipStream_t s);
+int surf_plan_bind(SurfPlan *p, const void *scan, void *mem, hipStream_t s, bool wait);
 
 // All of it, in device memory that the plan owns. *out is null when no pattern
 // is taken. Synchronises.

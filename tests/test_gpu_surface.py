@@ -417,11 +417,12 @@ def test_nfft_molecules_split_between_surface_and_grids(gpu, with_b, rotated):
     ("rod", (800, 800), 20_001, {"pixel": 60e-6}, True, False),
     ("dense", (720, 720), 24_000, {}, False, True),
     ("unordered", (640, 640), 30_011, {}, False, False),
+    ("pieces", (640, 640), 30_011, {}, False, False),
 ])
 def test_sums_by_cells(gpu, shape, n, natoms, geometry, with_b, rotated):
     """Large patterns, whose node sums go by cells: octants and plain nodes, atom
     counts that end within every piece, a rod (empty cells), nearly all atoms
-    in a few cells, and species that are not in order (no cells). The same bits
+    in a few cells, and species that are not in order or in many pieces (no cells). The same bits
     on every call and replay."""
     import torch
 
@@ -435,6 +436,10 @@ def test_sums_by_cells(gpu, shape, n, natoms, geometry, with_b, rotated):
     atoms = dv.DeviceAtoms(dv.pack_atoms(Z, pos, atom_b=b if with_b else None), gpu)
     if shape == "unordered":
         atoms.segs = torch.flip(atoms.segs.reshape(-1, 4), [0]).contiguous()
+    if shape == "pieces":  # more segments than species
+        pieces = [[i, min(100, int(s + c) - i), int(z), 0] for s, c, z, _ in atoms.segs.reshape(-1, 4).tolist()
+                  for i in range(int(s), int(s + c), 100)]
+        atoms.segs, atoms.nsegs = torch.tensor(pieces, dtype=torch.int32, device=gpu), len(pieces)
     R = wl.uniform_rotations(1, rng)[0] if rotated else None
     ff = dv.form_factor_table(device=gpu)
     q = _list(nx, ny, **geometry)
