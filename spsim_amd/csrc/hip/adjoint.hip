@@ -263,7 +263,7 @@ extern "C" int spsim_hip_sf_adjoint(const float *d_hkl, int npix, const spsim_hi
   // device's check catches a wrong guess, which costs its launches (60 us of
   // 350 us and more), and the direct kernel stays behind it.
   const int side = (int)std::lround(std::sqrt((double)npix));
-  const bool smooth = (long long)side * side == npix && surf_worth(side, side, natoms, 500000000LL);
+  bool smooth = (long long)side * side == npix && surf_worth(side, side, natoms, 500000000LL);
   const size_t segs_bytes = (((size_t)nsegs * sizeof(spsim_hip_segment) + 255) / 256) * 256;
   // one round of the node sums' workgroups (four resident per CU)
   const int node_splits = (int)std::max<long long>(1, std::min<long long>(32, 4LL * cus / (long long)tiles.size()));
@@ -272,7 +272,9 @@ extern "C" int spsim_hip_sf_adjoint(const float *d_hkl, int npix, const spsim_hi
   const size_t head = tiles_bytes + segs_bytes + partial_bytes + node_bytes;
   const size_t surf_at = (head + 255) / 256 * 256;
   void *ws = nullptr;
-  SPSIM_TRY(workspace(smooth ? surf_at + surf_adjoint_bytes(side, side, natoms) : head, &ws));
+  if (smooth && workspace(surf_at + surf_adjoint_bytes(side, side, natoms), &ws) != SPSIM_HIP_OK)
+    smooth = false;  // no memory for the nodes: the direct sums, which need less
+  if (!smooth) SPSIM_TRY(workspace(head - node_bytes, &ws));
   AtomTile *d_tiles = (AtomTile *)ws;
   spsim_hip_segment *d_segs = (spsim_hip_segment *)((char *)ws + tiles_bytes);
   double4 *partial = (double4 *)((char *)ws + tiles_bytes + segs_bytes);

@@ -352,10 +352,12 @@ int spsim_hip_batch_create(const float *hkl, int nx, int ny, int nmol, const int
   if (tile) b->direct = true;
   const SurfInput surf{b->hkl, nx,        ny,          b->atoms, b->atom_b, b->segs,  b->mols, b->h_mols.data(),
                        nmol,   npatterns, pattern_mol, rot9,     b->ff,     b_global, cus,     nullptr};
-  if (!tile && (rc = surf_plan_create(surf, &b->surf)) != SPSIM_HIP_OK) {
+  // without memory for it the direct kernels run every pattern
+  if (!tile && (rc = surf_plan_create(surf, &b->surf)) != SPSIM_HIP_OK && rc != SPSIM_HIP_ERR_NOMEM) {
     free_batch(b);
     return rc;
   }
+  rc = SPSIM_HIP_OK;
   const int avg_atoms = packed_total / std::max(nmol, 1);
   spsim_hip_tile t = tile ? *tile : default_tile(avg_atoms, npix, b->grid);
   if (!tile && b->square) t.pixels_per_lane = kOctantLane;

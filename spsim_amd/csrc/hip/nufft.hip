@@ -2238,7 +2238,8 @@ int nufft_impl(const float *d_hkl, int npix, const spsim_hip_atom *d_atoms, cons
   SurfInput in{d_hkl, side, side, d_atoms, d_atom_b, d_segs, nullptr, &mol, 1, nout, nullptr,
                npat > 0 ? rots : rot9, d_ff, b_global, cus, nullptr};
   void *ws = nullptr;
-  SPSIM_TRY(workspace(head + (side ? surf_scan_bytes(side, side, 1) : 0), &ws));
+  if (side && workspace(head + surf_scan_bytes(side, side, 1), &ws) != SPSIM_HIP_OK) side = 0;
+  if (!side) SPSIM_TRY(workspace(head, &ws));
   hipLaunchKernelGGL(bounds_partial, dim3(nblk), dim3(kThreads), 0, s, d_atoms, d_atom_b, natoms, d_hkl, npix, R,
                      (double *)((char *)ws + kDigest));
   SPSIM_HIP_TRY(hipGetLastError());
@@ -2675,7 +2676,8 @@ extern "C" int spsim_hip_sf_nfft_molecules(const float *d_hkl, int npix, int nmo
   int cus = 0;
   SPSIM_TRY(ensure_device(&cus));
   void *ws = nullptr;
-  SPSIM_TRY(workspace(head + b_scan, &ws));
+  bool look = side > 0 && workspace(head + b_scan, &ws) == SPSIM_HIP_OK;
+  if (!look) SPSIM_TRY(workspace(head, &ws));
   char *w = (char *)ws;
   double *qpart = (double *)(w + b_dig);
   double *part = (double *)(w + at_part);
@@ -2710,7 +2712,7 @@ extern "C" int spsim_hip_sf_nfft_molecules(const float *d_hkl, int npix, int nmo
     SPSIM_HIP_TRY(hipMemcpyAsync(base + at_mols, mols.data(), sizeof(MolInfo) * mols.size(), hipMemcpyHostToDevice, s));
     return surf_scan(in, base + head, base, s);
   };
-  if (side) SPSIM_TRY(scan_surface(w));
+  if (look) SPSIM_TRY(scan_surface(w));
   std::vector<char> h(at_off);
   SPSIM_HIP_TRY(hipMemcpyAsync(h.data(), w, total_atoms > 0 ? at_off : at_part, hipMemcpyDeviceToHost, s));
   SPSIM_HIP_TRY(hipStreamSynchronize(s));
@@ -2737,7 +2739,7 @@ extern "C" int spsim_hip_sf_nfft_molecules(const float *d_hkl, int npix, int nmo
   struct PlanOwner {
     SurfPlan *p;
     ~PlanOwner() { surf_plan_destroy(p); }
-  } plan{side ? surf_plan_choose(in, h.data()) : nullptr};
+  } plan{look ? surf_plan_choose(in, h.data()) : nullptr};
   // 3. The molecules that the plan leaves, their stages enqueued back to back
   // on kWorkers streams: the kHelperStreams streams forked from s, and s
   // itself. The i-th goes to worker i mod kWorkers, each worker with a

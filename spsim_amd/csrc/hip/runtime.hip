@@ -81,7 +81,11 @@ int workspace(size_t bytes, void **ptr) {
     }
     size_t want = bytes + bytes / 4;
     hipError_t e = hipMalloc(&st->ws, want);
-    if (e != hipSuccess) return fail(SPSIM_HIP_ERR_NOMEM, "workspace hipMalloc(%zu) failed: %s", want, hipGetErrorString(e));
+    if (e != hipSuccess) {
+      st->ws = nullptr;
+      (void)hipGetLastError();  // callers may go on with less
+      return fail(SPSIM_HIP_ERR_NOMEM, "workspace hipMalloc(%zu) failed: %s", want, hipGetErrorString(e));
+    }
     st->ws_bytes = want;
   }
   *ptr = st->ws;

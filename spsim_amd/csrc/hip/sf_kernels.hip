@@ -1131,7 +1131,8 @@ int launch_smooth(Kind kind, const PatternLaunch &a, int nx, int ny, const spsim
       return launch_single(kind, a, nx, ny, t, splits, s, spec);
   }
   void *ws = nullptr;
-  SPSIM_TRY(workspace(bytes, &ws));
+  // no memory for the interpolation: the direct kernel, which needs less
+  if (workspace(bytes, &ws) != SPSIM_HIP_OK) return launch_single(kind, a, nx, ny, t, splits, s, spec);
   PatternLaunch direct = a;
   SPSIM_TRY(launch_surface(a, nx, ny, spec, cus, ws, &direct.skip, s));
   return launch_single(kind, direct, nx, ny, t, splits, s, spec, (double2 *)((char *)ws + kFlag));
@@ -1352,7 +1353,7 @@ extern "C" int spsim_hip_sf_pattern(const float *d_hkl, int npix, const spsim_hi
     if (workspace_holds(bytes) ||
         (hipStreamIsCapturing((hipStream_t)stream, &st) == hipSuccess && st == hipStreamCaptureStatusNone)) {
       void *ws = nullptr;
-      SPSIM_TRY(workspace(bytes, &ws));
+      SPSIM_TRY(workspace(bytes, &ws));  // what launch_pattern asks for, and 256 bytes
       return d_atom_b ? launch_quads<true>(a, side, quad_tiles, t.pixels_per_lane, tiles, splits, ws, (hipStream_t)stream)
                       : launch_quads<false>(a, side, quad_tiles, t.pixels_per_lane, tiles, splits, ws,
                                             (hipStream_t)stream);

@@ -2939,8 +2939,9 @@ int surf_plan_create(const SurfInput &in, SurfPlan **out) {
   const size_t scan_bytes = surf_scan_bytes(in.nx, in.ny, in.nmol), digest_bytes = surf_digest_bytes(in.nmol);
   auto alloc = [](void **m, size_t bytes) {
     const hipError_t e = hipMalloc(m, bytes);
-    return e == hipSuccess ? SPSIM_HIP_OK
-                           : fail(SPSIM_HIP_ERR_NOMEM, "hipMalloc(%zu) failed: %s", bytes, hipGetErrorString(e));
+    if (e == hipSuccess) return SPSIM_HIP_OK;
+    (void)hipGetLastError();  // the caller may go on without the plan
+    return fail(SPSIM_HIP_ERR_NOMEM, "hipMalloc(%zu) failed: %s", bytes, hipGetErrorString(e));
   };
   void *scan = nullptr, *mem = nullptr;
   SPSIM_TRY(alloc(&scan, scan_bytes + digest_bytes));
