@@ -44,6 +44,7 @@
 #include <vector>
 
 #include "form_factor.hpp"
+#include "ranges.hpp"
 
 namespace spsim {
 
@@ -1373,8 +1374,8 @@ __global__ __launch_bounds__(kT) void surface_nodes_kernel(const SurfJob *jobs, 
                      (const NodeAtom *)jb.prep,
                      jb.segs,
                      jb.nsegs,
-                     (int)((long long)jb.natoms * m.split / jb.splits),
-                     (int)((long long)jb.natoms * (m.split + 1) / jb.splits)};
+                     range_begin(jb.natoms, m.split, jb.splits),
+                     range_begin(jb.natoms, m.split + 1, jb.splits)};
     any_item<HAS_B, SPEC, false>(w, m.tile, ff, b_global, sp, sm, [&](int e, double fc, double fs, float nc, float ns) {
       store_node(jb, m.tile, m.split, e, fc, fs, nc, ns);
     });
@@ -1551,8 +1552,8 @@ __global__ __launch_bounds__(kT, 4) void surface_cell_nodes_kernel(const SurfJob
     const SurfCell cell = c.cells[id];
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64), lane = threadIdx.x & 63;
     const int r = range - cell.range0;
-    const int begin = cell.start + cell.count * r / cell.ranges;
-    const int count = cell.start + cell.count * (r + 1) / cell.ranges - begin;
+    const int begin = cell.start + range_begin(cell.count, r, cell.ranges);
+    const int count = cell.start + range_begin(cell.count, r + 1, cell.ranges) - begin;
     const int nxn = c.co.ax.n, nyn = c.co.ay.n;
     const NodeWork w{c.co.nodes,
                      nxn,
@@ -1561,8 +1562,8 @@ __global__ __launch_bounds__(kT, 4) void surface_cell_nodes_kernel(const SurfJob
                      (const NodeAtom *)c.sorted,
                      c.segs + (size_t)id * jb.nsegs,
                      jb.nsegs,
-                     begin + count * wave / kWaves,
-                     begin + count * (wave + 1) / kWaves};
+                     begin + range_begin(count, wave, kWaves),
+                     begin + range_begin(count, wave + 1, kWaves)};
     NoSpectrum none;
     double fc[8] = {}, fs[8] = {};
     float nc[8] = {}, ns[8] = {};
