@@ -28,9 +28,12 @@
  * SPSIM_HIP_OK or a negative error code and never exits the process;
  * spsim_hip_last_error() describes the last failure on the calling thread.
  * Calls are stream-ordered and asynchronous unless stated otherwise. Entry
- * points that use "the library workspace" share one device buffer per GPU:
- * such calls on different streams must not overlap (issue them on one stream,
- * or synchronise between them); growing the buffer synchronises the device.
+ * points that use "the library workspace" share one device buffer per GPU and
+ * follow each other there, from any threads and streams: the later call's stream
+ * waits on the device for the earlier call's work, without the host. (The replays
+ * of a graph that such a call was captured into are not ordered in this way: they
+ * must not overlap other calls that use the workspace.) Growing the buffer
+ * synchronises the device.
  */
 #ifndef SPSIM_HIP_H
 #define SPSIM_HIP_H 1
@@ -121,9 +124,10 @@ int spsim_hip_hkl_detector_3d(int nx, int ny, int nz, float width, float height,
    kernels apply it exactly, in FP64, as R^T to the atoms. d_atom_b may be NULL
    (no per-atom Debye-Waller factor). d_F ([npix][2]) or d_I may be NULL. The
    nsegs segments must tile the packed atoms [0, natoms) in order (as
-   spsim_hip_pack_atoms writes them). tile may be NULL (default tiling). Uses a
-   library-owned device workspace when atom_splits > 1 (grown on demand, kept
-   until spsim_hip_release). */
+   spsim_hip_pack_atoms writes them). tile may be NULL (default tiling). Uses the
+   library workspace (grown on demand, kept until spsim_hip_release) for the
+   partial sums of several atom ranges, and, with tile == NULL, on lists of n^2
+   vectors and 2.5e9 terms or more for what the list's check found. */
 int spsim_hip_sf_pattern(const float *d_hkl, int npix, const spsim_hip_atom *d_atoms, const float *d_atom_b,
                          const spsim_hip_segment *d_segs, int nsegs, int natoms, const float *d_ff,
                          float b_global, const double *rot9, float *d_F, float *d_I, const spsim_hip_tile *tile,
@@ -286,8 +290,6 @@ int spsim_hip_sf_spectrum_nfft(const float *d_hkl, int npix, const spsim_hip_ato
    molecules. They run on `stream` and on 31 library-owned streams forked
    from it and joined back into it (work enqueued on `stream` afterwards runs
    after every pattern), each stream with its own slice of the library
-   workspace. Calls
-   that overlap on one device race, as for every entry point sharing the
    workspace. Same grids and accuracy as spsim_hip_sf_nfft; molecules that
    are cheaper by interpolation over a square detector's surface go that way,
    as in spsim_hip_sf_nfft_batch. */

@@ -234,6 +234,7 @@ extern "C" int spsim_hip_sf_adjoint(const float *d_hkl, int npix, const spsim_hi
   SPSIM_TRY(ensure_device(&cus));
   hipStream_t s = (hipStream_t)stream;
   if (natoms == 0) return SPSIM_HIP_OK;
+  WorkspaceUse use(s);
   constexpr int KA = kSurfAtomsPerLane;
   const int per_tile = kT * KA;
   std::vector<AtomTile> tiles;
@@ -325,6 +326,7 @@ extern "C" int spsim_hip_poisson_nll(const float *d_I, const float *d_y, const f
     return SPSIM_HIP_OK;
   }
   const int nb = (npix + kT - 1) / kT;
+  WorkspaceUse use(s);
   void *ws = nullptr;
   SPSIM_TRY(workspace(sizeof(double) * (size_t)nb, &ws));
   hipLaunchKernelGGL(nll_kernel, dim3(nb), dim3(kT), 0, s, d_I, d_y, d_K, npix, (double *)ws, d_gI);

@@ -17,8 +17,9 @@ namespace spsim {
 namespace {
 
 // What a call works with. Sessions are handed out one per call, so calls of
-// several threads never share one; idle ones wait in a list of at most
-// kMaxIdle, their buffers at most kKeepBytes each, until spsim_hip_release.
+// several threads never share one (they still follow each other where the entry
+// points that they call use the library workspace); idle ones wait in a list of
+// at most kMaxIdle, their buffers at most kKeepBytes each, until spsim_hip_release.
 struct Session {
   int device = -1;
   hipStream_t s = nullptr;

@@ -625,6 +625,7 @@ int launch_chain_bin_draws(const DetConst &d, const float *I, int npatterns, uin
   // the mark words (real output only): from the library workspace
   const long long nw = (nb + 63) / 64, nwords = nw * npatterns;
   unsigned long long *marks = nullptr;
+  WorkspaceUse use(s);
   if (real) {
     void *ws = nullptr;
     SPSIM_TRY(workspace(sizeof(unsigned long long) * (size_t)nwords, &ws));

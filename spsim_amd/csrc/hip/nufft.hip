@@ -2197,6 +2197,7 @@ int nufft_impl(const float *d_hkl, int npix, const spsim_hip_atom *d_atoms, cons
     return fail(SPSIM_HIP_ERR_INVALID, "NULL input pointer");
   if (npat > 0 && !rots) return fail(SPSIM_HIP_ERR_INVALID, "NULL rotations");
   SPSIM_TRY(ensure_device(nullptr));
+  WorkspaceUse use(s);
   const int W = width_for(eps);
   AtomRot R{};
   if (rot9) {
@@ -2656,6 +2657,7 @@ extern "C" int spsim_hip_sf_nfft_molecules(const float *d_hkl, int npix, int nmo
         if (!std::isfinite(rot9s[9 * (size_t)m + i])) return fail(SPSIM_HIP_ERR_INVALID, "non-finite rotation");
   }
   SPSIM_TRY(ensure_device(nullptr));
+  WorkspaceUse use(s);
   const int W = width_for(eps);
   // 1. Bounds: the q list's once (every molecule shares it) and every
   // molecule's atoms in one launch, and the look at the list's surface, read
@@ -2826,6 +2828,7 @@ extern "C" int spsim_hip_fft_pruned(const float *d_in, long long outer, long lon
   D.nf = nf;
   D.L = L;
   D.l_lo = l_lo;
+  WorkspaceUse use((hipStream_t)stream);
   void *ws = nullptr;
   SPSIM_TRY(workspace(sizeof(float2) * (size_t)nf, &ws));
   SPSIM_TRY(launch_twiddles(nf, (float2 *)ws, (hipStream_t)stream));

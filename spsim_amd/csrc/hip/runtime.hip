@@ -17,8 +17,7 @@ constexpr int kMaxDevices = 64;
 struct DeviceState {
   int checked = 0;  // 0 = not yet, 1 = ok, -1 = unusable
   int cus = 0;
-  void *ws = nullptr;
-  size_t ws_bytes = 0;
+  SharedWorkspace<WorkspaceApi> ws;
   int helpers = 0;  // 1 once hs and ev exist
   hipStream_t hs[kHelperStreams] = {};
   hipEvent_t ev[kHelperStreams + 1] = {};
@@ -67,34 +66,61 @@ int ensure_device(int *cus) {
   return SPSIM_HIP_OK;
 }
 
-int workspace(size_t bytes, void **ptr) {
-  int dev = 0;
-  DeviceState *st = state_for_current(&dev);
+bool WorkspaceApi::alloc(void **ptr, size_t bytes) {
+  if (hipMalloc(ptr, bytes) == hipSuccess) return true;
+  (void)hipGetLastError();  // callers may go on with less
+  return false;
+}
+void WorkspaceApi::free(void *ptr) { (void)hipFree(ptr); }
+bool WorkspaceApi::synchronize() { return hipDeviceSynchronize() == hipSuccess; }
+bool WorkspaceApi::capturing(hipStream_t s) {
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(s, &st) == hipSuccess) return st != hipStreamCaptureStatusNone;
+  (void)hipGetLastError();  // the default stream beside a capture: as good as captured itself
+  return true;
+}
+bool WorkspaceApi::lasting(hipStream_t s) { return s == nullptr; }
+bool WorkspaceApi::record(hipEvent_t *e, hipStream_t s) {
+  if ((*e || hipEventCreateWithFlags(e, hipEventDisableTiming) == hipSuccess) && hipEventRecord(*e, s) == hipSuccess)
+    return true;
+  (void)hipGetLastError();
+  return false;
+}
+bool WorkspaceApi::wait(hipStream_t s, hipEvent_t e) { return hipStreamWaitEvent(s, e, 0) == hipSuccess; }
+
+namespace {
+thread_local WorkspaceUse *g_use = nullptr;
+
+// The calling thread's use, with the current device's workspace.
+int acquire(WorkspaceUse **use) {
+  DeviceState *st = state_for_current(nullptr);
   if (!st) return fail(SPSIM_HIP_ERR_NODEVICE, "no HIP device is available");
-  if (st->ws_bytes < bytes) {
-    if (st->ws) {
-      // The previous workspace may still be in use by queued work on any stream.
-      SPSIM_HIP_TRY(hipDeviceSynchronize());
-      SPSIM_HIP_TRY(hipFree(st->ws));
-      st->ws = nullptr;
-      st->ws_bytes = 0;
-    }
-    size_t want = bytes + bytes / 4;
-    hipError_t e = hipMalloc(&st->ws, want);
-    if (e != hipSuccess) {
-      st->ws = nullptr;
-      (void)hipGetLastError();  // callers may go on with less
-      return fail(SPSIM_HIP_ERR_NOMEM, "workspace hipMalloc(%zu) failed: %s", want, hipGetErrorString(e));
-    }
-    st->ws_bytes = want;
-  }
-  *ptr = st->ws;
+  if (!g_use) return fail(SPSIM_HIP_ERR_HIP, "the workspace was asked for outside a call that shares it");
+  if (!g_use->acquire(&st->ws)) return fail(SPSIM_HIP_ERR_HIP, "waiting for the workspace failed");
+  *use = g_use;
   return SPSIM_HIP_OK;
+}
+}  // namespace
+
+WorkspaceUse::WorkspaceUse(hipStream_t s) : Use(s), outer_(g_use) { g_use = this; }
+WorkspaceUse::~WorkspaceUse() { g_use = outer_; }
+
+int workspace(size_t bytes, void **ptr) {
+  WorkspaceUse *use = nullptr;
+  SPSIM_TRY(acquire(&use));
+  switch (use->get(bytes, ptr)) {
+    case WorkspaceResult::kOk:
+      return SPSIM_HIP_OK;
+    case WorkspaceResult::kNoMemory:
+      return fail(SPSIM_HIP_ERR_NOMEM, "no memory for a workspace of %zu bytes", bytes);
+    default:
+      return fail(SPSIM_HIP_ERR_HIP, "the workspace cannot grow: the device could not be synchronised");
+  }
 }
 
 bool workspace_holds(size_t bytes) {
-  DeviceState *st = state_for_current(nullptr);
-  return st && st->ws_bytes >= bytes;
+  WorkspaceUse *use = nullptr;
+  return acquire(&use) == SPSIM_HIP_OK && use->holds(bytes);
 }
 
 int helper_streams(hipStream_t streams[kHelperStreams], hipEvent_t events[kHelperStreams + 1]) {
@@ -114,13 +140,8 @@ int helper_streams(hipStream_t streams[kHelperStreams], hipEvent_t events[kHelpe
 }
 
 void workspace_release() {
-  int dev = 0;
-  DeviceState *st = state_for_current(&dev);
-  if (!st || !st->ws) return;
-  (void)hipDeviceSynchronize();
-  (void)hipFree(st->ws);
-  st->ws = nullptr;
-  st->ws_bytes = 0;
+  DeviceState *st = state_for_current(nullptr);
+  if (st) st->ws.release();
 }
 
 }  // namespace spsim

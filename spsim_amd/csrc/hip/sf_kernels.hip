@@ -1326,6 +1326,7 @@ extern "C" int spsim_hip_sf_pattern(const float *d_hkl, int npix, const spsim_hi
   int cus = 0;
   SPSIM_TRY(ensure_device(&cus));
   if (npix == 0) return SPSIM_HIP_OK;
+  WorkspaceUse use((hipStream_t)stream);
   const spsim_hip_tile t = tile ? *tile : default_tile(natoms, npix, false);
   if (!tile_supported(t, false))
     return fail(SPSIM_HIP_ERR_INVALID, "unsupported tile (pixels_per_lane=%d waves=%d chunk_atoms=%d)",
@@ -1438,6 +1439,7 @@ extern "C" int spsim_hip_sf_grid(const float *d_hkl, int nx, int ny, const spsim
   SPSIM_TRY(grid_setup(d_hkl, nx, ny, d_atoms, d_atom_b != nullptr, d_segs, nsegs, natoms, d_ff, tile,
                        kWorkspacePartials, &t, &splits, &explicit_splits, &npix));
   if (npix == 0) return SPSIM_HIP_OK;
+  WorkspaceUse use((hipStream_t)stream);
   int cus = 0;
   SPSIM_TRY(ensure_device(&cus));
   const PatternLaunch a =
@@ -1488,6 +1490,7 @@ extern "C" int spsim_hip_sf_spectrum(const float *d_hkl, int npix, const spsim_h
   int cus = 0;
   SPSIM_TRY(ensure_device(&cus));
   if (npix == 0) return SPSIM_HIP_OK;
+  WorkspaceUse use((hipStream_t)stream);
   spsim_hip_tile t = tile ? *tile : default_tile(natoms, npix, true);
   // two pixels per lane share the atom loads and loop overhead (3 % on a
   // 512 x 512 detector); smaller lists keep one for more workgroups
