@@ -30,10 +30,11 @@
  * Calls are stream-ordered and asynchronous unless stated otherwise. Entry
  * points that use "the library workspace" share one device buffer per GPU and
  * follow each other there, from any threads and streams: the later call's stream
- * waits on the device for the earlier call's work, without the host. (The replays
- * of a graph that such a call was captured into are not ordered in this way: they
- * must not overlap other calls that use the workspace.) Growing the buffer
- * synchronises the device.
+ * waits on the device for the earlier call's work, without the host. Growing the
+ * buffer synchronises the device. A call that is captured into a graph needs a
+ * buffer that an earlier call has grown; the graph then holds its address, which
+ * stays valid until spsim_hip_release. Replays are not ordered with other calls
+ * that use the workspace: they must not overlap them, nor each other.
  */
 #ifndef SPSIM_HIP_H
 #define SPSIM_HIP_H 1
@@ -127,7 +128,8 @@ int spsim_hip_hkl_detector_3d(int nx, int ny, int nz, float width, float height,
    spsim_hip_pack_atoms writes them). tile may be NULL (default tiling). Uses the
    library workspace (grown on demand, kept until spsim_hip_release) for the
    partial sums of several atom ranges, and, with tile == NULL, on lists of n^2
-   vectors and 2.5e9 terms or more for what the list's check found. */
+   vectors and 2.5e9 terms or more for what the list's check found (while the
+   stream is being captured only beside such partial sums). */
 int spsim_hip_sf_pattern(const float *d_hkl, int npix, const spsim_hip_atom *d_atoms, const float *d_atom_b,
                          const spsim_hip_segment *d_segs, int nsegs, int natoms, const float *d_ff,
                          float b_global, const double *rot9, float *d_F, float *d_I, const spsim_hip_tile *tile,
@@ -152,7 +154,8 @@ int spsim_hip_sf_pattern(const float *d_hkl, int npix, const spsim_hip_atom *d_a
    own rounding), when the list and the molecule are smooth enough for it; the
    device checks both, and everything else takes the direct sum. Such a call
    uses the library workspace (about 100 MiB at 1024 x 1024); while the stream
-   is being captured it does so only if the workspace is already that large. */
+   is being captured it does so only if the workspace is already that large and the
+   direct sum would hold partial sums of several atom ranges there. */
 int spsim_hip_sf_grid(const float *d_hkl, int nx, int ny, const spsim_hip_atom *d_atoms, const float *d_atom_b,
                       const spsim_hip_segment *d_segs, int nsegs, int natoms, const float *d_ff, float b_global,
                       const double *rot9, float *d_F, float *d_I, const spsim_hip_tile *tile, void *stream);
@@ -308,7 +311,9 @@ int spsim_hip_sf_nfft_molecules(const float *d_hkl, int npix, int nmol, const sp
 int spsim_hip_fft_pruned(const float *d_in, long long outer, long long inner, int M, int m_lo, int nf, int L,
                          int l_lo, float *d_out, void *stream);
 
-/* Free the library's cached device workspace and graphs on the current device. */
+/* Free the library's cached device workspace and graphs on the current device.
+   Graphs that calls using the workspace were captured into must not be replayed
+   any more. */
 int spsim_hip_release(void);
 
 /* ---- Batched persistent launch over many molecules and orientations ---- */

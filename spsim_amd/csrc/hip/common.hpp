@@ -44,6 +44,7 @@ class WorkspaceUse : public SharedWorkspace<WorkspaceApi>::Use {
 };
 int workspace(size_t bytes, void **ptr);
 bool workspace_holds(size_t bytes);  // workspace(bytes) would not have to grow it
+bool workspace_captured();  // the call's stream is being captured, which cannot grow it
 void workspace_release();
 // Frees the idle buffers and streams of the host-array bridge on the current device.
 void bridge_release();

@@ -139,6 +139,11 @@ int helper_streams(hipStream_t streams[kHelperStreams], hipEvent_t events[kHelpe
   return SPSIM_HIP_OK;
 }
 
+bool workspace_captured() {
+  WorkspaceUse *use = nullptr;
+  return acquire(&use) != SPSIM_HIP_OK || use->capturing();
+}
+
 void workspace_release() {
   DeviceState *st = state_for_current(nullptr);
   if (st) st->ws.release();

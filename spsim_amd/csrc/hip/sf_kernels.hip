@@ -1124,12 +1124,11 @@ int launch_smooth(Kind kind, const PatternLaunch &a, int nx, int ny, const spsim
   if (!surf_worth(nx, ny, a.natoms, min_terms)) return launch_single(kind, a, nx, ny, t, splits, s, spec);
   constexpr size_t kFlag = (sizeof(SurfJob) + 255) / 256 * 256;
   const size_t bytes = std::max(surf_single_bytes(nx, ny, a.natoms, a.nsegs), kFlag + sizeof(double2) * (size_t)splits * a.npix);
-  if (!workspace_holds(bytes)) {
-    // A capture cannot grow the workspace: it takes the direct kernel, as long as that one's partials fit.
-    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-    if (hipStreamIsCapturing(s, &st) != hipSuccess || st != hipStreamCaptureStatusNone)
-      return launch_single(kind, a, nx, ny, t, splits, s, spec);
-  }
+  // A capture cannot grow the workspace, and its graph names the workspace only
+  // where the direct kernel's partials would be there as well: otherwise it takes
+  // the direct kernel.
+  if (workspace_captured() && (splits == 1 || !workspace_holds(bytes)))
+    return launch_single(kind, a, nx, ny, t, splits, s, spec);
   void *ws = nullptr;
   // no memory for the interpolation: the direct kernel, which needs less
   if (workspace(bytes, &ws) != SPSIM_HIP_OK) return launch_single(kind, a, nx, ny, t, splits, s, spec);
@@ -1349,10 +1348,8 @@ extern "C" int spsim_hip_sf_pattern(const float *d_hkl, int npix, const spsim_hi
   if (!tile && t.chunk_atoms == 256 && t.pixels_per_lane <= 2 && (long long)side * side == npix &&
       (long long)npix * natoms >= kQuadMinTerms && (long long)quad_tiles * splits >= 2LL * cus) {
     const size_t bytes = sizeof(int) * kMirrorBlocks + (splits > 1 ? sizeof(double2) * (size_t)splits * npix : 0);
-    // a capture cannot grow the workspace
-    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
-    if (workspace_holds(bytes) ||
-        (hipStreamIsCapturing((hipStream_t)stream, &st) == hipSuccess && st == hipStreamCaptureStatusNone)) {
+    // as in launch_smooth
+    if (!workspace_captured() || (splits > 1 && workspace_holds(bytes))) {
       void *ws = nullptr;
       SPSIM_TRY(workspace(bytes, &ws));  // what launch_pattern asks for, and 256 bytes
       return d_atom_b ? launch_quads<true>(a, side, quad_tiles, t.pixels_per_lane, tiles, splits, ws, (hipStream_t)stream)

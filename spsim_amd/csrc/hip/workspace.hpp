@@ -9,6 +9,9 @@
 // interpolated pattern became 75.5), so on a stream that never ends, where it can
 // be recorded later, it is only recorded once another stream's call comes.
 //
+// A graph keeps the addresses that were captured: a buffer that a captured call was
+// given outlives its replacement by a larger one, until release().
+//
 // Api: types Stream and Event, and static functions
 //   bool alloc(void **, size_t), void free(void *), bool synchronize() (the device),
 //   bool capturing(Stream), bool lasting(Stream) (it exists until the process ends,
@@ -18,6 +21,7 @@
 
 #include <cstddef>
 #include <mutex>
+#include <new>
 
 namespace spsim {
 
@@ -55,11 +59,11 @@ class SharedWorkspace {
 
     bool holds(size_t bytes) const { return ws_->bytes_ >= bytes; }
 
-    // At least `bytes` of the buffer, which grows if it has to (all work on the
-    // device has then ended).
+    // At least `bytes` of the buffer, which is replaced by a larger one if it has to
+    // grow (all work on the device has then ended).
     WorkspaceResult get(size_t bytes, void **ptr) {
       if (ws_->bytes_ < bytes) {
-        if (!ws_->clear()) return WorkspaceResult::kFailed;
+        if (!ws_->retire()) return WorkspaceResult::kFailed;
         void *p = nullptr;
         const size_t want = bytes + bytes / 4;
         if (!Api::alloc(&p, want)) return WorkspaceResult::kNoMemory;
@@ -68,6 +72,7 @@ class SharedWorkspace {
       }
       *ptr = ws_->ptr_;
       used_ = true;
+      ws_->captured_ = ws_->captured_ || capturing_;
       return WorkspaceResult::kOk;
     }
 
@@ -87,10 +92,17 @@ class SharedWorkspace {
     bool capturing_ = false, used_ = false;
   };
 
-  // Frees the buffer.
+  // Frees the buffer, and those that graphs may still name.
   void release() {
     std::lock_guard<std::mutex> lk(mu_);
-    (void)clear();
+    captured_ = false;
+    if (!retire()) return;
+    while (kept_) {
+      Kept *k = kept_;
+      kept_ = k->next;
+      Api::free(k->ptr);
+      delete k;
+    }
   }
 
  private:
@@ -104,17 +116,29 @@ class SharedWorkspace {
     else if (Api::synchronize())
       last_ = Last::kNone;
   }
-  bool clear() {
+  struct Kept {
+    void *ptr;
+    Kept *next;
+  };
+
+  // Leaves no buffer: it is freed, or kept if a graph may name it.
+  bool retire() {
     if (!ptr_) return true;
     if (!Api::synchronize()) return false;
-    Api::free(ptr_);
+    if (!captured_)
+      Api::free(ptr_);
+    else if (Kept *k = new (std::nothrow) Kept{ptr_, kept_})  // without it the buffer stays until the process ends
+      kept_ = k;
     ptr_ = nullptr;
     bytes_ = 0;
+    captured_ = false;
     return true;
   }
   std::mutex mu_;
   void *ptr_ = nullptr;
   size_t bytes_ = 0;
+  bool captured_ = false;
+  Kept *kept_ = nullptr;
   Last last_ = Last::kNone;
   Stream open_{};
   typename Api::Event done_{};

@@ -129,3 +129,63 @@ def test_threads_share_the_workspace(gpu):
     assert not failed
     for (F, I), (Fw, Iw) in zip(got, want):
         assert torch.equal(F, Fw) and torch.equal(I, Iw)
+
+
+def _replays(graph, F, I, want, between):
+    import torch
+
+    for _ in range(3):
+        F.fill_(float("nan"))
+        I.fill_(float("nan"))
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(F, want[0]) and torch.equal(I, want[1])
+        between()
+        torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize("kind,n,natoms", [("grid", 1500, 400), ("pattern", 2600, 400), ("spectrum", 1024, 300)])
+def test_captured_calls_of_one_atom_range_need_no_workspace(gpu, kind, n, natoms):
+    """They take the direct kernels, as with an explicit tile, and their graphs
+    replay after the library's buffers are released."""
+    import torch
+
+    run, npix = _input(gpu, kind, n, natoms, 1)
+    eager = _alone(gpu, run, npix)  # the workspace is large enough
+    F, I = _outputs(gpu, npix)
+    stream, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=stream):
+        run(torch.cuda.current_stream(), F, I)
+    _lib.load().spsim_hip_release()
+    graph.replay()
+    torch.cuda.synchronize()
+    direct = F.clone(), I.clone()
+    close = float(torch.linalg.norm(eager[1] - I) / torch.linalg.norm(I))
+    assert torch.equal(eager[1], I) if kind == "pattern" else 0 < close < 8e-7
+    _replays(graph, F, I, direct, lambda: _alone(gpu, run, npix))
+
+
+def test_captured_workspace_outlives_growth(gpu):
+    """A graph's calls of several atom ranges keep their buffer when a later call
+    needs a larger one."""
+    import torch
+
+    run, npix = _input(gpu, "grid", 512, 4_000, 1)
+    large, large_pix = _input(gpu, "grid", 1600, 3_000, 2)
+    _lib.load().spsim_hip_release()
+    want = _alone(gpu, run, npix)
+    F, I = _outputs(gpu, npix)
+    stream, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=stream):
+        run(torch.cuda.current_stream(), F, I)
+    before = torch.cuda.mem_get_info()[0]
+    F2, I2 = _outputs(gpu, large_pix)
+    large(None, F2, I2)
+    torch.cuda.synchronize()
+    assert torch.cuda.mem_get_info()[0] < before  # the buffer has grown
+    ones = torch.ones(64 << 20, dtype=torch.float32, device=gpu)  # would take up what was freed
+    _replays(graph, F, I, want, lambda: (large(None, F2, I2), ones.fill_(1.0)))
+    assert bool((ones == 1.0).all())
+    del graph
+    _lib.load().spsim_hip_release()

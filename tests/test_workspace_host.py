@@ -97,6 +97,26 @@ def test_a_capture_neither_waits_nor_records(tmp_path):
   ws.release();""") == ["alloc125", "work", "record1", "work", "wait3for1", "work", "record3", "sync", "free"]
 
 
+def test_a_captured_buffer_outlives_growth(tmp_path):
+    """It is kept through larger ones, eager or captured, until the release; a
+    buffer that no capture was given is freed at once."""
+    assert _run(tmp_path, """
+  use(ws, 1, 100);
+  use(ws, 1, 200);
+  capture[2] = true;
+  use(ws, 2, 200);
+  use(ws, 1, 400);
+  use(ws, 2, 400);
+  use(ws, 1, 800);
+  use(ws, 1, 2000);
+  ws.release();
+  use(ws, 1, 100);
+  ws.release();""") == ["alloc125", "work", "record1", "wait1for1", "sync", "free", "alloc250", "work", "record1",
+                        "work", "wait1for1", "sync", "alloc500", "work", "record1", "work", "wait1for1", "sync",
+                        "alloc1000", "work", "record1", "wait1for1", "sync", "free", "alloc2500", "work", "record1",
+                        "sync", "free", "free", "free", "wait1for1", "alloc125", "work", "record1", "sync", "free"]
+
+
 def test_growth_and_no_memory(tmp_path):
     """Growth frees the old buffer after the device is idle. Without memory for
     the larger one there is none, and the same call goes on with a smaller one."""
