@@ -839,6 +839,7 @@ __device__ void fold_records(const SurfRecord *list, int nlist, const SurfRecord
   double e[3] = {0.0, 0.0, 0.0};  // Gaussian, -weakest, no order for cells
   for (int i = t; i < nsegs; i += kT) {
     if (segs[i].count < 0 || (i > 0 && segs[i].start < segs[i - 1].start + segs[i - 1].count)) e[2] = 1.0;
+    if (segs[i].count <= 0) continue;  // no atom of it: the sums never look at its species
     const int sp = segs[i].species;
     species_terms(ff + sp * SPSIM_HIP_FF_STRIDE, sp == SPSIM_HIP_UNIT_SPECIES ? 0.0f : b_global,
                   has_b ? (float)-m[2] : 0.0f, has_b ? (float)m[3] : 0.0f, s2max, &bs, &weak);

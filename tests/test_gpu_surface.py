@@ -493,3 +493,32 @@ def test_flat_square_list_by_quads_keeps_the_bits(gpu, n, natoms, with_b, rotate
         torch.cuda.synchronize()
         assert np.array_equal(F.cpu().numpy(), Ft.cpu().numpy(), equal_nan=True)
         assert np.array_equal(I.cpu().numpy(), It.cpu().numpy(), equal_nan=True)
+
+
+@pytest.mark.parametrize("entry", ["grid", "spectrum", "nfft"])
+def test_empty_segments_change_nothing(gpu, entry):
+    """A segment without atoms does not take part in the choice of path, whatever
+    its species' form factor."""
+    import torch
+
+    rng = np.random.default_rng(41)
+    n, natoms = 256, 6_000
+    Z, pos, _ = wl.random_molecule(natoms, 4e-9, rng)
+    table = dv.default_form_factors().copy()
+    table[98] = np.nan
+    ff, q = dv.form_factor_table(table, device=gpu), torch.from_numpy(_list(n, n)).to(gpu)
+    sc, w = dv.spectrum_samples(0.2e-9, 0.02, 5)
+    got = []
+    for empty in (False, True):
+        atoms = dv.DeviceAtoms(dv.pack_atoms(Z, pos), gpu)
+        if empty:
+            last = torch.tensor([[natoms, 0, 98, 0]], dtype=torch.int32, device=gpu)
+            atoms.segs, atoms.nsegs = torch.cat([atoms.segs.reshape(-1, 4), last]).contiguous(), atoms.nsegs + 1
+        if entry == "grid":
+            got.append(dv.structure_factor_grid(q, n, n, atoms, ff)[1])
+        elif entry == "spectrum":
+            got.append(dv.structure_factor_spectrum(q, atoms, ff, sc, w)[1])
+        else:
+            got.append(dv.structure_factor_nfft(q, atoms, ff)[1])
+    torch.cuda.synchronize()
+    assert bool(torch.isfinite(got[0]).all()) and torch.equal(got[0], got[1])
