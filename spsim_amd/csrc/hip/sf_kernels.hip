@@ -1123,7 +1123,8 @@ int launch_smooth(Kind kind, const PatternLaunch &a, int nx, int ny, const spsim
                   long long min_terms, const Spectrum *spec, hipStream_t s) {
   if (!surf_worth(nx, ny, a.natoms, min_terms)) return launch_single(kind, a, nx, ny, t, splits, s, spec);
   constexpr size_t kFlag = (sizeof(SurfJob) + 255) / 256 * 256;
-  const size_t bytes = std::max(surf_single_bytes(nx, ny, a.natoms, a.nsegs), kFlag + sizeof(double2) * (size_t)splits * a.npix);
+  const size_t bytes = std::max(surf_single_bytes(nx, ny, a.natoms, a.nsegs, spec != nullptr),
+                                kFlag + sizeof(double2) * (size_t)splits * a.npix);
   // A capture cannot grow the workspace, and its graph names the workspace only
   // where the direct kernel's partials would be there as well: otherwise it takes
   // the direct kernel.

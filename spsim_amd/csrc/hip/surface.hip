@@ -413,7 +413,7 @@ __device__ void scan_atoms(const ScanArgs &a) {
     for (int k = 0; k < 3; ++k) a.centres[3 * mol + k] = c[k];
   // |r - r0|^2, -B, B, not finite
   double m[4] = {0.0, -3.4e38, -3.4e38, fabs(c[0]) + fabs(c[1]) + fabs(c[2]) < 1e30 ? 0.0 : 1.0};
-  for (int j = part * kT + t; j < n; j += kSurfAtomBlocks * kT) {
+  for (long long j = part * kT + t; j < n; j += kSurfAtomBlocks * kT) {
     const spsim_hip_atom at = atoms[j];
     const double x = at.x - c[0], y = at.y - c[1], z = at.z - c[2];
     const double d2 = x * x + y * y + z * z;
@@ -532,7 +532,7 @@ __device__ __forceinline__ int cell_index(double x, double extent, int g) {
 __device__ __forceinline__ void prepare_atoms(const SurfJob &jb, bool has_b, int first, int step) {
   NodeAtom *out = (NodeAtom *)jb.prep;
   const SurfCells &c = jb.c;
-  for (int j = first; j < jb.natoms; j += step) {
+  for (long long j = first; j < jb.natoms; j += step) {
     const spsim_hip_atom at = jb.atoms[j];
     const double x = at.x - jb.r0[0], y = at.y - jb.r0[1], z = at.z - jb.r0[2];
     NodeAtom r;
@@ -2197,7 +2197,7 @@ constexpr int kSlotSlack = 2 * kSurfMaxNodes + 8 * kT;
 struct SingleLayout {
   int max_nx, max_ny, slot_cap;
   size_t fit, records, centres, job, dev, nodes, tx, ty, tx32, ty32, prep, f, n, slot_f, slot_n, t64, t32, total;
-  // sums by cells, for large patterns
+  // sums by cells, for large patterns (not of spectra)
   int cells;
   long long cell_sums, cell_rows;
   size_t c_nodes, c_wx, c_wy, c_id, c_sorted, c_cells, c_segs, c_range, c_order, c_f, c_n, c_tf, c_tn;
@@ -2209,7 +2209,8 @@ constexpr long long kCellMinTerms = 10000000000;
 // Ranges and cells hold at most these for one pattern.
 constexpr long long kCellSums = 4 << 20, kCellRows = 4 << 20;
 
-SingleLayout single_layout(int nx, int ny, int natoms, int nsegs, bool adjoint) {
+SingleLayout single_layout(int nx, int ny, int natoms, int nsegs, SurfKind kind) {
+  const bool adjoint = kind == SurfKind::kAdjoint;
   SingleLayout l;
   auto cap = [](int n) { return std::max(kSurfMinNodes, std::min(kSurfMaxNodes, (int)(0.6 * n) / 4 * 4)); };
   l.max_nx = cap(nx);
@@ -2240,7 +2241,7 @@ SingleLayout single_layout(int nx, int ny, int natoms, int nsegs, bool adjoint) 
   l.slot_n = take(adjoint ? 0 : sizeof(float2) * (size_t)l.slot_cap);
   l.t64 = take(sizeof(double2) * rows);
   l.t32 = take(sizeof(float4) * rows);
-  l.cells = !adjoint && (long long)npix * natoms >= kCellMinTerms ? kMaxCells : 0;
+  l.cells = kind == SurfKind::kSum && (long long)npix * natoms >= kCellMinTerms ? kMaxCells : 0;
   l.cell_sums = l.cell_rows = 0;
   if (l.cells > 0) {
     l.cell_sums = kCellSums;
@@ -2327,8 +2328,8 @@ bool surf_worth(long long nx, long long ny, long long natoms, long long min_term
   return nx >= kSurfMinSide && ny >= kSurfMinSide && nx * ny * natoms >= min_terms;
 }
 
-size_t surf_single_bytes(int nx, int ny, int natoms, int nsegs) {
-  return single_layout(nx, ny, natoms, nsegs, false).total;
+size_t surf_single_bytes(int nx, int ny, int natoms, int nsegs, bool spectrum) {
+  return single_layout(nx, ny, natoms, nsegs, spectrum ? SurfKind::kSpectrum : SurfKind::kSum).total;
 }
 
 namespace {
@@ -2369,7 +2370,7 @@ int launch_plan(const PatternLaunch &a, int nx, int ny, const Spectrum *sp, Surf
   p.slot_cap = l.slot_cap;
   p.max_nx = l.max_nx;
   p.max_ny = l.max_ny;
-  const bool cells = l.cells > 0 && kind == SurfKind::kSum;
+  const bool cells = l.cells > 0;
   if (cells) {
     p.max_cells = l.cells;
     p.max_cell_sums = l.cell_sums;
@@ -2429,14 +2430,15 @@ int launch_plan(const PatternLaunch &a, int nx, int ny, const Spectrum *sp, Surf
 
 int launch_surface(const PatternLaunch &a, int nx, int ny, const Spectrum *sp, int cus, void *ws, const int **ok_flag,
                    hipStream_t s) {
-  const SingleLayout l = single_layout(nx, ny, a.natoms, a.nsegs, false);
+  const SurfKind kind = sp ? SurfKind::kSpectrum : SurfKind::kSum;
+  const SingleLayout l = single_layout(nx, ny, a.natoms, a.nsegs, kind);
   char *w = (char *)ws;
   const SurfJob *job = (const SurfJob *)(w + l.job);
   const bool has_b = a.atom_b != nullptr;
   const int slots = resident_slots(nodes_kernel(has_b, sp != nullptr), cus);
-  SPSIM_TRY(launch_plan(a, nx, ny, sp, sp ? SurfKind::kSpectrum : SurfKind::kSum, nullptr, l, w, slots, cus, s));
+  SPSIM_TRY(launch_plan(a, nx, ny, sp, kind, nullptr, l, w, slots, cus, s));
   SPSIM_TRY(launch_nodes(job, nullptr, 0, slots, a.ff, a.b_global, has_b, sp, s));
-  if (l.cells > 0 && !sp) {
+  if (l.cells > 0) {
     CellBounds b{};
     b.cells = l.cells;
     // ranges x ceil(nodes / 128) tiles of at most cell_sums range nodes
@@ -2454,12 +2456,14 @@ int launch_surface(const PatternLaunch &a, int nx, int ny, const Spectrum *sp, i
   return SPSIM_HIP_OK;
 }
 
-size_t surf_adjoint_bytes(int nx, int ny, int natoms) { return single_layout(nx, ny, natoms, 0, true).total; }
+size_t surf_adjoint_bytes(int nx, int ny, int natoms) {
+  return single_layout(nx, ny, natoms, 0, SurfKind::kAdjoint).total;
+}
 
 int launch_surface_adjoint(const PatternLaunch &a, const float *gI, int nx, int ny, const SurfAtomTile *tiles,
                            int ntiles, int splits, bool want_b, double4 *partial, int cus, void *ws,
                            const int **ok_flag, hipStream_t s) {
-  const SingleLayout l = single_layout(nx, ny, a.natoms, 0, true);
+  const SingleLayout l = single_layout(nx, ny, a.natoms, 0, SurfKind::kAdjoint);
   char *w = (char *)ws;
   const SurfJob *job = (const SurfJob *)(w + l.job);
   SPSIM_TRY(launch_plan(a, nx, ny, nullptr, SurfKind::kAdjoint, gI, l, w, cus, cus, s));

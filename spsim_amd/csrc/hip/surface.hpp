@@ -136,7 +136,7 @@ bool surf_worth(long long nx, long long ny, long long natoms, long long min_term
 // One pattern on the device alone (no host decision). On return *ok_flag points
 // to a device int that is non-zero when the outputs were written and zero when
 // the list or molecule is not smooth enough, in which case nothing was.
-size_t surf_single_bytes(int nx, int ny, int natoms, int nsegs);
+size_t surf_single_bytes(int nx, int ny, int natoms, int nsegs, bool spectrum);
 // sp: a wavelength spectrum, or null.
 int launch_surface(const PatternLaunch &a, int nx, int ny, const Spectrum *sp, int cus, void *ws, const int **ok_flag,
                    hipStream_t s);
