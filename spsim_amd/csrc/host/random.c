@@ -37,14 +37,20 @@ static uint64_t splitmix64(void) {
 
 double p_drand48(void) { return (double)(splitmix64() >> 11) * (1.0 / 9007199254740992.0); }
 
+uint64_t spsim_uniform_state(void) { return g_sm_state; }
+
+void spsim_set_uniform_state(uint64_t state) { g_sm_state = state; }
+
 uint64_t spsim_noise_seed(void) { return g_seed; }
 
 uint64_t spsim_next_poisson_pattern(void) { return g_poisson_calls++; }
 
 uint64_t spsim_next_readout_pattern(void) { return g_readout_calls++; }
 
+uint64_t spsim_shot_number(void) { return g_poisson_calls > g_readout_calls ? g_poisson_calls : g_readout_calls; }
+
 uint64_t spsim_next_shot_pattern(void) {
-  uint64_t p = g_poisson_calls > g_readout_calls ? g_poisson_calls : g_readout_calls;
+  uint64_t p = spsim_shot_number();
   g_poisson_calls = p + 1;
   g_readout_calls = p + 1;
   return p;

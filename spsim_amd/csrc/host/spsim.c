@@ -154,19 +154,18 @@ Diffraction_Pattern *simulate_shot(Molecule *mol, Options *opts) {
 
   /* The common shot, a direct structure factor on a 2-D detector, makes one trip
      to the device. Everything else, and whatever that cannot run, goes stage by
-     stage, which reports its errors. */
+     stage, which reports its errors. As there, an orientation is drawn only for a
+     q list that exists, and a shot is numbered only when it has a pattern. */
   Diffraction_Pattern *pattern = NULL;
   SpRotation *rot = NULL;
-  uint64_t shot = 0;
-  int have_shot = 0;
+  const uint64_t before = spsim_uniform_state();
   const int spectrum = opts->use_cuda && opts->experiment->bandwidth != 0 && opts->wavelength_samples > 1;
   if (allocated && n > 0 && nz == 1 && !opts->use_fft_for_sf && !opts->use_nfft_for_sf && !spectrum) {
     rot = spsim_orientation(opts);
     if (rot) {
       const int mode = opts->vectorize && !opts->use_cuda ? SPSIM_HIP_PACK_VECTOR : SPSIM_HIP_PACK_PLAIN;
-      shot = spsim_next_shot_pattern();
-      have_shot = 1;
-      pattern = spsim_shot_pattern(mol, opts, rot, mode, &p, spsim_noise_seed(), shot, out);
+      pattern = spsim_shot_pattern(mol, opts, rot, mode, &p, spsim_noise_seed(), spsim_shot_number(), out);
+      if (pattern) spsim_next_shot_pattern();
     }
   }
   int rc = SPSIM_HIP_OK;
@@ -176,12 +175,13 @@ Diffraction_Pattern *simulate_shot(Molecule *mol, Options *opts) {
       rot = apply_orientation_to_HKL_list(&HKL_list, &HKL_list_size, opts);
     else if (HKL_list)
       spsim_rotate_list(HKL_list, HKL_list_size, rot);
+    else
+      spsim_set_uniform_state(before);
     if (HKL_list) pattern = compute_sf(mol, HKL_list, HKL_list_size, opts);
     free(HKL_list);
-    if (pattern && !have_shot) shot = spsim_next_shot_pattern();
     if (pattern)
-      rc = allocated ? spsim_bridge_detector_chain(&p, pattern->ints, spsim_noise_seed(), shot, out[0], out[1], out[2],
-                                                   out[3], out[4], out[5], out[6])
+      rc = allocated ? spsim_bridge_detector_chain(&p, pattern->ints, spsim_noise_seed(), spsim_next_shot_pattern(),
+                                                   out[0], out[1], out[2], out[3], out[4], out[5], out[6])
                      : SPSIM_HIP_ERR_NOMEM;
   }
   if (!pattern || rc != SPSIM_HIP_OK) {

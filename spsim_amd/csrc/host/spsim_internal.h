@@ -17,7 +17,12 @@ extern "C" {
 uint64_t spsim_noise_seed(void);
 uint64_t spsim_next_poisson_pattern(void);
 uint64_t spsim_next_readout_pattern(void);
+/* The next shot's pattern counter, without and with taking it. */
+uint64_t spsim_shot_number(void);
 uint64_t spsim_next_shot_pattern(void);
+/* State of p_drand48's stream, to take draws back. */
+uint64_t spsim_uniform_state(void);
+void spsim_set_uniform_state(uint64_t state);
 
 /* diffraction.c: the form-factor table in use ([101][9], ./atomsf.lib applied). */
 const float *spsim_form_factor_table(void);
