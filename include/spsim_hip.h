@@ -150,8 +150,8 @@ int spsim_hip_sf_pattern(const float *d_hkl, int npix, const spsim_hip_atom *d_a
    GPU). tile may be NULL.
    With tile == NULL, a detector of at least 64 x 64 pixels and 2e8 pixel-atom
    terms, F is summed only at the nodes of a grid over the detector surface and
-   interpolated from there (error below 3e-8 of |F|, less than the direct sums'
-   own rounding), when the list and the molecule are smooth enough for it; the
+   interpolated from there (3e-8 to 2e-7 of |F|, in the norm over the detector, where
+   the direct sums' rounding is 1e-7 to 3e-7), when the list and the molecule are smooth enough for it; the
    device checks both, and everything else takes the direct sum. Such a call
    uses the library workspace (about 100 MiB at 1024 x 1024); while the stream
    is being captured it does so only if the workspace is already that large and the

@@ -16,11 +16,15 @@
 //     not taken.
 //  2. Nodes. u_i = asin(a cos t_i) / asin(a), t_i = (2 i + 1) pi / (2 n), the
 //     Chebyshev points stretched towards even spacing (Kosloff & Tal-Ezer,
-//     J. Comput. Phys. 104 (1993) 457), with a = 1 / cosh(20.7 / n), so that
-//     the stretch itself errs by e^-20.7 = 1e-9. Chebyshev coefficients of
-//     exp(i theta u) fall off like Bessel functions beyond theta:
-//     n = theta + 4 theta^(1/3) + 8 leaves 1e-9..1e-8 of |F| (measured against
-//     FP64 sums), a tenth of the FP32 sums' own error.
+//     J. Comput. Phys. 104 (1993) 457), with a = 1 / cosh(40 / n): the stretch
+//     itself errs by e^-40 times what exp(i theta u) grows by off the axis. (With
+//     e^-20.7 atoms all at the molecule's ends, 240 to 330 rad per unit of u, lost
+//     4e-7 and 8e-7 of |F|; now 5e-8, with as many nodes.) Beyond theta, the largest
+//     phase per unit of t, the Chebyshev coefficients of the phases fall off like Bessel
+//     functions, and those of a form factor's e^{-b s^2} like a Gaussian's:
+//     n = theta + sqrt((3 theta^(1/3) + 8.5)^2 + 64 b (ds/dt)^2)
+//     leaves at most 5e-9 of the steepest phase (rms over u, FP64, up to 560 rad per
+//     unit of u; 1e-13 in the median) and 2e-8 of a Gaussian with exponents up to 60.
 //  3. Node sums. F and its derivative N = n.dF/dq at the nodes, of large molecules
 //     by cells (below), by the arithmetic
 //     of the direct kernels (FP64 phase reduced to turns, FP32 sine and
@@ -35,8 +39,8 @@
 //     order: (2 pi R |d|)^2 / 2 <= 2e-8).
 //
 // The cost is n_x n_y natoms terms instead of npix natoms: 30 times fewer on
-// 100,000 atoms x 1024^2 at 0.15 nm (n = 188). The interpolation weights add
-// no error of their own: the sum of their squares is 1 at every pixel.
+// 100,000 atoms x 1024^2 at 0.15 nm (n = 192). The interpolation weights add
+// no error of their own: the sum of their squares is 1 over an axis (2 at its ends).
 #include "surface.hpp"
 
 #include <algorithm>
@@ -54,7 +58,7 @@ constexpr int kT = 256;
 constexpr int D = kSurfDeg;
 constexpr int kLines = kSurfLines;
 constexpr double kPi = 3.14159265358979323846;
-constexpr float kStretch = 20.7f;       // -ln of the node map's own error
+constexpr float kStretch = 40.0f;       // of the node map, see step 2 above
 constexpr double kMaxPhaseDev = 2e-4;   // largest 2 pi R |q - surface|
 constexpr double kMaxSpreadDev = 3e-7;  // the same times the spectrum's largest |s_k / sc - 1|
 constexpr float kMinWeakest = 0.02f;    // see species_terms
@@ -460,22 +464,33 @@ __host__ __device__ inline float line_density(int k, float a, float as) {
 #endif
 }
 
-// density(k) as line_density at the stretch whose asin is as.
-template <class Density>
-__host__ __device__ inline float axis_need(const SurfSlopes &slope, float radius, const float *h, float gauss, float as,
-                                           Density density) {
+// density(k) as line_density at the stretch whose asin is as; steepest(): the largest
+// slope.all[k] density(k), asked for behind the densities; b: the largest Gaussian
+// coefficient of the terms, A^2.
+template <class Density, class Steepest>
+__host__ __device__ inline float axis_need(const SurfSlopes &slope, float radius, const float *h, float b, float as,
+                                           Density density, Steepest steepest) {
   float w = 0.0f;
   for (int k = 0; k < kLines; ++k) {
     const float box = slope.part[0][k] * h[0] + slope.part[1][k] * h[1] + slope.part[2][k] * h[2];
     w = fmaxf(w, fminf(slope.all[k] * radius, box) * density(k));
   }
   const float theta = 1.02f * 2.0f * (float)kPi * w / as;
-  return theta + 4.0f * cbrtf(theta) + 8.0f + 2.0f * sqrtf(fmaxf(gauss, 0.0f));
+  const float tail = 3.0f * cbrtf(theta) + 8.5f, s = 0.5e-10f * steepest() / as;  // ds per node angle
+  return theta + sqrtf(tail * tail + 64.0f * fmaxf(b, 0.0f) * s * s);
 }
 
-__device__ __forceinline__ float axis_need(const SurfSlopes &slope, float radius, const float *h, float gauss, float a) {
+__device__ __forceinline__ float axis_need(const SurfSlopes &slope, float radius, const float *h, float b, float a) {
   const float as = asinf(a);
-  return axis_need(slope, radius, h, gauss, as, [&](int k) { return line_density(k, a, as); });
+  float steepest = 0.0f;
+  return axis_need(
+      slope, radius, h, b, as,
+      [&](int k) {
+        const float d = line_density(k, a, as);
+        steepest = fmaxf(steepest, slope.all[k] * d);
+        return d;
+      },
+      [&] { return steepest; });
 }
 
 enum class SurfKind { kSum, kSpectrum, kAdjoint };
@@ -804,7 +819,10 @@ __host__ __device__ inline void cell_tiling(int nx, int ny, bool octants, int *p
 // Issue cycles over all lanes of a pattern's node sums (nx x ny nodes), and of
 // the same by cells with mx x my nodes each: the sums, the two products
 // (290 cycles per 16 x 16 x 4 block, an FP64 sine and cosine per node and cell)
-// and the products' memory (about 33 cycles a byte).
+// and the products' memory (about 33 cycles a byte). The weights of the sums and
+// the products order the grids of boxes as they measured: on 100,000 atoms and 192^2
+// nodes 108 cells of 64^2 nodes take 239 us, 256 of 52^2 260 us (0.6 for the
+// products had them the other way round).
 __host__ __device__ inline double sums_cost(int nx, int ny, bool octants, double natoms, int *per_lane, int *tiles) {
   node_tiling(nx, ny, octants, 1LL << 25, per_lane, tiles);
   return (double)*tiles * kT * (*per_lane == 8 ? 321.0 : 57.0 * *per_lane) * natoms;
@@ -815,7 +833,7 @@ __host__ __device__ inline double cells_cost(int nx, int ny, int mx, int my, int
   const double sums = tiles * 64.0 * (per_lane == 8 ? 321.0 : 57.0 * per_lane) * natoms;
   auto up = [](int n) { return (n + 15) / 16; };
   const double rows = 290.0 * up(nx) * up(my) * (mx / 4), cols = up(nx) * up(ny) * (290.0 * (my / 4) + 2000.0);
-  return 1.2 * sums + 0.6 * ncells * (64.0 * (rows + cols) + 33.0 * 48.0 * my * nx);
+  return 1.2 * sums + 0.8 * ncells * (64.0 * (rows + cols) + 33.0 * 48.0 * my * nx);
 }
 
 // What the scan found about a molecule on its list, in *out (thread 0).
@@ -947,7 +965,7 @@ __global__ __launch_bounds__(kT) void surface_plan_kernel(PlanArgs a) {
     const int axis = t / 128, n = kSurfMinNodes + 4 * (t % 128);
     const SurfSlopes &slope = axis ? a.fit->slope_y : a.fit->slope_x;
     const float r = (float)mol.radius, h[3] = {r, r, r};
-    if (n <= kSurfMaxNodes && axis_need(slope, r, h, mol.b_smooth * a.fit->s2max, axis_stretch(n)) <= (float)n)
+    if (n <= kSurfMaxNodes && axis_need(slope, r, h, mol.b_smooth, axis_stretch(n)) <= (float)n)
       atomicMin(&best[axis], n);
   }
   if (a.max_cells > 0)  // and of the cells of every grid of boxes
@@ -958,7 +976,7 @@ __global__ __launch_bounds__(kT) void surface_plan_kernel(PlanArgs a) {
       const SurfSlopes &slope = axis ? a.fit->slope_y : a.fit->slope_x;
       const float r = (float)mol.radius, h[3] = {r / g, r / g, r / gz};
       if (n <= kCellMaxNodes && axis_need(slope, sqrtf(h[0] * h[0] + h[1] * h[1] + h[2] * h[2]), h,
-                                          mol.b_smooth * a.fit->s2max, axis_stretch(n)) <= (float)n)
+                                          mol.b_smooth, axis_stretch(n)) <= (float)n)
         atomicMin(&cell_best[k][axis], n);
     }
   __syncthreads();
@@ -2636,9 +2654,17 @@ ScanLayout scan_layout(int nx, int ny, int nmol) {
 // count grows and the stretch with it.
 int axis_count(int k) { return k <= 12 ? kSurfMinNodes + 4 * k : 64 + 8 * (k - 12); }
 
+// An axis with the largest slope times density of the counts that were asked for
+// (negative: not yet).
+struct AxisSlopes {
+  explicit AxisSlopes(const SurfSlopes &s) : slope(s) { std::fill(steepest, steepest + kSurfMaxNodes / 4 + 1, -1.0f); }
+  const SurfSlopes &slope;
+  float steepest[kSurfMaxNodes / 4 + 1];
+};
+
 // Whether n nodes (a multiple of 4) are enough: axis_need() with the densities of
 // every count formed once.
-bool enough_nodes(const SurfSlopes &slope, float radius, const float *h, float gauss, int n) {
+bool enough_nodes(AxisSlopes &axis, float radius, const float *h, float b, int n) {
   struct Line {
     float as, density[kLines];
   };
@@ -2652,28 +2678,31 @@ bool enough_nodes(const SurfSlopes &slope, float radius, const float *h, float g
     return l;
   }();
   const Line &l = lines[n / 4];
-  return axis_need(slope, radius, h, gauss, l.as, [&](int k) { return l.density[k]; }) <= (float)n;
+  float &steepest = axis.steepest[n / 4];
+  if (steepest < 0.0f)
+    for (int k = 0; k < kLines; ++k) steepest = std::max(steepest, axis.slope.all[k] * l.density[k]);
+  return axis_need(axis.slope, radius, h, b, l.as, [&](int k) { return l.density[k]; }, [&] { return steepest; }) <= (float)n;
 }
 
-int axis_nodes(const SurfSlopes &slope, double radius, float gauss) {
+int axis_nodes(AxisSlopes &axis, double radius, float b) {
   const float r = (float)radius, h[3] = {r, r, r};
   int lo = -1, hi = 12 + (kSurfMaxNodes - 64) / 8;
-  if (!enough_nodes(slope, r, h, gauss, axis_count(hi))) return 0;
+  if (!enough_nodes(axis, r, h, b, axis_count(hi))) return 0;
   while (hi - lo > 1) {
     const int mid = (lo + hi) / 2;
-    (enough_nodes(slope, r, h, gauss, axis_count(mid)) ? hi : lo) = mid;
+    (enough_nodes(axis, r, h, b, axis_count(mid)) ? hi : lo) = mid;
   }
   return axis_count(hi);
 }
 
 // The same for a box of half edges h, in multiples of 4 up to kCellMaxNodes.
-int box_nodes(const SurfSlopes &slope, const float *h, float gauss) {
+int box_nodes(AxisSlopes &axis, const float *h, float b) {
   const float r = std::sqrt(h[0] * h[0] + h[1] * h[1] + h[2] * h[2]);
   int lo = -1, hi = (kCellMaxNodes - kCellMinNodes) / 4;
-  if (!enough_nodes(slope, r, h, gauss, kCellMaxNodes)) return 0;
+  if (!enough_nodes(axis, r, h, b, kCellMaxNodes)) return 0;
   while (hi - lo > 1) {
     const int mid = (lo + hi) / 2;
-    (enough_nodes(slope, r, h, gauss, kCellMinNodes + 4 * mid) ? hi : lo) = mid;
+    (enough_nodes(axis, r, h, b, kCellMinNodes + 4 * mid) ? hi : lo) = mid;
   }
   return kCellMinNodes + 4 * hi;
 }
@@ -2693,13 +2722,14 @@ SurfAxis axis_of(int n) {
   return a;
 }
 
-Choice choose(const SurfHead &head, SurfMol mol, double norm, int nx, int ny, int natoms, const double *limit) {
+Choice choose(const SurfHead &head, AxisSlopes &along_x, AxisSlopes &along_y, SurfMol mol, double norm, int nx, int ny,
+              int natoms, const double *limit) {
   Choice c;
   c.norm = norm;
   mol.radius *= norm;
   if (natoms <= 0 || !smooth(mol, head.s2max)) return c;
-  const float gauss = mol.b_smooth * head.s2max;
-  const int n[2] = {axis_nodes(head.slope_x, mol.radius, gauss), axis_nodes(head.slope_y, mol.radius, gauss)};
+  const float b = mol.b_smooth;
+  const int n[2] = {axis_nodes(along_x, mol.radius, b), axis_nodes(along_y, mol.radius, b)};
   if (n[0] == 0 || n[1] == 0) return c;
   c.ax = axis_of(n[0]);
   c.ay = axis_of(n[1]);
@@ -2712,7 +2742,7 @@ Choice choose(const SurfHead &head, SurfMol mol, double norm, int nx, int ny, in
     int g, gz;
     cell_grid(k, &g, &gz);
     const float r = (float)mol.radius, h[3] = {r / g, r / g, r / gz};
-    const int mx = box_nodes(head.slope_x, h, gauss), my = box_nodes(head.slope_y, h, gauss);
+    const int mx = box_nodes(along_x, h, b), my = box_nodes(along_y, h, b);
     if (mx == 0 || my == 0 || (long long)(natoms / cell_range(natoms) + g * g * gz) * mx * my > kCellSums ||
         (long long)g * g * gz * my * n[0] > kCellRows)
       continue;
@@ -2762,6 +2792,7 @@ int surf_scan(const SurfInput &in, void *scan, void *digest, hipStream_t s) {
 SurfPlan *surf_plan_choose(const SurfInput &in, const void *digest) {
   const SurfHead &head = *(const SurfHead *)digest;
   const SurfDigest *mols = (const SurfDigest *)((const char *)digest + sizeof(SurfHead));
+  AxisSlopes along_x(head.slope_x), along_y(head.slope_y);
   SurfPlan *p = new SurfPlan;
   p->in = in;
   p->takes.assign(in.npatterns, 0);
@@ -2775,7 +2806,7 @@ SurfPlan *surf_plan_choose(const SurfInput &in, const void *digest) {
     if (std::fabs(norm - 1.0) < 1e-6) norm = 1.0;
     Choice &ch = last[m];
     if (ch.norm != norm) {
-      ch = choose(head, mols[m].mol, norm, in.nx, in.ny, natoms, in.limit ? in.limit + m : nullptr);
+      ch = choose(head, along_x, along_y, mols[m].mol, norm, in.nx, in.ny, natoms, in.limit ? in.limit + m : nullptr);
       if (ch.taken) {
         auto find = [](auto &list, auto same) {
           for (size_t k = 0; k < list.size(); ++k)

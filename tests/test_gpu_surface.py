@@ -522,3 +522,71 @@ def test_empty_segments_change_nothing(gpu, entry):
             got.append(dv.structure_factor_nfft(q, atoms, ff)[1])
     torch.cuda.synchronize()
     assert bool(torch.isfinite(got[0]).all()) and torch.equal(got[0], got[1])
+
+
+def _ends(natoms, radius, rng):
+    """Two clusters of carbon at the ends of the x axis: every phase is the steepest."""
+    pos = np.zeros((natoms, 3))
+    pos[:, 0] = np.where(np.arange(natoms) % 2, radius, -radius) * (1 - 1e-3 * rng.uniform(size=natoms))
+    return np.full(natoms, 6, np.int32), pos.astype(np.float32)
+
+
+@pytest.mark.parametrize("entry", ["grid", "plan"])
+@pytest.mark.parametrize("n,width,radius", [(512, 0.0384, 6e-8), (1024, 0.04, 8e-8)])
+def test_atoms_at_the_ends_of_the_molecule(gpu, entry, n, width, radius):
+    """240 to 330 radians from the middle of the detector to its edge, with all atoms at
+    the ends: the nodes serve the steepest phase as well as a ball's average one."""
+    import ctypes as C
+
+    import torch
+
+    from spsim_amd import _lib
+    from tests.test_gpu_batch import make_plan
+
+    rng = np.random.default_rng(51)
+    Z, pos = _ends(1_500, radius, rng)
+    hkl = oracle.hkl_detector(n, n, np.float32(width).item(), np.float32(width).item(), 0.2, 0.0, 0.0, 0, 0.15e-9)
+    if entry == "grid":
+        F, I = _run(gpu, hkl, n, n, Z, pos)
+    else:
+        plan, *_ = make_plan([(Z, pos)], np.eye(3)[None], np.zeros(1, np.int32), hkl, n, n)
+        try:
+            It = torch.empty((1, n * n), dtype=torch.float32, device=gpu)
+            Ft = torch.empty((1, n * n, 2), dtype=torch.float32, device=gpu)
+            _lib.check(_lib.load().spsim_hip_batch_run(plan, C.c_void_p(Ft.data_ptr()), C.c_void_p(It.data_ptr()), 0,
+                                                       None), "run")
+            torch.cuda.synchronize()
+        finally:
+            _lib.load().spsim_hip_batch_destroy(plan)
+        Fh = Ft.cpu().numpy()[0]
+        F, I = Fh[:, 0] + 1j * Fh[:, 1], It.cpu().numpy()[0]
+    sub = np.sort(rng.choice(n * n, 3000, replace=False))
+    Fr, Ir = oracle.sf_f64(hkl[sub], Z, pos, threads=oracle_threads())
+    e, ef = rel_l2(I[sub], Ir), np.linalg.norm(F[sub] - Fr) / np.linalg.norm(Fr)
+    print(f"{entry} {n}: I {e:.2e}, F {ef:.2e}", flush=True)
+    assert e < TOL and ef < TOL
+
+
+def test_sharp_form_factors(gpu):
+    """A form factor of one wide Gaussian (200 A^2, exponents up to 42 on this detector)
+    and a constant, on a molecule of 0.2 nm, whose phases need few nodes."""
+    import torch
+
+    rng = np.random.default_rng(52)
+    n, natoms = 1500, 150
+    Z, pos, _ = wl.random_molecule(natoms, 2e-10, rng)
+    Z[:] = 6
+    table = dv.default_form_factors().copy()
+    table[6] = [4.0, 0, 0, 0, 200.0, 0, 0, 0, 2.0]
+    hkl = oracle.hkl_detector(n, n, np.float32(0.1).item(), np.float32(0.1).item(), 0.05, 0.0, 0.0, 0, 1e-10)
+    atoms, ff = dv.DeviceAtoms(dv.pack_atoms(Z, pos), gpu), dv.form_factor_table(table, device=gpu)
+    q = torch.from_numpy(hkl).to(gpu)
+    _, I = dv.structure_factor_grid(q, n, n, atoms, ff)
+    _, Id = dv.structure_factor_grid(q, n, n, atoms, ff, tile=dv.make_tile(1, 256, 0))
+    torch.cuda.synchronize()
+    assert not torch.equal(I, Id)
+    sub = np.sort(rng.choice(n * n, 3000, replace=False))
+    _, Ir = oracle.sf_f64(hkl[sub], Z, pos, ff=table, threads=oracle_threads())
+    e = rel_l2(I.cpu().numpy()[sub], Ir)
+    print(f"sharp: I {e:.2e} (direct {rel_l2(Id.cpu().numpy()[sub], Ir):.2e})", flush=True)
+    assert e < TOL
