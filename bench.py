@@ -188,7 +188,8 @@ def surface_roofline(nbytes, kernel_ms, terms):
     achieved = nbytes / (kernel_ms * 1e-3) / 1e9
     return {
         "bound": "hbm", "achieved": round(achieved, 2), "peak": HBM_PEAK_GBS, "unit": "GB/s",
-        "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": None, "kernel": "surface_nodes_kernel",
+        "frac": round(achieved / HBM_PEAK_GBS, 4), "traffic": None,
+        "kernel": "node sums (surface_nodes_kernel, by cells surface_cell_nodes_kernel) and interpolation",
         "work": {"bytes": float(nbytes), "kernel_ms": round(kernel_ms, 4)},
         "textbook": {"w_eq_per_term": W_TEXTBOOK, "terms_per_launch": terms,
                      "note": "terms of the direct sum; the sums are formed at a few nodes per detector axis "
