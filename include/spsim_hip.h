@@ -148,14 +148,17 @@ int spsim_hip_sf_pattern(const float *d_hkl, int npix, const spsim_hip_atom *d_a
    is the quads per lane here (1 or 2), or 8 for one octant per lane (nx == ny
    only; the default for square detectors, with atom_splits chosen to fill the
    GPU). tile may be NULL.
-   With tile == NULL, a detector of at least 64 x 64 pixels and 2e8 pixel-atom
+   With tile == NULL and a detector of at least 64 x 64 pixels and 2e8 pixel-atom
    terms, F is summed only at the nodes of a grid over the detector surface and
-   interpolated from there (3e-8 to 2e-7 of |F|, in the norm over the detector, where
-   the direct sums' rounding is 1e-7 to 3e-7), when the list and the molecule are smooth enough for it; the
-   device checks both, and everything else takes the direct sum. Such a call
-   uses the library workspace (about 100 MiB at 1024 x 1024); while the stream
-   is being captured it does so only if the workspace is already that large and the
-   direct sum would hold partial sums of several atom ranges there. */
+   interpolated from there, when the list and the molecule are smooth enough for it;
+   the device checks both, and everything else takes the direct sum. Its error,
+   in the norm over the detector, is 3e-8 to 2e-7 of |F| where the direct sums' is
+   1e-7 to 3e-7. Such a call uses the library workspace: 80 MiB at 1024 x 1024, from
+   1e10 terms on 200 MiB and 54 bytes an atom more (280 MiB with 100,000 atoms), or
+   what the direct sum's partials take (up to 512 MiB) if that is more; a quarter
+   more is allocated. While the stream is being captured it does so only if the
+   workspace is already that large and the direct sum would hold partial sums of
+   several atom ranges there. */
 int spsim_hip_sf_grid(const float *d_hkl, int nx, int ny, const spsim_hip_atom *d_atoms, const float *d_atom_b,
                       const spsim_hip_segment *d_segs, int nsegs, int natoms, const float *d_ff, float b_global,
                       const double *rot9, float *d_F, float *d_I, const spsim_hip_tile *tile, void *stream);

@@ -1409,9 +1409,9 @@ __global__ __launch_bounds__(kT) void surface_nodes_kernel(const SurfJob *jobs, 
 // pattern's nodes like the pattern's to the pixels (FP64 products for F, FP32 for
 // N), turned by the centre's phase and added up. Terms fall with the square of
 // the coarse nodes, the interpolation grows with the cells: cells_cost. On
-// 100,000 atoms with B and 188^2 nodes, 108 cells of 64^2 nodes: 33 us for the
-// sort, 161 us for the sums, 36 and 84 us for the products, against 1140 us for
-// the plain sums.
+// 100,000 atoms with B and 192^2 nodes, 108 cells of 64^2 nodes: 27 us for the
+// sort, 162 us for the sums, 36 and 86 us for the products, against 1140 us for
+// the plain sums (at 188^2).
 
 // The records of one cell (blockIdx.x), in their order, which is that of the
 // species: every wave goes over one section of the atoms' cell indexes, 512 at a
@@ -1548,8 +1548,8 @@ __global__ __launch_bounds__(kSortT) void surface_sort_kernel(const SurfJob *job
 
 // One (range, tile of 64 lanes) per workgroup at a time, of pattern
 // first + blockIdx.y: every wave sums a quarter of the range's atoms, and the first
-// one adds them up. Bound by the issue of the sums (58 % of it; ranges of 1024
-// atoms take 204 us for 161 us, their last ones run alone).
+// one adds them up. Bound by the vector units, busy 87 % (77 % of the issue slots;
+// ranges of 1024 atoms take 204 us for 161 us, their last ones run alone).
 template <bool HAS_B>
 __global__ __launch_bounds__(kT, 4) void surface_cell_nodes_kernel(const SurfJob *jobs, int first,
                                                                    const float *__restrict__ ff, float b_global) {
